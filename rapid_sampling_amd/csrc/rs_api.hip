@@ -766,6 +766,7 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
     // general kernel in calls of fewer than 2^24 tokens, the row kernel (whose time does not depend on the
     // kept set) in every call it suits
     p.tell_lists = ((uint64_t)B * (uint64_t)V < (1ull << 24) || row_suits(B, V)) ? 1u : 0u;
+    p.long_list = 0xFFFFFFFFu;
     dim3 grid((uint32_t)B * g.G);
     const int path = choose_path(B, V, top_k, top_p, pen, opt);
     if (path == kPathRow) return launch_row(logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
@@ -774,6 +775,7 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
                      : (path == kPathWide1 || path == kPathKeep) ? wide_r(B, V, workspace_bytes) : stream_r(B, V, pen);
         StreamView v;
         v.G = stream_parts(V, sr);
+        v.slice_log2 = sr == 4 ? 12u : sr == 8 ? 13u : (uint32_t)kStreamLongLog2;
         const bool pen_stream = pen && path == kPathStream;                  // long slices: their layout has room for the notes
         const StreamLayout l = stream_layout((size_t)B * v.G, sizeof(WsHeader), pen_stream);
         // (rs_workspace_bytes sets aside room for every slice length chosen above; checked all the same: a
@@ -808,6 +810,19 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
         p.report = path == kPathKeep ? 0u : (uint32_t)policy_word(kind, size_class(B, V));
         p.attempt = path == kPathAttempt ? 1u : 0u;
         p.probe = path == kPathProbe ? 1u : 0u;
+        // A nucleus of thousands of tokens is finished from the stashes all the same, but one workgroup going through
+        // such a list a dozen times takes longer than the general kernel needs for the whole call (measured:
+        // 128 rows of 50304, about 4000 tokens each, 54 against 36 us; the two meet at about 2400 tokens
+        // there and, the general kernel's time growing with the row, at about 4700 for rows of 100256): a
+        // call that is only an attempt (no top_k bounds the kept set) says so to the caller's policy, and so
+        // does a call of moderate size with a bounding top_k (a lone flat row of 32768 tokens with top_k 1000:
+        // 26.7 us here against 17.5 on the general kernel).  Small calls in rows of up to 100256 tokens meet the
+        // general kernel earlier: a list of a thousand tokens takes one to sixteen such rows 21-27 us here
+        // against 18-21 there (lists of a few hundred: 12-14 us here).
+        if (p.attempt || p.tell_lists) {
+            const bool small_call = (uint64_t)B * (uint64_t)V < (1ull << 20) && V < 131072;
+            p.long_list = small_call ? 768u : max(2048u, (uint32_t)V / 20u);
+        }
         if (path == kPathKeep) { p.stash_k = 1u; v.list_cap = 2048u; }
         if (path == kPathWide || path == kPathProbe) {
             // the list holds the tokens of ONE sub-bin of the boundary bin: 1/128 of it for a smooth distribution

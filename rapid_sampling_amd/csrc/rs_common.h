@@ -85,6 +85,7 @@ struct Params {
     uint32_t     report;       // index of the report word of the caller's policy a streaming call writes (4..12: kind of call x size class), 0 none
     uint32_t     attempt;      // the call has no bounding top_k: its streaming pass is an attempt
     uint32_t     tell_lists;   // streaming finish: a row whose list is long enough for another kernel to be faster says so to the policy
+    uint32_t     long_list;    // ... and how long that is (0xFFFFFFFF: never)
     uint32_t     probe;        // wide path as a probe for the streaming path: rows whose kept set the stashes would not hold are reported as slow
     int32_t     *host_words;   // the caller's rs_policy: pinned host memory, [2] error, [4..12] routing reports; or null
     int32_t      defer_pen;    // penalties enter x and are not rewritten from the registers at the end: 1 a later pass over them
@@ -605,11 +606,13 @@ __device__ inline Target tie_and_target(const Params &p, uint32_t row, uint64_t 
 {
     const uint64_t w_thr = w_of_bits(thr);
     u128 a = (P > Gm) ? (P - Gm) : (u128)0;
-    u128 bk = ((uint32_t)p.top_k > n_gt) ? (u128)w_thr * ((uint32_t)p.top_k - n_gt) : (u128)0;
-    if (n_eq > 1) { a = div_u32(a, n_eq); bk = div_u32(bk, n_eq); }
     u128 wt = w_thr;
+    if (n_eq > 1 || (uint32_t)p.top_k <= n_gt) {         // (a single token at the threshold is never more than top_k allows)
+        u128 bk = ((uint32_t)p.top_k > n_gt) ? (u128)w_thr * ((uint32_t)p.top_k - n_gt) : (u128)0;
+        if (n_eq > 1) { a = div_u32(a, n_eq); bk = div_u32(bk, n_eq); }
+        if (bk < wt) wt = bk;
+    }
     if (a < wt) wt = a;
-    if (bk < wt) wt = bk;
     if (wt == 0 && Gm == 0) wt = 1;
     Target t;
     t.w_tie = (uint64_t)wt;
@@ -671,6 +674,7 @@ struct StreamView {
     uint64_t *shist;      // [B][G][kSB]   the slice's own bins (slice frame), as it added them to the row's
     uint32_t  G;          // slices per row
     uint32_t  list_cap;   // entries of the finishing workgroup's token list (a power of two up to kFinCap)
+    uint32_t  slice_log2; // log2 of the tokens per slice
 };
 
 

@@ -115,16 +115,23 @@ __device__ __forceinline__ u128 r_from_bits(uint64_t u64, u128 S)
     return (u128)u64 * s_hi + __umul64hi(u64, s_lo) + 1;
 }
 
-// floor(a / d) for a < 2^96 and a 32-bit divisor, by 32-bit long division
+// floor(a / d) for a < 2^96 and 1 <= d <= 2^20 (a count of tokens), by long division with 32-bit digits.
+// Each step divides less than d * 2^32 <= 2^52, which a double holds exactly, by multiplying with 1 / d: off
+// by one at most, put right with the remainder.  (The compiler's own 64-bit division takes a few hundred
+// dependent instructions per digit.)
 __device__ inline u128 div_u32(u128 a, uint32_t d)
 {
+    const double inv = 1.0 / (double)d;
     uint64_t rem = 0;
     u128 q = 0;
 #pragma unroll
     for (int i = 2; i >= 0; --i) {
         const uint64_t cur = (rem << 32) | (uint32_t)(a >> (32 * i));
-        const uint64_t qi = cur / d;
-        rem = cur - qi * d;
+        uint64_t qi = (uint64_t)((double)cur * inv);
+        int64_t r = (int64_t)(cur - qi * d);
+        if (r < 0) { qi -= 1u; r += d; }
+        if (r >= (int64_t)d) { qi += 1u; r -= d; }
+        rem = (uint64_t)r;
         q |= (u128)qi << (32 * i);
     }
     return q;

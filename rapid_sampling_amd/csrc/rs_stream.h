@@ -3,6 +3,7 @@
 
 #include "rs_common.h"
 #include "rs_cluster.h"
+#include "rs_mass.h"
 
 namespace rs {
 
@@ -379,46 +380,10 @@ struct LdsB {
     uint32_t m4[kMaxParts];      // 4 (M mod 128) of slice g's frame: where its bins sit among the row's positions
     uint32_t take[kMaxParts];    // inclusive prefix of the entries taken from each stash
     uint64_t rand64;
+    struct { M96 D, P, above; uint32_t place, cnt_above, cnt_bin, found; } one;   // what one wave worked out for all (finish_row)
     uint32_t nsmall, bucket, fail;
-    uint32_t result;             // one-launch path: sampled token + 1 once the row is finished here
+    uint32_t result;             // sampled token + 1 once the row is finished
 };
-
-// Inverse CDF by buckets of the token index: sum the kept weights per bucket
-// (bucket = (index >> shift) & 255, tokens outside [lo_idx, hi_idx) ignored),
-// scan, and return the bucket that holds target r, with r reduced to an offset
-// inside it.  Weights are < 2^64 and a sum has < 2^12 terms, so the halves
-// summed separately stay below 2^44 + 2^32.
-template <typename W>
-__device__ __forceinline__ uint32_t bucket_step(Lds &s, LdsB &t, uint32_t nlist, uint32_t shift, uint32_t lo_idx, uint32_t hi_idx,
-                                                u128 &r, W weight, int lane, int wave)
-{
-    const int tid = threadIdx.x;
-    t.blo[tid] = 0; t.bhi[tid] = 0;
-    __syncthreads();
-    for (uint32_t i = tid; i < nlist; i += kThreads) {
-        const uint64_t e = t.list[i];
-        const uint32_t idx = (uint32_t)e;
-        if (idx >= lo_idx && idx < hi_idx) {
-            const uint64_t w = weight((uint32_t)(e >> 32));
-            if (w) {
-                const uint32_t bk = (idx >> shift) & 255u;
-                atomicAdd(reinterpret_cast<unsigned long long *>(&t.blo[bk]), (unsigned long long)(w & 0xFFFFFFFFull));
-                atomicAdd(reinterpret_cast<unsigned long long *>(&t.bhi[bk]), (unsigned long long)(w >> 32));
-            }
-        }
-    }
-    __syncthreads();
-    const u128 mine = (u128)t.blo[tid] + ((u128)t.bhi[tid] << 32);
-    u128 inc = wave_inclusive_scan(mine);
-    if (lane == kWave - 1) s.q128[wave] = inc;
-    __syncthreads();
-    for (int w = 0; w < wave; ++w) inc += s.q128[w];
-    const u128 exc = inc - mine;
-    if (exc < r && r <= inc) { t.bucket = (uint32_t)tid; s.bc128[1] = r - exc; }
-    __syncthreads();
-    r = s.bc128[1];
-    return t.bucket;
-}
 
 // A row the stashes cannot finish (a nucleus or a tie of thousands of tokens, more kept tokens than
 // the list holds): the finishing workgroup does it alone, from the logits, in a few passes over the
@@ -762,21 +727,86 @@ __device__ __forceinline__ void pen_patch(const Params &p, const StreamView &v, 
     }
 }
 
+// The last step of a pick: the token among at most 64 (index, weight) entries, in any order, at which the
+// running sum of weights in index order reaches r.  One wave; lane i holds entry i, rank = the number of
+// entries with a smaller index.  The entries go through LDS into index order, one scan does the rest.
+__device__ __forceinline__ void pick_of_wave(const Params &p, LdsB &t, const uint32_t row, const int lane, const uint32_t n, const uint32_t rank,
+                                             const uint32_t idx, const uint64_t w, const M96 r)
+{
+    if ((uint32_t)lane < n) { t.small[rank] = w; t.take[rank] = idx; }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint64_t wr = (uint32_t)lane < n ? t.small[lane] : 0ull;
+    const uint32_t ir = t.take[lane];
+    const Limbs mine = limbs(M96{wr, 0u}), upto = wave_inclusive_scan(mine);
+    const M96 inc = m96(upto), exc = m96(upto - mine);
+    if (exc < r && inc >= r) {
+        p.out[row] = (int32_t)ir;
+        if (p.diag) p.diag[row].index = (int32_t)ir;
+        t.result = ir + 1u;
+    }
+}
+
 // Finishes a row from what its slices published.  Returns true when the row is done (token written),
 // false when it cannot be finished from the stashes: only on the one-launch path (FUSED = true: the
 // caller is the last workgroup of the row to publish, the data was written by workgroups of this same
 // launch and is read with device-scope atomic loads), where the caller then tells the row's other
 // workgroups and the row's histogram is left in place for them.  With FUSED = false such a row is
-// done here the slow way, from the logits.
-template <int SLICE_LOG2, bool FUSED, bool KEEP = false>     // SLICE_LOG2: log2 of the tokens per slice of the view
-__device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v, Lds &s, LdsB &t, const uint32_t row)
+// done here the slow way, from the logits, by the first four waves (the others have left: NT = 1024).
+//
+// What bounds it: nothing but the length of its chain.  A finish touches a few KB, and every step waits for
+// the one before: trips to memory, scans, threshold, pick, with a workgroup barrier between most of them.
+//   * The first 64 stashed tokens of every slice are asked for together with the headers and the row's
+//     bins, before it is known which of them count: for the usual call that is all of them.  That nothing is
+//     missing is checked by counting: the row's bins say how many tokens lie at or above the boundary bin.
+//   * With one wave per SIMD (NT = 256) every wave works the one-wave steps out for itself: no barrier and no
+//     trip through LDS for what all of them hold.
+//   * The row's random number is drawn by a wave of its own (NT = 256: a fifth one, which leaves at its second
+//     barrier; NT = 1024: the last; FUSED: drawn by the caller while its slice was on its way).
+//   * Threshold and pick of a list of at most 64 tokens are one all-pairs step and one scan.
+//   * Sums over a wave that need no carries (Limbs), no branch per list entry.
+// Measured (cycles of 2.4 GHz in the workgroup, before: counts per slice fetched first, one wave for the scans with
+// 128-bit sums, digits and buckets for every list): 13 rows of 50260, top_k 40: 14300 -> 9200; the kernel 7.6 -> 5.2 us;
+// 256 rows of 151936: 9.2 -> 5.8 us; one row of 262144 with top_p 0.3: 8.0 -> 7.3.  Where they go now: the first trip to memory 2000,
+// the level-1 scan 1800 (400 instructions), the list 1200, all pairs 650, threshold and target 1500, the pick 860.
+// PRE: slices per wave whose first tokens are asked for ahead (W * PRE >= G for the short way).
+// list: room for v.list_cap tokens in LDS.
+template <int NT, int PRE, bool FUSED>
+__device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v, Lds &s, LdsB &t, uint64_t *list, const uint32_t row, const uint64_t drawn = 0)
 {
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    constexpr int  W = NT / kWave;
+    constexpr bool kEach = NT == kThreads;               // every wave for itself
+    static_assert(NT == 256 || NT == 1024, "one or four waves per SIMD");
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = (int)uniform((uint32_t)tid >> 6);
     const uint32_t G = v.G;
     const PartHdr *hdrs = v.hdr + (size_t)row * G;
+    const uint64_t *stash = v.stash + (size_t)row * G * kStashCap;
     uint64_t *rowhist = FUSED ? (p.ctl_end - 1 - row)->h[0] : (p.ctl_end - 1 - row)->rowhist;
 
-    if (tid == 0) { s.abort = 0; s.host_words = p.host_words; t.fail = 0; t.result = 0u; }
+    uint32_t rs[6] = {0u, 0u, 0u, 0u, 0u, 0u};
+    uint32_t *rng_st = p.rng + (size_t)row * 16;
+    const bool draws = !FUSED && wave == (kEach ? W : W - 1);
+    if (draws && !p.inj_u) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) rs[i] = rng_st[i];
+    }
+    auto draw = [&]() {                                  // a row is always finished here unless FUSED: the state is advanced at once
+        if (!p.inj_u) {
+            uint32_t o[4];
+            philox4x32_10(rs[2], rs[3], rs[4], rs[5], rs[0], rs[1], o);
+            if (lane == 0) {
+                t.rand64 = ((uint64_t)o[0] << 32) | o[1];
+                rng_st[2] = rs[2] + 1u;
+                if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
+            }
+        }
+    };
+    if (!FUSED && kEach && wave == W) {
+        __syncthreads();
+        draw();
+        __syncthreads();
+        return true;
+    }
     PartHdr ph;
     ph.mkey = 0; ph.cov = 0; ph.n = 0; ph.cut = 0;
     if ((uint32_t)tid < G) {
@@ -786,7 +816,516 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             ph.mkey = (uint32_t)w0; ph.cov = (uint32_t)(w0 >> 32); ph.n = (uint32_t)w1; ph.cut = (uint32_t)(w1 >> 32);
         } else ph = hdrs[tid];
     }
-    const uint64_t h0 = get<FUSED>(&rowhist[tid]), h1 = get<FUSED>(&rowhist[tid + kThreads]);
+    uint64_t h0 = 0, h1 = 0;
+    if (kEach || tid < kThreads) { h0 = get<FUSED>(&rowhist[tid]); h1 = get<FUSED>(&rowhist[tid + kThreads]); }
+    uint64_t pre[PRE];                                   // (slices beyond the row's read its last slice again and are set aside below)
+#pragma unroll
+    for (int i = 0; i < PRE; ++i) pre[i] = get<FUSED>(&stash[(size_t)min((uint32_t)(wave + W * i), G - 1u) * kStashCap + lane]);
+    uint64_t *bk_lo = kEach ? t.blo : s.hr, *bk_hi = kEach ? t.bhi : s.hr + NT;       // buckets of the pick: NT of them
+    static_assert(kEach || sizeof(s.hr) >= 2 * NT * sizeof(uint64_t), "room for the buckets");
+    if (tid == 0) { s.abort = 0; s.host_words = p.host_words; t.result = 0u; s.ctr = 0u; t.nsmall = 0u; }
+    if (FUSED && tid == kWave) t.rand64 = drawn;
+    if (tid < 384) s.hm[tid] = 0;
+    if (kEach && tid < 128) s.hm[256 + tid] = 0;
+    bk_lo[tid] = 0; bk_hi[tid] = 0;
+
+    // The headers and the row's bins into LDS, the row's frame from the slices' maxima.  Bins are read where they
+    // lie, by absolute octave: bin r of the row's frame (octave M - 40 + r/4) sits at position 4 (M mod 128) + r - 160;
+    // the 348 positions no bin of that frame falls on hold tokens below 2^-40, which are dead there.
+    uint2 *hd = reinterpret_cast<uint2 *>(s.cand);       // per slice: key of its maximum, length of its stash
+    static_assert(sizeof(s.cand) >= kMaxParts * sizeof(uint2), "the headers lie in s.cand");
+    uint32_t kmax, kmin;
+    {
+        const uint32_t a = wave_max_u32(ph.mkey), b = wave_max_u32((uint32_t)tid < G ? ~ph.mkey : 0u);
+        if (lane == 0) { t.take[wave] = a; t.take[W + wave] = b; }
+        if (tid < kMaxParts) hd[tid] = make_uint2(ph.mkey, min(ph.n, (uint32_t)kStashCap));
+        if (kEach || tid < kThreads) {
+            s.g[tid] = h0; s.g[tid + kThreads] = h1;
+            if (!FUSED) { rowhist[tid] = 0; rowhist[tid + kThreads] = 0; }               // left clean for the next call
+        }
+        __syncthreads();
+        kmax = t.take[0]; kmin = t.take[W];
+        constexpr int kHdrWaves = kEach ? W : kMaxParts / kWave;       // the waves that hold headers
+#pragma unroll
+        for (int w = 1; w < kHdrWaves; ++w) { kmax = max(kmax, t.take[w]); kmin = max(kmin, t.take[W + w]); }
+        kmax = uniform(kmax); kmin = ~uniform(kmin);
+    }
+    if (!kEach && draws) draw();
+    const float xmax = fkey_inv(kmax);
+    const float M = __builtin_floorf(xmax);
+    // frames further apart than this may have put different octaves into one bin
+    const bool mixed = !(M - __builtin_floorf(fkey_inv(kmin)) < 88.0f);
+    const float mm = M - 128.0f * __builtin_floorf(M * 0.0078125f);
+    const uint32_t m4 = (uint32_t)(int)mm * 4u;
+    auto octaves_below = [&](uint32_t key) {             // of a slice's frame below the row's, at most 64
+        const float d = M - __builtin_floorf(fkey_inv(key));          // >= 0, a whole number or huge
+        return d >= 64.0f ? 64u : (uint32_t)d;
+    };
+    auto pos = [&](uint32_t b) { return (m4 + b - kBin0 - 160u) & 511u; };       // position of level-1 bin b
+    if (__builtin_expect(mixed, 0)) {
+        // Slices whose maxima lie 88 octaves or more apart may have put different octaves into
+        // one position.  Every token of a slice 41 octaves or more below the row's frame is
+        // dead there, whatever its bin: what such a slice added is taken out again, bin by bin
+        // (its own bins are on record).  The slices that remain lie within 40 octaves of each
+        // other.
+        for (uint32_t i = (uint32_t)tid; i < G * (uint32_t)kSB; i += NT) {
+            const uint32_t g = i / (uint32_t)kSB, r = i - g * (uint32_t)kSB;
+            if (octaves_below(hd[g].x) >= 41u) {
+                const uint64_t w = get<FUSED>(&v.shist[((size_t)row * G + g) * kSB + r]);
+                if (w) {
+                    const float Mg = __builtin_floorf(fkey_inv(hd[g].x));
+                    const uint32_t mg4 = (uint32_t)(int)(Mg - 128.0f * __builtin_floorf(Mg * 0.0078125f)) * 4u;
+                    atomicAdd(reinterpret_cast<unsigned long long *>(&s.g[(mg4 + r - 160u) & 511u]), 0ull - (unsigned long long)w);
+                }
+            }
+        }
+        __syncthreads();
+    }
+    if (__builtin_expect(p.e_bits != nullptr, 0)) {
+        // diagnostics: the slices' e into the row's frame, dead tokens as 0
+        uint4 *eb4 = reinterpret_cast<uint4 *>(p.e_bits + (int64_t)row * p.V);
+        auto fix = [&](uint32_t b, uint32_t d) { b = rebase_bits(min(b, 0x3FFFFFFFu), d); return b < kEMinBits ? 0u : b; };
+        for (uint32_t i4 = (uint32_t)tid; i4 < ((uint32_t)p.V >> 2); i4 += NT) {
+            const uint32_t d = octaves_below(hd[i4 >> (v.slice_log2 - 2u)].x);
+            uint4 q;
+            if (FUSED) {
+                const uint32_t *w = reinterpret_cast<const uint32_t *>(&eb4[i4]);
+                q = make_uint4(a_load(&w[0]), a_load(&w[1]), a_load(&w[2]), a_load(&w[3]));
+            } else q = eb4[i4];
+            q.x = fix(q.x, d); q.y = fix(q.y, d); q.z = fix(q.z, d); q.w = fix(q.w, d);
+            if (FUSED) {
+                // written through: a workgroup that falls back rewrites its slice of this later
+                uint32_t *w = reinterpret_cast<uint32_t *>(&eb4[i4]);
+                a_store(&w[0], q.x); a_store(&w[1], q.y); a_store(&w[2], q.z); a_store(&w[3], q.w);
+            } else eb4[i4] = q;
+        }
+    }
+
+    // A step one wave does: the first wave's result by way of LDS, unless every wave does it for itself.
+    struct { uint32_t place, cnt_above, cnt_bin; M96 above; } f;
+    f.place = 0; f.cnt_above = 0; f.cnt_bin = 0; f.above = M96{0ull, 0u};
+    M96 D{0ull, 0u}, P{0ull, 0u};
+    auto hand_on = [&](bool found) -> bool {
+        if constexpr (kEach) return found;
+        if (tid == 0) {
+            t.one.D = D; t.one.P = P; t.one.above = f.above;
+            t.one.place = f.place; t.one.cnt_above = f.cnt_above; t.one.cnt_bin = f.cnt_bin; t.one.found = found ? 1u : 0u;
+        }
+        __syncthreads();
+        D = uniform(t.one.D); P = uniform(t.one.P); f.above = uniform(t.one.above);
+        f.place = uniform(t.one.place); f.cnt_above = uniform(t.one.cnt_above); f.cnt_bin = uniform(t.one.cnt_bin);
+        return uniform(t.one.found) != 0u;
+    };
+    const uint32_t top_k = (uint32_t)p.top_k;
+    // boundary bin of the row, with D and P (whole_row), or of the listed tokens alone (counted in s.g by bin)
+    auto level1 = [&](bool whole_row) -> bool {
+        bool found = false;
+        if (kEach || wave == 0) {
+            BinScan<3> sc;
+            auto at = [&](int i) { return (uint32_t)max((int)kTop1 - 3 * lane - i, (int)kBin0); };
+            auto live = [&](int i) { return (int)kTop1 - 3 * lane - i >= (int)kBin0; };
+            sc.load([&](int i) { const uint64_t w = s.g[whole_row ? pos(at(i)) : at(i)]; return live(i) ? w : 0ull; }, [&](int i) { return at(i) >> 2; });
+            if (whole_row) { D = sc.total(); P = ceil_mul(p.top_p, D); }
+            found = sc.search(0u, M96{0ull, 0u}, top_k, P, f.place, f.cnt_above, f.cnt_bin, f.above);
+        }
+        return hand_on(found);
+    };
+    level1(true);
+    uint32_t bin = kTop1 - f.place;
+
+    // What the stashes cannot finish, this workgroup does alone from the logits.  Such rows are
+    // counted, and the first of a call tells the caller's policy at once (that a call went well is
+    // reported by the call after it, see report_begin).
+    auto tell_policy = [&]() {
+        if (tid == 0) {
+            const uint32_t c = __hip_atomic_fetch_add(&p.hdr->n_need, 1u, __ATOMIC_RELAXED, RS_AGENT);
+            if (c == 0u && p.host_words)                 // the call's first such row tells the caller's policy at once
+                __hip_atomic_store(p.host_words + p.report, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    };
+
+    // A row that is one tie of all its tokens (rows of equal logits) needs no stash at all: the
+    // threshold is the largest token's value, every token weighs the tie weight, and the token at
+    // which the running sum reaches r follows by division.
+    if (__builtin_expect(f.cnt_bin == (uint32_t)p.V, 0)) {
+        const uint32_t emax = e_bits_of(xmax, M);
+        if (bin_is_one_tie(uniform(s.g[pos(bin)]), bin, emax)) {
+            __syncthreads();                             // the random number is there
+            if (tid == 0) {
+                const Target tg = tie_and_target(p, row, t.rand64, xmax, wide(D), wide(P), emax, 0u, f.cnt_bin, (u128)0, 0u, true);
+                // smallest i with (i + 1) * w_tie >= r; r <= V * w_tie
+                uint32_t lo_i = 0, hi_i = (uint32_t)p.V - 1u;
+                while (lo_i < hi_i) {
+                    const uint32_t mid = (lo_i + hi_i) >> 1;
+                    if ((u128)(mid + 1u) * tg.w_tie >= tg.r) hi_i = mid; else lo_i = mid + 1u;
+                }
+                p.out[row] = (int32_t)lo_i;
+                if (p.diag) p.diag[row].index = (int32_t)lo_i;
+                t.result = lo_i + 1u;
+            }
+            return true;
+        }
+    }
+
+    // ---- the list: the row's tokens at or above the boundary bin ----
+    // The tokens of a chunk of 64 stash entries at or above `from`, side by side behind what is in the list
+    // already; at: the wave's place in it (claimed for what the wave is about to add).
+    auto put_listed = [&](uint32_t b, uint32_t idx, uint32_t &at) {
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(b != 0u);
+        const uint32_t o = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0u));
+        if (b != 0u && o < v.list_cap) list[o] = ((uint64_t)b << 32) | idx;
+        at += (uint32_t)__builtin_popcountll(vote);
+    };
+    auto claim = [&](uint32_t n) {
+        uint32_t at = 0;
+        if (lane == 0 && n) at = atomicAdd(&s.ctr, n);
+        return uniform(at);
+    };
+    const uint32_t total = f.cnt_above + f.cnt_bin;
+    const uint32_t cut = bin << 21;
+    uint32_t n = 0;                                      // tokens listed
+    bool listed = false, subset = false;
+    if (total <= v.list_cap && G <= (uint32_t)(W * PRE)) {
+        // lane i looks after the wave's i-th slice: how far its frame lies below the row's, how many tokens it stashed
+        const uint32_t sl = (uint32_t)(wave + W * lane);
+        const uint2 h = hd[min(sl, G - 1u)];
+        const uint32_t below = octaves_below(h.x), len = sl < G ? min(h.y, (uint32_t)kWave) : 0u;
+        uint32_t mine = 0;                               // of this lane's tokens, how many
+#pragma unroll
+        for (int i = 0; i < PRE; ++i) {
+            const uint32_t b = rebase_bits((uint32_t)(pre[i] >> 32), lane_of(below, (uint32_t)i));
+            const bool in = (uint32_t)lane < lane_of(len, (uint32_t)i) && b >= cut;
+            pre[i] = ((uint64_t)(in ? b : 0u) << 32) | (uint32_t)pre[i];
+            mine += in ? 1u : 0u;
+        }
+        const uint32_t upto = wave_inclusive_scan(mine);
+        uint32_t at = claim(lane63(upto)) + upto - mine;
+#pragma unroll
+        for (int i = 0; i < PRE; ++i)
+        {
+            // (a branch per entry would cost more than the store: what is not listed goes into a corner of its own)
+            typedef __attribute__((address_space(3))) uint64_t lds_u64;
+            const bool in = (uint32_t)(pre[i] >> 32) != 0u;
+            lds_u64 *to = in ? (lds_u64 *)list + at : (lds_u64 *)t.small + lane;
+            *to = pre[i];
+            at += in ? 1u : 0u;
+        }
+        __syncthreads();
+        n = uniform(s.ctr);
+        listed = n == total;                             // every token at or above the boundary bin is there
+    }
+    if (!listed) {
+        const uint32_t dl = (uint32_t)tid < G ? octaves_below(ph.mkey) : 0u;
+        if ((uint32_t)tid < G) { t.delta[tid] = dl; t.m4[tid] = min(ph.n, (uint32_t)kStashCap); }      // (m4: the stashes' lengths here)
+        // fn(bits of e in the row's frame, 0 past the end of a stash; token) for all stashes whole, 64 entries at a
+        // time, eight loads in flight; called by all lanes of a wave together
+        auto stashed = [&](auto fn) {
+            constexpr int kBatch = 8;
+            uint32_t sl = (uint32_t)wave, c = 0, len = sl < G ? uniform(t.m4[sl]) : 0u;
+            for (;;) {
+                uint64_t e[kBatch];
+                uint32_t d[kBatch];
+                bool live[kBatch];
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) {
+                    while (sl < G && c >= len) { sl += W; c = 0; len = sl < G ? uniform(t.m4[sl]) : 0u; }
+                    live[u] = sl < G && c + (uint32_t)lane < len;
+                    d[u] = sl < G ? t.delta[sl] : 0u;
+                    e[u] = live[u] ? get<FUSED>(&stash[(size_t)sl * kStashCap + c + (uint32_t)lane]) : 0ull;
+                    c += (uint32_t)kWave;
+                }
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) fn(live[u] ? rebase_bits((uint32_t)(e[u] >> 32), d[u]) : 0u, (uint32_t)e[u]);
+                if (sl >= G) break;
+            }
+        };
+        auto list_from = [&](uint32_t from) {
+            __syncthreads();                             // the list's counter has been read
+            if (tid == 0) s.ctr = 0u;
+            __syncthreads();
+            stashed([&](uint32_t b, uint32_t idx) {
+                if (b < from) b = 0u;
+                uint32_t at = claim((uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b != 0u)));
+                put_listed(b, idx, at);
+            });
+            __syncthreads();
+            return uniform(s.ctr);
+        };
+        // Together the stashes hold every token of the row at or above `from`, the largest of the slices' cuts.  (A
+        // cut that lands below 2^-40 in the row's frame: what the stash lacks is dead there.)
+        uint32_t from = (uint32_t)tid < G ? max(rebase_bits(ph.cut, dl), kEMinBits) : 0u;
+        uint32_t all = (uint32_t)tid < G ? min(ph.n, (uint32_t)kStashCap) : 0u;       // stashed tokens of the row
+        {
+            const uint32_t a = wave_max_u32(from), b = wave_sum(all);
+            __syncthreads();
+            if (lane == 0) { t.take[wave] = a; t.take[W + wave] = b; }
+            __syncthreads();
+            from = 0; all = 0;
+            for (int w = 0; w < W; ++w) { from = max(from, t.take[w]); all += t.take[W + w]; }
+            from = uniform(from); all = uniform(all);
+        }
+        bool slow = false;
+        if (from <= cut && total <= v.list_cap) {        // plan A: every stash reaches down to the boundary bin
+            n = list_from(cut);
+            slow = n != total;
+        } else if (!FUSED && all > min(v.list_cap, max(2048u, 3u * top_k)) && top_k <= v.list_cap / 2u) {
+            // Plan B (flat distributions: the boundary bin holds thousands of tokens, but top_k is small) with more
+            // stashed tokens than the list holds, or several times top_k of them.  The kept set is at most
+            // top_k tokens, so only the stashed tokens down to some value T at or above which there are at least
+            // top_k of them are needed: T from a count of the stashed tokens in steps of 1/512 octave below the
+            // row's largest (one pass over the stashes, which sit in the L2), the tokens at or above T into the
+            // list by a second pass.  T is at or above `from`, so the list is complete above T.
+            const uint32_t topkey = e_bits_of(xmax, M) >> 14;
+            uint32_t *cnt = reinterpret_cast<uint32_t *>(s.cand);                // 512 counters
+            if (tid < 512) cnt[tid] = 0u;
+            if (kEach) cnt[256 + tid] = 0u;
+            if (tid == 0) { s.bc32[4] = 0xFFFFFFFFu; s.bc32[5] = 0u; }
+            __syncthreads();
+            stashed([&](uint32_t b, uint32_t) {
+                if (b >= from) atomicAdd(&cnt[min(511u, topkey - (b >> 14))], 1u);
+            });
+            __syncthreads();
+            if (wave == 0) {
+                uint32_t c8 = 0;
+#pragma unroll
+                for (int q = 0; q < 8; ++q) c8 += cnt[lane * 8 + q];
+                const uint32_t inc = wave_inclusive_scan(c8);
+                uint32_t run = inc - c8;
+                if (run < top_k && top_k <= inc) {
+                    bool done = false;
+#pragma unroll
+                    for (int q = 0; q < 8; ++q) {
+                        run += cnt[lane * 8 + q];
+                        if (!done && run >= top_k) { s.bc32[4] = (uint32_t)(lane * 8 + q); s.bc32[5] = run; done = true; }
+                    }
+                }
+            }
+            __syncthreads();
+            const uint32_t step = uniform(s.bc32[4]), nge = uniform(s.bc32[5]);
+            slow = step >= 511u || nge > v.list_cap;     // fewer than top_k at or above `from`, or one value thousands of times
+            if (!slow) {
+                n = list_from(max(from, (topkey - step) << 14));
+                subset = true;
+                // Two more passes over the stashes make this finish slower than the general kernel's whole
+                // call while the call is of moderate size (measured: 64 flat rows of 131072 with top_k 1000,
+                // 51 against 38 us; 128 rows of 262144, 77 against 117): such a call says so to the caller's
+                // policy, as it did when these rows still went the slow way.
+                // (p.tell_lists: calls of fewer than 2^24 tokens, and calls whose rows the row kernel would take)
+                if (p.tell_lists) tell_policy();
+            }
+        } else {                                         // plan B, the stashes whole
+            slow = all > v.list_cap || all == 0u;
+            if (!slow) { n = list_from(from); subset = true; }
+        }
+        if (!slow && subset) {
+            // level 1 again, on the listed tokens alone
+            __syncthreads();
+            for (int b = tid; b < kSB; b += NT) s.g[kBin0 + b] = 0;
+            __syncthreads();
+            for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+                const uint32_t b = (uint32_t)(list[i] >> 32);
+                atomicAdd(reinterpret_cast<unsigned long long *>(&s.g[b >> 21]), (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
+            }
+            __syncthreads();
+            slow = !level1(false);                       // even all of them are neither top_k tokens nor top_p of the mass
+            bin = kTop1 - f.place;
+        }
+        if (slow) {
+            if (FUSED) return false;
+            __syncthreads();                             // the random number is there
+            if (NT > kThreads && tid >= kThreads) return true;
+            if (p.penalties && p.defer_pen == 2) pen_restore(p, v, row);
+            finish_row_slow(p, s, t, row, xmax, p.inj_u ? 0ull : t.rand64);
+            tell_policy();
+            return true;
+        }
+    }
+
+    // a list so long that another kernel is faster (the host's rule): said to the caller's policy
+    if (!FUSED && n > p.long_list) tell_policy();
+
+    if (!subset && n <= (uint32_t)kWave) {
+        // ---- a short list: every pair of its tokens ----
+        // Lane i of each of four waves holds token i and goes through a quarter of the others: how many are larger,
+        // what they weigh, how many come before it in index order.  A token is kept when what is larger is neither
+        // top_k tokens nor P; the threshold is the smallest kept value.
+        struct Part { uint64_t lo; uint32_t hi, cnt; };              // cnt: larger | before << 16
+        Part *part = reinterpret_cast<Part *>(s.cand);               // [4][64]
+        static_assert(sizeof(Part) == 16 && sizeof(s.cand) >= 4 * kWave * sizeof(Part) && offsetof(Lds, cand) % 16 == 0, "partial sums live in s.cand");
+        const uint64_t e = list[min((uint32_t)lane, n - 1u)];
+        const uint32_t b = (uint32_t)(e >> 32), idx = (uint32_t)e;
+        if (wave < 4) {
+            M96 sum{0ull, 0u};
+            uint32_t larger = 0, before = 0;
+            const uint32_t per = (n + 3u) >> 2, j1 = min(n, ((uint32_t)wave + 1u) * per);
+#pragma unroll 4
+            for (uint32_t j = (uint32_t)wave * per; j < j1; ++j) {
+                const uint64_t o = list[j];
+                const bool gt = (uint32_t)(o >> 32) > b;
+                sum = sum + M96{gt ? w_of_bits((uint32_t)(o >> 32)) : 0ull, 0u};
+                larger += gt ? 1u : 0u;
+                before += (uint32_t)o < idx ? 1u : 0u;
+            }
+            part[wave * kWave + lane] = Part{sum.lo, sum.hi, larger | before << 16};
+        }
+        __syncthreads();
+        if (wave == 0) {
+            M96 above{0ull, 0u};
+            uint32_t cnt = 0;
+#pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const Part q = part[w * kWave + lane];
+                above = above + M96{q.lo, q.hi};
+                cnt += q.cnt;
+            }
+            const uint32_t larger = cnt & 0xFFFFu, rank = cnt >> 16;
+            const bool in = (uint32_t)lane < n;
+            const bool kept = in && larger < top_k && above < P;
+            const uint32_t thr = ~wave_max_u32(kept ? ~b : 0u);
+            const uint64_t ties = __builtin_amdgcn_ballot_w64(in && b == thr);
+            const uint32_t l = (uint32_t)__builtin_ctzll(ties);
+            const Target tg = tie_and_target(p, row, t.rand64, xmax, wide(D), wide(P), thr, lane_of(larger, l), (uint32_t)__builtin_popcountll(ties),
+                                             wide(lane_of(above, l)), 0u, lane == 0);            // rounds = 0: no cluster histogram
+            pick_of_wave(p, t, row, lane, n, rank, idx, b > thr ? w_of_bits(b) : b == thr ? tg.w_tie : 0ull, m96(tg.r));
+        }
+        return true;
+    }
+
+    // ---- a longer list: the remaining digits of the threshold ----
+    uint32_t lo = bin << 21, span = (1u << 21) - 1u;
+    const uint32_t exb = bin >> 2;
+    for (uint32_t lv = 2; lv <= (uint32_t)kLevels && f.cnt_bin > 1u; ++lv) {
+        const uint32_t dsh = level_shift(lv);
+        uint64_t *hist = s.hm + (lv - 2u) * 128u;
+        for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+            const uint32_t b = (uint32_t)(list[i] >> 32);
+            if (b - lo <= span) atomicAdd(reinterpret_cast<unsigned long long *>(&hist[(b >> dsh) & 127u]), (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
+        }
+        __syncthreads();
+        bool found = true;
+        if (kEach || wave == 0) {
+            BinScan<2> sc;
+            sc.load([&](int i) { return hist[127 - 2 * lane - i]; }, [&](int) { return exb; });
+            const uint32_t c0 = f.cnt_above;
+            const M96 m0 = f.above;
+            found = sc.search(c0, m0, top_k, P, f.place, f.cnt_above, f.cnt_bin, f.above);
+        }
+        hand_on(found);
+        lo |= (127u - f.place) << dsh;
+        span = (1u << dsh) - 1u;
+    }
+    if (span != 0u) {                                    // a single token left in the range: the threshold itself
+        for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+            const uint32_t b = (uint32_t)(list[i] >> 32);
+            if (b - lo <= span) s.bc32[6] = b;
+        }
+        __syncthreads();
+        lo = uniform(s.bc32[6]);
+    }
+    const uint32_t thr = lo;
+    uint64_t w_tie = 0;
+    M96 r{0ull, 0u};
+    if (kEach || wave == 0) {
+        const Target tg = tie_and_target(p, row, t.rand64, xmax, wide(D), wide(P), thr, f.cnt_above, f.cnt_bin, wide(f.above), 0u, tid == 0);
+        w_tie = tg.w_tie; r = m96(tg.r);
+    }
+    if constexpr (!kEach) {
+        if (tid == 0) { s.bc64[1] = w_tie; t.one.P = r; }
+        __syncthreads();
+        w_tie = uniform(s.bc64[1]); r = uniform(t.one.P);
+    }
+
+    // ---- the pick: kept weights by bucket of the token index, NT buckets a step, then the bucket's tokens ----
+    // (a weight is below 2^64 and a bucket has fewer than 2^14 listed tokens: the halves summed apart stay below 2^46)
+    auto weight = [=](uint32_t b) -> uint64_t { return (b > thr) ? w_of_bits(b) : (b == thr ? w_tie : 0ull); };
+    constexpr uint32_t kLogNT = NT == 256 ? 8u : 10u;
+    uint32_t sh = 32u - (uint32_t)__builtin_clz((uint32_t)p.V - 1u | 1u);
+    sh = sh > kLogNT ? sh - kLogNT : 0u;
+    uint32_t lo_idx = 0, len = (uint32_t)p.V;
+    for (int step = 0;; ++step) {
+        for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+            const uint64_t e = list[i];
+            const uint32_t off = (uint32_t)e - lo_idx;
+            const uint64_t w = weight((uint32_t)(e >> 32));
+            if (w && off < len) {
+                atomicAdd(reinterpret_cast<unsigned long long *>(&bk_lo[off >> sh]), (unsigned long long)(w & 0xFFFFFFFFull));
+                atomicAdd(reinterpret_cast<unsigned long long *>(&bk_hi[off >> sh]), (unsigned long long)(w >> 32));
+            }
+        }
+        __syncthreads();
+        const M96 mine = m96((u128)bk_lo[tid] + ((u128)bk_hi[tid] << 32));
+        bk_lo[tid] = 0; bk_hi[tid] = 0;
+        M96 inc = m96(wave_inclusive_scan(limbs(mine)));
+        M96 *waves = reinterpret_cast<M96 *>(&s.wj[0][0]);
+        static_assert(sizeof(s.wj) >= 16 * sizeof(M96), "one mass per wave");
+        if (lane == kWave - 1) waves[wave] = inc;
+        __syncthreads();
+        {
+            const Limbs tot = wave_inclusive_scan(limbs(lane < W ? waves[lane] : M96{0ull, 0u}));
+            if (wave) inc = inc + m96(lane_of(tot, (uint32_t)wave - 1u));
+        }
+        const M96 exc = inc - mine;
+        if (exc < r && inc >= r) { t.bucket = (uint32_t)tid; t.one.above = r - exc; }
+        __syncthreads();
+        lo_idx += uniform(t.bucket) << sh; len = 1u << sh;
+        r = uniform(t.one.above);
+        // the kept tokens of the bucket: few enough for one wave, as a rule; otherwise the bucket is cut into NT again
+        for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+            const uint64_t e = list[i];
+            if ((uint32_t)e - lo_idx < len && weight((uint32_t)(e >> 32))) {
+                const uint32_t o = atomicAdd(&t.nsmall, 1u);
+                if (o < (uint32_t)kWave) s.cand[o] = e;
+            }
+        }
+        __syncthreads();
+        const uint32_t ns = uniform(t.nsmall);
+        if (ns <= (uint32_t)kWave) {
+            if (wave == 0) {
+                const uint64_t e = s.cand[min((uint32_t)lane, ns - 1u)];
+                uint32_t rank = 0;
+                for (uint32_t j = 0; j < ns; ++j) rank += (uint32_t)s.cand[j] < (uint32_t)e ? 1u : 0u;
+                pick_of_wave(p, t, row, lane, ns, rank, (uint32_t)e, weight((uint32_t)(e >> 32)), r);
+            }
+            return true;
+        }
+        __syncthreads();                                 // everyone has read the count
+        if (tid == 0) t.nsmall = 0u;
+        sh = sh > kLogNT ? sh - kLogNT : 0u;
+        __syncthreads();
+    }
+}
+
+// NT: 256 threads and the wave that draws the random number, or 1024 for calls whose lists are long (the host's choice).
+template <int NT> constexpr int finish_threads() { return NT == kThreads ? NT + kWave : NT; }
+template <int NT, int PRE>
+__global__ void __launch_bounds__(finish_threads<NT>()) finish_kernel(const Params p, const StreamView v)
+{
+    __shared__ Lds s;
+    __shared__ LdsB t;
+    extern __shared__ __align__(16) unsigned char finish_dyn[];
+    finish_row<NT, PRE, false>(p, v, s, t, reinterpret_cast<uint64_t *>(finish_dyn), blockIdx.x);
+    if (p.penalties && p.defer_pen == 2) {
+        if (threadIdx.x >= kThreads) return;
+        __syncthreads();
+        pen_patch(p, v, s, blockIdx.x, t.result - 1u, v.slice_log2);
+    }
+}
+
+// The finish of a call that keeps every live token (top_k = V, top_p = 1; the counting-only pass left the
+// slices' masses where their stashes would begin).
+template <int SLICE_LOG2>
+__device__ __forceinline__ void keep_finish_row(const Params &p, const StreamView &v, Lds &s, LdsB &t, const uint32_t row)
+{
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
+    const uint32_t G = v.G;
+    const PartHdr *hdrs = v.hdr + (size_t)row * G;
+    uint64_t *rowhist = (p.ctl_end - 1 - row)->rowhist;
+
+    if (tid == 0) { s.abort = 0; s.host_words = p.host_words; t.fail = 0; t.result = 0u; }
+    PartHdr ph;
+    ph.mkey = 0; ph.cov = 0; ph.n = 0; ph.cut = 0;
+    if ((uint32_t)tid < G) ph = hdrs[tid];
+    const uint64_t h0 = rowhist[tid], h1 = rowhist[tid + kThreads];
     // the first lane of wave 1 draws the row's random number while wave 0 scans the histogram;
     // the state is advanced only once the row is certain to be finished here
     const bool drawer = tid == kWave && !p.inj_u;
@@ -796,7 +1335,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
 #pragma unroll
         for (int i = 0; i < 6; ++i) rs[i] = rng_st[i];
     }
-    if (!FUSED) { rowhist[tid] = 0; rowhist[tid + kThreads] = 0; }   // left clean for the next call
+    rowhist[tid] = 0; rowhist[tid + kThreads] = 0;       // left clean for the next call
     uint32_t kmax, kmin;
     {
         const uint32_t a = wave_max_u32(ph.mkey), b = wave_max_u32((uint32_t)tid < G ? ~ph.mkey : 0u);
@@ -839,7 +1378,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             for (uint32_t i = (uint32_t)tid; i < G * (uint32_t)kSB; i += kThreads) {
                 const uint32_t g = i / (uint32_t)kSB, r = i - g * (uint32_t)kSB;
                 if (t.delta[g] >= 41u) {
-                    const uint64_t w = get<FUSED>(&v.shist[((size_t)row * G + g) * kSB + r]);
+                    const uint64_t w = v.shist[((size_t)row * G + g) * kSB + r];
                     if (w) {
                         const uint32_t rr = (t.m4[g] + r - m4) & 511u;
                         if (rr < (uint32_t)kSB)
@@ -856,17 +1395,9 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         auto fix = [&](uint32_t b, uint32_t d) { b = rebase_bits(min(b, 0x3FFFFFFFu), d); return b < kEMinBits ? 0u : b; };
         for (uint32_t i4 = (uint32_t)tid; i4 < ((uint32_t)p.V >> 2); i4 += kThreads) {
             const uint32_t d = t.delta[i4 >> (SLICE_LOG2 - 2)];
-            uint4 q;
-            if (FUSED) {
-                const uint32_t *w = reinterpret_cast<const uint32_t *>(&eb4[i4]);
-                q = make_uint4(a_load(&w[0]), a_load(&w[1]), a_load(&w[2]), a_load(&w[3]));
-            } else q = eb4[i4];
+            uint4 q = eb4[i4];
             q.x = fix(q.x, d); q.y = fix(q.y, d); q.z = fix(q.z, d); q.w = fix(q.w, d);
-            if (FUSED) {
-                // written through: a workgroup that falls back rewrites its slice of this later
-                uint32_t *w = reinterpret_cast<uint32_t *>(&eb4[i4]);
-                a_store(&w[0], q.x); a_store(&w[1], q.y); a_store(&w[2], q.z); a_store(&w[3], q.w);
-            } else eb4[i4] = q;
+            eb4[i4] = q;
         }
     }
     if (drawer) {
@@ -877,27 +1408,6 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     const uint64_t top_k = (uint64_t)p.top_k;
     Found f = hist_find_level1<false>(s, top_k, p.top_p, lane, wave);
     const u128 D = s.D, P = s.P;
-    // What the stashes cannot finish, this workgroup does alone from the logits.  Such rows are
-    // counted, and the first of a call tells the caller's policy at once (that a call went well is
-    // reported by the call after it, see report_begin).
-    auto tell_policy = [&]() {
-        if (tid == 0) {
-            const uint32_t c = __hip_atomic_fetch_add(&p.hdr->n_need, 1u, __ATOMIC_RELAXED, RS_AGENT);
-            if (c == 0u && p.host_words)                 // the call's first such row tells the caller's policy at once
-                __hip_atomic_store(p.host_words + p.report, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
-        }
-    };
-    auto slow = [&]() -> bool {
-        if (drawer) {                                    // the row is finished here: this draw is used up
-            rng_st[2] = rs[2] + 1u;
-            if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
-        }
-        if (!FUSED && p.penalties && p.defer_pen == 2) pen_restore(p, v, row);
-        finish_row_slow(p, s, t, row, xmax, p.inj_u ? 0ull : t.rand64);
-        tell_policy();
-        return true;
-    };
-
     // A row that is one tie of all its tokens (rows of equal logits) needs no stash at all: the
     // threshold is the largest token's value, every token weighs the tie weight, and the token at
     // which the running sum reaches r follows by division.
@@ -919,357 +1429,55 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             if (p.diag) p.diag[row].index = (int32_t)lo_i;
             t.result = lo_i + 1u;
         }
-        return true;
+        return;
     }
 
-    if constexpr (KEEP) {
-        // Every live token is kept with its full weight (S = D).  Each slice's mass, moved into the
-        // row's frame, is exact (a bin is dead in the row's frame as a whole or not at all: frames
-        // differ by whole octaves); a scan over the slices finds the one that holds the target, and
-        // only that slice's logits are looked at again.
-        if (drawer) {
-            rng_st[2] = rs[2] + 1u;
-            if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
-        }
-        u128 mine = 0;
-        if ((uint32_t)tid < G && dl < 41u) {                          // 41 octaves and more below: nothing of the slice is live
-            const uint64_t *sm = v.stash + ((size_t)row * G + tid) * kStashCap;
-            mine = (u128)sm[0] | ((u128)sm[1] << 64);
-            if (dl) {
-                // the slice's lowest 4 dl bins are dead in the row's frame; the rest is a multiple of 2^dl
-                const uint64_t *sh = v.shist + ((size_t)row * G + tid) * kSB;
-                u128 low = 0;
-                for (uint32_t b = 0; b < 4u * dl; ++b) {
-                    const uint64_t w = sh[b];
-                    if (w) low += pack_mass(w, (kBin0 + b) >> 2);
-                }
-                mine = (mine - low) >> dl;
-            }
-        }
-        const u128 r = p.inj_u ? ceil_mul(p.inj_u[row], D) : r_from_bits(t.rand64, D);
-        u128 inc = wave_inclusive_scan(mine);
-        if (lane == kWave - 1) s.q128[wave] = inc;
-        __syncthreads();
-        for (int w = 0; w < wave; ++w) inc += s.q128[w];
-        const u128 exc = inc - mine;
-        if (exc < r && r <= inc) { t.bucket = (uint32_t)tid; s.bc128[1] = r - exc; }
-        __syncthreads();
-        const uint32_t g = t.bucket;
-        const u128 r_in = s.bc128[1];
-        __syncthreads();
-        if (p.diag) finish_row_slow<true>(p, s, t, row, xmax, p.inj_u ? 0ull : t.rand64, f.cnt_above + f.cnt_bin);
-        keep_pick<SLICE_LOG2>(p, s, t, row, M, g << SLICE_LOG2, r_in,
-                              [](uint32_t b) -> uint64_t { return b >= kEMinBits ? w_of_bits(b) : 0ull; });
-        return true;
-    }
-
-    // Plan A: every stash reaches down to the row's boundary bin.  Then exactly the tokens at or
-    // above that bin are taken, a prefix of each stash whose length is one cumulative count.
-    uint32_t total = f.cnt_above + f.cnt_bin;
-    uint32_t mtake = 0;
-    bool bad = total > v.list_cap;
-    if ((uint32_t)tid < G) {
-        const int lb = (int)(f.bin - kBin0) + 4 * (int)dl;            // boundary bin in the slice's frame
-        if (dl >= 64u) mtake = 0;                                      // the whole slice is dead in the row's frame
-        else if (lb < kSB) mtake = get<FUSED>(&v.cum[((size_t)row * G + tid) * kSB + lb]);
-        if (mtake && ((int)ph.cov > lb || mtake > ph.n)) bad = true;
-    }
-    if (bad) t.fail = 1;
-    auto take_prefix = [&](uint32_t mine) {                           // inclusive prefix over the slices, into t.take
-        uint32_t inc = wave_inclusive_scan(mine);
-        __syncthreads();
-        if (lane == kWave - 1) s.u32[wave] = inc;
-        __syncthreads();
-        for (int w = 0; w < wave; ++w) inc += s.u32[w];
-        t.take[tid] = inc;
-        __syncthreads();
-    };
-    // fn(i, e in the row's frame, token) for the first n entries of the stashes' prefixes as t.take has
-    // them (entry i belongs to the first slice whose inclusive prefix exceeds i): a thread takes a run of
-    // consecutive entries, so that it looks up its first slice once and walks on from there, eight
-    // loads in flight
-    auto stashed = [&](const uint32_t n_all, auto fn) {
-        constexpr int kBatch = 8;
-        const uint32_t per = (n_all + kThreads - 1u) / kThreads;
-        uint32_t i = (uint32_t)tid * per;
-        const uint32_t iend = min(n_all, i + per);
-        uint32_t g = 0, gbase = 0, gend = 0;
-        if (i < iend) {
-            uint32_t lo_g = 0, hi_g = G - 1;                           // first slice whose prefix exceeds i
-            while (lo_g < hi_g) {
-                const uint32_t mid = (lo_g + hi_g) >> 1;
-                if (t.take[mid] > i) hi_g = mid; else lo_g = mid + 1;
-            }
-            g = lo_g; gbase = g ? t.take[g - 1] : 0u; gend = t.take[g];
-        }
-        if (per == 1u) {                                               // a short list: one entry, no walking
-            if (i < iend) {
-                const uint64_t e = get<FUSED>(&v.stash[((size_t)row * G + g) * kStashCap + (i - gbase)]);
-                fn(i, rebase_bits((uint32_t)(e >> 32), t.delta[g]), (uint32_t)e);
-            }
-            i = iend;
-        }
-        while (i < iend) {
-            uint64_t e[kBatch];
-            uint32_t sl[kBatch];
-            const uint32_t n = min((uint32_t)kBatch, iend - i);
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u) {
-                e[u] = 0; sl[u] = 0;
-                if ((uint32_t)u < n) {
-                    while (i + (uint32_t)u >= gend) { ++g; gbase = gend; gend = t.take[g]; }    // slices that give nothing are skipped
-                    e[u] = get<FUSED>(&v.stash[((size_t)row * G + g) * kStashCap + (i + (uint32_t)u - gbase)]);
-                    sl[u] = g;
-                }
-            }
-#pragma unroll
-            for (int u = 0; u < kBatch; ++u)
-                if ((uint32_t)u < n) fn(i + (uint32_t)u, rebase_bits((uint32_t)(e[u] >> 32), t.delta[sl[u]]), (uint32_t)e[u]);
-            i += n;
-        }
-    };
-    take_prefix(mtake);
-    bool subset = false;                                               // plan B in force
-    bool listed = false;                                               // the list has been filled already
-    uint32_t cutrow = 0;
-    if (t.fail || t.take[kThreads - 1] != total) {
-        // Plan B (flat distributions: the boundary bin holds thousands of tokens, but top_k is small):
-        // take the stashes whole.  Together they hold every token of the row at or above
-        // cutrow = the largest of the slices' cuts, so a threshold found among those is the row's.
-        uint32_t mycut = 0;
-        if ((uint32_t)tid < G) {
-            // a cut that lands below 2^-40 in the row's frame: what the stash lacks is dead there
-            mycut = max(rebase_bits(ph.cut, dl), kEMinBits);
-        }
-        cutrow = block_max_u32(s, mycut, lane, wave);
-        take_prefix((uint32_t)tid < G ? min(ph.n, (uint32_t)kStashCap) : 0u);
-        total = t.take[kThreads - 1];
-        if (!FUSED && total > min(v.list_cap, max(2048u, 3u * (uint32_t)p.top_k)) && (uint32_t)p.top_k <= v.list_cap / 2u) {
-            // More stashed tokens than the list holds (a flat row cut into many slices, each of which
-            // stashed several times its share of top_k), or several times top_k of them (going through
-            // a list of thousands a dozen times costs more than these two passes: 128 flat rows of
-            // 100256 with top_k 1000, 60 against 70 us).  The kept set is at most top_k tokens, so only
-            // the stashed tokens down to some value T at or above which there are at least top_k of
-            // them are needed: T from a count of the stashed tokens in steps of 1/512 octave below the
-            // row's largest (one pass over the stashes, which sit in the L2), the tokens at or above T
-            // into the list by a second pass.  T is at or above cutrow, so the list is complete above T.
-            const uint32_t topkey = e_bits_of(xmax, M) >> 14;
-            uint32_t *cnt = reinterpret_cast<uint32_t *>(t.blo);                // 512 counters
-            cnt[tid] = 0u; cnt[tid + kThreads] = 0u;
-            if (tid == 0) { s.ctr = 0u; s.bc32[4] = 0xFFFFFFFFu; s.bc32[5] = 0u; }
-            __syncthreads();
-            stashed(total, [&](uint32_t, uint32_t b, uint32_t) {
-                if (b >= cutrow) atomicAdd(&cnt[min(511u, topkey - (b >> 14))], 1u);
-            });
-            __syncthreads();
-            if (wave == 0) {
-                uint32_t c8 = 0;
-#pragma unroll
-                for (int q = 0; q < 8; ++q) c8 += cnt[lane * 8 + q];
-                const uint32_t inc = wave_inclusive_scan(c8);
-                uint32_t run = inc - c8;
-                if (run < (uint32_t)p.top_k && (uint32_t)p.top_k <= inc) {
-                    bool done = false;
-#pragma unroll
-                    for (int q = 0; q < 8; ++q) {
-                        run += cnt[lane * 8 + q];
-                        if (!done && run >= (uint32_t)p.top_k) { s.bc32[4] = (uint32_t)(lane * 8 + q); s.bc32[5] = run; done = true; }
-                    }
-                }
-            }
-            __syncthreads();
-            const uint32_t step = s.bc32[4], nge = s.bc32[5];
-            if (step >= 511u || nge > v.list_cap) return slow();              // fewer than top_k at or above cutrow, or one value thousands of times
-            cutrow = max(cutrow, (topkey - step) << 14);
-            stashed(total, [&](uint32_t, uint32_t b, uint32_t idx) {
-                if (b >= cutrow) {
-                    const uint32_t o = atomicAdd(&s.ctr, 1u);
-                    if (o < v.list_cap) t.list[o] = ((uint64_t)b << 32) | idx;
-                }
-            });
-            __syncthreads();
-            total = nge;
-            subset = true; listed = true;
-            // Two more passes over the stashes make this finish slower than the general kernel's whole
-            // call while the call is of moderate size (measured: 64 flat rows of 131072 with top_k 1000,
-            // 51 against 38 us; 128 rows of 262144, 77 against 117): such a call says so to the caller's
-            // policy, as it did when these rows still went the slow way.
-            // (p.tell_lists: calls of fewer than 2^24 tokens, and calls whose rows the row kernel would take)
-            if (p.tell_lists) tell_policy();
-        } else {
-        if (total > v.list_cap || total == 0u) {
-            // not resolvable from the stashes
-            if (FUSED) return false;
-            return slow();
-        }
-        subset = true;
-        }
-    }
-
-    // A nucleus of thousands of tokens is finished here all the same, but one workgroup going through
-    // such a list a dozen times takes longer than the general kernel needs for the whole call (measured:
-    // 128 rows of 50304, about 4000 tokens each, 54 against 36 us; the two meet at about 2400 tokens
-    // there and, the general kernel's time growing with the row, at about 4700 for rows of 100256): a
-    // call that is only an attempt (no top_k bounds the kept set) says so to the caller's policy, and so
-    // does a call of moderate size with a bounding top_k (a lone flat row of 32768 tokens with top_k 1000:
-    // 26.7 us here against 17.5 on the general kernel).  Small calls in rows of up to 100256 tokens meet the
-    // general kernel earlier: a list of a thousand tokens takes one to sixteen such rows 21-27 us here
-    // against 18-21 there (lists of a few hundred: 12-14 us here).
-    const bool small_call = (uint64_t)p.B * (uint64_t)p.V < (1ull << 20) && p.V < 131072;
-    const uint32_t long_list = small_call ? 768u : max(2048u, (uint32_t)p.V / 20u);
-    if (!FUSED && (p.attempt || p.tell_lists) && total > long_list) tell_policy();
-
-    // gather the tokens, re-based to the row's frame
-    if (!listed)
-        stashed(total, [&](uint32_t i, uint32_t b, uint32_t idx) {
-            if (b < cutrow) b = 0;                                     // plan B: below the complete part; 0 matches nothing
-            t.list[i] = ((uint64_t)b << 32) | idx;
-        });
-    __syncthreads();
-    uint32_t exb = f.bin >> 2;
-    if (subset) {
-        // level 1 again, on the gathered tokens alone
-        for (int b = tid; b < kSB; b += kThreads) s.g[kBin0 + b] = 0;
-        __syncthreads();
-        for (uint32_t i = tid; i < total; i += kThreads) {
-            const uint32_t b = (uint32_t)(t.list[i] >> 32);
-            if (b) atomicAdd(reinterpret_cast<unsigned long long *>(&s.g[b >> 21]), (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
-        }
-        __syncthreads();
-        f = hist_find_level1<false, true>(s, top_k, p.top_p, lane, wave);
-        if (f.bin == 0u) {
-            // even all of them are neither top_k tokens nor top_p of the mass
-            if (FUSED) return false;
-            return slow();
-        }
-        exb = f.bin >> 2;
-    }
-
-    // remaining digits of the threshold, on the gathered tokens
-    uint32_t lo = f.bin << 21, span = (1u << 21) - 1u;
-    for (uint32_t lv = 2; lv <= (uint32_t)kLevels && f.cnt_bin > 1u; ++lv) {
-        const uint32_t dsh = level_shift(lv);
-        lds_hist_zero(s, 128);
-        __syncthreads();
-        for (uint32_t i = tid; i < total; i += kThreads) {
-            const uint32_t b = (uint32_t)(t.list[i] >> 32);
-            if (b - lo <= span) lds_hist_add(s, (b >> dsh) & 127u, b);
-        }
-        __syncthreads();
-        f = hist_find128(s, s.hm, f.cnt_above, f.mass_above, top_k, exb, lane, wave);
-        lo |= f.bin << dsh;
-        span = (1u << dsh) - 1u;
-    }
-    if (span != 0u) {                                    // a single token left in the range: the threshold itself
-        for (uint32_t i = tid; i < total; i += kThreads) {
-            const uint32_t b = (uint32_t)(t.list[i] >> 32);
-            if (b - lo <= span) s.bc32[6] = b;
-        }
-        __syncthreads();
-        lo = s.bc32[6];
-    }
-    const uint32_t thr = lo;
-    if (drawer) {                                        // the row is finished here: this draw is used up
+    // Every live token is kept with its full weight (S = D).  Each slice's mass, moved into the
+    // row's frame, is exact (a bin is dead in the row's frame as a whole or not at all: frames
+    // differ by whole octaves); a scan over the slices finds the one that holds the target, and
+    // only that slice's logits are looked at again.
+    if (drawer) {
         rng_st[2] = rs[2] + 1u;
         if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
     }
-    if (tid == 0) {
-        const Target tg = tie_and_target(p, row, p.inj_u ? 0ull : t.rand64, xmax, D, P, thr, f.cnt_above, f.cnt_bin, f.mass_above, 0u, true);   // rounds = 0: no cluster histogram
-        s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
-    }
-    __syncthreads();
-    const uint64_t w_tie = s.bc64[1];
-    u128 r = s.bc128[0];
-    auto weight = [&](uint32_t b) -> uint64_t { return (b > thr) ? w_of_bits(b) : (b == thr ? w_tie : 0); };
-
-    // inverse CDF in index order: slice, then run of tokens, then token
-    constexpr uint32_t sh_slice = SLICE_LOG2;
-    constexpr uint32_t sh_run = sh_slice - 8;                                  // 256 runs of at most 64 tokens
-    static_assert(SLICE_LOG2 >= 8 && SLICE_LOG2 <= 14, "runs must fit the final all-pairs step");
-    constexpr uint32_t kPairs = 64;
-    const uint64_t *cands = t.small;                                           // what the all-pairs step works on
-    uint32_t nkept = total;
-    if (total <= kPairs) cands = t.list;                                       // the whole list is few enough as it is
-    else {
-    const uint32_t ga = bucket_step(s, t, total, sh_slice, 0u, 0xFFFFFFFFu, r, weight, lane, wave);
-    uint32_t lo_b = ga << sh_slice, len_b = 1u << sh_slice;
-    // the kept tokens of that slice: few enough for the all-pairs step as they are, as a rule;
-    // otherwise the slice is narrowed to one of its 256 runs first
-    auto collect = [&]() {
-        if (tid == 0) t.nsmall = 0;
-        __syncthreads();
-        for (uint32_t i = tid; i < total; i += kThreads) {
-            const uint64_t e = t.list[i];
-            const uint32_t idx = (uint32_t)e;
-            if (idx - lo_b < len_b && weight((uint32_t)(e >> 32))) {
-                const uint32_t o = atomicAdd(&t.nsmall, 1u);
-                if (o < kPairs) t.small[o] = e;
+    u128 mine = 0;
+    if ((uint32_t)tid < G && dl < 41u) {                          // 41 octaves and more below: nothing of the slice is live
+        const uint64_t *sm = v.stash + ((size_t)row * G + tid) * kStashCap;
+        mine = (u128)sm[0] | ((u128)sm[1] << 64);
+        if (dl) {
+            // the slice's lowest 4 dl bins are dead in the row's frame; the rest is a multiple of 2^dl
+            const uint64_t *sh = v.shist + ((size_t)row * G + tid) * kSB;
+            u128 low = 0;
+            for (uint32_t b = 0; b < 4u * dl; ++b) {
+                const uint64_t w = sh[b];
+                if (w) low += pack_mass(w, (kBin0 + b) >> 2);
             }
+            mine = (mine - low) >> dl;
         }
-        __syncthreads();
-        return t.nsmall;
-    };
-    nkept = collect();
-    if (nkept > kPairs) {
-        __syncthreads();                                                       // everyone has read the count
-        const uint32_t gb = bucket_step(s, t, total, sh_run, lo_b, lo_b + len_b, r, weight, lane, wave);
-        lo_b += gb << sh_run; len_b = 1u << sh_run;
-        nkept = collect();
     }
-    }
-    // all pairs: every kept token of the range adds up the weights at or before it in index order;
-    // the four waves take a quarter of the addends each
-    static_assert(kWaves == 4 && offsetof(Lds, cand) % 16 == 0 && sizeof(s.cand) >= 64 * 16 + 4 * 64 * 16, "records and partial sums live in s.cand");
-    const uint32_t ns = min(nkept, kPairs);
-    uint4 *rec = reinterpret_cast<uint4 *>(s.cand);                             // weight (x, y), index (z)
-    u128 *partial = reinterpret_cast<u128 *>(s.cand) + kPairs;
-    uint64_t me = 0, wme = 0;
-    if ((uint32_t)tid < ns) {
-        me = cands[tid];
-        wme = weight((uint32_t)(me >> 32));
-        rec[tid] = make_uint4((uint32_t)wme, (uint32_t)(wme >> 32), (uint32_t)me, 0u);
-    }
+    const u128 r = p.inj_u ? ceil_mul(p.inj_u[row], D) : r_from_bits(t.rand64, D);
+    u128 inc = wave_inclusive_scan(mine);
+    if (lane == kWave - 1) s.q128[wave] = inc;
     __syncthreads();
-    {
-        const uint32_t per = (ns + 3u) >> 2, j0 = (uint32_t)wave * per, j1 = min(ns, j0 + per);
-        const uint32_t mine = (uint32_t)lane < ns ? rec[lane].z : 0u;
-        uint64_t lo32 = 0, hi32 = 0;                                              // halves summed apart: no carries
-#pragma unroll 4
-        for (uint32_t j = j0; j < j1; ++j) {
-            const uint4 o = rec[j];
-            const bool c = o.z <= mine;
-            lo32 += c ? o.x : 0u;
-            hi32 += c ? o.y : 0u;
-        }
-        partial[wave * (int)kPairs + lane] = (u128)lo32 + ((u128)hi32 << 32);
-    }
+    for (int w = 0; w < wave; ++w) inc += s.q128[w];
+    const u128 exc = inc - mine;
+    if (exc < r && r <= inc) { t.bucket = (uint32_t)tid; s.bc128[1] = r - exc; }
     __syncthreads();
-    if ((uint32_t)tid < ns) {
-        const u128 upto = partial[tid] + partial[kPairs + tid] + partial[2 * kPairs + tid] + partial[3 * kPairs + tid];
-        if (upto - wme < r && r <= upto) {
-            p.out[row] = (int32_t)(uint32_t)me;
-            if (p.diag) p.diag[row].index = (int32_t)(uint32_t)me;
-            t.result = (uint32_t)me + 1u;
-        }
-    }
-    return true;
+    const uint32_t g = t.bucket;
+    const u128 r_in = s.bc128[1];
+    __syncthreads();
+    if (p.diag) finish_row_slow<true>(p, s, t, row, xmax, p.inj_u ? 0ull : t.rand64, f.cnt_above + f.cnt_bin);
+    keep_pick<SLICE_LOG2>(p, s, t, row, M, g << SLICE_LOG2, r_in,
+                          [](uint32_t b) -> uint64_t { return b >= kEMinBits ? w_of_bits(b) : 0ull; });
 }
 
-template <int SLICE_LOG2, bool KEEP = false>
-__global__ void __launch_bounds__(kThreads) finish_kernel(const Params p, const StreamView v)
+template <int SLICE_LOG2>
+__global__ void __launch_bounds__(kThreads) keep_finish_kernel(const Params p, const StreamView v)
 {
     __shared__ Lds s;
     __shared__ LdsB t;
-    extern __shared__ __align__(16) unsigned char finish_dyn[];
-    t.list = reinterpret_cast<uint64_t *>(finish_dyn);       // every thread writes the same value (KEEP: no list, not used)
-    finish_row<SLICE_LOG2, false, KEEP>(p, v, s, t, blockIdx.x);
-    if (!KEEP && p.penalties && p.defer_pen == 2) {
-        __syncthreads();
-        pen_patch(p, v, s, blockIdx.x, t.result - 1u, SLICE_LOG2);
-    }
+    keep_finish_row<SLICE_LOG2>(p, v, s, t, blockIdx.x);
 }
-
-
 
 // The streaming pass for calls with penalties too large for the one-launch path: logits and penalties
 // are read once, x = sf((sf(l) - pen) * c) as in the cluster kernel, everything after that is the
@@ -1483,7 +1691,6 @@ template <int R, bool PEN>
 __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, const StreamView v)
 {
     constexpr int kRep = stream_copies<R>();
-    constexpr int kSliceLog2 = R == 16 ? 14 : R == 8 ? 13 : 12;
     static_assert(R == 4 || R == 8 || R == 16, "slices of 4096, 8192 or 16384 tokens");
     __shared__ FusedLds<R, PEN> u;
     const int tid = threadIdx.x;
@@ -1503,6 +1710,14 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
     Slice<R, PEN> sl;
     slice_setup(p, sl, row, part, G);
     RowCtl *rc = sl.rc;
+    // the row's random number, should this workgroup be the one that finishes the row: drawn while the slice is on its way
+    uint64_t drawn = 0;
+    if (tid == kWave && !p.inj_u) {
+        const uint32_t *st = p.rng + (size_t)row * 16;
+        uint32_t o[4];
+        philox4x32_10(st[2], st[3], st[4], st[5], st[0], st[1], o);
+        drawn = ((uint64_t)o[0] << 32) | o[1];
+    }
     const float lmax = slice_load(p, sl);
     const uint32_t key = slice_count_and_stash<R, kThreads, kRep, true>(p, v, u.a, sl.eb, lmax, row, part, sl.base4, sl.nv);
 
@@ -1529,8 +1744,13 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
         // the token list: the cluster rounds' histogram copies, which are not in use while a row is
         // finished from the stashes (no dynamic LDS in this kernel: see rs_sample_ex)
         static_assert(sizeof(s.hr) == 2048 * sizeof(uint64_t), "room for a list of 2048 tokens");
-        t.list = s.hr;
-        const bool done = finish_row<kSliceLog2, true>(p, v, s, t, row);
+        const bool done = finish_row<kThreads, 16, true>(p, v, s, t, s.hr, row, drawn);
+        if (done && tid == kWave && !p.inj_u) {
+            uint32_t *st = p.rng + (size_t)row * 16;     // the row is finished: this draw is used up
+            const uint32_t next = st[2] + 1u;
+            st[2] = next;
+            if (next == 0u) st[3] += 1u;
+        }
         __syncthreads();
         verdict = done && t.result != 0u ? t.result : kVerdictFallback;
         if (tid == 0) a_store(&rc->verdict, verdict);

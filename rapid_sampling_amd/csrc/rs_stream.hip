@@ -5,6 +5,19 @@ namespace rs {
 
 constexpr int kStreamNT = 256;
 
+// The finishing workgroup's size.  Lists of hundreds of tokens (a bounding top_k above 256): 1024 threads (128 rows of
+// 1M with top_k 1024: 10.8 us where 256 threads took 13.7).  Short ones: 256 threads -- a nucleus whose list is not
+// known to be long too (one row of 262144: 7.3 us, with 1024 threads 8.4, the scans then go from one wave to
+// the others by way of LDS) -- asking ahead for the first 64 tokens of 4, 8 or 16 slices per wave, which is 16 instructions
+// per slice whether the row has it or not (64 rows of 19 slices: 7.3 us with 16, 6.5 with 8).
+static void launch_finish(uint32_t B, size_t lds_bytes, hipStream_t st, const Params &p, const StreamView &v)
+{
+    if (p.top_k > 256 && !p.attempt) hipLaunchKernelGGL((finish_kernel<1024, 8>), dim3(B), dim3(finish_threads<1024>()), lds_bytes, st, p, v);
+    else if (v.G <= 16u) hipLaunchKernelGGL((finish_kernel<kThreads, 4>), dim3(B), dim3(finish_threads<kThreads>()), lds_bytes, st, p, v);
+    else if (v.G <= 32u) hipLaunchKernelGGL((finish_kernel<kThreads, 8>), dim3(B), dim3(finish_threads<kThreads>()), lds_bytes, st, p, v);
+    else hipLaunchKernelGGL((finish_kernel<kThreads, 16>), dim3(B), dim3(finish_threads<kThreads>()), lds_bytes, st, p, v);
+}
+
 hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p,
                          const StreamView &v)
 {
@@ -18,7 +31,8 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
         if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F32, KEEPv>), sgrid, dim3(NTv), 0, st, p, v);       \
         else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_BF16, KEEPv>), sgrid, dim3(NTv), 0, st, p, v); \
         else hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F16, KEEPv>), sgrid, dim3(NTv), 0, st, p, v);                             \
-        hipLaunchKernelGGL((finish_kernel<Lv, KEEPv>), dim3(B), dim3(kThreads), KEEPv ? 0 : finish_lds_bytes, st, p, v); } while (0)
+        if (KEEPv) hipLaunchKernelGGL((keep_finish_kernel<Lv>), dim3(B), dim3(kThreads), 0, st, p, v);                                    \
+        else launch_finish(B, finish_lds_bytes, st, p, v); } while (0)
     if (slice_r == 4) { if (keep) RS_STREAM(4, 256, 12, true); else RS_STREAM(4, 256, 12, false); }
     else if (slice_r == 8) { if (keep) RS_STREAM(8, 256, 13, true); else RS_STREAM(8, 256, 13, false); }
     else { if (keep) RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, true); else RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, false); }
@@ -29,7 +43,7 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
 hipError_t launch_stream_pen(uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v)
 {
     hipLaunchKernelGGL((stream_pen_kernel<kStreamLongR>), dim3(B * v.G), dim3(kThreads), 0, st, p, v);
-    hipLaunchKernelGGL((finish_kernel<kStreamLongLog2>), dim3(B), dim3(kThreads), finish_lds_bytes, st, p, v);
+    launch_finish(B, finish_lds_bytes, st, p, v);
     return hipGetLastError();
 }
 

@@ -1686,3 +1686,19 @@ def test_chi_square_one_million_draws(torch_cuda, oracle):
     chi2, pval = stats.chisquare(counts[keep], n * w[keep] / w.sum())
     print("chi2", chi2, "dof", keep.sum() - 1, "p", pval)
     assert pval > 0.01
+
+
+@pytest.mark.parametrize("V", [65536, 65540, 131072, 131076, 262144, 262148])
+def test_finish_at_the_edges_of_its_variants(torch_cuda, oracle, V):
+    """The streaming finish asks ahead for the first tokens of 16, 32 or 64 slices (rows of that many slices and of
+    one more), takes lists of up to 64 tokens by pairs and longer ones by digits, and has 1024 threads from
+    a top_k of 257 on: rows of distinct values, of ties at the threshold and a row with few live tokens, lists
+    just below and above each bound, every path against the oracle in every field (integers: equal)."""
+    from tests import capi
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal((4, V)) * 1.5).astype(np.float32)
+    lg[1] = np.round(lg[1] * 64) / 64
+    lg[2, V // 3:] = -np.inf
+    lg[3] -= 200.0 * (rng.random(V) < 1.0 - 40.0 / V)
+    for (k, p) in [(1, 1.0), (40, 0.95), (63, 1.0), (66, 1.0), (256, 0.999), (257, 1.0)]:
+        _run_case(torch_cuda, oracle, capi, lg, 1.0, k, p, u_np=H.uniforms(4, k), what="finish edges V=%d k=%d" % (V, k))
