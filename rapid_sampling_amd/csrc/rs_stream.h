@@ -136,7 +136,8 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
         }
         return w;
     };
-    if (tid < kSB) {
+    const bool plain = KEEP && p.report == 0u;           // (not the first pass of the two-pass wide path)
+    if (!plain && tid < kSB) {
         const uint64_t w = bin_total(tid);
         const float mm = M - 128.0f * __builtin_floorf(M * 0.0078125f);          // M mod 128, exact
         put<FUSED>(&v.shist[((size_t)row * G + part) * kSB + tid], w);          // kept for rows whose slices lie far apart
@@ -144,20 +145,22 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
         if (w) a_add(&rowbins[((uint32_t)(int)mm * 4u + (uint32_t)tid - 160u) & 511u], w);
     }
     if constexpr (KEEP) {
-        // every live token is kept: the bins and their mass (in this slice's frame, left where the
-        // stash would begin) are all the finishing workgroup needs of this slice
-        if (wave == 0) {
-            u128 ms = 0;
+        // every live token is kept: what the finishing workgroup needs of this slice is its mass in the row's frame, which
+        // may lie d octaves above this one's and leaves the lowest 4 d bins dead: the mass of the bins from 4 d on, for
+        // every d, left where the stash would begin
+        if (plain && wave == 0) {
+            BinScan<3> sc;
+            auto at = [&](int i) { return kSB - 1 - 3 * lane - i; };
+            sc.load([&](int i) { return at(i) >= 0 ? bin_total(max(at(i), 0)) : 0ull; }, [&](int i) { return (kBin0 + (uint32_t)max(at(i), 0)) >> 2; });
+            uint64_t *st = v.stash + ((size_t)row * G + part) * kStashCap;
+            Limbs from = sc.mb;
 #pragma unroll
             for (int i = 0; i < 3; ++i) {
-                const int b = kSB - 1 - 3 * lane - i;
-                const uint64_t w = b >= 0 ? bin_total(b) : 0ull;
-                if (w) ms += pack_mass(w, (kBin0 + (uint32_t)b) >> 2);
-            }
-            const u128 tot = wave_inclusive_scan(ms);
-            if (lane == kWave - 1) {
-                uint64_t *st = v.stash + ((size_t)row * G + part) * kStashCap;
-                st[0] = (uint64_t)tot; st[1] = (uint64_t)(tot >> 64);
+                from = from + sc.m[i];
+                if (at(i) >= 0 && (at(i) & 3) == 0) {
+                    const M96 q = m96(from);
+                    reinterpret_cast<uint4 *>(st)[at(i) >> 2] = make_uint4((uint32_t)q.lo, (uint32_t)(q.lo >> 32), q.hi, 0u);
+                }
             }
         }
         if (tid == 0) {
@@ -393,14 +396,7 @@ struct LdsB {
 // by token.  A few passes of one workgroup over one row take tens of microseconds (a row of a
 // million tokens: more than a hundred): fine for the odd row, and calls whose rows mostly end here
 // are routed to the cluster kernel by the caller's policy.  Same integers as every other path.
-//
-// KEEP_DIAG: the call keeps every live token (top_k = V, top_p = 1) and its token is picked from the
-// slices' masses (keep_pick); what is left to do here is the diagnostics record, which names the
-// threshold -- the smallest live token of the row -- and how many tokens tie there: one pass over
-// the row, paid by callers that ask for the record (tests, mostly).  keep_live: live tokens of the row.
-template <bool KEEP_DIAG = false>
-__device__ __forceinline__ void finish_row_slow(const Params &p, Lds &s, LdsB &t, const uint32_t row, const float xmax, const uint64_t rand64,
-                                                const uint32_t keep_live = 0u)
+__device__ __forceinline__ void finish_row_slow(const Params &p, Lds &s, LdsB &t, const uint32_t row, const float xmax, const uint64_t rand64)
 {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     const uint32_t V4 = (uint32_t)p.V >> 2;
@@ -439,36 +435,6 @@ __device__ __forceinline__ void finish_row_slow(const Params &p, Lds &s, LdsB &t
         }
     };
     const uint64_t top_k = (uint64_t)p.top_k;
-    if constexpr (KEEP_DIAG) {
-        uint32_t mn = 0xFFFFFFFFu, cnt = 0u;
-        row_pass(0u, V4, [&](uint32_t, uint32_t b) {
-            if (b >= kEMinBits) {
-                if (b < mn) { mn = b; cnt = 1u; }
-                else if (b == mn) ++cnt;
-            }
-        });
-        const uint32_t wm = ~wave_max_u32(~mn);
-        __syncthreads();
-        if (lane == 0) s.u32[wave] = wm;
-        __syncthreads();
-        uint32_t bm = s.u32[0];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) bm = min(bm, s.u32[w]);
-        const uint32_t ci = wave_inclusive_scan(mn == bm ? cnt : 0u);
-        __syncthreads();
-        if (lane == kWave - 1) s.u32[wave] = ci;
-        __syncthreads();
-        if (tid == 0) {
-            uint32_t n_eq = 0;
-#pragma unroll
-            for (int w = 0; w < kWaves; ++w) n_eq += s.u32[w];
-            const u128 D = s.D;
-            tie_and_target(p, row, rand64, xmax, D, s.P, bm, keep_live - n_eq, n_eq, D - (u128)n_eq * w_of_bits(bm), 9u, true);
-        }
-        __syncthreads();
-        return;
-    }
-
     // level 1 (dead tokens, below 2^-40, are left out)
     __syncthreads();
     for (int b = tid; b < kNB * kRepC; b += kThreads) s.hr[b] = 0;
@@ -1311,172 +1277,197 @@ __global__ void __launch_bounds__(finish_threads<NT>()) finish_kernel(const Para
     }
 }
 
-// The finish of a call that keeps every live token (top_k = V, top_p = 1; the counting-only pass left the
-// slices' masses where their stashes would begin).
-template <int SLICE_LOG2>
-__device__ __forceinline__ void keep_finish_row(const Params &p, const StreamView &v, Lds &s, LdsB &t, const uint32_t row)
+// ---- calls that keep every live token (top_k = V, top_p = 1): one workgroup per row behind the counting-only pass ----
+// The pass left, per slice, its mass without its lowest 4 d bins for every d (41 sums): a slice whose frame lies d
+// octaves below the row's has just those bins dead in the row's frame, and what is left is a multiple of 2^d.  So
+// the row's total and the slice that holds the target come from one load and one scan per wave -- every wave does
+// them for itself -- and only that slice's logits are looked at again.
+//
+// What bounds it: the length of the chain (headers -> target -> slice -> token), two trips to memory of a
+// microsecond each.  The slice comes in coalesced and goes through LDS, so that every thread then owns consecutive
+// tokens: one sum per thread, one scan over the workgroup, and one wave finds the token among the owner's T.
+// (Chunks of 256 consecutive tokens summed wave by wave, two 64-bit wave sums each, behind the general finish's bins and
+// boundary: 16.1 us for 512 rows of 50304 tokens; this way 10.8, of which some 5 are the 16 MB of slices.)
+constexpr int kKeepT = 512;                              // threads that look at the slice; one more wave draws the random number
+template <int LOG2>
+struct LdsK {
+    static constexpr int U = (1 << LOG2) / 4 / kKeepT;   // float4 groups per thread
+    float4   x[kKeepT * U + kKeepT];                     // group g of the slice at g + g / U: threads read their U groups an odd number of groups apart
+    M96      waves[kKeepT / kWave];
+    uint64_t rand64;
+    uint32_t u32[kKeepT / kWave];
+};
+
+// The diagnostics record of such a call names the threshold -- the smallest live token of the row -- and how many
+// tokens tie there: one pass over the row, paid by callers that ask for the record (tests, mostly).
+template <typename L>
+__device__ __forceinline__ void keep_diag(const Params &p, L &s, const uint32_t row, const float xmax, const M96 D, const uint64_t rand64)
 {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
-    const uint32_t G = v.G;
-    const PartHdr *hdrs = v.hdr + (size_t)row * G;
-    uint64_t *rowhist = (p.ctl_end - 1 - row)->rowhist;
-
-    if (tid == 0) { s.abort = 0; s.host_words = p.host_words; t.fail = 0; t.result = 0u; }
-    PartHdr ph;
-    ph.mkey = 0; ph.cov = 0; ph.n = 0; ph.cut = 0;
-    if ((uint32_t)tid < G) ph = hdrs[tid];
-    const uint64_t h0 = rowhist[tid], h1 = rowhist[tid + kThreads];
-    // the first lane of wave 1 draws the row's random number while wave 0 scans the histogram;
-    // the state is advanced only once the row is certain to be finished here
-    const bool drawer = tid == kWave && !p.inj_u;
-    uint32_t *rng_st = p.rng + (size_t)row * 16;
-    uint32_t rs[6] = {0u, 0u, 0u, 0u, 0u, 0u};
-    if (drawer) {
-#pragma unroll
-        for (int i = 0; i < 6; ++i) rs[i] = rng_st[i];
-    }
-    rowhist[tid] = 0; rowhist[tid + kThreads] = 0;       // left clean for the next call
-    uint32_t kmax, kmin;
-    {
-        const uint32_t a = wave_max_u32(ph.mkey), b = wave_max_u32((uint32_t)tid < G ? ~ph.mkey : 0u);
-        if (lane == 0) { s.u32[wave] = a; s.u32[kWaves + wave] = b; }
-        __syncthreads();
-        kmax = s.u32[0]; kmin = s.u32[kWaves];
-#pragma unroll
-        for (int w = 1; w < kWaves; ++w) { kmax = max(kmax, s.u32[w]); kmin = max(kmin, s.u32[kWaves + w]); }
-        kmin = ~kmin;
-    }
-    const float xmax = fkey_inv(kmax);
     const float M = __builtin_floorf(xmax);
-    // frames further apart than this may have put different octaves into one bin
-    const bool mixed = !(M - __builtin_floorf(fkey_inv(kmin)) < 88.0f);
-    uint32_t dl = 0;
-    if ((uint32_t)tid < G) {
-        const float d = M - __builtin_floorf(fkey_inv(ph.mkey));      // >= 0, a whole number or huge
-        dl = d >= 64.0f ? 64u : (uint32_t)d;
-        t.delta[tid] = dl;
-        const float Mg = __builtin_floorf(fkey_inv(ph.mkey));
-        t.m4[tid] = (uint32_t)(int)(Mg - 128.0f * __builtin_floorf(Mg * 0.0078125f)) * 4u;
-    }
-    // the row's level-1 histogram in the row's frame: bin r (octave M - 40 + r/4) sits at absolute
-    // position 4 (M mod 128) + r - 160; the other 348 positions hold tokens below 2^-40 of this
-    // frame, which are dead there: dropped
-    {
-        const float mm = M - 128.0f * __builtin_floorf(M * 0.0078125f);
-        const uint32_t m4 = (uint32_t)(int)mm * 4u;
-        const uint32_t r0 = ((uint32_t)tid + 160u - m4) & 511u, r1 = ((uint32_t)tid + kThreads + 160u - m4) & 511u;
-        if (r0 < (uint32_t)kSB) s.g[kBin0 + r0] = h0;
-        if (r1 < (uint32_t)kSB) s.g[kBin0 + r1] = h1;
-        for (int b = tid; b < (int)kBin0; b += kThreads) s.g[b] = 0;
+    const char *lrow = logits_row(p, row);
+    auto each = [&](auto fn) {
+        for (uint32_t i4 = (uint32_t)tid; i4 < (uint32_t)p.V >> 2; i4 += kKeepT) {
+            const float4 l = load_logits4(lrow, i4, p.dtype);
+            fn(e_bits_of(sf(l.x * p.c), M)); fn(e_bits_of(sf(l.y * p.c), M)); fn(e_bits_of(sf(l.z * p.c), M)); fn(e_bits_of(sf(l.w * p.c), M));
+        }
+    };
+    auto over_waves = [&](uint32_t v, bool sum) {        // sum or minimum over the workgroup
+        v = sum ? wave_sum(v) : ~wave_max_u32(~v);
         __syncthreads();
-        if (mixed) {
-            // Slices whose maxima lie 88 octaves or more apart may have put different octaves into
-            // one position.  Every token of a slice 41 octaves or more below the row's frame is
-            // dead there, whatever its bin: what such a slice added is taken out again, bin by bin
-            // (its own bins are on record).  The slices that remain lie within 40 octaves of each
-            // other.
-            for (uint32_t i = (uint32_t)tid; i < G * (uint32_t)kSB; i += kThreads) {
-                const uint32_t g = i / (uint32_t)kSB, r = i - g * (uint32_t)kSB;
-                if (t.delta[g] >= 41u) {
-                    const uint64_t w = v.shist[((size_t)row * G + g) * kSB + r];
-                    if (w) {
-                        const uint32_t rr = (t.m4[g] + r - m4) & 511u;
-                        if (rr < (uint32_t)kSB)
-                            atomicAdd(reinterpret_cast<unsigned long long *>(&s.g[kBin0 + rr]), 0ull - (unsigned long long)w);
-                    }
-                }
+        if (lane == 0) s.u32[wave] = v;
+        __syncthreads();
+        uint32_t r = s.u32[0];
+        for (int w = 1; w < kKeepT / kWave; ++w) r = sum ? r + s.u32[w] : min(r, s.u32[w]);
+        return r;
+    };
+    uint32_t mn = 0xFFFFFFFFu, n_live = 0, n_eq = 0;
+    each([&](uint32_t b) { if (b >= kEMinBits) { mn = min(mn, b); ++n_live; } });
+    mn = over_waves(mn, false);
+    each([&](uint32_t b) { if (b == mn) ++n_eq; });
+    n_live = over_waves(n_live, true); n_eq = over_waves(n_eq, true);
+    if (tid == 0)
+        tie_and_target(p, row, rand64, xmax, wide(D), wide(D), mn, n_live - n_eq, n_eq, wide(D) - (u128)n_eq * w_of_bits(mn), 9u, true);
+}
+
+template <int LOG2>
+__global__ void __launch_bounds__(kKeepT + kWave) keep_finish_kernel(const Params p, const StreamView v)
+{
+    __shared__ LdsK<LOG2> s;
+    constexpr int U = LdsK<LOG2>::U, T = 4 * U;          // groups and tokens per thread
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = (int)uniform((uint32_t)tid >> 6);
+    const uint32_t row = blockIdx.x, G = v.G, V4 = (uint32_t)p.V >> 2;
+    if (wave == kKeepT / kWave) {
+        if (!p.inj_u) {
+            uint32_t *st = p.rng + (size_t)row * 16, rs[6], o[4];
+#pragma unroll
+            for (int i = 0; i < 6; ++i) rs[i] = st[i];
+            philox4x32_10(rs[2], rs[3], rs[4], rs[5], rs[0], rs[1], o);
+            if (lane == 0) {
+                s.rand64 = ((uint64_t)o[0] << 32) | o[1];
+                st[2] = rs[2] + 1u;
+                if (rs[2] + 1u == 0u) st[3] = rs[3] + 1u;
             }
         }
+        __syncthreads();
+        return;
     }
+
+    // the slices' masses in the row's frame: lane l holds slice l, or slices 2l and 2l + 1 of a row of more than 64
+    constexpr int kAhead = 4;                            // sums asked for before the frames are known: slices up to 3 octaves below the row's
+    const PartHdr *hdrs = v.hdr + (size_t)row * G;
+    const uint64_t *sums = v.stash + (size_t)row * G * kStashCap;
+    const uint32_t per = G > (uint32_t)kWave ? 2u : 1u;
+    uint32_t key[2];
+    uint4 ahead[2][kAhead];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t g = min((uint32_t)lane * per + (uint32_t)k, G - 1u);
+        key[k] = hdrs[g].mkey;
+        const uint4 *q = reinterpret_cast<const uint4 *>(sums + (size_t)g * kStashCap);
+#pragma unroll
+        for (int d = 0; d < kAhead; ++d) ahead[k][d] = q[d];
+    }
+    const float xmax = fkey_inv(wave_max_u32(max(key[0], key[1])));
+    const float M = __builtin_floorf(xmax);
+    M96 mass[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        const uint32_t g = (uint32_t)lane * per + (uint32_t)k;
+        const float df = M - __builtin_floorf(fkey_inv(key[k]));
+        const uint32_t d = df >= 64.0f ? 64u : (uint32_t)df;
+        uint4 q = ahead[k][0];
+#pragma unroll
+        for (int i = 1; i < kAhead; ++i)
+            if (d == (uint32_t)i) q = ahead[k][i];
+        if (d >= (uint32_t)kAhead && d <= 40u) q = reinterpret_cast<const uint4 *>(sums + (size_t)min(g, G - 1u) * kStashCap)[d];
+        const uint64_t lo = ((uint64_t)q.y << 32) | q.x, hi = q.z;
+        mass[k] = M96{d == 0u ? lo : (lo >> (d & 63u)) | (hi << ((64u - d) & 63u)), (uint32_t)(hi >> (d & 63u))};
+        if (d > 40u || (uint32_t)k >= per || g >= G) mass[k] = M96{0ull, 0u};        // 41 octaves and more below: nothing of the slice is live
+    }
+    const Limbs both = limbs(mass[0] + mass[1]), upto = wave_inclusive_scan(both);
+    const M96 D = m96(lane_of(upto, 63u));
     __syncthreads();
-    if (p.e_bits) {
+    const uint64_t rand64 = uniform(s.rand64);
+    const M96 r = p.inj_u ? m96(ceil_mul(p.inj_u[row], wide(D))) : m96(r_from_bits(rand64, wide(D)));
+    uint32_t g;
+    M96 r_in;
+    {
+        const M96 inc = m96(upto), exc = m96(upto - both);
+        const uint32_t l = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(inc >= r));         // 1 <= r <= D: there is one
+        r_in = r - lane_of(exc, l);
+        g = l * per;
+        const M96 first = lane_of(mass[0], l);
+        if (!(first >= r_in)) { r_in = r_in - first; g += 1u; }
+    }
+    if (__builtin_expect(p.e_bits != nullptr, 0)) {
         // diagnostics: the slices' e into the row's frame, dead tokens as 0
         uint4 *eb4 = reinterpret_cast<uint4 *>(p.e_bits + (int64_t)row * p.V);
         auto fix = [&](uint32_t b, uint32_t d) { b = rebase_bits(min(b, 0x3FFFFFFFu), d); return b < kEMinBits ? 0u : b; };
-        for (uint32_t i4 = (uint32_t)tid; i4 < ((uint32_t)p.V >> 2); i4 += kThreads) {
-            const uint32_t d = t.delta[i4 >> (SLICE_LOG2 - 2)];
+        for (uint32_t i4 = (uint32_t)tid; i4 < V4; i4 += kKeepT) {
+            const float df = M - __builtin_floorf(fkey_inv(hdrs[i4 >> (LOG2 - 2)].mkey));
+            const uint32_t d = df >= 64.0f ? 64u : (uint32_t)df;
             uint4 q = eb4[i4];
             q.x = fix(q.x, d); q.y = fix(q.y, d); q.z = fix(q.z, d); q.w = fix(q.w, d);
             eb4[i4] = q;
         }
     }
-    if (drawer) {
-        uint32_t o[4];
-        philox4x32_10(rs[2], rs[3], rs[4], rs[5], rs[0], rs[1], o);
-        t.rand64 = ((uint64_t)o[0] << 32) | o[1];
-    }
-    const uint64_t top_k = (uint64_t)p.top_k;
-    Found f = hist_find_level1<false>(s, top_k, p.top_p, lane, wave);
-    const u128 D = s.D, P = s.P;
-    // A row that is one tie of all its tokens (rows of equal logits) needs no stash at all: the
-    // threshold is the largest token's value, every token weighs the tie weight, and the token at
-    // which the running sum reaches r follows by division.
-    if (f.cnt_bin == (uint32_t)p.V && bin_is_one_tie(s.g[f.bin], f.bin, e_bits_of(xmax, M))) {
-        if (drawer) {
-            rng_st[2] = rs[2] + 1u;
-            if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
-        }
-        if (tid == 0) {
-            const uint32_t thr1 = e_bits_of(xmax, M);
-            const Target tg = tie_and_target(p, row, p.inj_u ? 0ull : t.rand64, xmax, D, P, thr1, 0u, f.cnt_bin, (u128)0, 0u, true);
-            // smallest i with (i + 1) * w_tie >= r; r <= V * w_tie
-            uint32_t lo_i = 0, hi_i = (uint32_t)p.V - 1u;
-            while (lo_i < hi_i) {
-                const uint32_t mid = (lo_i + hi_i) >> 1;
-                if ((u128)(mid + 1u) * tg.w_tie >= tg.r) hi_i = mid; else lo_i = mid + 1u;
-            }
-            p.out[row] = (int32_t)lo_i;
-            if (p.diag) p.diag[row].index = (int32_t)lo_i;
-            t.result = lo_i + 1u;
-        }
-        return;
-    }
+    if (__builtin_expect(p.diag != nullptr, 0)) keep_diag(p, s, row, xmax, D, rand64);
 
-    // Every live token is kept with its full weight (S = D).  Each slice's mass, moved into the
-    // row's frame, is exact (a bin is dead in the row's frame as a whole or not at all: frames
-    // differ by whole octaves); a scan over the slices finds the one that holds the target, and
-    // only that slice's logits are looked at again.
-    if (drawer) {
-        rng_st[2] = rs[2] + 1u;
-        if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
-    }
-    u128 mine = 0;
-    if ((uint32_t)tid < G && dl < 41u) {                          // 41 octaves and more below: nothing of the slice is live
-        const uint64_t *sm = v.stash + ((size_t)row * G + tid) * kStashCap;
-        mine = (u128)sm[0] | ((u128)sm[1] << 64);
-        if (dl) {
-            // the slice's lowest 4 dl bins are dead in the row's frame; the rest is a multiple of 2^dl
-            const uint64_t *sh = v.shist + ((size_t)row * G + tid) * kSB;
-            u128 low = 0;
-            for (uint32_t b = 0; b < 4u * dl; ++b) {
-                const uint64_t w = sh[b];
-                if (w) low += pack_mass(w, (kBin0 + b) >> 2);
-            }
-            mine = (mine - low) >> dl;
+    // that slice's tokens, through LDS
+    const uint32_t g0 = g << (LOG2 - 2);
+    const char *lrow = logits_row(p, row);
+    {
+        float4 l[U];
+#pragma unroll
+        for (int j = 0; j < U; ++j) l[j] = load_logits4(lrow, min(g0 + (uint32_t)(j * kKeepT + tid), V4 - 1u), p.dtype);
+#pragma unroll
+        for (int j = 0; j < U; ++j) {
+            const uint32_t at = (uint32_t)(j * kKeepT + tid);
+            s.x[at + at / (uint32_t)U] = make_float4(sf(l[j].x * p.c), sf(l[j].y * p.c), sf(l[j].z * p.c), sf(l[j].w * p.c));
         }
     }
-    const u128 r = p.inj_u ? ceil_mul(p.inj_u[row], D) : r_from_bits(t.rand64, D);
-    u128 inc = wave_inclusive_scan(mine);
-    if (lane == kWave - 1) s.q128[wave] = inc;
     __syncthreads();
-    for (int w = 0; w < wave; ++w) inc += s.q128[w];
-    const u128 exc = inc - mine;
-    if (exc < r && r <= inc) { t.bucket = (uint32_t)tid; s.bc128[1] = r - exc; }
+    auto weight = [&](float x) -> uint64_t {
+        const uint32_t b = e_bits_of(x, M);
+        return b >= kEMinBits ? w_of_bits(b) : 0ull;
+    };
+    uint64_t lo = 0, hi = 0;                             // halves summed apart: T * 2^32 at most
+#pragma unroll
+    for (int j = 0; j < U; ++j)
+        if (g0 + (uint32_t)(tid * U + j) < V4) {         // past the end of the row: no weight
+            const float4 x = s.x[tid * U + j + tid];
+            const uint64_t w0 = weight(x.x), w1 = weight(x.y), w2 = weight(x.z), w3 = weight(x.w);
+            lo += (w0 & 0xFFFFFFFFull) + (w1 & 0xFFFFFFFFull) + (w2 & 0xFFFFFFFFull) + (w3 & 0xFFFFFFFFull);
+            hi += (w0 >> 32) + (w1 >> 32) + (w2 >> 32) + (w3 >> 32);
+        }
+    const Limbs mine = limbs(m96((u128)lo + ((u128)hi << 32))), run = wave_inclusive_scan(mine);
+    M96 inc = m96(run);
+    if (lane == kWave - 1) s.waves[wave] = inc;
     __syncthreads();
-    const uint32_t g = t.bucket;
-    const u128 r_in = s.bc128[1];
-    __syncthreads();
-    if (p.diag) finish_row_slow<true>(p, s, t, row, xmax, p.inj_u ? 0ull : t.rand64, f.cnt_above + f.cnt_bin);
-    keep_pick<SLICE_LOG2>(p, s, t, row, M, g << SLICE_LOG2, r_in,
-                          [](uint32_t b) -> uint64_t { return b >= kEMinBits ? w_of_bits(b) : 0ull; });
-}
-
-template <int SLICE_LOG2>
-__global__ void __launch_bounds__(kThreads) keep_finish_kernel(const Params p, const StreamView v)
-{
-    __shared__ Lds s;
-    __shared__ LdsB t;
-    keep_finish_row<SLICE_LOG2>(p, v, s, t, blockIdx.x);
+    if (wave) {
+        const Limbs before = wave_inclusive_scan(limbs(lane < wave ? s.waves[lane] : M96{0ull, 0u}));
+        inc = inc + m96(lane_of(before, 63u));
+    }
+    const M96 exc = inc - m96(mine);
+    const uint64_t vote = __builtin_amdgcn_ballot_w64(exc < r_in && inc >= r_in);
+    if (vote == 0ull) return;                            // another wave's thread owns the target
+    const uint32_t o = (uint32_t)__builtin_ctzll(vote), t0 = (uint32_t)(wave * kWave) + o;
+    const M96 r2 = r_in - lane_of(exc, o);
+    const uint32_t at = t0 * (uint32_t)U + ((uint32_t)lane >> 2);
+    uint64_t w = 0;
+    if (lane < T && g0 + at < V4) {
+        const float4 q = s.x[at + t0];
+        const uint32_t c = (uint32_t)lane & 3u;
+        w = weight(c == 0u ? q.x : c == 1u ? q.y : c == 2u ? q.z : q.w);
+    }
+    const Limbs one = limbs(M96{w, 0u}), sofar = wave_inclusive_scan(one);
+    if (m96(sofar - one) < r2 && m96(sofar) >= r2) {
+        const int32_t pick = (int32_t)((g0 + at) * 4u + ((uint32_t)lane & 3u));
+        p.out[row] = pick;
+        if (p.diag) p.diag[row].index = pick;
+    }
 }
 
 // The streaming pass for calls with penalties too large for the one-launch path: logits and penalties

@@ -22,6 +22,7 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
                          const StreamView &v)
 {
     const dim3 sgrid(B * v.G);
+    if (keep && v.G > 2u * kWave) return hipErrorInvalidValue;             // keep_finish_kernel holds two slices per lane
     // keep: the call keeps every live token; its kernels neither fill nor read stashes, and the finish needs no list.
     // NTv threads with Rv groups of four tokens each: a slice of 4 Rv NTv tokens
 #ifndef RS_LONG_NT
@@ -31,7 +32,7 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
         if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F32, KEEPv>), sgrid, dim3(NTv), 0, st, p, v);       \
         else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_BF16, KEEPv>), sgrid, dim3(NTv), 0, st, p, v); \
         else hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F16, KEEPv>), sgrid, dim3(NTv), 0, st, p, v);                             \
-        if (KEEPv) hipLaunchKernelGGL((keep_finish_kernel<Lv>), dim3(B), dim3(kThreads), 0, st, p, v);                                    \
+        if (KEEPv) hipLaunchKernelGGL((keep_finish_kernel<Lv>), dim3(B), dim3(kKeepT + kWave), 0, st, p, v);                              \
         else launch_finish(B, finish_lds_bytes, st, p, v); } while (0)
     if (slice_r == 4) { if (keep) RS_STREAM(4, 256, 12, true); else RS_STREAM(4, 256, 12, false); }
     else if (slice_r == 8) { if (keep) RS_STREAM(8, 256, 13, true); else RS_STREAM(8, 256, 13, false); }
