@@ -145,12 +145,13 @@ __global__ void __launch_bounds__(kRowT) row_kernel(const Params p)
     const float M = __builtin_floorf(xmax);
 
     // e (not clamped at 2^-40: what lies below is dead and lands in bins nobody looks at) and level 1
+    const Frame fr = frame_of(M, eb);
 #pragma unroll
     for (int j = 0; j < kRowR; ++j) {
         if (g0 + (uint32_t)(j * kWave) < g_end) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const uint32_t b = e_bits_raw(__uint_as_float(eb[j * 4 + q]), M);
+                const uint32_t b = fr.raw(__uint_as_float(eb[j * 4 + q]));
                 eb[j * 4 + q] = b;
                 atomicAdd(reinterpret_cast<unsigned long long *>(&L.hr8[(b >> 21) * 8u + (uint32_t)(lane & 7)]),
                           (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));

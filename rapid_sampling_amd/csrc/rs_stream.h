@@ -96,12 +96,13 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
 
     // e in the slice's frame, not yet clamped at 2^-40, and its histogram; slots past the end of
     // the row become 0
+    const Frame fr = frame_of(M, eb);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         if (j < nv) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const uint32_t b = e_bits_raw(__uint_as_float(eb[j * 4 + q]), M);
+                const uint32_t b = fr.raw(__uint_as_float(eb[j * 4 + q]));
                 eb[j * 4 + q] = b;
                 atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * kRep + (lane & (kRep - 1))]),
                           (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));

@@ -117,12 +117,13 @@ __global__ void __launch_bounds__(kW1SampleT) wide_sample_kernel(const Params p,
     static_assert(kW1SampleT / kWave <= 16, "LdsS::u32");
     const float M = __builtin_floorf(fkey_inv(kmax));
     // e in the sample's frame; live tokens into the histogram
+    const Frame frm = frame_of(M, eb);
 #pragma unroll
     for (int j = 0; j < kW1SampleR; ++j) {
         const bool in = (uint32_t)tid + (uint32_t)j * kThreads < ng;
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const uint32_t b = in ? e_bits_raw(__uint_as_float(eb[j * 4 + q]), M) : 0u;
+            const uint32_t b = in ? frm.raw(__uint_as_float(eb[j * 4 + q])) : 0u;
             eb[j * 4 + q] = b;
             if (b >= kEMinBits)
                 atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * 8u + (uint32_t)(lane & 7)]),
@@ -331,12 +332,13 @@ __global__ void __launch_bounds__(kThreads, (R <= 8 ? 5 : RS_STREAM_WAVES)) wide
     // address is selected, nothing is branched on (a conditional per token keeps the compiler from
     // interleaving the tokens' polynomials and is issued whenever some lane of the wave takes it).  Slots
     // past the end of the row become 0.
+    const Frame frm = frame_of(M, eb);
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         if (j < nv) {
 #pragma unroll
             for (int q = 0; q < 4; ++q) {
-                const uint32_t b = e_bits_raw(__uint_as_float(eb[j * 4 + q]), M);
+                const uint32_t b = frm.raw(__uint_as_float(eb[j * 4 + q]));
                 eb[j * 4 + q] = b;
                 uint64_t *bin = &s.hm[(b >> 21) * kRep + (lane & (kRep - 1))];
                 uint64_t *sub = &s.sub[(((b - lo_bits) >> sh) & 127u) * kW1Rep + (lane & (kW1Rep - 1))];

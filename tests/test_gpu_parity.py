@@ -1702,3 +1702,25 @@ def test_finish_at_the_edges_of_its_variants(torch_cuda, oracle, V):
     lg[3] -= 200.0 * (rng.random(V) < 1.0 - 40.0 / V)
     for (k, p) in [(1, 1.0), (40, 0.95), (63, 1.0), (66, 1.0), (256, 0.999), (257, 1.0)]:
         _run_case(torch_cuda, oracle, capi, lg, 1.0, k, p, u_np=H.uniforms(4, k), what="finish edges V=%d k=%d" % (V, k))
+
+
+@pytest.mark.parametrize("V", [256, 20484, 131076])
+def test_frames_near_zero_and_far_from_it(torch_cuda, oracle, V):
+    """e with the frame in the polynomial's coefficients (|M| <= 100) and with the frame taken off the tokens first:
+    rows on both sides of +-100, thousands and 10^9 away, of the largest floats there are, of slices in frames of
+    both kinds, of values just below a whole number (where a token less its floor rounds to 1) and of subnormals."""
+    from tests import capi
+    rng = np.random.default_rng(V)
+    lg = np.zeros((12, V), dtype=np.float32)
+    for b, off in enumerate([0.0, 98.5, 101.5, -99.0, -103.0, 5000.0, -5000.0, 1e9]):
+        lg[b] = (rng.standard_normal(V) * 2.0 + off).astype(np.float32)
+    lg[8] = np.where(rng.random(V) < 0.5, np.float32(3.0e38), np.float32(-3.0e38))
+    lg[9] = (-np.exp2(-rng.uniform(20, 149, V))).astype(np.float32)
+    lg[9, ::7] *= -1
+    lg[10] = np.nextafter(rng.integers(-30, 3, V).astype(np.float32), np.float32(-1e9))
+    lg[11] = (rng.standard_normal(V)).astype(np.float32)
+    lg[11, : V // 2] -= 150.0
+    lg[11, :3] = -np.inf
+    # log2(e) / T = 1 up to rounding: x is the logit
+    for (temp, k, p) in [(1.4426950408889634, 40, 0.95), (1.4426950408889634, -1, 0.7)]:
+        _run_case(torch_cuda, oracle, capi, lg, temp, k, p, u_np=H.uniforms(12, 71), what="frames V=%d k=%d" % (V, k))
