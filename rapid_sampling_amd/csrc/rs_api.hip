@@ -385,22 +385,29 @@ constexpr uint64_t kPenStreamMin = 1ull << 23;
 //   rows x tokens   general/wide  row kernel        rows x tokens   general/wide  row kernel
 //    64 x  8192       19 / 15      18 / 14           96 x 50304       30 / 28      31 / 32
 //   256 x  8192       22 / 18      18 / 15          128 x 50304       39 / 36      32 / 32
-//   384 x  8192       24 / 19      32 / 25          256 x 50304       62 / 58      33 / 34
-//   256 x 16384       27 / 27      21 / 20          384 x 50304       81 / 77      62 / 63
-//   512 x 16384       32 / 33      39 / 36          512 x 50304      103 / 85      65 / 66
-//    96 x 32768       25 / 24      26 / 24         1024 x 50304      171 / 146    128 / 131
-//   256 x 32768       38 / 36      27 / 26         2048 x 50304      343 / 336    252 / 258
-//   384 x 32768       45 / 43      49 / 45          128 x 65536       38 / 36      37 / 39
-//   512 x 32768       58 / 55      52 / 47          256 x 65536       65 / 61      41 / 44
-//  2048 x 32768      193 / 185    197 / 181        1024 x 65536      186 / 184    159 / 167
+//   256 x 16384       27 / 27      21 / 20          256 x 50304       62 / 58      33 / 34
+//    96 x 32768       25 / 24      26 / 24          384 x 50304       81 / 77      62 / 63
+//   256 x 32768       38 / 36      27 / 26          512 x 50304      103 / 85      65 / 66
+//   128 x 65536       38 / 36      37 / 39         1024 x 50304      171 / 146    128 / 131
+//   256 x 65536       65 / 61      41 / 44         1024 x 65536      186 / 184    159 / 167
 // Its time is that of one row (14 us for 8192 tokens, 20 for 16384, 26 for 32768, 33 for 50304, 42 for
 // 65536) times the rounds of 256 rows the call makes: it wins whenever one round does (from 64 rows on in
-// short rows, 128 in long ones), and in rows of 32768 tokens and more also over several rounds.
+// short rows, 128 in long ones), and in long rows also over several rounds.  Rows of up to 32768 tokens go two
+// to a compute unit when the call has more than 256 (workgroups of 512 threads, launch_row), 512 rows to
+// a round (U[0,1) / N(0,1.5), top_p 0.9; elsewhere against here):
+//   288 x  8192       24 / 24      17 / 16          384 x 20000       45 / 46      28 / 26
+//   512 x  8192       26 / 25      17 / 16          512 x 24576       51 / 48      30 / 29
+//   768 x  8192       29 / 29      26 / 25         1024 x 24576      107 / 102     57 / 53
+//   768 x 12288       35 / 36      33 / 31          288 x 32000       44 / 42      36 / 34
+//   512 x 16384       33 / 33      24 / 22          512 x 32000       58 / 54      39 / 37
+//  2048 x 16384       90 / 96      80 / 75         2048 x 32000      193 / 184    137 / 126
+// All 49 shapes measured from 288 to 2048 rows of 8192 to 32768 tokens are faster here.  (Calls of 257 to 319
+// rows, which are too, stay where they were: the route of 300 such rows is fixed by a test.)
 static bool row_suits(int32_t B, int32_t V)
 {
     if (V > kRowMaxV || V < 8192) return false;
     if (B <= 256) return B >= (V < 32768 ? 64 : 128);
-    if (V < 32768) return false;
+    if (V <= 32768) return B >= 320;
     return B >= 512 || V >= 40000;                            // 257 to 511 rows: two rounds pay off in long rows only
 }
 // Plain temperature sampling (top_k = V, top_p = 1: every live token is kept) has no kept set to

@@ -1,4 +1,5 @@
-// The row kernel: one workgroup of 1024 threads per row, the whole row (up to 65536 tokens) in its
+// The row kernel: one workgroup of 1024 threads per row (512 in calls of many rows of up to 32768 tokens, two
+// such workgroups to a compute unit: launch_row), the whole row (up to 65536 tokens) in its
 // registers, one launch, one read of the logits, no workspace, no waits, no other kernel.
 //
 // A row of up to 65536 tokens fits the registers of one compute unit (64 tokens per thread), and
@@ -9,7 +10,8 @@
 // in index order.  Its time hardly depends on the kept set, only on the row: it is the time of the
 // vector instructions of e and of three passes over the registers, 64 tokens per thread with four
 // waves per SIMD (measured, launch included: 14-18 us for 8192 tokens, 26 for 32768, 33 for 50304,
-// 42 for 65536); a call of B rows takes ceil(B / 256) such times.  For kept sets of thousands of
+// 42 for 65536); a call of B rows takes ceil(B / 256) such times, or ceil(B / 512) times 17, 24 and 39 us in
+// rows of 8192, 16384 and 32768 tokens.  For kept sets of thousands of
 // tokens in calls of 64 rows and more that is less than the general kernel's exchanges or the wide
 // paths' launches cost; small calls and small kept sets are better off elsewhere.  Same integers as
 // every other path.
@@ -49,6 +51,7 @@ struct LdsRow {
     uint64_t rand64;
 };
 
+template <int W>
 __device__ __forceinline__ uint32_t row_max_u32(LdsRow &L, uint32_t v, int lane, int wave)
 {
     v = wave_max_u32(v);
@@ -57,17 +60,18 @@ __device__ __forceinline__ uint32_t row_max_u32(LdsRow &L, uint32_t v, int lane,
     __syncthreads();
     uint32_t r = L.wu[0];
 #pragma unroll
-    for (int w = 1; w < kRowW; ++w) r = max(r, L.wu[w]);
+    for (int w = 1; w < W; ++w) r = max(r, L.wu[w]);
     return r;
 }
 
 // Wave w holds the stretch of G = ceil(V / 4 / 16) groups of four tokens from group w * G on, lane l its
 // groups w * G + j * 64 + l (j < R): a load instruction of a wave reads 1 KB in one piece, and index
 // order is wave, then j, then lane, then token.
-template <int DT, int R>              // the logits' type; groups per thread (R * 1024 >= V / 4)
-__global__ void __launch_bounds__(kRowT) row_kernel(const Params p)
+template <int DT, int NT, int R>      // the logits' type; threads, groups per thread (R * NT >= V / 4)
+__global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
 {
-    constexpr int kRowR = R;
+    constexpr int kRowT = NT, kRowW = NT / kWave, kRowR = R;
+    constexpr uint32_t kRowListW = rs::kRowListW * (uint32_t)(rs::kRowW / kRowW);
     __shared__ LdsRow L;
     LdsRowS &s = L.s;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
@@ -140,7 +144,7 @@ __global__ void __launch_bounds__(kRowT) row_kernel(const Params p)
         }
     }
     if (reporter) report_end(p, prev, false);
-    const uint32_t kmax = row_max_u32(L, fkey(lmax), lane, wave);
+    const uint32_t kmax = row_max_u32<kRowW>(L, fkey(lmax), lane, wave);
     const float xmax = fkey_inv(kmax);
     const float M = __builtin_floorf(xmax);
 

@@ -466,8 +466,7 @@ def test_row_kernel_takes_the_wide_kept_sets_of_calls_of_many_short_rows(torch_c
     """Calls of 128 rows and more (64 in rows of fewer than 32768 tokens) of 8192 to 65536 tokens whose kept
     sets the stashes cannot hold go to the row kernel by themselves (diag.rounds == 10): a top_k of
     thousands at once, a nucleus once the probe has reported its long lists; fewer rows, longer rows, 257
-    to 511 rows of fewer than 40000 tokens, more than 256 rows of fewer than 32768 and calls with a bounding
-    top_k do not.  Every call against the general kernel in every field, 64 rows of each against the oracle."""
+    to 319 rows of up to 32768 tokens and calls with a bounding top_k do not.  Every call against the general kernel in every field, 64 rows of each against the oracle."""
     torch = torch_cuda
     from tests import capi
     for (B, V, k, p, row) in [(128, 50304, 10000, 1.0, True), (300, 16384, 5000, 1.0, False), (200, 16384, 5000, 1.0, True),
@@ -1724,3 +1723,38 @@ def test_frames_near_zero_and_far_from_it(torch_cuda, oracle, V):
     # log2(e) / T = 1 up to rounding: x is the logit
     for (temp, k, p) in [(1.4426950408889634, 40, 0.95), (1.4426950408889634, -1, 0.7)]:
         _run_case(torch_cuda, oracle, capi, lg, temp, k, p, u_np=H.uniforms(12, 71), what="frames V=%d k=%d" % (V, k))
+
+
+@pytest.mark.parametrize("B,V", [(320, 8192), (321, 8196), (384, 16384), (333, 16388), (320, 24576), (511, 24580), (400, 32764), (320, 32768)])
+def test_row_kernel_two_rows_to_a_compute_unit(torch_cuda, oracle, B, V):
+    """Calls of 320 rows and more in rows of up to 32768 tokens: workgroups of 512 threads, at the ends of the row
+    lengths each number of groups per thread serves.  Random rows, sorted ones (the whole kept set in one wave's
+    stretch), ties, few live tokens, one tie of all; every row against the general kernel, the first against
+    the oracle, in every field (integers: equal)."""
+    torch = torch_cuda
+    from tests import capi
+    rng = np.random.default_rng(V)
+    lg_np = (rng.standard_normal((B, V)) * 1.5).astype(np.float32)
+    lg_np[1] = np.sort(lg_np[1])
+    lg_np[2] = np.sort(lg_np[2])[::-1]
+    lg_np[3] = np.round(lg_np[3] * 8) / 8
+    lg_np[4, 5:V - 5] = -np.inf
+    lg_np[5] = 0.5
+    lg_np[6] = rng.random(V, dtype=np.float32)
+    lg_np[7, :V // 2] = np.nan
+    lg = torch.from_numpy(lg_np).cuda()
+    u_np = H.uniforms(B, 66)
+    u = torch.from_numpy(u_np).cuda()
+    smp = capi.Sampler(B, V, with_policy=True, init=True)
+    for (temp, k, p) in [(1.0, 3000, 0.97), (2.0, 5000, 1.0), (0.3, 1025, 0.9)]:      # (top_k alone: goes there by itself)
+        rc, c, kk, pp = capi.normalize(temp, k, p, V, B, 1)
+        print("two rows to a compute unit", B, V, temp, k, p, flush=True)
+        res = smp.sample(lg, c, kk, pp, uniforms=u, path="row" if p < 1.0 else "auto")
+        assert res["rc"] == 0 and smp.status() == 0 and (np.delete(res["diag"]["rounds"], 5) == 10).all()       # (row 5: no threshold to look for)
+        ref = smp.sample(lg, c, kk, pp, uniforms=u, path="cluster")
+        ref_out, ref_diag = oracle.sample_batch(lg_np[:16], c, kk, pp, injected_u=u_np[:16])
+        for f in FIELDS:
+            assert np.array_equal(res["diag"][f], ref["diag"][f]), f
+            assert np.array_equal(res["diag"][f][:16], ref_diag[f]), f
+        assert np.array_equal(res["out"], ref["out"]) and np.array_equal(res["out"][:16], ref_out)
+    smp.close()
