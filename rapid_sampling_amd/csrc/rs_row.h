@@ -18,6 +18,7 @@
 #pragma once
 
 #include "rs_common.h"
+#include "rs_mass.h"
 
 namespace rs {
 
@@ -27,6 +28,8 @@ constexpr int      kRowR      = 16;                      // groups of four token
 static_assert(kRowMaxV == kRowT * kRowR * 4, "the row kernel's registers hold kRowMaxV tokens");
 constexpr uint32_t kRowListW  = 768u;                    // tokens of the boundary bin a wave can list for levels 3 and 4
 constexpr uint32_t kRowList   = kRowListW * 12u;         // the row's boundary bin is listed when it holds no more than this (16 waves: room to spare for uneven shares)
+constexpr uint32_t kRowKeptW  = kRowListW / 2u;          // the same lists with 64-bit entries: tokens at or above the boundary bin, with their places
+constexpr uint32_t kRowKept   = kRowKeptW * 12u;         // listed when there are no more than this in the row
 constexpr uint32_t kRowRounds = 10u;                     // DiagRow::rounds of a row finished here
 
 struct LdsRowS {                      // what the shared helpers work on
@@ -47,6 +50,7 @@ struct LdsRow {
     u128     wq[kRowW];               // per wave: kept weight of its stretch of the row
     u128     wq4[kRowW][4];           // the same, a quarter of the wave's groups at a time
     uint32_t nolist;                  // a wave's share of the boundary bin did not fit its list
+    uint32_t nokept;                  // the same for the list of all tokens at or above the boundary bin
     uint32_t wu[kRowW];
     uint64_t rand64;
 };
@@ -71,7 +75,7 @@ template <int DT, int NT, int R>      // the logits' type; threads, groups per t
 __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
 {
     constexpr int kRowT = NT, kRowW = NT / kWave, kRowR = R;
-    constexpr uint32_t kRowListW = rs::kRowListW * (uint32_t)(rs::kRowW / kRowW);
+    constexpr uint32_t kRowListW = rs::kRowListW * (uint32_t)(rs::kRowW / kRowW), kRowKeptW = rs::kRowKeptW * (uint32_t)(rs::kRowW / kRowW);
     __shared__ LdsRow L;
     LdsRowS &s = L.s;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
@@ -87,7 +91,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     prev.slow_rows = 0; prev.meta = 0;
     if (reporter) prev = report_begin(p);
     for (int i = tid; i < kNB * 8; i += kRowT) L.hr8[i] = 0;
-    if (tid == 0) L.nolist = 0u;
+    if (tid == 0) { L.nolist = 0u; L.nokept = 0u; }
 
     // token (g0 + j * 64) * 4 + q sits in register j * 4 + q; slots past the end of the stretch read the
     // row's last group again (harmless for the maximum and the probe) and are set aside before anything is counted
@@ -185,14 +189,17 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     __syncthreads();
     const uint64_t top_k = (uint64_t)p.top_k;
     Found f = hist_find_level1<false, false, LdsRowS>(s, top_k, p.top_p, lane, wave);
-    const u128 D = s.D, P = s.P;
-    const uint64_t rand64 = p.inj_u ? 0ull : L.rand64;
+    // (what is the same for all threads stays in scalar registers, or in LDS until it is used)
+    f.bin = uniform(f.bin); f.cnt_above = uniform(f.cnt_above); f.cnt_bin = uniform(f.cnt_bin);
+    auto target = [&](uint32_t thr, uint32_t n_gt, uint32_t n_eq, u128 above, uint32_t rounds) {
+        return tie_and_target(p, row, p.inj_u ? 0ull : L.rand64, xmax, s.D, s.P, thr, n_gt, n_eq, above, rounds, true);
+    };
 
     // one tie of all the row's tokens: as on the streaming path
     if (f.cnt_bin == (uint32_t)p.V && bin_is_one_tie(s.g[f.bin], f.bin, e_bits_of(xmax, M))) {
         if (tid == 0) {
             const uint32_t thr1 = e_bits_of(xmax, M);
-            const Target tg = tie_and_target(p, row, rand64, xmax, D, P, thr1, 0u, f.cnt_bin, (u128)0, 0u, true);
+            const Target tg = target(thr1, 0u, f.cnt_bin, (u128)0, 0u);
             uint32_t lo_i = 0, hi_i = (uint32_t)p.V - 1u;
             while (lo_i < hi_i) {
                 const uint32_t mid = (lo_i + hi_i) >> 1;
@@ -214,6 +221,119 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
         const uint32_t emax = e_bits_of(xmax, M);
         one_tie = bin_is_one_tie(s.g[f.bin], f.bin, emax);
         if (one_tie) { lo = emax; span = 0u; }
+    }
+    // A moderate number of tokens at or above the boundary bin: every wave lists its own, bits of e and place in its
+    // stretch, and everything behind -- the levels, the sums of the pick -- reads a few list entries per thread instead
+    // of the registers (the first pass of the pick alone takes 15 instructions per token, listing 8).  Up to a sixth of
+    // the row, that is: where more is kept the lists themselves cost as much as the registers (1024 rows of 8192, more
+    // than half of each kept: 28 us from the registers, 38 from lists).  512 x 32768 float16, 4 % kept: 31.3 -> 26.8
+    // us a call; 512 x 50304: 55.5 -> 46.3; 200 x 50304: 27.6 -> 22.9; flat rows with top_k 1000, 512 x 32768: 38.3 -> 30.4.
+    // (The bits are copied out of the compiler's sight: it kept what it had worked out from them in 200 registers.)
+    uint64_t *kept = L.hr8 + (uint32_t)wave * kRowKeptW;             // group by group, then token of the group, then lane
+    uint32_t nkept = 0u, kept_from = 0u;                             // kept_from: lane j, where those of the wave's group j begin
+    const uint32_t bin_lo = f.bin << 21;
+    const uint32_t at_or_above = f.cnt_above + f.cnt_bin;
+    bool have_kept = at_or_above <= kRowKept && at_or_above * 6u <= (uint32_t)p.V;
+    if (have_kept) {
+        uint32_t lane4 = (uint32_t)lane * 4u;
+#pragma unroll
+        for (int j = 0; j < kRowR; ++j) {
+            asm volatile("" : "+s"(nkept), "+v"(lane4));
+            kept_from = lane == j ? nkept : kept_from;
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                uint32_t b = eb[j * 4 + q];
+                asm volatile("" : "+v"(b));
+                const uint64_t cand = __builtin_amdgcn_ballot_w64(b >= bin_lo);
+                const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(cand >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cand, nkept));
+                if (b >= bin_lo && at < kRowKeptW) kept[at] = ((uint64_t)b << 32) | (lane4 + (uint32_t)(j * 256 + q));
+                nkept += (uint32_t)__builtin_popcountll(cand);
+            }
+        }
+        if (nkept > kRowKeptW && lane == 0) L.nokept = 1u;
+        __syncthreads();
+        have_kept = L.nokept == 0u;
+    }
+    if (have_kept) {
+        // fn(bits of e, place in the wave's stretch) for the wave's listed tokens
+        auto listed = [&](auto fn) {
+            for (uint32_t i = (uint32_t)lane; i < nkept; i += (uint32_t)kWave) {
+                const uint64_t e = kept[i];
+                fn((uint32_t)(e >> 32), (uint32_t)e);
+            }
+        };
+        for (uint32_t lv = 2; lv <= (uint32_t)kLevels && !one_tie && f.cnt_bin > 1u; ++lv) {
+            const uint32_t dsh = level_shift(lv);
+            if (tid < 128 * 4) L.lev[tid] = 0;
+            __syncthreads();
+            listed([&](uint32_t b, uint32_t) {
+                if (b - lo <= span)
+                    atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[((b >> dsh) & 127u) * 4u + (uint32_t)(lane & 3)]),
+                              (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
+            });
+            __syncthreads();
+            if (tid < 128) s.hm[tid] = L.lev[tid * 4] + L.lev[tid * 4 + 1] + L.lev[tid * 4 + 2] + L.lev[tid * 4 + 3];
+            __syncthreads();
+            f = hist_find128(s, s.hm, f.cnt_above, f.mass_above, top_k, exb, lane, wave);
+            lo |= f.bin << dsh;
+            span = (1u << dsh) - 1u;
+        }
+        if (span != 0u) {
+            listed([&](uint32_t b, uint32_t) { if (b - lo <= span) s.bc32[6] = b; });
+            __syncthreads();
+            lo = s.bc32[6];
+        }
+        const uint32_t thr = lo;
+        if (tid == 0) {
+            const Target tg = target(thr, f.cnt_above, f.cnt_bin, f.mass_above, kRowRounds);
+            s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
+        }
+        __syncthreads();
+        const uint64_t w_tie = s.bc64[1];
+        const u128 r = s.bc128[0];
+        auto weight = [=](uint32_t b) -> uint64_t { return (b > thr) ? w_of_bits(b) : (b == thr ? w_tie : 0ull); };
+        uint64_t a = 0, h = 0;                           // halves summed apart
+        listed([&](uint32_t b, uint32_t) { const uint64_t w = weight(b); a += w & 0xFFFFFFFFull; h += w >> 32; });
+        a = wave_sum(a); h = wave_sum(h);
+        if (lane == 0) L.wq[wave] = (u128)a + ((u128)h << 32);
+        __syncthreads();
+        // every wave looks which stretch holds the target (1 <= r <= the sum of all kept weights); that wave goes on
+        const u128 wt = lane < kRowW ? L.wq[lane] : (u128)0, winc = wave_inclusive_scan(wt);
+        const uint32_t wstar = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(winc >= r));
+        if ((uint32_t)wave != wstar) return;
+        u128 rl = r - wide(lane_of(m96(winc - wt), wstar));
+        // the wave's groups one per lane, then the tokens of one group, four per lane
+        auto in_order = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
+        if (lane < 32) L.lev[lane] = 0ull;
+        in_order();
+        for (uint32_t i = (uint32_t)lane; i < nkept; i += (uint32_t)kWave) {
+            const uint64_t e = kept[i], w = weight((uint32_t)(e >> 32));
+            const uint32_t g = (uint32_t)e >> 8;         // < 16
+            atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[g]), (unsigned long long)(w & 0xFFFFFFFFull));
+            atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[16 + g]), (unsigned long long)(w >> 32));
+        }
+        in_order();
+        const u128 gm = lane < 16 ? (u128)L.lev[lane] + ((u128)L.lev[16 + lane] << 32) : (u128)0;
+        const u128 ginc = wave_inclusive_scan(gm);
+        const uint32_t j = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(ginc >= rl));       // there is one
+        rl -= wide(lane_of(m96(ginc - gm), j));
+        const uint32_t from = lane_of(kept_from, j), to = j + 1u < (uint32_t)kRowR ? lane_of(kept_from, j + 1u) : nkept;
+        in_order();
+#pragma unroll
+        for (int k = 0; k < 4; ++k) L.lev[k * kWave + lane] = 0ull;
+        in_order();
+        for (uint32_t i = from + (uint32_t)lane; i < to; i += (uint32_t)kWave) L.lev[(uint32_t)kept[i] & 255u] = weight((uint32_t)(kept[i] >> 32));
+        in_order();
+        const uint64_t w0 = L.lev[lane * 4], w1 = L.lev[lane * 4 + 1], w2 = L.lev[lane * 4 + 2], w3 = L.lev[lane * 4 + 3];
+        const u128 m4 = (u128)w0 + w1 + w2 + w3, inc = wave_inclusive_scan(m4), exc = inc - m4;
+        if (exc < rl && rl <= inc) {                     // exactly one lane
+            const u128 rr = rl - exc;
+            const uint32_t kk = (rr <= w0) ? 0u : (rr <= (u128)w0 + w1) ? 1u : (rr <= (u128)w0 + w1 + w2) ? 2u : 3u;
+            const int32_t idx = (int32_t)(((uint32_t)wave * G + j * (uint32_t)kWave + (uint32_t)lane) * 4u + kk);
+            p.out[row] = idx;
+            if (p.diag) p.diag[row].index = idx;
+        }
+        return;
     }
     // The tokens of the boundary bin are listed while level 2 counts them (where the bin's copies were: they
     // are done with), every wave its own in a list of its own -- no counter to share, no wait: the place is
@@ -292,7 +412,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     }
     const uint32_t thr = lo;
     if (tid == 0) {
-        const Target tg = tie_and_target(p, row, rand64, xmax, D, P, thr, f.cnt_above, f.cnt_bin, f.mass_above, kRowRounds, true);
+        const Target tg = target(thr, f.cnt_above, f.cnt_bin, f.mass_above, kRowRounds);
         s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
     }
     __syncthreads();
