@@ -5,14 +5,15 @@ namespace rs {
 
 constexpr int kStreamNT = 256;
 
-// The finishing workgroup's size.  Lists of hundreds of tokens (a bounding top_k above 256): 1024 threads (128 rows of
-// 1M with top_k 1024: 10.8 us where 256 threads took 13.7).  Short ones: 256 threads -- a nucleus whose list is not
-// known to be long too (one row of 262144: 7.3 us, with 1024 threads 8.4, the scans then go from one wave to
-// the others by way of LDS) -- asking ahead for the first 64 tokens of 4, 8 or 16 slices per wave, which is 16 instructions
-// per slice whether the row has it or not (64 rows of 19 slices: 7.3 us with 16, 6.5 with 8).
+// The finishing workgroup's size.  Lists of hundreds of tokens (a bounding top_k above 256) out of 32 slices and more: 1024
+// threads (128 rows of 1M with top_k 1024: 10.8 us where 256 threads took 13.7; 32 rows of 131072 with top_k 1000, the
+// call: 23.0 -> 19.9) while every row has a compute unit to itself (1024 rows of 8192 with top_k 1000: 77 us a call with 1024
+// threads, 48 with 256).  Else 256 threads, the scans then stay inside a wave, asking ahead for the first 64 tokens of
+// 4, 8 or 16 slices per wave, which is 16 instructions per slice whether the row has it or not (64 rows of 19
+// slices: 7.3 us with 16, 6.5 with 8).
 static void launch_finish(uint32_t B, size_t lds_bytes, hipStream_t st, const Params &p, const StreamView &v)
 {
-    if (p.top_k > 256 && !p.attempt) hipLaunchKernelGGL((finish_kernel<1024, 8>), dim3(B), dim3(finish_threads<1024>()), lds_bytes, st, p, v);
+    if (B <= 256u && v.G >= 32u && p.top_k > 256 && !p.attempt) hipLaunchKernelGGL((finish_kernel<1024, 8>), dim3(B), dim3(finish_threads<1024>()), lds_bytes, st, p, v);
     else if (v.G <= 16u) hipLaunchKernelGGL((finish_kernel<kThreads, 4>), dim3(B), dim3(finish_threads<kThreads>()), lds_bytes, st, p, v);
     else if (v.G <= 32u) hipLaunchKernelGGL((finish_kernel<kThreads, 8>), dim3(B), dim3(finish_threads<kThreads>()), lds_bytes, st, p, v);
     else hipLaunchKernelGGL((finish_kernel<kThreads, 16>), dim3(B), dim3(finish_threads<kThreads>()), lds_bytes, st, p, v);
