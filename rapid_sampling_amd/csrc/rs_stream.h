@@ -724,7 +724,11 @@ __device__ __forceinline__ void pick_of_wave(const Params &p, LdsB &t, const uin
 // the one before: trips to memory, scans, threshold, pick, with a workgroup barrier between most of them.
 //   * The first 64 stashed tokens of every slice are asked for together with the headers and the row's
 //     bins, before it is known which of them count: for the usual call that is all of them.  That nothing is
-//     missing is checked by counting: the row's bins say how many tokens lie at or above the boundary bin.
+//     missing is checked by counting: the row's bins say how many tokens lie at or above the boundary bin.  A list
+//     that may hold more takes the rest of each stash's prefix, as long as the slice's counts by bin say; those counts
+//     are on their way while the first tokens are listed.  (Going through the stashes whole instead: 128 rows of 32768 with
+//     top_k 1000 31.5 us a call against 21.7, one row of 524288 in 128 slices with top_k 50 24.4 against 14.5,
+//     8 rows of 50304 with penalties and top_k 1000, in one launch, 28.6 against 19.5.)
 //   * With one wave per SIMD (NT = 256) every wave works the one-wave steps out for itself: no barrier and no
 //     trip through LDS for what all of them hold.
 //   * The row's random number is drawn by a wave of its own (NT = 256: a fifth one, which leaves at its second
@@ -935,14 +939,6 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     }
 
     // ---- the list: the row's tokens at or above the boundary bin ----
-    // The tokens of a chunk of 64 stash entries at or above `from`, side by side behind what is in the list
-    // already; at: the wave's place in it (claimed for what the wave is about to add).
-    auto put_listed = [&](uint32_t b, uint32_t idx, uint32_t &at) {
-        const uint64_t vote = __builtin_amdgcn_ballot_w64(b != 0u);
-        const uint32_t o = at + __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0u));
-        if (b != 0u && o < v.list_cap) list[o] = ((uint64_t)b << 32) | idx;
-        at += (uint32_t)__builtin_popcountll(vote);
-    };
     auto claim = [&](uint32_t n) {
         uint32_t at = 0;
         if (lane == 0 && n) at = atomicAdd(&s.ctr, n);
@@ -952,7 +948,16 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     const uint32_t cut = bin << 21;
     uint32_t n = 0;                                      // tokens listed
     bool listed = false, subset = false;
-    if (total <= v.list_cap && G <= (uint32_t)(W * PRE)) {
+    const bool ahead = total <= v.list_cap && G <= (uint32_t)(W * PRE);
+    // How many tokens of slice tid lie at or above the boundary bin, as its workgroup counted them: asked for while the
+    // first ones go into the list, unless those are certain to be all.
+    const uint32_t dl = (uint32_t)tid < G ? octaves_below(ph.mkey) : 0u;
+    uint32_t above_cut = 0;
+    if ((total > (uint32_t)kWave || !ahead) && (uint32_t)tid < G) {
+        const uint32_t lb = bin - kBin0 + 4u * dl;       // the boundary bin in the slice's frame; past its last bin: nothing of the slice is live
+        if (lb < (uint32_t)kSB) above_cut = get<FUSED>(&v.cum[((size_t)row * G + (uint32_t)tid) * kSB + lb]);
+    }
+    if (ahead) {
         // lane i looks after the wave's i-th slice: how far its frame lies below the row's, how many tokens it stashed
         const uint32_t sl = (uint32_t)(wave + W * lane);
         const uint2 h = hd[min(sl, G - 1u)];
@@ -982,60 +987,108 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         listed = n == total;                             // every token at or above the boundary bin is there
     }
     if (!listed) {
-        const uint32_t dl = (uint32_t)tid < G ? octaves_below(ph.mkey) : 0u;
-        if ((uint32_t)tid < G) { t.delta[tid] = dl; t.m4[tid] = min(ph.n, (uint32_t)kStashCap); }      // (m4: the stashes' lengths here)
-        // fn(bits of e in the row's frame, 0 past the end of a stash; token) for all stashes whole, 64 entries at a
-        // time, eight loads in flight; called by all lanes of a wave together
-        auto stashed = [&](auto fn) {
-            constexpr int kBatch = 8;
-            uint32_t sl = (uint32_t)wave, c = 0, len = sl < G ? uniform(t.m4[sl]) : 0u;
-            for (;;) {
+        // Prefixes of the stashes, one after the other: t.take[g] = entries of slices 0..g.  Returns how many in all.
+        auto take_prefix = [&](uint32_t mine) -> uint32_t {
+            uint32_t inc = wave_inclusive_scan(mine);
+            __syncthreads();
+            if (lane == kWave - 1) s.u32[wave] = inc;
+            __syncthreads();
+            uint32_t sum = 0;
+#pragma unroll
+            for (int w = 0; w < kMaxParts / kWave; ++w) {              // the waves that hold slices
+                if (w < wave) inc += s.u32[w];
+                sum += s.u32[w];
+            }
+            if (tid < kMaxParts) t.take[tid] = inc;
+            __syncthreads();
+            return uniform(sum);
+        };
+        // fn(first, how many, bits of e in the row's frame, tokens) for the n_all entries t.take speaks of, those of a
+        // slice from entry `skip` on, eight of a thread at a time and in flight together; a thread has a run of consecutive ones, so that
+        // all threads have as many wherever they lie, and looks up its first slice once.  Called by all threads together.
+        constexpr int kBatch = 8;
+        auto stashed = [&](const uint32_t n_all, const uint32_t skip, auto fn) {
+            const uint32_t per = (n_all + (uint32_t)NT - 1u) / (uint32_t)NT;
+            const uint32_t i0 = (uint32_t)tid * per, iend = min(n_all, i0 + per);
+            uint32_t g = 0, hi_g = G - 1u;                             // first slice whose prefix exceeds i0
+            while (g < hi_g) {
+                const uint32_t mid = (g + hi_g) >> 1;
+                if (t.take[mid] > i0) hi_g = mid; else g = mid + 1u;
+            }
+            uint32_t gend = t.take[g];
+            const uint64_t *from_g = stash + (size_t)g * kStashCap + skip - (g ? t.take[g - 1u] : 0u);
+            for (uint32_t k = 0; k < per; k += (uint32_t)kBatch) {
+                const uint32_t i = i0 + k, m = i < iend ? min((uint32_t)kBatch, iend - i) : 0u;
                 uint64_t e[kBatch];
                 uint32_t d[kBatch];
-                bool live[kBatch];
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
-                    while (sl < G && c >= len) { sl += W; c = 0; len = sl < G ? uniform(t.m4[sl]) : 0u; }
-                    live[u] = sl < G && c + (uint32_t)lane < len;
-                    d[u] = sl < G ? t.delta[sl] : 0u;
-                    e[u] = live[u] ? get<FUSED>(&stash[(size_t)sl * kStashCap + c + (uint32_t)lane]) : 0ull;
-                    c += (uint32_t)kWave;
+                    e[u] = 0; d[u] = 0;
+                    if ((uint32_t)u < m) {
+                        while (i + (uint32_t)u >= gend) {              // slices that give nothing are skipped
+                            ++g; from_g = stash + (size_t)g * kStashCap + skip - gend; gend = t.take[g];
+                        }
+                        e[u] = get<FUSED>(&from_g[i + (uint32_t)u]);
+                        d[u] = t.delta[g];
+                    }
                 }
+                uint32_t bits[kBatch], idx[kBatch];
 #pragma unroll
-                for (int u = 0; u < kBatch; ++u) fn(live[u] ? rebase_bits((uint32_t)(e[u] >> 32), d[u]) : 0u, (uint32_t)e[u]);
-                if (sl >= G) break;
+                for (int u = 0; u < kBatch; ++u) {
+                    bits[u] = (uint32_t)u < m ? rebase_bits((uint32_t)(e[u] >> 32), d[u]) : 0u;
+                    idx[u] = (uint32_t)e[u];
+                }
+                fn(i, m, bits, idx);
             }
         };
-        auto list_from = [&](uint32_t from) {
+        // the tokens at or above `from` among them, side by side
+        auto list_from = [&](const uint32_t n_all, const uint32_t from) -> uint32_t {
             __syncthreads();                             // the list's counter has been read
             if (tid == 0) s.ctr = 0u;
             __syncthreads();
-            stashed([&](uint32_t b, uint32_t idx) {
-                if (b < from) b = 0u;
-                uint32_t at = claim((uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b != 0u)));
-                put_listed(b, idx, at);
+            stashed(n_all, 0u, [&](uint32_t, uint32_t, const uint32_t (&bits)[kBatch], const uint32_t (&idx)[kBatch]) {
+                uint32_t mine = 0;
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u) mine += bits[u] >= from ? 1u : 0u;
+                const uint32_t upto = wave_inclusive_scan(mine);
+                uint32_t at = claim(lane63(upto)) + upto - mine;
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u)
+                    if (bits[u] >= from) {
+                        if (at < v.list_cap) list[at] = ((uint64_t)bits[u] << 32) | idx[u];
+                        ++at;
+                    }
             });
             __syncthreads();
             return uniform(s.ctr);
         };
+        if ((uint32_t)tid < G) t.delta[tid] = dl;
         // Together the stashes hold every token of the row at or above `from`, the largest of the slices' cuts.  (A
         // cut that lands below 2^-40 in the row's frame: what the stash lacks is dead there.)
+        const uint32_t len = (uint32_t)tid < G ? min(ph.n, (uint32_t)kStashCap) : 0u;
         uint32_t from = (uint32_t)tid < G ? max(rebase_bits(ph.cut, dl), kEMinBits) : 0u;
-        uint32_t all = (uint32_t)tid < G ? min(ph.n, (uint32_t)kStashCap) : 0u;       // stashed tokens of the row
-        {
-            const uint32_t a = wave_max_u32(from), b = wave_sum(all);
-            __syncthreads();
-            if (lane == 0) { t.take[wave] = a; t.take[W + wave] = b; }
-            __syncthreads();
-            from = 0; all = 0;
-            for (int w = 0; w < W; ++w) { from = max(from, t.take[w]); all += t.take[W + w]; }
-            from = uniform(from); all = uniform(all);
-        }
+        from = wave_max_u32(from);
+        __syncthreads();
+        if (lane == 0) t.take[wave] = from;
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kMaxParts / kWave; ++w) from = max(from, t.take[w]);
+        from = uniform(from);
         bool slow = false;
         if (from <= cut && total <= v.list_cap) {        // plan A: every stash reaches down to the boundary bin
-            n = list_from(cut);
+            // exactly the tokens at or above that bin: of every stash a prefix, whose first 64 are listed already
+            const uint32_t skip = ahead ? (uint32_t)kWave : 0u, had = n, take = min(above_cut, len);
+            const uint32_t rest = take_prefix(take > skip ? take - skip : 0u);
+            n = had + rest;
             slow = n != total;
-        } else if (!FUSED && all > min(v.list_cap, max(2048u, 3u * top_k)) && top_k <= v.list_cap / 2u) {
+            if (!slow)
+                stashed(rest, skip, [&](uint32_t i, uint32_t m, const uint32_t (&bits)[kBatch], const uint32_t (&idx)[kBatch]) {
+#pragma unroll
+                    for (int u = 0; u < kBatch; ++u)
+                        if ((uint32_t)u < m) list[had + i + (uint32_t)u] = ((uint64_t)bits[u] << 32) | idx[u];
+                });
+            __syncthreads();
+        } else if (const uint32_t all = take_prefix(len); !FUSED && all > min(v.list_cap, max(2048u, 3u * top_k)) && top_k <= v.list_cap / 2u) {
             // Plan B (flat distributions: the boundary bin holds thousands of tokens, but top_k is small) with more
             // stashed tokens than the list holds, or several times top_k of them.  The kept set is at most
             // top_k tokens, so only the stashed tokens down to some value T at or above which there are at least
@@ -1048,8 +1101,10 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             if (kEach) cnt[256 + tid] = 0u;
             if (tid == 0) { s.bc32[4] = 0xFFFFFFFFu; s.bc32[5] = 0u; }
             __syncthreads();
-            stashed([&](uint32_t b, uint32_t) {
-                if (b >= from) atomicAdd(&cnt[min(511u, topkey - (b >> 14))], 1u);
+            stashed(all, 0u, [&](uint32_t, uint32_t, const uint32_t (&bits)[kBatch], const uint32_t (&)[kBatch]) {
+#pragma unroll
+                for (int u = 0; u < kBatch; ++u)
+                    if (bits[u] >= from) atomicAdd(&cnt[min(511u, topkey - (bits[u] >> 14))], 1u);
             });
             __syncthreads();
             if (wave == 0) {
@@ -1071,7 +1126,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             const uint32_t step = uniform(s.bc32[4]), nge = uniform(s.bc32[5]);
             slow = step >= 511u || nge > v.list_cap;     // fewer than top_k at or above `from`, or one value thousands of times
             if (!slow) {
-                n = list_from(max(from, (topkey - step) << 14));
+                n = list_from(all, max(from, (topkey - step) << 14));
                 subset = true;
                 // Two more passes over the stashes make this finish slower than the general kernel's whole
                 // call while the call is of moderate size (measured: 64 flat rows of 131072 with top_k 1000,
@@ -1082,7 +1137,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             }
         } else {                                         // plan B, the stashes whole
             slow = all > v.list_cap || all == 0u;
-            if (!slow) { n = list_from(from); subset = true; }
+            if (!slow) { n = list_from(all, from); subset = true; }
         }
         if (!slow && subset) {
             // level 1 again, on the listed tokens alone

@@ -1758,3 +1758,82 @@ def test_row_kernel_two_rows_to_a_compute_unit(torch_cuda, oracle, B, V):
             assert np.array_equal(res["diag"][f][:16], ref_diag[f]), f
         assert np.array_equal(res["out"], ref["out"]) and np.array_equal(res["out"][:16], ref_out)
     smp.close()
+
+
+def _us_per_call(torch, sample, fn):
+    """Microseconds per call of fn, back to back on the current stream, routed as a program's calls are: the best of
+    seven batches of 30, after twelve calls that settle the route."""
+    sample.reset_routing()
+    for _ in range(12):
+        fn()
+        torch.cuda.synchronize()
+    best = float("inf")
+    for _ in range(7):
+        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        e0.record()
+        for _ in range(30):
+            fn()
+        e1.record()
+        e1.synchronize()
+        best = min(best, e0.elapsed_time(e1) * 1000.0 / 30)
+    return best
+
+
+def _top_tokens_per_slice(rng, B, V, slice_tokens, counts):
+    """Rows with counts[g] tokens of distinct values within two octaves in slice g, everything else far below: the kept
+    set of a top_k of their number, and how much of it each slice holds."""
+    lg = (rng.standard_normal((B, V)) - 30.0).astype(np.float32)
+    n = int(sum(counts))
+    for b in range(B):
+        vals = (5.0 + rng.permutation(n) / np.float32(n)).astype(np.float32)
+        at = 0
+        for g, c in enumerate(counts):
+            lo, hi = g * slice_tokens, min(V, (g + 1) * slice_tokens)
+            lg[b, lo + rng.choice(hi - lo, c, replace=False)] = vals[at:at + c]
+            at += c
+    return lg
+
+
+@pytest.mark.parametrize("V,counts", [
+    (32768, [63, 64, 65, 0, 66, 1, 64, 64]), (32768, [1000, 0, 0, 0, 0, 0, 0, 1]), (32768, [0, 0, 0, 0, 0, 0, 65, 65]),
+    (50260, [65] * 13), (4096 * 33, [70] + [0] * 31 + [70]), (4096 * 64, [20, 66] * 32), (4096 * 65, [1] * 65),
+    (4096 * 128, [8, 7] * 64), (4096 * 127 + 4, [33] + [0] * 126 + [1]), (262144 * 4, [30, 1, 2, 0] * 32)])
+def test_streaming_finish_takes_prefixes_of_the_stashes(torch_cuda, oracle, V, counts):
+    """Lists of which a slice holds more than the 64 tokens that are asked for ahead, or out of more slices than are: a
+    prefix of every stash, the first 64 of it listed already or not, of 0, 1, 63 to 66 and a thousand tokens, at both ends
+    of the row, with top_k at and around the number of such tokens.  Every path (with penalties the one-launch path too)
+    against the oracle in every field (integers: equal)."""
+    from tests import capi
+    rng = np.random.default_rng(V + len(counts))
+    lg = _top_tokens_per_slice(rng, 2, V, 8192 if V == 1 << 20 else 4096, counts)
+    n = sum(counts)
+    for k in sorted({max(1, n // 2), n, min(1024, n + 5)}):
+        _run_case(torch_cuda, oracle, capi, lg, 1.0, k, 1.0, u_np=H.uniforms(2, k), what="prefixes V=%d k=%d" % (V, k))
+    if V <= 262144:
+        pen = np.where(rng.random((2, V)) < 0.02, rng.exponential(1.0, (2, V)), 0.0).astype(np.float32)
+        _run_case(torch_cuda, oracle, capi, lg, 1.0, min(1024, n), 0.99, u_np=H.uniforms(2, 7), pen_np=pen, presence=0.1,
+                  repetition=0.1, decay=0.95, what="prefixes with penalties V=%d" % V)
+
+
+def test_streaming_finish_costs_what_its_list_holds(torch_cuda):
+    """The finish reads the tokens its list will hold, not the stashes whole: calls whose first 64 tokens per slice are
+    not all, or whose rows have more slices than are asked for ahead, against calls of the same pass for which they
+    are.  Time ratios, measured 1.05, 1.56 and 1.40 with prefixes, 1.9, 2.2 and 2.0 with whole stashes."""
+    torch = torch_cuda
+    import rapid_sampling_amd as sample
+    gen = torch.Generator(device="cuda").manual_seed(3)
+
+    def us(B, V, k, pen=False):
+        lg = torch.randn((B, V), generator=gen, device="cuda").mul_(1.5)
+        st = sample.setup_rand(1, B)
+        if not pen:
+            return _us_per_call(torch, sample, lambda: sample.batch_sampling_temperature_topk_topp(lg, st, 1.0, k, 1.0))
+        pn = torch.zeros((B, V), device="cuda")
+        return _us_per_call(torch, sample, lambda: sample.batch_sampling_repetition_temperature_topk_topp(
+            lg, pn, st, 0.1, 0.1, 0.95, 1.0, k, 0.95))
+
+    for what, more, fewer, bound in [("128 slices and 64", us(1, 524288, 50), us(1, 262144, 50), 1.4),
+                                     ("8 slices, top_k 1000 and 50", us(128, 32768, 1000), us(128, 32768, 50), 1.85),
+                                     ("13 slices with penalties, top_k 1000 and 50", us(8, 50304, 1000, True), us(8, 50304, 50, True), 1.7)]:
+        print(what, "%.1f us, %.1f us: %.2f" % (more, fewer, more / fewer), flush=True)
+        assert more < bound * fewer, (what, more, fewer)
