@@ -830,7 +830,6 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
             const bool small_call = (uint64_t)B * (uint64_t)V < (1ull << 20) && V < 131072;
             p.long_list = small_call ? 768u : max(2048u, (uint32_t)V / 20u);
         }
-        if (path == kPathKeep) { p.stash_k = 1u; v.list_cap = 2048u; }
         if (path == kPathWide || path == kPathProbe) {
             // the list holds the tokens of ONE sub-bin of the boundary bin: 1/128 of it for a smooth distribution
             p.stash_k = 1u; v.list_cap = 4096u;

@@ -653,10 +653,9 @@ constexpr int      kFinCap   = 8192;          // tokens the finishing workgroup 
 
 struct PartHdr {
     uint32_t mkey;        // fkey(max x of the slice)
-    uint32_t cov;         // the stash holds every token of the slice with bin - 348 >= cov
+    uint32_t window;      // wide paths: which level-1 bins the slice's window covers (kWideValid); 0 elsewhere
     uint32_t n;           // entries in the stash
-    uint32_t cut;         // the stash holds every token of the slice with bits(e) >= cut (slice frame); cut lies in
-                          // bin cov or, when only part of a bin fitted, in bin cov - 1
+    uint32_t cut;         // the stash holds every token of the slice with bits(e) >= cut (slice frame)
 };
 
 // A slice's note of its penalties (stream_pen_kernel): word 0 = count, or kPenDeferred when the slice left its

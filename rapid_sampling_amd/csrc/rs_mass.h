@@ -29,18 +29,6 @@ __device__ __forceinline__ M96 operator-(M96 a, M96 b)
 __device__ __forceinline__ bool operator>=(M96 a, M96 b) { return a.hi > b.hi || (a.hi == b.hi && a.lo >= b.lo); }
 __device__ __forceinline__ bool operator<(M96 a, M96 b) { return !(a >= b); }
 
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ M96 dpp0_m96(M96 v) { return M96{dpp0<CTRL, ROW_MASK>(v.lo), dpp0<CTRL, ROW_MASK>(v.hi)}; }
-__device__ __forceinline__ M96 wave_inclusive_scan(M96 v)
-{
-    v = v + dpp0_m96<0x111, 0xf>(v);
-    v = v + dpp0_m96<0x112, 0xf>(v);
-    v = v + dpp0_m96<0x114, 0xf>(v);
-    v = v + dpp0_m96<0x118, 0xf>(v);
-    v = v + dpp0_m96<0x142, 0xa>(v);
-    v = v + dpp0_m96<0x143, 0xc>(v);
-    return v;
-}
 __device__ __forceinline__ uint32_t lane_of(uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); }
 __device__ __forceinline__ uint64_t lane_of(uint64_t v, uint32_t l) { return ((uint64_t)lane_of((uint32_t)(v >> 32), l) << 32) | lane_of((uint32_t)v, l); }
 __device__ __forceinline__ M96 lane_of(M96 v, uint32_t l) { return M96{lane_of(v.lo, l), lane_of(v.hi, l)}; }

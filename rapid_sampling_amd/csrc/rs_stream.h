@@ -51,7 +51,7 @@ struct LdsA {
     uint32_t off[kSB];
     uint32_t sub[128];           // level-2 counts inside a boundary bin too large for the stash
     uint32_t u32[16];
-    uint32_t cov, n, cut, over;
+    uint32_t n, cut, over;
 };
 
 #ifndef RS_STREAM_WAVES
@@ -166,7 +166,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
         }
         if (tid == 0) {
             PartHdr ph;
-            ph.mkey = k; ph.cov = 0u; ph.n = 0u; ph.cut = 0u;
+            ph.mkey = k; ph.window = 0u; ph.n = 0u; ph.cut = 0u;
             v.hdr[(size_t)row * G + part] = ph;
         }
         return k;
@@ -191,7 +191,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
         uint32_t run = ci - cs;
         const uint32_t total = lane63(ci);
         if (lane == 0) s.over = 0xFFFFFFFFu;
-        if (lane == 0 && total < Ks) { s.cov = 0u; s.n = total; s.cut = kBin0 << 21; }   // a short slice: all its live tokens
+        if (lane == 0 && total < Ks) { s.n = total; s.cut = kBin0 << 21; }   // a short slice: all its live tokens
 #pragma unroll
         for (int i = 0; i < 3; ++i) {
             const int b = kSB - 1 - 3 * lane - i;
@@ -202,8 +202,8 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
             }
             if (run < Ks && nx >= Ks) {
                 // the whole bin if that stays close to stash_k, else only part of it (found below)
-                if (nx <= min((uint32_t)kStashCap, Ks + max(64u, Ks >> 2))) { s.cov = (uint32_t)b; s.n = nx; s.cut = ((uint32_t)b + kBin0) << 21; }
-                else { s.cov = (uint32_t)b + 1u; s.n = run; s.cut = ((uint32_t)b + 1u + kBin0) << 21; s.over = (uint32_t)b; }
+                if (nx <= min((uint32_t)kStashCap, Ks + max(64u, Ks >> 2))) { s.n = nx; s.cut = ((uint32_t)b + kBin0) << 21; }
+                else { s.n = run; s.cut = ((uint32_t)b + 1u + kBin0) << 21; s.over = (uint32_t)b; }
             }
             run = nx;
         }
@@ -250,8 +250,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
         }
         __syncthreads();
     }
-    const uint32_t cov = s.cov, n = s.n;
-    const uint32_t cut = s.cut;
+    const uint32_t n = s.n, cut = s.cut;
     // From here on the bits in the registers are compared with the cut, which is never below
     // 2^-40: dead tokens are no candidates.
 
@@ -298,11 +297,11 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     if (tid == 0) {
         if (FUSED) {
             uint64_t *h2 = reinterpret_cast<uint64_t *>(&v.hdr[(size_t)row * G + part]);
-            a_store(&h2[0], ((uint64_t)cov << 32) | k);
+            a_store(&h2[0], (uint64_t)k);
             a_store(&h2[1], ((uint64_t)cut << 32) | n);
         } else {
             PartHdr ph;
-            ph.mkey = k; ph.cov = cov; ph.n = n; ph.cut = cut;
+            ph.mkey = k; ph.window = 0u; ph.n = n; ph.cut = cut;
             v.hdr[(size_t)row * G + part] = ph;
         }
     }
@@ -779,12 +778,12 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         return true;
     }
     PartHdr ph;
-    ph.mkey = 0; ph.cov = 0; ph.n = 0; ph.cut = 0;
+    ph.mkey = 0; ph.window = 0; ph.n = 0; ph.cut = 0;
     if ((uint32_t)tid < G) {
         if (FUSED) {
             const uint64_t *h2 = reinterpret_cast<const uint64_t *>(&hdrs[tid]);
             const uint64_t w0 = a_load(&h2[0]), w1 = a_load(&h2[1]);
-            ph.mkey = (uint32_t)w0; ph.cov = (uint32_t)(w0 >> 32); ph.n = (uint32_t)w1; ph.cut = (uint32_t)(w1 >> 32);
+            ph.mkey = (uint32_t)w0; ph.n = (uint32_t)w1; ph.cut = (uint32_t)(w1 >> 32);
         } else ph = hdrs[tid];
     }
     uint64_t h0 = 0, h1 = 0;

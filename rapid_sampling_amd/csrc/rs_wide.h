@@ -35,7 +35,7 @@ namespace rs {
 constexpr int      kWideHead  = 132;                     // words at the head of a slice's stash region: kept mass above the bin (2), running sums (129)
 constexpr int      kWideCap   = kStashCap - kWideHead;   // tokens a slice can set aside
 constexpr int      kWideRep   = 4;                       // copies of each sub-bin while it is counted
-constexpr uint32_t kWideValid = 1u << 16;                // PartHdr::cov of a slice the second pass has been over: window lo | hi << 8 | this
+constexpr uint32_t kWideValid = 1u << 16;                // PartHdr::window of a slice the second pass has been over: window lo | hi << 8 | this
 
 // What the plan kernel leaves for a row (in the first words of RowCtl::A, which the wide path does not
 // use otherwise; the finishing workgroup puts them back to zero).
@@ -371,7 +371,7 @@ __global__ void __launch_bounds__(NT) wide_kernel(const Params p, const StreamVi
         if (lane == 0) {
             s.win_lo = wl; s.win_hi = wh; s.n = wn;
             PartHdr *ph = &v.hdr[(size_t)row * G + part];
-            ph->cov = wl | wh << 8 | kWideValid;
+            ph->window = wl | wh << 8 | kWideValid;
             ph->n = wn;
         }
     } else if (wave == 1) {
@@ -430,7 +430,7 @@ __device__ __forceinline__ void wide_finish_row(const Params &p, const StreamVie
 
     if (tid == 0) { s.abort = 0; s.host_words = p.host_words; t.fail = 0; t.result = 0u; }
     PartHdr ph;
-    ph.mkey = 0; ph.cov = 0; ph.n = 0; ph.cut = 0;
+    ph.mkey = 0; ph.window = 0; ph.n = 0; ph.cut = 0;
     if ((uint32_t)tid < G) ph = hdrs[tid];
     // the row's level 2: a thread sums half of the slices' running sums at one of the 128 sub-bin edges (the
     // 129th is zero by definition; a load instruction reads one slice's consecutive words, sixteen slices'
@@ -527,9 +527,9 @@ __device__ __forceinline__ void wide_finish_row(const Params &p, const StreamVie
     bool bad = false;
     if ((uint32_t)tid < G) {
         const uint64_t *st = v.stash + ((size_t)row * G + tid) * kStashCap;
-        if (!(ph.cov & kWideValid)) bad = true;
+        if (!(ph.window & kWideValid)) bad = true;
         else {
-            const uint32_t wl = ph.cov & 255u, wh = (ph.cov >> 8) & 255u;
+            const uint32_t wl = ph.window & 255u, wh = (ph.window >> 8) & 255u;
             const uint64_t c_hi = st[2 + b2 + 1], c_lo = st[2 + b2];
             mine = pack_count(c_lo) - pack_count(c_hi);
             if (mine) {

@@ -442,7 +442,7 @@ __global__ void __launch_bounds__(kThreads, (R <= 8 ? 5 : RS_STREAM_WAVES)) wide
         if (lane == 0) {
             s.win_lo = wl; s.win_hi = wh; s.n = wn;
             PartHdr ph;
-            ph.mkey = k; ph.cov = ranged ? (wl | wh << 8 | kWideValid) : 0u; ph.n = wn; ph.cut = 0u;
+            ph.mkey = k; ph.window = ranged ? (wl | wh << 8 | kWideValid) : 0u; ph.n = wn; ph.cut = 0u;
             v.hdr[(size_t)row * G + part] = ph;
         }
     }
@@ -477,7 +477,7 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
 
     if (tid == 0) { s.abort = 0; s.host_words = p.host_words; t.fail = 0; t.result = 0u; }
     PartHdr ph;
-    ph.mkey = 0; ph.cov = 0; ph.n = 0; ph.cut = 0;
+    ph.mkey = 0; ph.window = 0; ph.n = 0; ph.cut = 0;
     if ((uint32_t)tid < G) ph = hdrs[tid];
     const uint64_t h0 = rc->rowhist[tid], h1 = rc->rowhist[tid + kThreads];
     rc->rowhist[tid] = 0; rc->rowhist[tid + kThreads] = 0;          // left clean for the next call
@@ -580,7 +580,7 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
     // The row's running sums at the sub-bin edges: the slices' added up (edge 128 is zero by definition).
     // Every thread takes one edge and half of the slices, sixteen slices' loads in flight at a time; what a
     // slice that said nothing left behind is not added.
-    if ((uint32_t)tid < G) t.take[tid] = ph.cov & kWideValid;
+    if ((uint32_t)tid < G) t.take[tid] = ph.window & kWideValid;
     __syncthreads();
     uint32_t Rc = 0;
     u128 Rm = 0;
@@ -642,10 +642,10 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
     uint32_t mine = 0, offs = 0;
     u128 kept_g = 0;                                     // kept weight of slice tid, so far without its listed tokens
     bool bad = false;
-    if ((uint32_t)tid < G && (ph.cov & kWideValid)) {
+    if ((uint32_t)tid < G && (ph.window & kWideValid)) {
         const uint64_t *st = v.stash + ((size_t)row * G + tid) * kStashCap;
         const uint32_t *cum = v.cum + ((size_t)row * G + tid) * kSB;
-        const uint32_t wl = ph.cov & 255u, wh = (ph.cov >> 8) & 255u;
+        const uint32_t wl = ph.window & 255u, wh = (ph.window >> 8) & 255u;
         const uint32_t c_hi = cum[jb + 1], c_lo = cum[jb];
         mine = c_lo - c_hi;
         if (mine) {
