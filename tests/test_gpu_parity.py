@@ -1760,6 +1760,50 @@ def test_row_kernel_two_rows_to_a_compute_unit(torch_cuda, oracle, B, V):
     smp.close()
 
 
+@pytest.mark.parametrize("fmt", ["float32", "bfloat16", "float16"])
+@pytest.mark.parametrize("V", [8192, 12288, 16384, 24576, 32768])
+def test_row_kernel_512_threads_in_every_format_at_the_bounds_of_the_lists(torch_cuda, oracle, V, fmt):
+    """Workgroups of 512 threads with 4, 8, 12 and 16 groups per thread on logits of each format, e of every token
+    included.  The tokens at or above the boundary bin are listed when they are at most a sixth of the row and at most
+    4608, unless one wave's share exceeds 768: rows with that many, one fewer and one more, spread over the row and
+    side by side in one wave's stretch, every row against the general kernel and the first ones against the oracle, in
+    every field (integers: equal)."""
+    torch = torch_cuda
+    from tests import capi
+    B = 320
+    rng = np.random.default_rng(V)
+    bound = min(V // 6, 4608)
+    stretch = (V // 4 + 7) // 8 * 4
+    lg = (-3.0 - 8.0 * rng.random((B, V))).astype(np.float32)
+    want = []
+    for b, (n, spread) in enumerate([(bound - 1, True), (bound, True), (bound + 1, True), (bound + 700, True),
+                                     (767, False), (768, False), (769, False), (min(bound, stretch), False)]):
+        at = rng.choice(V, n, replace=False) if spread else (b % 8) * stretch + np.arange(n)
+        lg[b, at] = 0.25 * rng.random(n)                 # one quarter octave: the boundary bin
+        want.append(n)
+    lg[8:] = 1.5 * rng.standard_normal((B - 8, V))
+    lg = torch.from_numpy(lg).to(getattr(torch, fmt))
+    lg_np = lg[:12].float().numpy()
+    lg = lg.cuda()
+    u_np = H.uniforms(B, V)
+    u = torch.from_numpy(u_np).cuda()
+    smp = capi.Sampler(B, V)
+    for k, p in [(600, 1.0), (V, 0.05)]:
+        rc, c, kk, pp = capi.normalize(1.4426950408889634, k, p, V, B, 1)        # x is the logit, up to rounding
+        print("lists of the row kernel", fmt, V, k, p, flush=True)
+        ref_out, ref_diag, ref_e = oracle.sample_batch(lg_np, c, kk, pp, injected_u=u_np[:12], want_e=True)
+        at_or_above = (ref_e >= (ref_diag["thr_bits"] >> 21 << 21)[:, None]).sum(axis=1)
+        assert list(at_or_above[:8]) == want, at_or_above
+        res = smp.sample(lg, c, kk, pp, uniforms=u, path="row", want_e=True)
+        assert res["rc"] == 0 and smp.status() == 0 and (res["diag"]["rounds"] == 10).all()
+        ref = smp.sample(lg, c, kk, pp, uniforms=u, path="cluster")
+        for f in FIELDS:
+            assert np.array_equal(res["diag"][f], ref["diag"][f]), f
+            assert np.array_equal(res["diag"][f][:12], ref_diag[f]), f
+        assert np.array_equal(res["out"], ref["out"]) and np.array_equal(res["out"][:12], ref_out)
+        assert np.array_equal(res["e_bits"][:12], ref_e)
+
+
 def _us_per_call(torch, sample, fn):
     """Microseconds per call of fn, back to back on the current stream, routed as a program's calls are: the best of
     seven batches of 30, after twelve calls that settle the route."""
