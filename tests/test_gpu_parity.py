@@ -1881,3 +1881,34 @@ def test_streaming_finish_costs_what_its_list_holds(torch_cuda):
                                      ("13 slices with penalties, top_k 1000 and 50", us(8, 50304, 1000, True), us(8, 50304, 50, True), 1.7)]:
         print(what, "%.1f us, %.1f us: %.2f" % (more, fewer, more / fewer), flush=True)
         assert more < bound * fewer, (what, more, fewer)
+
+
+@pytest.mark.parametrize("V,first", [(4096, 0), (4100, 0), (16384, 0), (32772, 0), (262144, 3000), (50260, 500)])
+def test_streaming_finish_short_lists_of_whole_stashes(torch_cuda, oracle, V, first):
+    """A boundary bin of hundreds of tokens of which the stashes hold the largest: lists of up to 64 tokens and of a few
+    more, of top_k tokens and more (the kept set is among them), and of fewer, of which the nucleus needs only some or
+    more than there are (all but the first slice far below: its stash alone counts).  Flat rows and rows of few values,
+    every path against the oracle in every field (integers: equal)."""
+    from tests import capi
+    rng = np.random.default_rng(V)
+    lg = (0.3 * rng.random((3, V))).astype(np.float32)
+    if first:
+        lg[:, first:] -= 5.0
+    lg[1] = np.round(lg[1] * 512) / 512
+    for (k, p) in [(1, 1.0), (2, 0.9), (31, 1.0), (33, 1.0), (40, 0.002), (60, 0.02), (60, 1.0), (63, 1.0), (64, 1.0), (65, 1.0), (70, 0.5)]:
+        _run_case(torch_cuda, oracle, capi, lg, 1.4426950408889634, k, p, u_np=H.uniforms(3, k), what="short lists V=%d k=%d p=%g" % (V, k, p))
+
+
+def test_streaming_finish_of_flat_rows_in_calls_of_many(torch_cuda):
+    """Flat rows of 4096 tokens with a small top_k, whose lists come out of whole stashes, against rows of the same call
+    that leave short lists at once: short lists are finished the same way wherever they come from.  Time ratio,
+    measured 1.40; 1.83 when lists out of whole stashes took the digits of longer ones."""
+    torch = torch_cuda
+    import rapid_sampling_amd as sample
+    gen = torch.Generator(device="cuda").manual_seed(4)
+    flat = torch.rand((1024, 4096), generator=gen, device="cuda")
+    peaked = torch.randn((1024, 4096), generator=gen, device="cuda").mul_(3.0)
+    st = sample.setup_rand(1, 1024)
+    a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_temperature_topk_topp(x, st, 1.0, 1, 1.0)) for x in (flat, peaked))
+    print("flat %.1f us, peaked %.1f us: %.2f" % (a, b, a / b), flush=True)
+    assert a < 1.6 * b, (a, b)
