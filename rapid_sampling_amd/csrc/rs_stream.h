@@ -748,6 +748,9 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     constexpr int  W = NT / kWave;
     constexpr bool kEach = NT == kThreads;               // every wave for itself
     static_assert(NT == 256 || NT == 1024, "one or four waves per SIMD");
+    // the tokens asked for ahead may be listed a second time (FUSED with PRE = 16 never would, its list holds 2048 tokens, and has
+    // no registers to keep them in)
+    constexpr bool kAgain = !(FUSED && PRE > 8);
     const int tid = threadIdx.x, lane = tid & (kWave - 1);
     const int wave = (int)uniform((uint32_t)tid >> 6);
     const uint32_t G = v.G;
@@ -958,17 +961,19 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         const uint32_t lb = bin - kBin0 + 4u * dl;       // the boundary bin in the slice's frame; past its last bin: nothing of the slice is live
         if (lb < (uint32_t)kSB) above_cut = get<FUSED>(&v.cum[((size_t)row * G + (uint32_t)tid) * kSB + lb]);
     }
-    if (ahead) {
+    // The tokens asked for ahead, those at or above `from` of them into the list.  Called by all threads together, s.ctr = 0.
+    auto list_ahead = [&](const uint32_t from) -> uint32_t {
         // lane i looks after the wave's i-th slice: how far its frame lies below the row's, how many tokens it stashed
         const uint32_t sl = (uint32_t)(wave + W * lane);
         const uint2 h = hd[min(sl, G - 1u)];
         const uint32_t below = octaves_below(h.x), len = sl < G ? min(h.y, (uint32_t)kWave) : 0u;
+        uint64_t e[PRE];
         uint32_t mine = 0;                               // of this lane's tokens, how many
 #pragma unroll
         for (int i = 0; i < PRE; ++i) {
             const uint32_t b = rebase_bits((uint32_t)(pre[i] >> 32), lane_of(below, (uint32_t)i));
-            const bool in = (uint32_t)lane < lane_of(len, (uint32_t)i) && b >= cut;
-            pre[i] = ((uint64_t)(in ? b : 0u) << 32) | (uint32_t)pre[i];
+            const bool in = (uint32_t)lane < lane_of(len, (uint32_t)i) && b >= from;
+            e[i] = ((uint64_t)(in ? b : 0u) << 32) | (uint32_t)pre[i];
             mine += in ? 1u : 0u;
         }
         const uint32_t upto = wave_inclusive_scan(mine);
@@ -978,13 +983,16 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         {
             // (a branch per entry would cost more than the store: what is not listed goes into a corner of its own)
             typedef __attribute__((address_space(3))) uint64_t lds_u64;
-            const bool in = (uint32_t)(pre[i] >> 32) != 0u;
+            const bool in = (uint32_t)(e[i] >> 32) != 0u;
             lds_u64 *to = in ? (lds_u64 *)list + at : (lds_u64 *)t.small + lane;
-            *to = pre[i];
+            *to = e[i];
             at += in ? 1u : 0u;
         }
         __syncthreads();
-        n = uniform(s.ctr);
+        return uniform(s.ctr);
+    };
+    if (ahead) {
+        n = list_ahead(cut);
         listed = n == total;                             // every token at or above the boundary bin is there
     }
     if (!listed) {
@@ -1069,12 +1077,13 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         const uint32_t len = (uint32_t)tid < G ? min(ph.n, (uint32_t)kStashCap) : 0u;
         uint32_t from = (uint32_t)tid < G ? max(rebase_bits(ph.cut, dl), kEMinBits) : 0u;
         from = wave_max_u32(from);
+        uint32_t longer = __builtin_amdgcn_ballot_w64(len > (uint32_t)kWave) != 0ull ? 1u : 0u;        // some stash than what was asked for ahead
         __syncthreads();
-        if (lane == 0) t.take[wave] = from;
+        if (lane == 0) { t.take[wave] = from; t.take[W + wave] = longer; }
         __syncthreads();
 #pragma unroll
-        for (int w = 0; w < kMaxParts / kWave; ++w) from = max(from, t.take[w]);
-        from = uniform(from);
+        for (int w = 0; w < kMaxParts / kWave; ++w) { from = max(from, t.take[w]); longer |= t.take[W + w]; }
+        from = uniform(from); longer = uniform(longer);
         bool slow = false;
         if (from <= cut && total <= v.list_cap) {        // plan A: every stash reaches down to the boundary bin
             // exactly the tokens at or above that bin: of every stash a prefix, whose first 64 are listed already
@@ -1089,6 +1098,13 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
                         if ((uint32_t)u < m) list[had + i + (uint32_t)u] = ((uint64_t)bits[u] << 32) | idx[u];
                 });
             __syncthreads();
+        } else if (kAgain && !longer && G <= (uint32_t)(W * PRE) && G * (uint32_t)kWave <= v.list_cap) {
+            // plan B, the stashes whole, every one of them asked for ahead (320 flat rows of 8192 with penalties, top_k 50:
+            // 23.2 us a call from the stashes again, 22.6 this way)
+            if (tid == 0) s.ctr = 0u;                    // (it has been read)
+            __syncthreads();
+            n = list_ahead(from);
+            subset = true;
         } else if (const uint32_t all = take_prefix(len); !FUSED && all > min(v.list_cap, max(2048u, 3u * top_k)) && top_k <= v.list_cap / 2u) {
             // Plan B (flat distributions: the boundary bin holds thousands of tokens, but top_k is small) with more
             // stashed tokens than the list holds, or several times top_k of them.  The kept set is at most
@@ -1267,33 +1283,37 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     uint32_t sh = 32u - (uint32_t)__builtin_clz((uint32_t)p.V - 1u | 1u);
     sh = sh > kLogNT ? sh - kLogNT : 0u;
     uint32_t lo_idx = 0, len = (uint32_t)p.V;
-    for (int step = 0;; ++step) {
-        for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
-            const uint64_t e = list[i];
-            const uint32_t off = (uint32_t)e - lo_idx;
-            const uint64_t w = weight((uint32_t)(e >> 32));
-            if (w && off < len) {
-                atomicAdd(reinterpret_cast<unsigned long long *>(&bk_lo[off >> sh]), (unsigned long long)(w & 0xFFFFFFFFull));
-                atomicAdd(reinterpret_cast<unsigned long long *>(&bk_hi[off >> sh]), (unsigned long long)(w >> 32));
+    // (kept tokens few enough for one wave as they are: no buckets.  320 flat rows of 8192 with penalties, top_k 50: 23.6 -> 23.2 us a call)
+    bool few = f.cnt_above + f.cnt_bin <= (uint32_t)kWave;
+    for (;; few = false) {
+        if (!few) {
+            for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+                const uint64_t e = list[i];
+                const uint32_t off = (uint32_t)e - lo_idx;
+                const uint64_t w = weight((uint32_t)(e >> 32));
+                if (w && off < len) {
+                    atomicAdd(reinterpret_cast<unsigned long long *>(&bk_lo[off >> sh]), (unsigned long long)(w & 0xFFFFFFFFull));
+                    atomicAdd(reinterpret_cast<unsigned long long *>(&bk_hi[off >> sh]), (unsigned long long)(w >> 32));
+                }
             }
+            __syncthreads();
+            const M96 mine = m96((u128)bk_lo[tid] + ((u128)bk_hi[tid] << 32));
+            bk_lo[tid] = 0; bk_hi[tid] = 0;
+            M96 inc = m96(wave_inclusive_scan(limbs(mine)));
+            M96 *waves = reinterpret_cast<M96 *>(&s.wj[0][0]);
+            static_assert(sizeof(s.wj) >= 16 * sizeof(M96), "one mass per wave");
+            if (lane == kWave - 1) waves[wave] = inc;
+            __syncthreads();
+            {
+                const Limbs tot = wave_inclusive_scan(limbs(lane < W ? waves[lane] : M96{0ull, 0u}));
+                if (wave) inc = inc + m96(lane_of(tot, (uint32_t)wave - 1u));
+            }
+            const M96 exc = inc - mine;
+            if (exc < r && inc >= r) { t.bucket = (uint32_t)tid; t.one.above = r - exc; }
+            __syncthreads();
+            lo_idx += uniform(t.bucket) << sh; len = 1u << sh;
+            r = uniform(t.one.above);
         }
-        __syncthreads();
-        const M96 mine = m96((u128)bk_lo[tid] + ((u128)bk_hi[tid] << 32));
-        bk_lo[tid] = 0; bk_hi[tid] = 0;
-        M96 inc = m96(wave_inclusive_scan(limbs(mine)));
-        M96 *waves = reinterpret_cast<M96 *>(&s.wj[0][0]);
-        static_assert(sizeof(s.wj) >= 16 * sizeof(M96), "one mass per wave");
-        if (lane == kWave - 1) waves[wave] = inc;
-        __syncthreads();
-        {
-            const Limbs tot = wave_inclusive_scan(limbs(lane < W ? waves[lane] : M96{0ull, 0u}));
-            if (wave) inc = inc + m96(lane_of(tot, (uint32_t)wave - 1u));
-        }
-        const M96 exc = inc - mine;
-        if (exc < r && inc >= r) { t.bucket = (uint32_t)tid; t.one.above = r - exc; }
-        __syncthreads();
-        lo_idx += uniform(t.bucket) << sh; len = 1u << sh;
-        r = uniform(t.one.above);
         // the kept tokens of the bucket: few enough for one wave, as a rule; otherwise the bucket is cut into NT again
         for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
             const uint64_t e = list[i];
@@ -1737,7 +1757,10 @@ __device__ __forceinline__ bool fused_fallback(const Params &p, const StreamView
     return slice_finish(p, s, sl);
 }
 
-template <int R, bool PEN>
+// PRE: slices per wave whose first tokens the finishing workgroup asks for ahead (the host's choice, as for finish_kernel).
+// With 16 whatever the row and the random number drawn before the slice was asked for, 320 rows of 8192 tokens, two slices
+// each, N(0,2) with 16 large logits in 4096, top_k 50, took 19.0 us a call; 17.4 this way.
+template <int R, bool PEN, int PRE>
 __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, const StreamView v)
 {
     constexpr int kRep = stream_copies<R>();
@@ -1760,13 +1783,12 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
     Slice<R, PEN> sl;
     slice_setup(p, sl, row, part, G);
     RowCtl *rc = sl.rc;
-    // the row's random number, should this workgroup be the one that finishes the row: drawn while the slice is on its way
-    uint64_t drawn = 0;
+    // the row's generator state is asked for ahead of the slice and used behind it
+    uint32_t rs[6] = {0u, 0u, 0u, 0u, 0u, 0u};
+    uint32_t *st = p.rng + (size_t)row * 16;
     if (tid == kWave && !p.inj_u) {
-        const uint32_t *st = p.rng + (size_t)row * 16;
-        uint32_t o[4];
-        philox4x32_10(st[2], st[3], st[4], st[5], st[0], st[1], o);
-        drawn = ((uint64_t)o[0] << 32) | o[1];
+#pragma unroll
+        for (int i = 0; i < 6; ++i) rs[i] = st[i];
     }
     const float lmax = slice_load(p, sl);
     const uint32_t key = slice_count_and_stash<R, kThreads, kRep, true>(p, v, u.a, sl.eb, lmax, row, part, sl.base4, sl.nv);
@@ -1778,6 +1800,13 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
 #ifndef RS_FUSED_RELAXED
 #define RS_FUSED_RELAXED 1
 #endif
+    // the row's random number, should this workgroup be the one that finishes the row: drawn while the stores are on their way
+    uint64_t drawn = 0;
+    if (tid == kWave && !p.inj_u) {
+        uint32_t o[4];
+        philox4x32_10(rs[2], rs[3], rs[4], rs[5], rs[0], rs[1], o);
+        drawn = ((uint64_t)o[0] << 32) | o[1];
+    }
     wait_vmem();
     __syncthreads();
     if (tid == 0)
@@ -1794,12 +1823,10 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
         // the token list: the cluster rounds' histogram copies, which are not in use while a row is
         // finished from the stashes (no dynamic LDS in this kernel: see rs_sample_ex)
         static_assert(sizeof(s.hr) == 2048 * sizeof(uint64_t), "room for a list of 2048 tokens");
-        const bool done = finish_row<kThreads, 16, true>(p, v, s, t, s.hr, row, drawn);
+        const bool done = finish_row<kThreads, PRE, true>(p, v, s, t, s.hr, row, drawn);
         if (done && tid == kWave && !p.inj_u) {
-            uint32_t *st = p.rng + (size_t)row * 16;     // the row is finished: this draw is used up
-            const uint32_t next = st[2] + 1u;
-            st[2] = next;
-            if (next == 0u) st[3] += 1u;
+            st[2] = rs[2] + 1u;                          // the row is finished: this draw is used up
+            if (rs[2] + 1u == 0u) st[3] = rs[3] + 1u;
         }
         __syncthreads();
         verdict = done && t.result != 0u ? t.result : kVerdictFallback;

@@ -59,14 +59,17 @@ hipError_t launch_fused(int slice_r, bool pen, uint32_t B, hipStream_t st, const
 {
     const dim3 grid(B * v.G), block(kThreads);
     if (v.list_cap > 2048u) return hipErrorInvalidValue;      // the list lives in static LDS
-#define RS_FUSED(Rv) do { if (pen) hipLaunchKernelGGL((fused_kernel<Rv, true>), grid, block, 0, st, p, v);          \
-                          else hipLaunchKernelGGL((fused_kernel<Rv, false>), grid, block, 0, st, p, v); } while (0)
+    // (slices asked for ahead: launch_finish)
+#define RS_FUSED_PRE(Rv, PREv) do { if (pen) hipLaunchKernelGGL((fused_kernel<Rv, true, PREv>), grid, block, 0, st, p, v);          \
+                                    else hipLaunchKernelGGL((fused_kernel<Rv, false, PREv>), grid, block, 0, st, p, v); } while (0)
+#define RS_FUSED(Rv) do { if (v.G <= 16u) RS_FUSED_PRE(Rv, 4); else if (v.G <= 32u) RS_FUSED_PRE(Rv, 8); else RS_FUSED_PRE(Rv, 16); } while (0)
     switch (slice_r) {
     case 4:  RS_FUSED(4); break;
     case 8:  RS_FUSED(8); break;
     default: RS_FUSED(16); break;
     }
 #undef RS_FUSED
+#undef RS_FUSED_PRE
     return hipGetLastError();
 }
 
