@@ -261,8 +261,8 @@ int rs_philox_init(void *state_device, uint64_t seed, int32_t B, void *stream);
  * the guess against the exact counts), one again for such kept sets in rows of
  * 8192 to 65536 tokens when the call has 64 rows (128 from 32768 tokens on)
  * or more (the row kernel: one workgroup of 512 or 1024 threads per row, the
- * row in its registers; not calls of 257 to 319 rows, nor of 320 to 511 rows
- * of 32769 to 39999 tokens), or three for calls of at least
+ * row in its registers; not calls of 257 to 319 rows of up to 32768 tokens, nor
+ * of 257 to 511 rows of 32769 to 39999 tokens), or three for calls of at least
  * 2^23 tokens with penalties and top_k <= 1024 (a pass over logits and
  * penalties that also writes the decayed penalties, the finish, which patches
  * the sampled tokens' penalties, and a fix-up kernel for slices the pass left

@@ -401,8 +401,9 @@ constexpr uint64_t kPenStreamMin = 1ull << 23;
 //   768 x 12288       35 / 36      33 / 31          288 x 32000       44 / 42      36 / 34
 //   512 x 16384       33 / 33      24 / 22          512 x 32000       58 / 54      39 / 37
 //  2048 x 16384       90 / 96      80 / 75         2048 x 32000      193 / 184    137 / 126
-// All 49 shapes measured from 288 to 2048 rows of 8192 to 32768 tokens are faster here.  (Calls of 257 to 319
-// rows, which are too, stay where they were: the route of 300 such rows is fixed by a test.)
+// All 49 shapes measured from 288 to 2048 rows of 8192 to 32768 tokens are faster here.  The 320 below is no
+// crossover: calls of 257 to 319 such rows stay where they always were, a bound kept for compatibility (the route
+// of 300 of them is fixed by a test).
 static bool row_suits(int32_t B, int32_t V)
 {
     if (V > kRowMaxV || V < 8192) return false;
@@ -542,7 +543,7 @@ using namespace rs;
 
 extern "C" {
 
-int rs_version(void) { return 415; }
+int rs_version(void) { return 416; }
 
 const char *rs_error_string(int code)
 {
@@ -817,15 +818,19 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
         p.report = path == kPathKeep ? 0u : (uint32_t)policy_word(kind, size_class(B, V));
         p.attempt = path == kPathAttempt ? 1u : 0u;
         p.probe = path == kPathProbe ? 1u : 0u;
-        // A nucleus of thousands of tokens is finished from the stashes all the same, but one workgroup going through
-        // such a list a dozen times takes longer than the general kernel needs for the whole call (measured:
-        // 128 rows of 50304, about 4000 tokens each, 54 against 36 us; the two meet at about 2400 tokens
-        // there and, the general kernel's time growing with the row, at about 4700 for rows of 100256): a
-        // call that is only an attempt (no top_k bounds the kept set) says so to the caller's policy, and so
-        // does a call of moderate size with a bounding top_k (a lone flat row of 32768 tokens with top_k 1000:
-        // 26.7 us here against 17.5 on the general kernel).  Small calls in rows of up to 100256 tokens meet the
-        // general kernel earlier: a list of a thousand tokens takes one to sixteen such rows 21-27 us here
-        // against 18-21 there (lists of a few hundred: 12-14 us here).
+        // A list of thousands of tokens is finished all the same, but one workgroup going through it a dozen
+        // times may take longer than the general kernel needs for the whole call: a call that is only an attempt
+        // (no top_k bounds the kept set) says so to the caller's policy, and so does a call of moderate size with a
+        // bounding top_k.  Counted are the tokens of the list: those at or above the boundary bin or, out of
+        // whole stashes, at or above the value down to which all stashes are complete.  Here / general kernel, us a call:
+        //   128 x  50304 N(0,1.5), 400 / 1000 / 2000 / 2600 tokens kept      23 / 33   25 / 35   28 / 35   31 / 37
+        //    64 x 100256 N(0,1.5), 600 / 1000 / 2100                         21 / 27   23 / 28   28 / 29
+        //     8 x  50304 N(0,1.5), 140 / 450 / 1100 / 2000                   13 / 16   14 / 17   18 / 17   21 / 17
+        //     1 x  32768, 50304 and 100256 N(0,1.5), top_k 300               13 / 15   13 / 15   13 / 17
+        //                                            top_k 1000              18 / 16   17 / 17   15 / 17
+        //    16 x  32768, 50304 and 100256 N(0,1.5), top_k 1000              18 / 17   18 / 19   18 / 22
+        // So small calls meet the general kernel at lists of about a thousand tokens in rows of 32768 and later in
+        // longer ones, larger calls beyond 2600; the bounds below are a little on the general kernel's side.
         if (p.attempt || p.tell_lists) {
             const bool small_call = (uint64_t)B * (uint64_t)V < (1ull << 20) && V < 131072;
             p.long_list = small_call ? 768u : max(2048u, (uint32_t)V / 20u);

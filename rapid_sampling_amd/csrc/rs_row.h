@@ -7,10 +7,11 @@
 // workgroup: the maximum, e, the level-1 histogram in LDS, the radix selection of the threshold
 // level by level (level 2 on the registers, the deeper ones on a list of the boundary bin's tokens
 // in LDS when they fit), tie weight and target, and the pick by sums and scans of the kept weights
-// in index order.  Its time hardly depends on the kept set, only on the row: it is the time of the
-// vector instructions of e and of three passes over the registers, 64 tokens per thread with four
-// waves per SIMD (measured, launch included: 14-18 us for 8192 tokens, 26 for 32768, 33 for 50304,
-// 42 for 65536); a call of B rows takes ceil(B / 256) such times, or ceil(B / 512) times 17, 24 and 39 us in
+// in index order.  With more than a sixth of the row at or above the boundary bin its time hardly depends on the
+// kept set, only on the row: it is the time of the vector instructions of e and of three passes over the
+// registers, 64 tokens per thread with four waves per SIMD; with less, everything behind e and level 1 reads lists
+// (below), and the call takes a sixth to a fifth less.  Measured with more, launch included: 14-18 us for 8192 tokens,
+// 26 for 32768, 33 for 50304, 42 for 65536; a call of B rows takes ceil(B / 256) such times, or ceil(B / 512) times 17, 24 and 39 us in
 // rows of 8192, 16384 and 32768 tokens.  For kept sets of thousands of
 // tokens in calls of 64 rows and more that is less than the general kernel's exchanges or the wide
 // paths' launches cost; small calls and small kept sets are better off elsewhere.  Same integers as

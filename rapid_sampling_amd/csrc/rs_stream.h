@@ -26,9 +26,9 @@ namespace rs {
 //                   that cannot be finished from the stashes (a huge tie, a
 //                   nucleus of thousands of tokens) it does alone, from the
 //                   logits (finish_row_slow).
-// A call that keeps every live token (top_k = V, top_p = 1) runs both kernels as a variant (KEEP):
-// the pass stops behind the histogram and leaves each slice's mass, the finishing workgroup picks
-// the slice from the masses and reads that one slice again (keep_pick).
+// For a call that keeps every live token (top_k = V, top_p = 1) the pass (KEEP) stops behind the histogram
+// and leaves each slice's mass, one sum for every distance its frame may lie below the row's, where the
+// stash would begin; keep_finish_kernel picks the slice from those and reads that one slice again.
 // Lanes of a wave that add to one LDS address are served one after the other, and rows often put
 // most of their tokens into a few bins.  So each bin is kept in kRep copies (lane l adds to copy
 // l % kRep), and e is not clamped before it is counted: the histogram spans all 512 values of
@@ -579,7 +579,7 @@ __device__ __forceinline__ void finish_row_slow(const Params &p, Lds &s, LdsB &t
     }
 }
 
-// The token of a row of a call that keeps everything: the slice that begins at token lo_idx holds
+// The last step of the wide paths' finishes: the slice that begins at token lo_idx holds
 // the target, r is the target's offset inside the slice.  The slice is gone through in chunks of
 // 64 float4 groups (256 consecutive tokens, one KB that a wave loads in one go): chunk c belongs
 // to wave c mod 4, which sums its tokens' weights (two 64-bit wave sums of the weights' halves);
@@ -588,8 +588,8 @@ __device__ __forceinline__ void finish_row_slow(const Params &p, Lds &s, LdsB &t
 // atomics, no list.  (An earlier version gave every thread 16 consecutive groups: its loads, 64
 // cache lines per instruction and every line touched by 8 instructions, cost a microsecond per
 // group.)  No penalties on this path.
-// `kept`: weight of a token from the bit pattern of its e in the row's frame (its full weight when the
-// call keeps every live token; on the wide path what the threshold and the tie weight leave of it).
+// `kept`: what the threshold and the tie weight leave of a token's weight, from the bit pattern of its e in the
+// row's frame.
 template <int SLICE_LOG2, typename WF>
 __device__ __forceinline__ void keep_pick(const Params &p, Lds &s, LdsB &t, const uint32_t row, const float M, const uint32_t lo_idx, const u128 r,
                                           WF kept)
@@ -1147,7 +1147,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
                 subset = true;
                 // Two more passes over the stashes make this finish slower than the general kernel's whole
                 // call while the call is of moderate size (measured: 64 flat rows of 131072 with top_k 1000,
-                // 51 against 38 us; 128 rows of 262144, 77 against 117): such a call says so to the caller's
+                // 44 against 38 us; 128 rows of 262144, 68 against 116): such a call says so to the caller's
                 // policy, as it did when these rows still went the slow way.
                 // (p.tell_lists: calls of fewer than 2^24 tokens, and calls whose rows the row kernel would take)
                 if (p.tell_lists) tell_policy();

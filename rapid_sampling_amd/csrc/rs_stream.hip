@@ -24,7 +24,8 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
 {
     const dim3 sgrid(B * v.G);
     if (keep && v.G > 2u * kWave) return hipErrorInvalidValue;             // keep_finish_kernel holds two slices per lane
-    // keep: the call keeps every live token; its kernels neither fill nor read stashes, and the finish needs no list.
+    // keep: the call keeps every live token; what its pass leaves at the head of each slice's stash are masses, and its finish
+    // needs no list.
     // NTv threads with Rv groups of four tokens each: a slice of 4 Rv NTv tokens
 #ifndef RS_LONG_NT
 #define RS_LONG_NT 256

@@ -466,7 +466,7 @@ def test_row_kernel_takes_the_wide_kept_sets_of_calls_of_many_short_rows(torch_c
     """Calls of 128 rows and more (64 in rows of fewer than 32768 tokens) of 8192 to 65536 tokens whose kept
     sets the stashes cannot hold go to the row kernel by themselves (diag.rounds == 10): a top_k of
     thousands at once, a nucleus once the probe has reported its long lists; fewer rows, longer rows, 257
-    to 319 rows of up to 32768 tokens and calls with a bounding top_k do not.  Every call against the general kernel in every field, 64 rows of each against the oracle."""
+    to 319 rows of up to 32768 tokens (and 257 to 511 of 32769 to 39999) and calls with a bounding top_k do not.  Every call against the general kernel in every field, 64 rows of each against the oracle."""
     torch = torch_cuda
     from tests import capi
     for (B, V, k, p, row) in [(128, 50304, 10000, 1.0, True), (300, 16384, 5000, 1.0, False), (200, 16384, 5000, 1.0, True),
@@ -1691,7 +1691,7 @@ def test_chi_square_one_million_draws(torch_cuda, oracle):
 def test_finish_at_the_edges_of_its_variants(torch_cuda, oracle, V):
     """The streaming finish asks ahead for the first tokens of 16, 32 or 64 slices (rows of that many slices and of
     one more), takes lists of up to 64 tokens by pairs and longer ones by digits, and has 1024 threads from
-    a top_k of 257 on: rows of distinct values, of ties at the threshold and a row with few live tokens, lists
+    a top_k of 257 on in rows of 32 slices and more: rows of distinct values, of ties at the threshold and a row with few live tokens, lists
     just below and above each bound, every path against the oracle in every field (integers: equal)."""
     from tests import capi
     rng = np.random.default_rng(V)
