@@ -173,10 +173,13 @@ __device__ __forceinline__ bool slice_level1(const Params &p, Lds &s, Slice<R, P
     // back with the histogram, in the same polling rounds.
     const float Mloc = __builtin_floorf(fkey_inv(kmax_row));
     const uint32_t pos0 = G > 1 ? (uint32_t)(int)(Mloc - 128.0f * __builtin_floorf(Mloc * 0.0078125f)) * 4u - 508u : 0u;
+    auto frame = [&]() { if constexpr (PEN) return Mloc; else return frame_of(Mloc, eb); };        // (which form is the faster: see Frame)
+    const auto fr = frame();
+    auto bits_of = [&](float x) { if constexpr (PEN) return e_bits_of(x, fr); else return fr.bits(x); };
 #pragma unroll
     for (int j = 0; j < R; ++j) {
 #pragma unroll
-        for (int k = 0; k < 4; ++k) eb[j * 4 + k] = e_bits_of(__uint_as_float(eb[j * 4 + k]), Mloc);
+        for (int k = 0; k < 4; ++k) eb[j * 4 + k] = bits_of(__uint_as_float(eb[j * 4 + k]));
         if (j < nv) {
 #pragma unroll
             for (int k = 0; k < 4; ++k) {
