@@ -954,12 +954,19 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     bool listed = false, subset = false;
     const bool ahead = total <= v.list_cap && G <= (uint32_t)(W * PRE);
     // How many tokens of slice tid lie at or above the boundary bin, as its workgroup counted them: asked for while the
-    // first ones go into the list, unless those are certain to be all.
-    const uint32_t dl = (uint32_t)tid < G ? octaves_below(ph.mkey) : 0u;
+    // first ones go into the list if those may well not be all (more than 40 a slice on average), else when they are not.
+    auto octaves = [&]() { return (uint32_t)tid < G ? octaves_below(ph.mkey) : 0u; };
+    auto count_above = [&]() -> uint32_t {
+        const uint32_t lb = bin - kBin0 + 4u * octaves();   // the boundary bin in the slice's frame; past its last bin: nothing of the slice is live
+        return (uint32_t)tid < G && lb < (uint32_t)kSB ? get<FUSED>(&v.cum[((size_t)row * G + (uint32_t)tid) * kSB + lb]) : 0u;
+    };
+    const bool likely = !ahead || total > max((uint32_t)kWave, 40u * G);
     uint32_t above_cut = 0;
-    if ((total > (uint32_t)kWave || !ahead) && (uint32_t)tid < G) {
-        const uint32_t lb = bin - kBin0 + 4u * dl;       // the boundary bin in the slice's frame; past its last bin: nothing of the slice is live
-        if (lb < (uint32_t)kSB) above_cut = get<FUSED>(&v.cum[((size_t)row * G + (uint32_t)tid) * kSB + lb]);
+    if (likely) {
+        // (The first tokens have long arrived.  Said here, because behind a load that not every thread makes the compiler
+        // waits for that load, too, before it touches them.)
+        __builtin_amdgcn_s_waitcnt(0x0F70);              // vmcnt(0)
+        above_cut = count_above();
     }
     // The tokens asked for ahead, those at or above `from` of them into the list.  Called by all threads together, s.ctr = 0.
     auto list_ahead = [&](const uint32_t from) -> uint32_t {
@@ -995,7 +1002,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         n = list_ahead(cut);
         listed = n == total;                             // every token at or above the boundary bin is there
     }
-    if (!listed) {
+    if (__builtin_expect(!listed, 0)) {                  // (out of the way of the usual call's instructions)
         // Prefixes of the stashes, one after the other: t.take[g] = entries of slices 0..g.  Returns how many in all.
         auto take_prefix = [&](uint32_t mine) -> uint32_t {
             uint32_t inc = wave_inclusive_scan(mine);
@@ -1012,42 +1019,46 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             __syncthreads();
             return uniform(sum);
         };
-        // fn(first, how many, bits of e in the row's frame, tokens) for the n_all entries t.take speaks of, those of a
-        // slice from entry `skip` on, eight of a thread at a time and in flight together; a thread has a run of consecutive ones, so that
-        // all threads have as many wherever they lie, and looks up its first slice once.  Called by all threads together.
+        // fn(i, step, bits of e in the row's frame, tokens) for the n_all entries t.take speaks of, those of a slice from entry
+        // `skip` on: eight of a thread at a time and in flight together, entries i, i + step, ... (bits 0 past the last).  A
+        // thread looks up the slice of its first entry and walks on from there.  Many entries per slice: neighbouring
+        // threads read neighbouring entries (512 flat rows of 131072 with top_k 1000 104 us a call, 114 in runs); few: a thread reads a run of them, which
+        // takes it over fewer slices (one row of 524288 in 128 slices with top_k 200: 15 us a call, 19.7 with neighbours).
+        // Called by all threads together.
         constexpr int kBatch = 8;
         auto stashed = [&](const uint32_t n_all, const uint32_t skip, auto fn) {
             const uint32_t per = (n_all + (uint32_t)NT - 1u) / (uint32_t)NT;
-            const uint32_t i0 = (uint32_t)tid * per, iend = min(n_all, i0 + per);
-            uint32_t g = 0, hi_g = G - 1u;                             // first slice whose prefix exceeds i0
+            const bool dense = n_all >= 64u * G;
+            const uint32_t first = dense ? (uint32_t)tid : (uint32_t)tid * per, step = dense ? (uint32_t)NT : 1u;
+            uint32_t g = 0, hi_g = G - 1u;                             // first slice whose prefix exceeds the first entry
             while (g < hi_g) {
                 const uint32_t mid = (g + hi_g) >> 1;
-                if (t.take[mid] > i0) hi_g = mid; else g = mid + 1u;
+                if (t.take[mid] > first) hi_g = mid; else g = mid + 1u;
             }
             uint32_t gend = t.take[g];
             const uint64_t *from_g = stash + (size_t)g * kStashCap + skip - (g ? t.take[g - 1u] : 0u);
             for (uint32_t k = 0; k < per; k += (uint32_t)kBatch) {
-                const uint32_t i = i0 + k, m = i < iend ? min((uint32_t)kBatch, iend - i) : 0u;
                 uint64_t e[kBatch];
                 uint32_t d[kBatch];
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
+                    const uint32_t i = first + (k + (uint32_t)u) * step;
                     e[u] = 0; d[u] = 0;
-                    if ((uint32_t)u < m) {
-                        while (i + (uint32_t)u >= gend) {              // slices that give nothing are skipped
+                    if (k + (uint32_t)u < per && i < n_all) {
+                        while (i >= gend) {                            // slices that give nothing are skipped
                             ++g; from_g = stash + (size_t)g * kStashCap + skip - gend; gend = t.take[g];
                         }
-                        e[u] = get<FUSED>(&from_g[i + (uint32_t)u]);
+                        e[u] = get<FUSED>(&from_g[i]);
                         d[u] = t.delta[g];
                     }
                 }
                 uint32_t bits[kBatch], idx[kBatch];
 #pragma unroll
                 for (int u = 0; u < kBatch; ++u) {
-                    bits[u] = (uint32_t)u < m ? rebase_bits((uint32_t)(e[u] >> 32), d[u]) : 0u;
+                    bits[u] = (uint32_t)(e[u] >> 32) ? rebase_bits((uint32_t)(e[u] >> 32), d[u]) : 0u;
                     idx[u] = (uint32_t)e[u];
                 }
-                fn(i, m, bits, idx);
+                fn(first + k * step, step, bits, idx);
             }
         };
         // the tokens at or above `from` among them, side by side
@@ -1071,7 +1082,9 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             __syncthreads();
             return uniform(s.ctr);
         };
+        const uint32_t dl = octaves();
         if ((uint32_t)tid < G) t.delta[tid] = dl;
+        if (!likely) above_cut = count_above();
         // Together the stashes hold every token of the row at or above `from`, the largest of the slices' cuts.  (A
         // cut that lands below 2^-40 in the row's frame: what the stash lacks is dead there.)
         const uint32_t len = (uint32_t)tid < G ? min(ph.n, (uint32_t)kStashCap) : 0u;
@@ -1085,6 +1098,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         for (int w = 0; w < kMaxParts / kWave; ++w) { from = max(from, t.take[w]); longer |= t.take[W + w]; }
         from = uniform(from); longer = uniform(longer);
         bool slow = false;
+        uint32_t list_all = 0;                           // stashed tokens to go through for those at or above `from`
         if (from <= cut && total <= v.list_cap) {        // plan A: every stash reaches down to the boundary bin
             // exactly the tokens at or above that bin: of every stash a prefix, whose first 64 are listed already
             const uint32_t skip = ahead ? (uint32_t)kWave : 0u, had = n, take = min(above_cut, len);
@@ -1092,10 +1106,10 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             n = had + rest;
             slow = n != total;
             if (!slow)
-                stashed(rest, skip, [&](uint32_t i, uint32_t m, const uint32_t (&bits)[kBatch], const uint32_t (&idx)[kBatch]) {
+                stashed(rest, skip, [&](uint32_t i, uint32_t step, const uint32_t (&bits)[kBatch], const uint32_t (&idx)[kBatch]) {
 #pragma unroll
                     for (int u = 0; u < kBatch; ++u)
-                        if ((uint32_t)u < m) list[had + i + (uint32_t)u] = ((uint64_t)bits[u] << 32) | idx[u];
+                        if (bits[u]) list[had + i + (uint32_t)u * step] = ((uint64_t)bits[u] << 32) | idx[u];
                 });
             __syncthreads();
         } else if (kAgain && !longer && G <= (uint32_t)(W * PRE) && G * (uint32_t)kWave <= v.list_cap) {
@@ -1143,8 +1157,8 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             const uint32_t step = uniform(s.bc32[4]), nge = uniform(s.bc32[5]);
             slow = step >= 511u || nge > v.list_cap;     // fewer than top_k at or above `from`, or one value thousands of times
             if (!slow) {
-                n = list_from(all, max(from, (topkey - step) << 14));
-                subset = true;
+                list_all = all;
+                from = max(from, (topkey - step) << 14);
                 // Two more passes over the stashes make this finish slower than the general kernel's whole
                 // call while the call is of moderate size (measured: 64 flat rows of 131072 with top_k 1000,
                 // 44 against 38 us; 128 rows of 262144, 68 against 116): such a call says so to the caller's
@@ -1154,8 +1168,9 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             }
         } else {                                         // plan B, the stashes whole
             slow = all > v.list_cap || all == 0u;
-            if (!slow) { n = list_from(all, from); subset = true; }
+            if (!slow) list_all = all;
         }
+        if (list_all) { n = list_from(list_all, from); subset = true; }
         // A short list of at least top_k tokens holds the kept set; of any other it is the listed tokens' own bins that say
         // whether it does.
         if (!slow && subset && (n < top_k || n > (uint32_t)kWave)) {
@@ -1285,6 +1300,8 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     uint32_t lo_idx = 0, len = (uint32_t)p.V;
     // (kept tokens few enough for one wave as they are: no buckets.  320 flat rows of 8192 with penalties, top_k 50: 23.6 -> 23.2 us a call)
     bool few = f.cnt_above + f.cnt_bin <= (uint32_t)kWave;
+    uint32_t *ranks = reinterpret_cast<uint32_t *>(s.cand + kWave);    // [4][64]
+    static_assert(sizeof(s.cand) >= 3 * kWave * sizeof(uint64_t), "the ranks lie behind the tokens in s.cand");
     for (;; few = false) {
         if (!few) {
             for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
@@ -1325,10 +1342,19 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
         __syncthreads();
         const uint32_t ns = uniform(t.nsmall);
         if (ns <= (uint32_t)kWave) {
+            // how many of them come before each: one wave alone or, of more than a few, four with a quarter each
+            const uint64_t e = s.cand[min((uint32_t)lane, ns - 1u)];
+            const bool split = ns > 16u;
+            const uint32_t per = split ? (ns + 3u) >> 2 : ns, j1 = min(ns, ((uint32_t)wave + 1u) * per);
+            uint32_t rank = 0;
+#pragma unroll 4
+            for (uint32_t j = (uint32_t)wave * per; j < j1; ++j) rank += (uint32_t)s.cand[j] < (uint32_t)e ? 1u : 0u;
+            if (split) {
+                if (wave < 4) ranks[wave * kWave + lane] = rank;
+                __syncthreads();
+                rank = ranks[lane] + ranks[kWave + lane] + ranks[2 * kWave + lane] + ranks[3 * kWave + lane];
+            }
             if (wave == 0) {
-                const uint64_t e = s.cand[min((uint32_t)lane, ns - 1u)];
-                uint32_t rank = 0;
-                for (uint32_t j = 0; j < ns; ++j) rank += (uint32_t)s.cand[j] < (uint32_t)e ? 1u : 0u;
                 pick_of_wave(p, t, row, lane, ns, rank, (uint32_t)e, weight((uint32_t)(e >> 32)), r);
             }
             return true;
