@@ -1932,4 +1932,4 @@ def test_one_launch_path_of_rows_of_few_slices(torch_cuda):
     a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_repetition_temperature_topk_topp(
         lg, pen, st, 0.1, 0.1, 0.95, 1.0, k, p)) for k, p in ((50, 0.95), (-1, 0.9)))
     print("one launch %.1f us, general kernel %.1f us: %.2f" % (a, b, a / b), flush=True)
-    assert a < 0.91 * b, (a, b)
+    assert a < 0.93 * b, (a, b)
