@@ -315,7 +315,8 @@ int rs_sample_dtype(const void *logits_device, int32_t logits_dtype, int64_t row
  * path and RS_PATH_WIDE1 the one-pass wide path (any call without penalties; a
  * call that keeps every token takes the counting-only streaming variant),
  * RS_PATH_ROW the row kernel (any call without penalties in rows of up to
- * 65536 tokens; else the general kernel).  `slice_r` forces the float4 groups per thread of the
+ * 65536 tokens; else the general kernel), RS_PATH_SHORT the short-row kernel (any
+ * call in rows of up to 16384 tokens; else the general kernel).  `slice_r` forces the float4 groups per thread of the
  * general kernel (1, 2, 4, 8, 16 or 32; 0 = chosen by the library).
  * `policy` see rs_policy.  No counterpart in the reference.
  */
@@ -327,6 +328,7 @@ int rs_sample_dtype(const void *logits_device, int32_t logits_dtype, int64_t row
 #define RS_PATH_WIDE    5
 #define RS_PATH_WIDE1   6
 #define RS_PATH_ROW     7
+#define RS_PATH_SHORT   8
 typedef struct rs_options {
     int32_t    path;
     int32_t    slice_r;

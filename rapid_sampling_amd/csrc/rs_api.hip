@@ -356,7 +356,7 @@ namespace rs {
 // Measured on MI355X, back to back: with a bounding top_k the streaming path beats the cluster
 // kernel from 131072 tokens per call upwards (15-17 us for small calls against 16-31 us, 2-3
 // times faster for large ones); below that the single launch wins by up to a microsecond.
-enum { kPathCluster = 0, kPathStream = 1, kPathAttempt = 2, kPathFused = 3, kPathKeep = 4, kPathWide = 5, kPathProbe = 6, kPathWide1 = 7, kPathRow = 8 };
+enum { kPathCluster = 0, kPathStream = 1, kPathAttempt = 2, kPathFused = 3, kPathKeep = 4, kPathWide = 5, kPathProbe = 6, kPathWide1 = 7, kPathRow = 8, kPathShort = 9 };
 // The wide path (four launches, two reads of the logits) against the general kernel (one launch, its
 // exchanges), measured on flat rows (U[0,1), top_p 0.9) and on N(0,1.5) with top_k 10000: the wide path
 // wins from about 25 million tokens per call on in rows of 50304 tokens and more (96 x 262144: 88 against
@@ -411,6 +411,30 @@ static bool row_suits(int32_t B, int32_t V)
     if (V <= 32768) return B >= 320;
     return B >= 512 || V >= 40000;                            // 257 to 511 rows: two rounds pay off in long rows only
 }
+// The short-row kernel (one workgroup per row, one launch, any kept set) against what such calls took before it -- the general
+// kernel, the streaming path, the row kernel -- us a call, top_k 40 of peaked rows / top_p 0.9 of N(0,3) / the same two with
+// penalties:
+//   rows x tokens          before                    here
+//      1 x   256      8.4 /  8.2 /  8.4 /  8.4     4.6 / 4.9 / 4.8 / 4.7
+//   2048 x   256     45.9 / 45.7 / 61.7 / 61.3    10.6 / 10.4 / 12.7 / 12.5
+//      1 x  4096     12.0 / 13.3 / 13.2 / 14.5     5.6 /  7.1 /  5.9 /  7.7
+//   1024 x  4096     18.6 / 31.7 / 37.5 / 39.6     8.7 / 14.3 / 13.1 / 19.2
+//     64 x  8192     10.0 / 10.4 / 11.6 / 18.3     6.5 /  9.8 /  7.2 / 10.5
+//   1024 x  8192     21.7 / 23.9 / 47.0 / 50.1    18.1 / 24.9 / 27.8 / 31.6
+//      1 x 16384      9.3 / 15.2 / 10.9 / 15.9     7.7 / 12.5 /  9.1 / 13.2
+//     64 x 16384     10.2 / 12.0 / 12.2 / 20.0     8.0 / 13.2 /  9.3 / 14.5
+//    256 x 16384     12.6 / 13.1 / 17.6 / 28.3     8.6 / 13.9 / 13.6 / 15.9
+//    512 x 16384     15.9 / 17.0 / 36.4 / 38.4    14.4 / 24.5 / 24.6 / 33.7
+//   1024 x 16384     28.5 / 31.5 / 64.3 / 68.9    29.2 / 46.7 / 47.0 / 62.6
+// So it takes every call with penalties and every call in rows below 8192 tokens; in longer ones, the kept sets of thousands
+// stay with the row kernel where that takes them, and calls of more than 512 rows where they were.
+static bool short_suits(int32_t B, int32_t V, bool bounded, bool pen)
+{
+    if (V > kShortMaxV) return false;
+    if (pen || V < 8192) return true;
+    if (bounded) return B <= 512 || V == 8192;
+    return B <= 256 && (V == 8192 || !row_suits(B, V));
+}
 // Plain temperature sampling (top_k = V, top_p = 1: every live token is kept) has no kept set to
 // stash, but the streaming pass's bins alone say which slice holds the target: one pass at
 // bandwidth that only counts, plus a second look at one slice per row, beats the general kernel's
@@ -445,6 +469,8 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
 {
     const bool bounded = top_k <= kStreamK;
     const int force = opt ? opt->path : RS_PATH_AUTO;
+    if (force == RS_PATH_SHORT) return V <= kShortMaxV ? kPathShort : kPathCluster;
+    if (force == RS_PATH_AUTO && !(opt && opt->slice_r) && short_suits(B, V, bounded, pen)) return kPathShort;
     if (force == RS_PATH_FUSED) return fused_r(B, V, pen, true) ? kPathFused : kPathCluster;
     // The one-launch path by default: calls with penalties whose kept set is bounded by top_k (the
     // general kernel, the only other way with penalties, spends most of its time in exchanges).
@@ -543,7 +569,7 @@ using namespace rs;
 
 extern "C" {
 
-int rs_version(void) { return 416; }
+int rs_version(void) { return 417; }
 
 const char *rs_error_string(int code)
 {
@@ -715,7 +741,7 @@ static int check_call(const void *logits, int32_t logits_dtype, int64_t row_stri
     if (!(V > 0 && V <= 1048576 && V % 4 == 0)) return RS_ERR_VOCAB;
     if (B <= 0) return RS_ERR_BATCH;
     if (!(top_k >= 1 && top_k <= V) || !(top_p > 0.0f && top_p <= 1.0f) || !(log2e_inv_temp > 0.0f)) return RS_ERR_ARG;
-    if (opt && (opt->path < RS_PATH_AUTO || opt->path > RS_PATH_ROW || opt->slice_r < 0)) return RS_ERR_ARG;
+    if (opt && (opt->path < RS_PATH_AUTO || opt->path > RS_PATH_SHORT || opt->slice_r < 0)) return RS_ERR_ARG;
     if (((uintptr_t)logits & (logits_dtype == RS_DTYPE_F32 ? 15 : 7)) || (B > 1 && (row_stride & 3)) || ((uintptr_t)penalties & 15) || ((uintptr_t)e_bits & 15))
         return RS_ERR_ALIGN;
     return RS_OK;
@@ -777,6 +803,7 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
     p.long_list = 0xFFFFFFFFu;
     dim3 grid((uint32_t)B * g.G);
     const int path = choose_path(B, V, top_k, top_p, pen, opt);
+    if (path == kPathShort) return launch_short(pen, logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     if (path == kPathRow) return launch_row(logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     if (path != kPathCluster) {
         const int sr = path == kPathFused ? fused_r(B, V, pen, opt && opt->path == RS_PATH_FUSED)

@@ -687,6 +687,8 @@ hipError_t launch_fused(int slice_r, bool pen, uint32_t B, hipStream_t st, const
 hipError_t launch_wide(int slice_r, int32_t dtype, uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v);
 hipError_t launch_wide1(int slice_r, int32_t dtype, uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v);
 constexpr int32_t kRowMaxV = 65536;                      // the longest row the row kernel holds in its registers
+constexpr int32_t kShortMaxV = 16384;                    // the longest row of the short-row kernel
+hipError_t launch_short(bool pen, int32_t dtype, uint32_t B, hipStream_t st, const Params &p);
 hipError_t launch_row(int32_t dtype, uint32_t B, hipStream_t st, const Params &p);
 
 }  // namespace rs

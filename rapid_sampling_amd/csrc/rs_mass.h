@@ -151,4 +151,152 @@ struct BinScan {
     }
 };
 
+// What is left to a bin's tokens of one exponent: the mass that must be reached, `above` of which there is already, in units of
+// the exponent's weights (2^(ex - 87)), rounded up; all ones when it is out of their reach.
+__device__ __forceinline__ uint64_t need_of(M96 P, M96 above, uint32_t ex)
+{
+    const uint32_t sh = ex - 87u;
+    const M96 left = (P - above) + M96{(1ull << sh) - 1ull, 0u};
+    return (uint64_t)left.hi >> sh ? ~0ull : (left.lo >> sh) | (((uint64_t)left.hi << 1) << (63u - sh));
+}
+// A sum in those units as a mass.
+__device__ __forceinline__ M96 mass_of(uint64_t sum, uint32_t ex)
+{
+    const uint32_t sh = ex - 87u;
+    return M96{sum << sh, (uint32_t)((sum >> 24) >> (40u - sh))};
+}
+// Where a scan in order of falling e stopped: the first place at which there are top_k tokens or the mass P, what lies before
+// it and what is there (wave-uniform).
+struct Edge {
+    uint32_t at, cnt_above, cnt_bin;
+    uint64_t sum;                                        // of the levels below the first: mass before it since the first level's place, in units of the exponent
+    M96      above;                                      // of the first level: mass before it
+    uint64_t bin_sum;                                    // of the first level: mass there, in units of the exponent
+};
+
+// The 164 bins of level 1 looked at by one wave, an octave of four bins a lane, largest e first: the bins of a lane share
+// their exponent, so the lane shifts one sum, a scan over 41 lanes finds the octave, and the bin in it is found on scalars.
+struct OctScan {
+    uint32_t c[4], cs, before;                           // tokens of the lane's bins, of the lane, of the lanes before
+    uint64_t s[4];                                       // the bins' masses in units of the octave's exponent
+    Limbs    own, upto;                                  // the lane's mass; with the lanes before
+    // octave(o, w): the packed words of octave o (87 to 127), w[0] its smallest bin
+    template <typename F>
+    __device__ __forceinline__ void load(const int lane, F octave)
+    {
+        const uint32_t o = (uint32_t)max(127 - lane, 87);
+        uint64_t w[4], ss = 0;
+        octave(o, w);
+        cs = 0;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint64_t q = lane <= 40 ? w[3 - i] : 0ull;
+            c[i] = pack_count(q);
+            s[i] = (q & kPackMask) + ((uint64_t)c[i] << 23);
+            cs += c[i]; ss += s[i];
+        }
+        own = limbs(mass_of(ss, o));
+        before = wave_inclusive_scan(cs) - cs;
+        upto = wave_inclusive_scan(own);
+    }
+    __device__ __forceinline__ M96 total() const { return m96(lane_of(upto, 63u)); }
+    // The first bin at which there are top_k tokens or P > 0; false when there is none.
+    __device__ __forceinline__ bool search(uint32_t top_k, M96 P, Edge &e) const
+    {
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(before + cs >= top_k || m96(upto) >= P);
+        if (vote == 0ull) return false;
+        const uint32_t l = (uint32_t)__builtin_ctzll(vote), ex = 127u - l;
+        const M96 mb = m96(lane_of(upto - own, l));
+        const uint64_t need = need_of(P, mb, ex);
+        e.cnt_above = lane_of(before, l); e.cnt_bin = lane_of(c[0], l);
+        uint64_t here = lane_of(s[0], l), sum = 0;
+        uint32_t k = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 3u; ++i)
+            if (k == i && e.cnt_above + e.cnt_bin < top_k && sum + here < need) {
+                e.cnt_above += e.cnt_bin; sum += here;
+                e.cnt_bin = lane_of(c[i + 1], l); here = lane_of(s[i + 1], l);
+                k = i + 1u;
+            }
+        e.at = ex * 4u + 3u - k;
+        e.sum = 0; e.bin_sum = here;
+        e.above = mb + mass_of(sum, ex);
+        return true;
+    }
+};
+
+// The next seven bits of one bin's tokens, 128 bins two a lane: `word(i)` bin i, `from` the edge found so far, `need` what
+// need_of says of the first level's.  All tokens share the exponent, so masses are 64-bit sums, scanned as two limbs.
+template <typename F>
+__device__ __forceinline__ bool fine_search(const int lane, F word, const Edge &from, uint32_t top_k, uint64_t need, Edge &e)
+{
+    const uint64_t w0 = word(127 - 2 * lane), w1 = word(126 - 2 * lane);
+    const uint32_t c0 = pack_count(w0), c1 = pack_count(w1), cs = c0 + c1;
+    const uint64_t s0 = (w0 & kPackMask) + ((uint64_t)c0 << 23), s1 = (w1 & kPackMask) + ((uint64_t)c1 << 23), ss = s0 + s1;
+    const uint32_t ci = wave_inclusive_scan(cs) + from.cnt_above;
+    const uint32_t lo = wave_inclusive_scan((uint32_t)ss & 0xFFFFFFu), hi = wave_inclusive_scan((uint32_t)(ss >> 24));
+    const uint64_t si = ((uint64_t)hi << 24) + lo + from.sum;
+    const uint64_t vote = __builtin_amdgcn_ballot_w64(ci >= top_k || si >= need);
+    if (vote == 0ull) return false;
+    const uint32_t l = (uint32_t)__builtin_ctzll(vote);
+    const bool first = (__builtin_amdgcn_ballot_w64(ci - c1 >= top_k || si - s1 >= need) >> l & 1ull) != 0ull;
+    e.at = 127u - 2u * l - (first ? 0u : 1u);
+    e.cnt_above = lane_of(ci - cs, l) + (first ? 0u : lane_of(c0, l));
+    e.cnt_bin = first ? lane_of(c0, l) : lane_of(c1, l);
+    e.sum = lane_of(si - ss, l) + (first ? 0ull : lane_of(s0, l));
+    return true;
+}
+
+// ---- a row finished from a list of at most 64 tokens that holds its kept set and its threshold's ties ----
+struct LdsFew {
+    uint64_t sorted[kWave], w[kWave];
+    uint32_t part[4][kWave], idx[kWave];
+};
+// list: bits of e << 32 | index, in any order, n > 0 of them, with nothing larger left out.  Called by the first four waves
+// of the workgroup together (more may call; all meet at its barrier); one wave does it alone when there are few tokens.  Each token is
+// compared with every other: its place by falling e, where one scan finds the threshold, and its place by index, where
+// another finds the sampled token.  Returns that token + 1 in one lane of wave 0, 0 elsewhere.
+__device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const uint32_t row, const int lane, const int wave, const uint64_t *list,
+                                             const uint32_t n, const uint32_t top_k, const M96 D, const M96 P, const float xmax,
+                                             const uint64_t *rand64, const uint32_t rounds)
+{
+    const uint64_t e = list[min((uint32_t)lane, n - 1u)];
+    const bool split = n > 16u, in = (uint32_t)lane < n;
+    uint32_t larger = 0, before = 0;
+    if (wave < (split ? 4 : 1)) {
+        const uint32_t each = split ? (n + 3u) >> 2 : n, j1 = min(n, ((uint32_t)wave + 1u) * each);
+#pragma unroll 4
+        for (uint32_t j = (uint32_t)wave * each; j < j1; ++j) {
+            const uint64_t o = list[j];
+            larger += o > e ? 1u : 0u;                   // (equal e: the larger index first)
+            before += (uint32_t)o < (uint32_t)e ? 1u : 0u;
+        }
+        if (split) s.part[wave][lane] = larger | before << 16;
+    }
+    if (split) __syncthreads();
+    if (wave != 0) return 0u;
+    if (split) {
+        const uint32_t c = s.part[0][lane] + s.part[1][lane] + s.part[2][lane] + s.part[3][lane];
+        larger = c & 0xFFFFu; before = c >> 16;
+    }
+    if (in) s.sorted[larger] = e;
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const uint32_t b = in ? (uint32_t)(s.sorted[lane] >> 32) : 0u;
+    const Limbs own = limbs(M96{in ? w_of_bits(b) : 0ull, 0u}), upto = wave_inclusive_scan(own);
+    const uint64_t enough = __builtin_amdgcn_ballot_w64(in && ((uint32_t)lane + 1u >= top_k || m96(upto) >= P));
+    const uint32_t thr = lane_of(b, enough ? (uint32_t)__builtin_ctzll(enough) : n - 1u);
+    const uint32_t n_gt = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b > thr));
+    const uint32_t n_eq = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b == thr));
+    const Target tg = tie_and_target(p, row, uniform(*rand64), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(m96(lane_of(upto - own, n_gt))), rounds, lane == 0);
+    const M96 r = m96(tg.r);
+    if (in) {
+        const uint32_t be = (uint32_t)(e >> 32);
+        s.w[before] = be > thr ? w_of_bits(be) : be == thr ? tg.w_tie : 0ull;
+        s.idx[before] = (uint32_t)e;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    const Limbs mine = limbs(M96{in ? s.w[lane] : 0ull, 0u}), run = wave_inclusive_scan(mine);
+    return in && m96(run - mine) < r && m96(run) >= r ? s.idx[lane] + 1u : 0u;
+}
+
 }  // namespace rs

@@ -1933,3 +1933,92 @@ def test_one_launch_path_of_rows_of_few_slices(torch_cuda):
         lg, pen, st, 0.1, 0.1, 0.95, 1.0, k, p)) for k, p in ((50, 0.95), (-1, 0.9)))
     print("one launch %.1f us, general kernel %.1f us: %.2f" % (a, b, a / b), flush=True)
     assert a < 0.93 * b, (a, b)
+
+
+@pytest.mark.parametrize("pen_on", [False, True])
+@pytest.mark.parametrize("V", [4, 12, 252, 256, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8188, 8192, 8196, 16384])
+def test_short_row_kernel(torch_cuda, oracle, V, pen_on):
+    """Rows of up to 16384 tokens, at the edges of the kernel's variants (4, 8 and 16 waves with 1, 2 and 4 groups of four per
+    thread; waves without a token in the shortest rows): lists of 1, 16, 17, 64 and 65 tokens, kept sets of thousands, ties (of all tokens,
+    of the largest, of a few values), masked and sorted rows, frames far from zero, NaNs; penalties that are -0.0, infinite,
+    dense, and a decay that is not finite.  Every field against the oracle, and with the generator's own draws against
+    the general kernel, states included."""
+    torch = torch_cuda
+    from tests import capi
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal((14, V)) * 2.0).astype(np.float32)
+    lg[1] = rng.random(V, dtype=np.float32)
+    lg[2] = 0.5
+    lg[3, V // 2:] = -np.inf
+    lg[4] = np.sort(lg[4])
+    lg[5] = np.round(lg[5])
+    lg[6] = -1e30
+    lg[6, V // 3] = 1e30
+    lg[7, ::3] = np.nan
+    lg[8] += 4000.0
+    lg[9] = -np.inf
+    lg[10, : (V + 1) // 2] = 7.0
+    lg[11] = rng.random(V, dtype=np.float32) * 4
+    lg[12] = np.sort(lg[12])[::-1]
+    lg[13, rng.integers(0, V, min(V, 16))] += 10.0
+    pen = None
+    if pen_on:
+        pen = H.penalties_sparse(14, V, seed=V + 1)
+        pen[1, ::5] = -0.0
+        pen[4] = rng.exponential(0.1, V).astype(np.float32)
+        pen[5, :3] = np.inf
+        pen[8] = 0.0
+    kw = dict(presence=0.1, repetition=0.2, decay=0.95)
+    for temp, k, p in [(1.0, 1, 1.0), (0.8, 40, 0.95), (1.0, 16, 1.0), (1.0, 17, 1.0), (1.0, 64, 1.0), (1.0, 65, 1.0), (1.0, -1, 0.5), (1.3, -1, 1.0),
+                       (0.7, 1000, 0.9)]:
+        _run_case(torch, oracle, capi, lg, temp, k, p, pen_np=pen, u_np=H.uniforms(14, 90 + k % 7), what="short V=%d k=%d p=%g" % (V, k, p), **kw)
+    if pen_on:
+        zero = np.zeros_like(pen)
+        _run_case(torch, oracle, capi, lg, 1.0, 40, 0.9, pen_np=zero, u_np=H.uniforms(14, 5), presence=0.1, repetition=0.2, decay=float("inf"), what="short, infinite decay")
+    smp = capi.Sampler(14, V)
+    for fmt in (torch.float32, torch.bfloat16, torch.float16):
+        x = torch.from_numpy(lg).cuda().to(fmt)
+        rc, c, k, p = capi.normalize(0.9, 50, 0.95, V, 14, 1)
+        got = {}
+        for path in ("short", "cluster"):
+            state = torch.zeros(14 * 16, dtype=torch.int32, device="cuda")
+            assert capi.lib().rs_philox_init(state.data_ptr(), 77, 14, smp.stream()) == 0
+            state[2::16] = -1                                         # the draw counter carries into its next word
+            pn = torch.from_numpy(pen.copy()).cuda() if pen_on else None
+            runs = [smp.sample(x, c, k, p, rng=state, penalties=pn, path=path, **kw) for _ in range(3)]
+            got[path] = ([r["out"] for r in runs], [r["diag"][FIELDS] for r in runs], state.cpu().numpy(), pn.cpu().numpy().view(np.uint32) if pen_on else 0)
+            if path == "short":
+                assert all((r["diag"]["rounds"] == 10).all() for r in runs)
+        for a, b in zip(got["short"], got["cluster"]):
+            assert np.array_equal(np.asarray(a), np.asarray(b)), (V, pen_on, fmt)
+    assert smp.status() == 0
+    smp.close()
+
+
+@pytest.mark.parametrize("pen_on", [False, True])
+@pytest.mark.parametrize("V", [2048, 4092, 4096, 8188, 8192])
+def test_short_row_kernel_in_calls_of_more_rows_than_compute_units(torch_cuda, oracle, V, pen_on):
+    """257 rows: the smaller workgroups of such calls (4 waves with 2 and 4 groups of four per thread, 8 with 4)."""
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal((257, V)) * 2.0).astype(np.float32)
+    lg[::3] = rng.random((86, V), dtype=np.float32)
+    lg[1] = 0.25
+    lg[5, 7:] = -np.inf
+    pen = H.penalties_sparse(257, V, seed=V + 1) if pen_on else None
+    for temp, k, p in [(0.8, 40, 0.95), (1.0, -1, 0.9), (1.0, 300, 1.0)]:
+        torch = torch_cuda
+        from tests import capi
+        rc, c, kk, pp = capi.normalize(temp, k, p, V, 257, 1)
+        u_np = H.uniforms(257, 17)
+        pen_ref = None if pen is None else pen.copy()
+        ref_out, ref_diag, ref_e = oracle.sample_batch(lg, c, kk, pp, injected_u=u_np, penalties=pen_ref, presence=0.1, repetition=0.2, decay=0.95,
+                                                       want_e=True)
+        smp = capi.Sampler(257, V)
+        pn = None if pen is None else torch.from_numpy(pen.copy()).cuda()
+        res = smp.sample(torch.from_numpy(lg).cuda(), c, kk, pp, uniforms=torch.from_numpy(u_np).cuda(), penalties=pn, presence=0.1, repetition=0.2,
+                         decay=0.95, path="short", want_e=True)
+        _check(res, ref_out, ref_diag, "short, 257 rows V=%d k=%d" % (V, k), ref_e)
+        if pen_on:
+            assert np.array_equal(pn.cpu().numpy().view(np.uint32), pen_ref.view(np.uint32))
+        assert (res["diag"]["rounds"] == 10).all() and smp.status() == 0
+        smp.close()
