@@ -238,25 +238,24 @@ constexpr uint32_t kStreamSmallParts = 1536;
 constexpr int32_t kMidMaxV = 262144;                          // rows up to here may be cut into slices of 8192 tokens whatever the call's size (wide_r)
 constexpr uint64_t kFusedSmall = 1ull << 22;
 static uint32_t stream_parts(int32_t V, int R) { return ((uint32_t)V / 4 + kStreamNT * R - 1) / (kStreamNT * R); }
-// `pen`: the pass that also reads penalties exists for the long slices only
-static int stream_r(int32_t B, int32_t V, bool pen = false)
+static int stream_r(int32_t B, int32_t V)
 {
     if (V > 262144) {
         // a few long rows: shorter slices while a row has at most 128 of them and the call at most 512
         // (measured at 524288 and 1048576 tokens: 1-3.7 us faster up to there, slower beyond)
-        for (int R = 4; R <= 8 && !pen; R *= 2) {
+        for (int R = 4; R <= 8; R *= 2) {
             const uint32_t g = stream_parts(V, R);
             if (g <= 128u && (uint64_t)B * g <= 512u) return R;
         }
         return kStreamLongR;
     }
     if ((uint64_t)B * stream_parts(V, 4) <= kStreamSmallParts) return 4;
-    if (!pen && (uint64_t)B * stream_parts(V, 8) <= kStreamSmallParts) return 8;
+    if ((uint64_t)B * stream_parts(V, 8) <= kStreamSmallParts) return 8;
     return kStreamLongR;
 }
 static size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
 struct StreamLayout { size_t hdr, cum, shist, stash, pens, end; };
-// `with_pens`: room for every slice's note of its non-zero penalties behind the stashes (long slices only)
+// `with_pens`: room for every slice's note of its non-zero penalties behind the stashes
 static StreamLayout stream_layout(size_t parts, size_t base, bool with_pens = false)
 {
     StreamLayout l;
@@ -274,7 +273,8 @@ static StreamLayout stream_layout(size_t parts, size_t base, bool with_pens = fa
 // at most kFusedSmall tokens, fewer than kFusedSmall / 4096 + B slices), so that the size grows
 // with B and with V and a workspace for the largest B and V serves every smaller call.
 // (`least`: what every call needs; without it, also room for slices of 8192 tokens in rows of up to
-// 262144, which the one-pass wide path and the counting-only pass take when they are given it: see wide_r)
+// 262144, which the one-pass wide path, the counting-only pass and the pass with penalties take when they are given it: see
+// wide_r and pen_r)
 static size_t stream_bytes(int32_t B, int32_t V, bool least)
 {
     const size_t longs = stream_layout((size_t)B * stream_parts(V, kStreamLongR), sizeof(WsHeader), true).end;
@@ -303,6 +303,21 @@ static int wide_r(int32_t B, int32_t V, size_t workspace_bytes)
     if (r != kStreamLongR || V > kMidMaxV) return r;
     const size_t need = stream_layout((size_t)B * stream_parts(V, 8), sizeof(WsHeader)).end + (size_t)B * sizeof(RowCtl);
     return need <= (workspace_bytes & ~(size_t)255) ? 8 : r;
+}
+
+// Slice length of the streaming pass with penalties (calls of kPenStreamMin tokens and more): 8192 tokens in rows of up to
+// 262144 when the workspace has room for them (a workspace of rs_workspace_bytes has) and each stash leaves room for the slice's
+// notes behind it, else 16384, whose notes have room of their own.  A thread holds its
+// tokens and their penalties, so slices half as long let twice the workgroups share a compute unit and load in each other's scans:
+// 128 x 262144 73.0 -> 63.9 us a call, 256 x 131072 73.1 -> 64.0, 128 x 100256 42.2 -> 35.0, 512 x 32768 48.0 -> 41.1.  Rows of a million tokens would be cut into more slices than
+// their finish handles quickly (16 x 1048576: 55 us a call with slices of 16384, 67 with 8192).
+static uint32_t stash_aim(uint32_t top_k, uint32_t G) { return min(top_k, max(32u, 8u * top_k / G)); }    // eight times a slice's share of the row's top_k
+static int pen_r(int32_t B, int32_t V, int32_t top_k, size_t workspace_bytes)
+{
+    const uint32_t aim = stash_aim((uint32_t)top_k, stream_parts(V, 8));
+    if (V > kMidMaxV || aim + max(64u, aim / 4u) > (uint32_t)kPenStashCap) return kStreamLongR;
+    const size_t need = stream_layout((size_t)B * stream_parts(V, 8), sizeof(WsHeader)).end + (size_t)B * sizeof(RowCtl);
+    return need <= (workspace_bytes & ~(size_t)255) ? 8 : kStreamLongR;
 }
 
 }  // namespace rs
@@ -379,7 +394,12 @@ constexpr uint64_t kWide1Min = 1ull << 26;
 // below: 64 x 131072 48 against 38, 32 x 262144 50 against 40) and puts it ahead of the two-pass path
 // everywhere above (256 x 131072: 77 against 94; 512 x 262144: 191 against 266).
 constexpr uint64_t kWide1MinMid = 12000000ull;
-constexpr uint64_t kPenStreamMin = 1ull << 23;
+// Calls with penalties the one-launch path does not hold: three launches of the streaming path against the general kernel, us a
+// call, top_k 50 / 1000 of N(0,1.5): 400 x 20480 30.8 / 48.5 against 70.0 / 77.1, 260 x 24576 27.6 / 44.6 against 63.9 / 69.0, 160 x 50304
+// 29.8 / 37.7 against 67.8 / 73.8, 80 x 100256 29.2 / 36.7 against 66.0 / 72.2.  Where the one-launch path holds the call the two are
+// level from about 6 million tokens on (64 x 131072 29.4 one launch, 28.4 three; with 20 % of the penalties non-zero 29.7 against 34.9), and it
+// stays there.  The bound lies below every call of rows of more than 16384 tokens that the one-launch path does not hold.
+constexpr uint64_t kPenStreamMin = 1ull << 22;
 // The row kernel (one workgroup per row, the row in its registers, one launch; rows of up to 65536 tokens, no
 // penalties) against what else there is for kept sets the stashes cannot hold, same rows, us per call:
 //   rows x tokens   general/wide  row kernel        rows x tokens   general/wide  row kernel
@@ -475,8 +495,8 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
     // The one-launch path by default: calls with penalties whose kept set is bounded by top_k (the
     // general kernel, the only other way with penalties, spends most of its time in exchanges).
     if (force == RS_PATH_AUTO && pen && bounded && fused_r(B, V, pen, false)) return kPathFused;
-    // Larger calls with penalties: the streaming pass with a pass over the penalties behind it, from
-    // kPenStreamMin tokens on (measured crossover with the general kernel), long slices only.
+    // Larger calls with penalties: the streaming pass that also writes the decayed penalties, its finish and a fix-up, three
+    // launches, from kPenStreamMin tokens on.
     rs_policy *pol = opt ? opt->policy : nullptr;
     const int cls = size_class(B, V);
     // after a call of this kind with a slow row: the general kernel for a while, then another try
@@ -502,7 +522,7 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
         retry = true;
         return false;
     };
-    if (pen && bounded && stream_r(B, V, true) == kStreamLongR && stream_parts(V, kStreamLongR) >= 2u) {
+    if (pen && bounded && stream_parts(V, kStreamLongR) >= 2u) {
         if (force == RS_PATH_STREAM || force == RS_PATH_ATTEMPT) return kPathStream;
         if (force == RS_PATH_AUTO && (uint64_t)B * (uint64_t)V >= kPenStreamMin && !routed_away(0)) return kPathStream;
     }
@@ -807,23 +827,26 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
     if (path == kPathRow) return launch_row(logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     if (path != kPathCluster) {
         const int sr = path == kPathFused ? fused_r(B, V, pen, opt && opt->path == RS_PATH_FUSED)
-                     : (path == kPathWide1 || path == kPathKeep) ? wide_r(B, V, workspace_bytes) : stream_r(B, V, pen);
+                     : (path == kPathWide1 || path == kPathKeep) ? wide_r(B, V, workspace_bytes)
+                     : pen ? pen_r(B, V, top_k, workspace_bytes) : stream_r(B, V);
         StreamView v;
         v.G = stream_parts(V, sr);
         v.slice_log2 = sr == 4 ? 12u : sr == 8 ? 13u : (uint32_t)kStreamLongLog2;
-        const bool pen_stream = pen && path == kPathStream;                  // long slices: their layout has room for the notes
-        const StreamLayout l = stream_layout((size_t)B * v.G, sizeof(WsHeader), pen_stream);
+        const bool pen_stream = pen && path == kPathStream;
+        const StreamLayout l = stream_layout((size_t)B * v.G, sizeof(WsHeader), pen_stream && sr != 8);
         // (rs_workspace_bytes sets aside room for every slice length chosen above; checked all the same: a
         // layout that ran into the rows' records would be written out of bounds by thousands of workgroups)
         if (l.end + (size_t)B * sizeof(RowCtl) > (workspace_bytes & ~(size_t)255)) return RS_ERR_WORKSPACE;
         char *w = (char *)workspace;
         v.hdr = (PartHdr *)(w + l.hdr); v.stash = (uint64_t *)(w + l.stash); v.cum = (uint32_t *)(w + l.cum);
         v.shist = (uint64_t *)(w + l.shist);
-        v.pens = pen_stream ? (uint64_t *)(w + l.pens) : nullptr;
+        // a slice's notes: room of their own, or (slices of 8192 tokens) the end of its stash, which is then kept shorter
+        v.pens = !pen_stream ? nullptr : sr == 8 ? v.stash + kPenStashCap : (uint64_t *)(w + l.pens);
+        v.pen_stride = sr == 8 ? (uint32_t)kStashCap : (uint32_t)kPenCap;
         // without a bounding top_k the stashes are sized as for top_k = kStreamK: enough for a nucleus
         // of up to about a thousand tokens
         const uint32_t kk = min((uint32_t)top_k, (uint32_t)kStreamK);
-        p.stash_k = min(kk, max(32u, 8u * kk / v.G));            // eight times a slice's share of the row's top_k
+        p.stash_k = stash_aim(kk, v.G);
         hipStream_t st = (hipStream_t)stream;
         // The finishing workgroup's list: twice what a well-behaved row needs (its top_k tokens and
         // a boundary bin, or every stash whole), as a power of two; a row that needs more is handed
@@ -879,8 +902,8 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
             // finishing workgroup; slices the pass deferred are rewritten by a fix-up kernel at the end
             // a finite decay keeps +0.0 at +0.0, which is what lets the pass skip the groups that hold nothing
             p.defer_pen = (decay - decay == 0.0f) ? 2 : 1;
-            if (launch_stream_pen((uint32_t)B, dyn, st, p, v) != hipSuccess) return RS_ERR_LAUNCH;
-            return launch_penalty_fix(st, p, v) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
+            if (launch_stream_pen(sr, (uint32_t)B, dyn, st, p, v) != hipSuccess) return RS_ERR_LAUNCH;
+            return launch_penalty_fix(sr, st, p, v) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
         }
         return launch_stream(sr, logits_dtype, path == kPathKeep, (uint32_t)B, dyn, st, p, v) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     }

@@ -661,16 +661,18 @@ struct PartHdr {
 // A slice's note of its penalties (stream_pen_kernel): word 0 = count, or kPenDeferred when the slice left its
 // penalties untouched; then count entries (old value's bits << 32 | token index in the row), the penalties
 // whose bit pattern was not +0.0 before the call.
-constexpr int      kPenCap      = 512;        // words per slice: 511 non-zero penalties among 16384 tokens, 3.1 %
-constexpr int      kPenWave     = 160;        // of which one wave (4096 tokens) can note this many
+constexpr int      kPenCap      = 512;        // words per slice: 511 non-zero penalties among 16384 tokens, 3.1 %, or 8192
+constexpr int      kPenWave     = 160;        // of which one wave (4096 tokens or 2048) can note this many
+constexpr int      kPenStashCap = kStashCap - kPenCap;       // stash entries per slice where the notes lie at the stash's end
 constexpr uint64_t kPenDeferred = 1ull << 63;
 
 struct StreamView {
     PartHdr  *hdr;        // [B][G]
-    uint64_t *pens;       // [B][G][kPenCap]   penalties at scale only, else null
+    uint64_t *pens;       // [B][G][pen_stride]   kPenCap words each; penalties at scale only, else null
     uint64_t *stash;      // [B][G][kStashCap]   bits(e, slice frame) << 32 | index, by descending bin
     uint32_t *cum;        // [B][G][kSB]   tokens of the slice in this bin and the bins above it
     uint64_t *shist;      // [B][G][kSB]   the slice's own bins (slice frame), as it added them to the row's
+    uint32_t  pen_stride; // words from a slice's notes to the next one's
     uint32_t  G;          // slices per row
     uint32_t  list_cap;   // entries of the finishing workgroup's token list (a power of two up to kFinCap)
     uint32_t  slice_log2; // log2 of the tokens per slice
@@ -679,8 +681,8 @@ struct StreamView {
 
 // Launchers, one per translation unit that instantiates the kernels.
 hipError_t launch_sample(bool pen, int R, dim3 grid, hipStream_t st, const Params &p);
-hipError_t launch_stream_pen(uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v);
-hipError_t launch_penalty_fix(hipStream_t st, const Params &p, const StreamView &v);
+hipError_t launch_stream_pen(int slice_r, uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v);
+hipError_t launch_penalty_fix(int slice_r, hipStream_t st, const Params &p, const StreamView &v);
 hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p,
                          const StreamView &v);
 hipError_t launch_fused(int slice_r, bool pen, uint32_t B, hipStream_t st, const Params &p, const StreamView &v);

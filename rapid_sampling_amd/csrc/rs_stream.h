@@ -74,7 +74,7 @@ template <bool FUSED, typename T> __device__ __forceinline__ T get(const T *p)
 // in eb), the packed histogram added to the row's and kept under the slice's own name, cumulative
 // counts, and the stash of its largest tokens with the value down to which it is complete.
 // Returns the key of the slice's maximum.
-template <int R, int NT, int kRep, bool FUSED, bool KEEP = false>     // KEEP: a call that keeps every live token (top_k = V, top_p = 1)
+template <int R, int NT, int kRep, bool FUSED, bool KEEP = false, int kCap = kStashCap>     // KEEP: a call that keeps every live token (top_k = V, top_p = 1); kCap: room of the stash
 __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const StreamView &v, LdsA<kRep> &s, uint32_t (&eb)[R * 4],
                                                           const float lmax, const uint32_t row, const uint32_t part,
                                                           const uint32_t base4, const int nv)
@@ -202,7 +202,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
             }
             if (run < Ks && nx >= Ks) {
                 // the whole bin if that stays close to stash_k, else only part of it (found below)
-                if (nx <= min((uint32_t)kStashCap, Ks + max(64u, Ks >> 2))) { s.n = nx; s.cut = ((uint32_t)b + kBin0) << 21; }
+                if (nx <= min((uint32_t)kCap, Ks + max(64u, Ks >> 2))) { s.n = nx; s.cut = ((uint32_t)b + kBin0) << 21; }
                 else { s.n = run; s.cut = ((uint32_t)b + 1u + kBin0) << 21; s.over = (uint32_t)b; }
             }
             run = nx;
@@ -239,11 +239,11 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
             const uint32_t r0 = above + ci - c0 - c1, r1 = r0 + c0, r2 = r1 + c1;
             // first sub-bin at which the count reaches stash_k (there is one: the whole bin reaches it)
             if (r0 < Ks && r1 >= Ks) {
-                const bool fits = r1 <= (uint32_t)kStashCap;
+                const bool fits = r1 <= (uint32_t)kCap;
                 s.n = fits ? r1 : r0;
                 s.cut = (ob << 21) + ((127u - 2u * (uint32_t)lane + (fits ? 0u : 1u)) << 14);
             } else if (r1 < Ks && r2 >= Ks) {
-                const bool fits = r2 <= (uint32_t)kStashCap;
+                const bool fits = r2 <= (uint32_t)kCap;
                 s.n = fits ? r2 : r1;
                 s.cut = (ob << 21) + ((126u - 2u * (uint32_t)lane + (fits ? 0u : 1u)) << 14);
             }
@@ -254,7 +254,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     // From here on the bits in the registers are compared with the cut, which is never below
     // 2^-40: dead tokens are no candidates.
 
-    // Candidates (bits >= cut) are at most n <= kStashCap, so at most that many float4 groups
+    // Candidates (bits >= cut) are at most n <= kCap, so at most that many float4 groups
     // hold one.  Each thread copies its groups with a candidate into LDS at an offset from a scan
     // of the per-thread counts; the tokens of those groups are then gone through densely.
     uint32_t mine = 0;
@@ -274,7 +274,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
 #pragma unroll
     for (int j = 0; j < R; ++j) {
         if (max(max(eb[j * 4], eb[j * 4 + 1]), max(eb[j * 4 + 2], eb[j * 4 + 3])) >= cut) {
-            if (o < (uint32_t)kStashCap) {
+            if (o < (uint32_t)kCap) {
                 s.grp[o] = make_uint4(eb[j * 4], eb[j * 4 + 1], eb[j * 4 + 2], eb[j * 4 + 3]);
                 s.gidx[o] = (base4 + (uint32_t)j * NT) * 4;
             }
@@ -287,11 +287,11 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     uint64_t *st = v.stash + ((size_t)row * G + part) * kStashCap;
     const uint32_t *gb = reinterpret_cast<const uint32_t *>(s.grp);
 #pragma unroll 4
-    for (uint32_t i = tid; i < min(ngroups, (uint32_t)kStashCap) * 4u; i += NT) {
+    for (uint32_t i = tid; i < min(ngroups, (uint32_t)kCap) * 4u; i += NT) {
         const uint32_t b = gb[i];
         if (b >= cut) {
             const uint32_t slot = atomicAdd(&s.off[(b >> 21) - kBin0], 1u);
-            if (slot < (uint32_t)kStashCap) put<FUSED>(&st[slot], ((uint64_t)b << 32) | (s.gidx[i >> 2] + (i & 3u)));
+            if (slot < (uint32_t)kCap) put<FUSED>(&st[slot], ((uint64_t)b << 32) | (s.gidx[i >> 2] + (i & 3u)));
         }
     }
     if (tid == 0) {
@@ -657,7 +657,7 @@ __device__ __forceinline__ void pen_restore(const Params &p, const StreamView &v
     const int tid = threadIdx.x;
     float *pen = p.penalties + (int64_t)row * p.V;
     for (uint32_t g = 0; g < v.G; ++g) {
-        uint64_t *rec = v.pens + ((size_t)row * v.G + g) * kPenCap;
+        uint64_t *rec = v.pens + ((size_t)row * v.G + g) * v.pen_stride;
         const uint64_t h = rec[0];
         if (!(h & kPenDeferred))
             for (uint32_t i = (uint32_t)tid; i < (uint32_t)h; i += kThreads) {
@@ -666,7 +666,7 @@ __device__ __forceinline__ void pen_restore(const Params &p, const StreamView &v
             }
     }
     __syncthreads();
-    if ((uint32_t)tid < v.G) v.pens[((size_t)row * v.G + tid) * kPenCap] = kPenDeferred;
+    if ((uint32_t)tid < v.G) v.pens[((size_t)row * v.G + tid) * v.pen_stride] = kPenDeferred;
     wait_vmem();
     __syncthreads();
 }
@@ -677,7 +677,7 @@ __device__ __forceinline__ void pen_restore(const Params &p, const StreamView &v
 __device__ __forceinline__ void pen_patch(const Params &p, const StreamView &v, Lds &s, const uint32_t row, const uint32_t idx, const uint32_t slice_log2)
 {
     const int tid = threadIdx.x;
-    const uint64_t *rec = v.pens + ((size_t)row * v.G + (idx >> slice_log2)) * kPenCap;
+    const uint64_t *rec = v.pens + ((size_t)row * v.G + (idx >> slice_log2)) * v.pen_stride;
     const uint64_t h = rec[0];
     if (h & kPenDeferred) return;
     if (tid == 0) s.bc32[6] = 0u;
@@ -1587,7 +1587,7 @@ __global__ void __launch_bounds__(kKeepT + kWave) keep_finish_kernel(const Param
 // once the tokens are known).  Groups of four that are all +0.0 stay +0.0 under a finite decay and are
 // not written at all.
 template <int R>
-__global__ void __launch_bounds__(kThreads, 2) stream_pen_kernel(const Params p, const StreamView v)
+__global__ void __launch_bounds__(kThreads, R <= 8 ? 4 : 2) stream_pen_kernel(const Params p, const StreamView v)
 {
     constexpr int kRep = stream_copies<R>();
     __shared__ LdsA<kRep> s;
@@ -1633,7 +1633,7 @@ __global__ void __launch_bounds__(kThreads, 2) stream_pen_kernel(const Params p,
             fits = fits && n <= (uint32_t)kPenWave;
         }
         fits = fits && total < (uint32_t)kPenCap;
-        uint64_t *rec = v.pens + ((size_t)row * G + part) * kPenCap;
+        uint64_t *rec = v.pens + ((size_t)row * G + part) * v.pen_stride;
         if (fits) {
             for (uint32_t i = (uint32_t)lane; i < fill; i += kWave) rec[1 + before + i] = noted[wave][i];
             if (tid == 0) rec[0] = total;
@@ -1648,7 +1648,7 @@ __global__ void __launch_bounds__(kThreads, 2) stream_pen_kernel(const Params p,
             }
         } else if (tid == 0) rec[0] = kPenDeferred;
     }
-    slice_count_and_stash<R, kThreads, kRep, false>(p, v, s, sl.eb, lmax, row, part, sl.base4, sl.nv);
+    slice_count_and_stash<R, kThreads, kRep, false, false, R == 8 ? kPenStashCap : kStashCap>(p, v, s, sl.eb, lmax, row, part, sl.base4, sl.nv);
 }
 
 // pen <- fma(pen, decay, onehot * (pen == 0 ? presence : repetition)), the switch on the value before
@@ -1662,7 +1662,7 @@ __global__ void __launch_bounds__(kThreads) penalty_fix_kernel(const Params p, c
 {
     const uint32_t G = v.G;
     const uint32_t row = blockIdx.x / G, part = blockIdx.x - row * G;
-    if (p.defer_pen == 2 && !(v.pens[((size_t)row * G + part) * kPenCap] & kPenDeferred)) return;
+    if (p.defer_pen == 2 && !(v.pens[((size_t)row * G + part) * v.pen_stride] & kPenDeferred)) return;
     const uint32_t V4 = (uint32_t)p.V >> 2;
     const uint32_t idx = (uint32_t)p.out[row];
     float4 *pn4 = reinterpret_cast<float4 *>(p.penalties + (int64_t)row * p.V);

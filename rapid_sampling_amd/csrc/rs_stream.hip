@@ -43,16 +43,18 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
     return hipGetLastError();
 }
 
-hipError_t launch_stream_pen(uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v)
+hipError_t launch_stream_pen(int slice_r, uint32_t B, size_t finish_lds_bytes, hipStream_t st, const Params &p, const StreamView &v)
 {
-    hipLaunchKernelGGL((stream_pen_kernel<kStreamLongR>), dim3(B * v.G), dim3(kThreads), 0, st, p, v);
+    if (slice_r == 8) hipLaunchKernelGGL((stream_pen_kernel<8>), dim3(B * v.G), dim3(kThreads), 0, st, p, v);
+    else hipLaunchKernelGGL((stream_pen_kernel<kStreamLongR>), dim3(B * v.G), dim3(kThreads), 0, st, p, v);
     launch_finish(B, finish_lds_bytes, st, p, v);
     return hipGetLastError();
 }
 
-hipError_t launch_penalty_fix(hipStream_t st, const Params &p, const StreamView &v)
+hipError_t launch_penalty_fix(int slice_r, hipStream_t st, const Params &p, const StreamView &v)
 {
-    hipLaunchKernelGGL((penalty_fix_kernel<kStreamLongR>), dim3((uint32_t)p.B * v.G), dim3(kThreads), 0, st, p, v);
+    if (slice_r == 8) hipLaunchKernelGGL((penalty_fix_kernel<8>), dim3((uint32_t)p.B * v.G), dim3(kThreads), 0, st, p, v);
+    else hipLaunchKernelGGL((penalty_fix_kernel<kStreamLongR>), dim3((uint32_t)p.B * v.G), dim3(kThreads), 0, st, p, v);
     return hipGetLastError();
 }
 
