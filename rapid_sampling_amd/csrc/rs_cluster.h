@@ -3,6 +3,7 @@
 #pragma once
 
 #include "rs_common.h"
+#include "rs_mass.h"
 
 namespace rs {
 
@@ -423,8 +424,8 @@ __device__ __forceinline__ bool slice_finish(const Params &p, Lds &s, Slice<R, P
     const u128 Gm = f.mass_above;
 
     // ---- 5. tie weight, total S, target r (every workgroup, identically) ----
-    if (tid == 0) {
-        const Target t = tie_and_target(p, row, s.bc64[5], xmax, D, P, thr, n_gt, n_eq, Gm, levels, part == 0);
+    if (wave == 0) {
+        const Target t = target_of_wave(p, row, s.bc64[5], xmax, D, P, thr, n_gt, n_eq, Gm, levels, part == 0 && lane == 0);
         s.bc64[1] = t.w_tie; s.bc128[0] = t.r;
     }
     __syncthreads();

@@ -467,71 +467,6 @@ __device__ __forceinline__ int combine_level1(Lds &s, WsHeader *hdr, uint32_t G,
     return 0;
 }
 
-// Scan the level-1 histogram s.g from the top (index 511, largest e) down to
-// index 348 (e = 2^-40) and find the first bin at which (count so far >=
-// top_k) or (mass so far >= P).  The total mass of the histogram is the row
-// total D, and P = ceil(top_p * D) is derived from it here.  The 164 bins fit
-// one wave (lane l owns indices 511-3l, 510-3l, 509-3l), so the scan needs no
-// LDS exchange; the exponent of bin idx is idx >> 2.  With LOCAL the wave also
-// scans this workgroup's own histogram s.hm and returns its mass above the
-// boundary bin in local_above.  With GIVEN_P the histogram is that of a
-// subset of the row which is complete above some value: D and P are left alone.
-template <bool LOCAL, bool GIVEN_P = false, typename L = Lds>
-__device__ __forceinline__ Found hist_find_level1(L &s, uint64_t top_k, float top_p, int lane, int wave)
-{
-    if (wave == 0) {
-        uint32_t c[3]; u128 m[3], hl[3];
-        uint32_t cs = 0; u128 ms = 0, hs = 0;
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const int idx = (int)kTop1 - 3 * lane - i;
-            const uint64_t w = idx >= (int)kBin0 ? s.g[idx] : 0ull;
-            c[i] = pack_count(w);
-            m[i] = w ? pack_mass(w, (uint32_t)idx >> 2) : (u128)0;
-            cs += c[i]; ms += m[i];
-            if constexpr (LOCAL) {
-                const uint64_t h = idx >= (int)kBin0 ? s.hm[idx] : 0ull;
-                hl[i] = h ? pack_mass(h, (uint32_t)idx >> 2) : (u128)0;
-                hs += hl[i];
-            }
-        }
-        const u128 mi = wave_inclusive_scan(ms);
-        const uint32_t ci = wave_inclusive_scan(cs);
-        u128 hrun = 0;
-        if (LOCAL) hrun = wave_inclusive_scan(hs) - hs;
-        u128 P;
-        if (GIVEN_P) {
-            // the histogram holds only part of the row: P stands as it is, and the scan may end
-            // without the set becoming sufficient (bin 0 then)
-            P = s.P;
-            if (lane == 0) s.found.bin = 0;
-        } else {
-            const u128 D = lane63(mi);
-            P = ceil_mul(top_p, D);
-            if (lane == 0) { s.D = D; s.P = P; }
-        }
-        uint64_t rcnt = (uint64_t)ci - cs;               // count before my first bin
-        u128 rm = mi - ms;                               // mass before my first bin
-#pragma unroll
-        for (int i = 0; i < 3; ++i) {
-            const bool before = rcnt >= top_k || rm >= P;
-            const uint64_t nc = rcnt + c[i];
-            const u128 nm = rm + m[i];
-            const bool after = nc >= top_k || nm >= P;
-            if (!before && after) {
-                s.found.bin = kTop1 - (uint32_t)(3 * lane + i);
-                s.found.cnt_above = (uint32_t)rcnt; s.found.cnt_bin = c[i];
-                s.found.mass_above = rm;
-                s.found.local_above = hrun;
-            }
-            rcnt = nc; rm = nm;
-            if (LOCAL) hrun += hl[i];
-        }
-    }
-    __syncthreads();
-    return s.found;
-}
-
 // A boundary bin with nothing above it holds the row's largest token.  Every token of the bin
 // shares its exponent and none has a larger fraction, so a fraction sum of count times the largest
 // token's fraction proves that all of them equal it: one tie, whose value is then known without
@@ -539,38 +474,6 @@ __device__ __forceinline__ Found hist_find_level1(L &s, uint64_t top_k, float to
 __device__ __forceinline__ bool bin_is_one_tie(uint64_t word, uint32_t bin, uint32_t emax_bits)
 {
     return (emax_bits >> 21) == bin && (word & kPackMask) == (uint64_t)pack_count(word) * (uint64_t)(emax_bits & 0x7FFFFFu);
-}
-
-// The same for a 128-bin level (all tokens share the exponent ex): one wave,
-// lane l owns indices 127-2l and 126-2l, no LDS exchange inside the scan.
-template <typename L = Lds>
-__device__ __forceinline__ Found hist_find128(L &s, const uint64_t *arr, uint32_t cnt0, u128 mass0,
-                                              uint64_t top_k, uint32_t ex, int lane, int wave)
-{
-    if (wave == 0) {
-        const uint64_t w0 = arr[127 - 2 * lane], w1 = arr[126 - 2 * lane];
-        const uint32_t c0 = pack_count(w0), c1 = pack_count(w1);
-        const u128 m0 = pack_mass(w0, ex), m1 = pack_mass(w1, ex);
-        const uint32_t cs = c0 + c1;
-        const u128 ms = m0 + m1;
-        const u128 mi = wave_inclusive_scan(ms);
-        const uint32_t ci = wave_inclusive_scan(cs);
-        const u128 P = s.P;
-        const uint64_t r0 = (uint64_t)cnt0 + ci - cs;      // before my first bin
-        const u128 q0 = mass0 + mi - ms;
-        const uint64_t r1 = r0 + c0, r2 = r1 + c1;         // before my second bin, after it
-        const u128 q1 = q0 + m0, q2 = q1 + m1;
-        const bool s0 = r0 >= top_k || q0 >= P, s1 = r1 >= top_k || q1 >= P, s2 = r2 >= top_k || q2 >= P;
-        if (!s0 && s1) {
-            s.found.bin = 127u - 2u * (uint32_t)lane;
-            s.found.cnt_above = (uint32_t)r0; s.found.cnt_bin = c0; s.found.mass_above = q0;
-        } else if (!s1 && s2) {
-            s.found.bin = 126u - 2u * (uint32_t)lane;
-            s.found.cnt_above = (uint32_t)r1; s.found.cnt_bin = c1; s.found.mass_above = q1;
-        }
-    }
-    __syncthreads();
-    return s.found;
 }
 
 // Mass of this workgroup's own tokens in the bins above index `bin` of a

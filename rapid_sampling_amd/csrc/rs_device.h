@@ -281,4 +281,72 @@ __device__ __forceinline__ uint32_t wave_max_u32(uint32_t v)
     return lane63_u32(v);
 }
 
+// ---- 96-bit masses ------------------------------------------------------------
+struct M96 {
+    uint64_t lo;
+    uint32_t hi;
+};
+__device__ __forceinline__ M96 m96(u128 v) { return M96{(uint64_t)v, (uint32_t)(v >> 64)}; }
+__device__ __forceinline__ u128 wide(M96 a) { return ((u128)a.hi << 64) | a.lo; }
+__device__ __forceinline__ M96 operator+(M96 a, M96 b)
+{
+    M96 r;
+    const bool c = __builtin_add_overflow(a.lo, b.lo, &r.lo);
+    r.hi = a.hi + b.hi + (c ? 1u : 0u);
+    return r;
+}
+__device__ __forceinline__ M96 operator-(M96 a, M96 b)
+{
+    M96 r;
+    const bool c = __builtin_sub_overflow(a.lo, b.lo, &r.lo);
+    r.hi = a.hi - b.hi - (c ? 1u : 0u);
+    return r;
+}
+__device__ __forceinline__ bool operator>=(M96 a, M96 b) { return a.hi > b.hi || (a.hi == b.hi && a.lo >= b.lo); }
+__device__ __forceinline__ bool operator<(M96 a, M96 b) { return !(a >= b); }
+
+__device__ __forceinline__ uint32_t lane_of(uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); }
+__device__ __forceinline__ uint64_t lane_of(uint64_t v, uint32_t l) { return ((uint64_t)lane_of((uint32_t)(v >> 32), l) << 32) | lane_of((uint32_t)v, l); }
+__device__ __forceinline__ M96 lane_of(M96 v, uint32_t l) { return M96{lane_of(v.lo, l), lane_of(v.hi, l)}; }
+__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+__device__ __forceinline__ uint64_t uniform(uint64_t v) { return ((uint64_t)uniform((uint32_t)(v >> 32)) << 32) | uniform((uint32_t)v); }
+__device__ __forceinline__ M96 uniform(M96 v) { return M96{uniform(v.lo), uniform(v.hi)}; }
+
+// A mass as four limbs of 24 bits in 32-bit words: sums of up to 256 of them need no carries, so a scan
+// over a wave is four independent chains of fused DPP adds (a 96-bit add costs a carry through the VCC register
+// per word, with wait states between).
+struct Limbs {
+    uint32_t w[4];
+};
+__device__ __forceinline__ Limbs operator+(Limbs a, Limbs b) { return Limbs{{a.w[0] + b.w[0], a.w[1] + b.w[1], a.w[2] + b.w[2], a.w[3] + b.w[3]}}; }
+__device__ __forceinline__ Limbs operator-(Limbs a, Limbs b) { return Limbs{{a.w[0] - b.w[0], a.w[1] - b.w[1], a.w[2] - b.w[2], a.w[3] - b.w[3]}}; }
+__device__ __forceinline__ Limbs limbs(M96 m)
+{
+    const uint32_t x = (uint32_t)m.lo, y = (uint32_t)(m.lo >> 32), z = m.hi;
+    return Limbs{{x & 0xFFFFFFu, __builtin_amdgcn_alignbit(y, x, 24u) & 0xFFFFFFu, __builtin_amdgcn_alignbit(z, y, 16u) & 0xFFFFFFu, z >> 8}};
+}
+__device__ __forceinline__ M96 m96(Limbs l)
+{
+    const uint32_t w1 = l.w[1] + (l.w[0] >> 24), w2 = l.w[2] + (w1 >> 24), w3 = l.w[3] + (w2 >> 24);
+    const uint32_t x = (l.w[0] & 0xFFFFFFu) | w1 << 24, y = (w1 >> 8 & 0xFFFFu) | w2 << 16, z = (w2 >> 16 & 0xFFu) | w3 << 8;
+    return M96{((uint64_t)y << 32) | x, z};
+}
+template <int CTRL, int ROW_MASK>
+__device__ __forceinline__ void dpp_add(Limbs &v)
+{
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v.w[i] += dpp0_u32<CTRL, ROW_MASK>(v.w[i]);
+}
+__device__ __forceinline__ Limbs wave_inclusive_scan(Limbs v)
+{
+    dpp_add<0x111, 0xf>(v); dpp_add<0x112, 0xf>(v); dpp_add<0x114, 0xf>(v); dpp_add<0x118, 0xf>(v);
+    dpp_add<0x142, 0xa>(v); dpp_add<0x143, 0xc>(v);
+    return v;
+}
+__device__ __forceinline__ Limbs lane_of(Limbs v, uint32_t l) { return Limbs{{lane_of(v.w[0], l), lane_of(v.w[1], l), lane_of(v.w[2], l), lane_of(v.w[3], l)}}; }
+
+// 128-bit sums of masses (a row's total stays below 2^84) go the same way.
+__device__ __forceinline__ u128 wave_inclusive_scan(u128 v) { return wide(m96(wave_inclusive_scan(limbs(m96(v))))); }
+__device__ __forceinline__ u128 wave_sum(u128 v) { return wide(m96(lane_of(wave_inclusive_scan(limbs(m96(v))), 63u))); }
+
 }  // namespace rs

@@ -5,37 +5,6 @@
 
 namespace rs {
 
-// ---- 96-bit masses ------------------------------------------------------------
-struct M96 {
-    uint64_t lo;
-    uint32_t hi;
-};
-__device__ __forceinline__ M96 m96(u128 v) { return M96{(uint64_t)v, (uint32_t)(v >> 64)}; }
-__device__ __forceinline__ u128 wide(M96 a) { return ((u128)a.hi << 64) | a.lo; }
-__device__ __forceinline__ M96 operator+(M96 a, M96 b)
-{
-    M96 r;
-    const bool c = __builtin_add_overflow(a.lo, b.lo, &r.lo);
-    r.hi = a.hi + b.hi + (c ? 1u : 0u);
-    return r;
-}
-__device__ __forceinline__ M96 operator-(M96 a, M96 b)
-{
-    M96 r;
-    const bool c = __builtin_sub_overflow(a.lo, b.lo, &r.lo);
-    r.hi = a.hi - b.hi - (c ? 1u : 0u);
-    return r;
-}
-__device__ __forceinline__ bool operator>=(M96 a, M96 b) { return a.hi > b.hi || (a.hi == b.hi && a.lo >= b.lo); }
-__device__ __forceinline__ bool operator<(M96 a, M96 b) { return !(a >= b); }
-
-__device__ __forceinline__ uint32_t lane_of(uint32_t v, uint32_t l) { return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)l); }
-__device__ __forceinline__ uint64_t lane_of(uint64_t v, uint32_t l) { return ((uint64_t)lane_of((uint32_t)(v >> 32), l) << 32) | lane_of((uint32_t)v, l); }
-__device__ __forceinline__ M96 lane_of(M96 v, uint32_t l) { return M96{lane_of(v.lo, l), lane_of(v.hi, l)}; }
-__device__ __forceinline__ uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
-__device__ __forceinline__ uint64_t uniform(uint64_t v) { return ((uint64_t)uniform((uint32_t)(v >> 32)) << 32) | uniform((uint32_t)v); }
-__device__ __forceinline__ M96 uniform(M96 v) { return M96{uniform(v.lo), uniform(v.hi)}; }
-
 // Mass of a packed bin whose tokens share the exponent ex (87 <= ex <= 127): 44 bits shifted by up to 40.
 __device__ __forceinline__ M96 pack_m96(uint64_t w, uint32_t ex)
 {
@@ -43,39 +12,6 @@ __device__ __forceinline__ M96 pack_m96(uint64_t w, uint32_t ex)
     const uint32_t sh = ex - 87u;
     return M96{sum << sh, (uint32_t)((sum >> 24) >> (40u - sh))};
 }
-
-// The same mass as four limbs of 24 bits in 32-bit words: sums of up to 256 of them need no carries, so a scan
-// over a wave is four independent chains of fused DPP adds (a 96-bit add costs a carry through the VCC register
-// per word, with wait states between).
-struct Limbs {
-    uint32_t w[4];
-};
-__device__ __forceinline__ Limbs operator+(Limbs a, Limbs b) { return Limbs{{a.w[0] + b.w[0], a.w[1] + b.w[1], a.w[2] + b.w[2], a.w[3] + b.w[3]}}; }
-__device__ __forceinline__ Limbs operator-(Limbs a, Limbs b) { return Limbs{{a.w[0] - b.w[0], a.w[1] - b.w[1], a.w[2] - b.w[2], a.w[3] - b.w[3]}}; }
-__device__ __forceinline__ Limbs limbs(M96 m)
-{
-    const uint32_t x = (uint32_t)m.lo, y = (uint32_t)(m.lo >> 32), z = m.hi;
-    return Limbs{{x & 0xFFFFFFu, __builtin_amdgcn_alignbit(y, x, 24u) & 0xFFFFFFu, __builtin_amdgcn_alignbit(z, y, 16u) & 0xFFFFFFu, z >> 8}};
-}
-__device__ __forceinline__ M96 m96(Limbs l)
-{
-    const uint32_t w1 = l.w[1] + (l.w[0] >> 24), w2 = l.w[2] + (w1 >> 24), w3 = l.w[3] + (w2 >> 24);
-    const uint32_t x = (l.w[0] & 0xFFFFFFu) | w1 << 24, y = (w1 >> 8 & 0xFFFFu) | w2 << 16, z = (w2 >> 16 & 0xFFu) | w3 << 8;
-    return M96{((uint64_t)y << 32) | x, z};
-}
-template <int CTRL, int ROW_MASK>
-__device__ __forceinline__ void dpp_add(Limbs &v)
-{
-#pragma unroll
-    for (int i = 0; i < 4; ++i) v.w[i] += dpp0_u32<CTRL, ROW_MASK>(v.w[i]);
-}
-__device__ __forceinline__ Limbs wave_inclusive_scan(Limbs v)
-{
-    dpp_add<0x111, 0xf>(v); dpp_add<0x112, 0xf>(v); dpp_add<0x114, 0xf>(v); dpp_add<0x118, 0xf>(v);
-    dpp_add<0x142, 0xa>(v); dpp_add<0x143, 0xc>(v);
-    return v;
-}
-__device__ __forceinline__ Limbs lane_of(Limbs v, uint32_t l) { return Limbs{{lane_of(v.w[0], l), lane_of(v.w[1], l), lane_of(v.w[2], l), lane_of(v.w[3], l)}}; }
 
 // ceil(f * s) for a uniform s < 2^96 and a float 0 < f <= 1 (see ceil_mul), the usual 2^-7 <= f < 1 by one 32-bit multiplication
 // per word.
@@ -245,6 +181,83 @@ __device__ __forceinline__ bool fine_search(const int lane, F word, const Edge &
     e.cnt_bin = first ? lane_of(c0, l) : lane_of(c1, l);
     e.sum = lane_of(si - ss, l) + (first ? 0ull : lane_of(s0, l));
     return true;
+}
+
+// Scan the level-1 histogram s.g (the first wave; the others wait) for the first bin, largest e first, at which
+// (count so far >= top_k) or (mass so far >= P).  The total mass of the histogram is the row total D, and P = ceil(top_p * D)
+// is derived from it here.  With LOCAL this workgroup's own histogram s.hm is scanned along and its mass above the
+// boundary bin returned in local_above.  With GIVEN_P the histogram is that of a subset of the row which is complete above some
+// value: P stands as it is, D is left alone, and the scan may end without the set becoming sufficient (bin 0 then).
+template <bool LOCAL, bool GIVEN_P = false, typename L = Lds>
+__device__ __forceinline__ Found hist_find_level1(L &s, uint64_t top_k, float top_p, int lane, int wave)
+{
+    if (wave == 0) {
+        auto bins = [](const uint64_t *h) {
+            return [h](uint32_t o, uint64_t (&w)[4]) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = h[o * 4u + (uint32_t)i];
+            };
+        };
+        OctScan sc, own;
+        sc.load(lane, bins(s.g));
+        if constexpr (LOCAL) own.load(lane, bins(s.hm));
+        M96 P;
+        if constexpr (GIVEN_P) P = m96((u128)s.P);
+        else {
+            const M96 D = sc.total();
+            P = ceil_mul(top_p, D);
+            if (lane == 0) { s.D = wide(D); s.P = wide(P); }
+        }
+        Edge e{0u, 0u, 0u, 0ull, M96{0ull, 0u}, 0ull};
+        const bool found = sc.search((uint32_t)min(top_k, (uint64_t)0xFFFFFFFFull), P, e);
+        M96 mine{0ull, 0u};
+        if constexpr (LOCAL) {
+            const uint32_t ex = e.at >> 2, l = 127u - ex, k = 3u - (e.at & 3u);
+            if (found) {
+                uint64_t part = 0;
+#pragma unroll
+                for (uint32_t i = 0; i < 3u; ++i)
+                    if (i < k) part += lane_of(own.s[i], l);
+                mine = m96(lane_of(own.upto - own.own, l)) + mass_of(part, ex);
+            }
+        }
+        if (lane == 0) {
+            s.found.bin = found ? e.at : 0u;
+            s.found.cnt_above = e.cnt_above; s.found.cnt_bin = e.cnt_bin;
+            s.found.mass_above = wide(e.above);
+            s.found.local_above = wide(mine);
+        }
+    }
+    __syncthreads();
+    return s.found;
+}
+
+// The same for a 128-bin level (all tokens share the exponent ex).
+template <typename L = Lds>
+__device__ __forceinline__ Found hist_find128(L &s, const uint64_t *arr, uint32_t cnt0, u128 mass0, uint64_t top_k, uint32_t ex, int lane, int wave)
+{
+    if (wave == 0) {
+        const M96 above = m96(mass0);
+        const Edge from{0u, uniform(cnt0), 0u, 0ull, above, 0ull};
+        Edge e = from;
+        if (fine_search(lane, [&](int i) { return arr[i]; }, from, (uint32_t)min(top_k, (uint64_t)0xFFFFFFFFull), need_of(uniform(m96((u128)s.P)), uniform(above), ex), e) &&
+            lane == 0) {
+            s.found.bin = e.at;
+            s.found.cnt_above = e.cnt_above; s.found.cnt_bin = e.cnt_bin;
+            s.found.mass_above = wide(above + mass_of(e.sum, ex));
+        }
+    }
+    __syncthreads();
+    return s.found;
+}
+
+// tie_and_target by one wave on values that are the same for all its lanes: on scalars (one thread's 64- and 96-bit
+// multiplications and carries go through the vector unit one dependent instruction after the other).
+__device__ __forceinline__ Target target_of_wave(const Params &p, uint32_t row, uint64_t rand64, float xmax, u128 D, u128 P, uint32_t thr, uint32_t n_gt,
+                                                 uint32_t n_eq, u128 Gm, uint32_t levels, bool write_diag)
+{
+    return tie_and_target(p, row, uniform(rand64), xmax, wide(uniform(m96(D))), wide(uniform(m96(P))), uniform(thr), uniform(n_gt), uniform(n_eq),
+                          wide(uniform(m96(Gm))), levels, write_diag);
 }
 
 // ---- a row finished from a list of at most 64 tokens that holds its kept set and its threshold's ties ----

@@ -45,7 +45,7 @@ struct LdsRowS {                      // what the shared helpers work on
 static_assert(kRowW * kRowListW / 2 >= (uint32_t)kNB * 8u, "the lists lie where the copies of the level-1 bins were");
 struct LdsRow {
     LdsRowS  s;
-    uint64_t hr8[kRowW * kRowListW / 2];   // level 1 while it is counted: eight copies of each bin (the first kNB * 8
+    alignas(16) uint64_t hr8[kRowW * kRowListW / 2];   // level 1 while it is counted: eight copies of each bin (the first kNB * 8
                                       // words); later the waves' lists of the boundary bin's tokens (all of it)
     uint64_t lev[128 * 4];            // a deeper level while it is counted: four copies
     u128     wq[kRowW];               // per wave: kept weight of its stretch of the row
@@ -91,7 +91,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     PrevCall prev;
     prev.slow_rows = 0; prev.meta = 0;
     if (reporter) prev = report_begin(p);
-    for (int i = tid; i < kNB * 8; i += kRowT) L.hr8[i] = 0;
+    for (int i = (int)kBin0 * 4 + tid; i < kNB * 4; i += kRowT) reinterpret_cast<uint4 *>(L.hr8)[i] = make_uint4(0u, 0u, 0u, 0u);       // (the bins of live tokens)
     if (tid == 0) { L.nolist = 0u; L.nokept = 0u; }
 
     // token (g0 + j * 64) * 4 + q sits in register j * 4 + q; slots past the end of the stretch read the
@@ -154,19 +154,30 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     const float M = __builtin_floorf(xmax);
 
     // e (not clamped at 2^-40: what lies below is dead and lands in bins nobody looks at) and level 1
+    // (slots past the end of the stretch become dead tokens, spread over the bins of 32 octaves: see slice_count_and_stash)
     const Frame fr = frame_of(M, eb);
+    const uint32_t mine = uniform(g_end - min((uint32_t)wave * G, g_end));          // groups of the wave's stretch
+    // (the mask is made opaque, so that the fractions are not kept, a register each, for the levels and the weights further down)
+    uint32_t fmask0 = 0x7FFFFFu;
+    asm volatile("" : "+s"(fmask0));
+    const float dead = (__builtin_fabsf(M) <= 100.0f ? M : 0.0f) - 48.0f - (float)(lane & 31);
 #pragma unroll
     for (int j = 0; j < kRowR; ++j) {
-        if (g0 + (uint32_t)(j * kWave) < g_end) {
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t b = fr.raw(__uint_as_float(eb[j * 4 + q]));
-                eb[j * 4 + q] = b;
-                atomicAdd(reinterpret_cast<unsigned long long *>(&L.hr8[(b >> 21) * 8u + (uint32_t)(lane & 7)]),
-                          (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
-            }
-        } else {
+        if ((uint32_t)(j * kWave) >= mine) {             // nothing of the row (a scalar test)
             eb[j * 4] = 0; eb[j * 4 + 1] = 0; eb[j * 4 + 2] = 0; eb[j * 4 + 3] = 0;
+            continue;
+        }
+        if ((uint32_t)(j + 1) * (uint32_t)kWave > mine) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if ((uint32_t)(j * kWave + lane) >= mine) eb[j * 4 + q] = __float_as_uint(dead);
+        }
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t b = fr.raw(__uint_as_float(eb[j * 4 + q]));
+            eb[j * 4 + q] = b;
+            atomicAdd(reinterpret_cast<unsigned long long *>(&L.hr8[(b >> 21) * 8u + (uint32_t)(lane & 7)]),
+                      (unsigned long long)(kPackOne | (b & fmask0)));
         }
     }
     if (p.e_bits) {
@@ -193,12 +204,12 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     // (what is the same for all threads stays in scalar registers, or in LDS until it is used)
     f.bin = uniform(f.bin); f.cnt_above = uniform(f.cnt_above); f.cnt_bin = uniform(f.cnt_bin);
     auto target = [&](uint32_t thr, uint32_t n_gt, uint32_t n_eq, u128 above, uint32_t rounds) {
-        return tie_and_target(p, row, p.inj_u ? 0ull : L.rand64, xmax, s.D, s.P, thr, n_gt, n_eq, above, rounds, true);
+        return target_of_wave(p, row, p.inj_u ? 0ull : L.rand64, xmax, s.D, s.P, thr, n_gt, n_eq, above, rounds, lane == 0);
     };
 
     // one tie of all the row's tokens: as on the streaming path
     if (f.cnt_bin == (uint32_t)p.V && bin_is_one_tie(s.g[f.bin], f.bin, e_bits_of(xmax, M))) {
-        if (tid == 0) {
+        if (wave == 0) {
             const uint32_t thr1 = e_bits_of(xmax, M);
             const Target tg = target(thr1, 0u, f.cnt_bin, (u128)0, 0u);
             uint32_t lo_i = 0, hi_i = (uint32_t)p.V - 1u;
@@ -285,7 +296,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
             lo = s.bc32[6];
         }
         const uint32_t thr = lo;
-        if (tid == 0) {
+        if (wave == 0) {
             const Target tg = target(thr, f.cnt_above, f.cnt_bin, f.mass_above, kRowRounds);
             s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
         }
@@ -412,7 +423,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
         lo = s.bc32[6];
     }
     const uint32_t thr = lo;
-    if (tid == 0) {
+    if (wave == 0) {
         const Target tg = target(thr, f.cnt_above, f.cnt_bin, f.mass_above, kRowRounds);
         s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
     }

@@ -717,8 +717,8 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
         lo = s.bc32[6];
     }
     const uint32_t thr = lo;
-    if (tid == 0) {
-        const Target tg = tie_and_target(p, row, rand64, xmax, D, P, thr, f.cnt_above, f.cnt_bin, f.mass_above, kW1Rounds, true);
+    if (wave == 0) {
+        const Target tg = target_of_wave(p, row, rand64, xmax, D, P, thr, f.cnt_above, f.cnt_bin, f.mass_above, kW1Rounds, lane == 0);
         s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
     }
     __syncthreads();
