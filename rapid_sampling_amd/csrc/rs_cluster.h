@@ -547,11 +547,12 @@ __device__ __forceinline__ bool slice_finish(const Params &p, Lds &s, Slice<R, P
             if (s.abort) return false;
         }
         const uint32_t idx = s.bc32[7];
+        const bool finite = p.decay - p.decay == 0.0f;   // groups of four that are all +0.0 then stay that, but for the sampled token's
 #pragma unroll
         for (int j = 0; j < R; ++j) {
-            if (j < nv) {
-                const uint32_t i4 = base4 + (uint32_t)j * kThreads;
-                float4 v = pen[j];
+            const uint32_t i4 = base4 + (uint32_t)j * kThreads;
+            float4 v = pen[j];
+            if (j < nv && (!finite || i4 == idx >> 2 || (__float_as_uint(v.x) | __float_as_uint(v.y) | __float_as_uint(v.z) | __float_as_uint(v.w)) != 0u)) {
                 const uint32_t e0 = i4 * 4;
                 v.x = __builtin_fmaf(v.x, p.decay, (e0 + 0 != idx) ? 0.0f : (v.x == 0.0f ? p.presence : p.repetition));
                 v.y = __builtin_fmaf(v.y, p.decay, (e0 + 1 != idx) ? 0.0f : (v.y == 0.0f ? p.presence : p.repetition));

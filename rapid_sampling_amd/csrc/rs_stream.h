@@ -1847,6 +1847,21 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
     Lds &s = u.f.s;
     LdsB &t = u.f.t;
     if (tid == 0) { s.abort = 0; s.host_words = p.host_words; s.who = row << 16 | part; s.seen = 0; s.want = 0; }
+    // Every penalty but the sampled token's becomes fma(pen, decay, 0) whatever is sampled: the workgroups that wait write theirs
+    // while they do, the last one behind its verdict.  Groups of four that are all +0.0 stay that under a finite decay.  (Written
+    // behind the verdict, all of them: 32 rows of 131072 20.8 us a call, 19.4 this way.)  A row that falls back writes them once more.
+    auto decayed = [&]() {
+        if constexpr (PEN) {
+            const bool finite = p.decay - p.decay == 0.0f;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                const float4 q = sl.pen[j];
+                if (j < sl.nv && (!finite || (__float_as_uint(q.x) | __float_as_uint(q.y) | __float_as_uint(q.z) | __float_as_uint(q.w)) != 0u))
+                    sl.pn4[sl.base4 + (uint32_t)j * kThreads] = make_float4(__builtin_fmaf(q.x, p.decay, 0.0f), __builtin_fmaf(q.y, p.decay, 0.0f),
+                                                                            __builtin_fmaf(q.z, p.decay, 0.0f), __builtin_fmaf(q.w, p.decay, 0.0f));
+            }
+        }
+    };
     uint32_t verdict = 0;
     if (last) {
         // the token list: the cluster rounds' histogram copies, which are not in use while a row is
@@ -1860,7 +1875,9 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
         __syncthreads();
         verdict = done && t.result != 0u ? t.result : kVerdictFallback;
         if (tid == 0) a_store(&rc->verdict, verdict);
+        decayed();
     } else {
+        decayed();
         __syncthreads();
         if (tid == 0) {
             const uint64_t t0 = wall_clock64();
@@ -1881,20 +1898,14 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
     }
     const uint32_t idx = verdict - 1u;
     if (PEN) {
-        // penalties: decay and one-hot add, from registers (reference: sampling.cu:427-437)
+        // the sampled token's penalty, by the thread that wrote its group before (reference: sampling.cu:427-437)
 #pragma unroll
-        for (int j = 0; j < R; ++j) {
-            if (j < sl.nv) {
-                const uint32_t i4 = sl.base4 + (uint32_t)j * kThreads;
-                float4 q = sl.pen[j];
-                const uint32_t e0 = i4 * 4;
-                q.x = __builtin_fmaf(q.x, p.decay, (e0 + 0 != idx) ? 0.0f : (q.x == 0.0f ? p.presence : p.repetition));
-                q.y = __builtin_fmaf(q.y, p.decay, (e0 + 1 != idx) ? 0.0f : (q.y == 0.0f ? p.presence : p.repetition));
-                q.z = __builtin_fmaf(q.z, p.decay, (e0 + 2 != idx) ? 0.0f : (q.z == 0.0f ? p.presence : p.repetition));
-                q.w = __builtin_fmaf(q.w, p.decay, (e0 + 3 != idx) ? 0.0f : (q.w == 0.0f ? p.presence : p.repetition));
-                sl.pn4[i4] = q;
+        for (int j = 0; j < R; ++j)
+            if (sl.base4 + (uint32_t)j * kThreads == idx >> 2 && j < sl.nv) {
+                const uint32_t q = idx & 3u;
+                const float old = q == 0u ? sl.pen[j].x : q == 1u ? sl.pen[j].y : q == 2u ? sl.pen[j].z : sl.pen[j].w;
+                reinterpret_cast<float *>(sl.pn4)[idx] = __builtin_fmaf(old, p.decay, old == 0.0f ? p.presence : p.repetition);
             }
-        }
     }
     // leave: the last workgroup out of the row puts its record back to zero
     __syncthreads();

@@ -2026,7 +2026,8 @@ def test_short_row_kernel_in_calls_of_more_rows_than_compute_units(torch_cuda, o
 
 @pytest.mark.parametrize("B,V", [(11, 16388), (9, 40000), (9, 65536)])
 def test_penalties_on_the_streaming_path_in_slices_of_8192_tokens(torch_cuda, oracle, B, V):
-    """The pass with penalties on slices of 8192 tokens, a last one of a few tokens among them: a row done the slow way (half of it ties
+    """The pass with penalties on slices of 8192 tokens, a last one of a few tokens among them, and the one-launch and the general
+    kernel, which write only what is not +0.0: a row done the slow way (half of it ties
     at the top), slices with more non-zero penalties than they can note, penalties of -0.0, sampled tokens already penalised, rows
     without and with nothing but penalties, and a decay that is not finite; three chained steps, bit for bit against the oracle."""
     torch = torch_cuda
@@ -2046,18 +2047,18 @@ def test_penalties_on_the_streaming_path_in_slices_of_8192_tokens(torch_cuda, or
     pen0[6] = rng.exponential(0.1, V).astype(np.float32)
     rc, c, k, p = capi.normalize(0.8, 50, 0.9, V, B, 1)
     lg = torch.from_numpy(lg_np).cuda()
-    for decay in (0.95, float("inf")):
+    for decay, path in ((0.95, "stream"), (float("inf"), "stream"), (0.95, "fused"), (float("inf"), "fused"), (0.95, "cluster"), (float("inf"), "cluster")):
         pen_ref = pen0.copy() if decay == 0.95 else np.zeros_like(pen0)
         smp = capi.Sampler(B, V)
         pen = torch.from_numpy(pen_ref.copy()).cuda()
         for step in range(3):
             u_np = H.uniforms(B, 700 + step)
             ref_out, ref_diag = oracle.sample_batch(lg_np, c, k, p, injected_u=u_np, penalties=pen_ref, presence=0.1, repetition=0.2, decay=decay)
-            print("penalties, slices of 8192:", B, V, decay, step, flush=True)
-            res = smp.sample(lg, c, k, p, uniforms=torch.from_numpy(u_np).cuda(), penalties=pen, presence=0.1, repetition=0.2, decay=decay, path="stream")
-            _check(res, ref_out, ref_diag, "penalties, slices of 8192 tokens, decay %r step %d" % (decay, step))
-            assert np.array_equal(pen.cpu().numpy().view(np.uint32), pen_ref.view(np.uint32)), (decay, step)
-            if decay == 0.95 and step == 0:
+            print("penalties:", B, V, path, decay, step, flush=True)
+            res = smp.sample(lg, c, k, p, uniforms=torch.from_numpy(u_np).cuda(), penalties=pen, presence=0.1, repetition=0.2, decay=decay, path=path)
+            _check(res, ref_out, ref_diag, "penalties, path %s, decay %r step %d" % (path, decay, step))
+            assert np.array_equal(pen.cpu().numpy().view(np.uint32), pen_ref.view(np.uint32)), (path, decay, step)
+            if decay == 0.95 and step == 0 and path == "stream":
                 assert res["diag"]["rounds"][1] == 8 and res["diag"]["rounds"][0] == 0, res["diag"]["rounds"]
             assert smp.status() == 0
         smp.close()
