@@ -90,8 +90,8 @@ int rs_normalize_args(double temperature, int64_t top_k, double top_p,
  * stash of its largest tokens, its counts and bins, and 4 KB for its note of
  * the non-zero penalties; up to 3.2 bytes per token for the first 6M tokens,
  * where slices are shorter; 1.5 bytes per token in rows of up to 262144
- * tokens, for the slices of 8192 tokens the one-pass wide path and the
- * counting-only pass cut there); a quarter to two fifths of the reference's
+ * tokens, for the slices of 8192 tokens the one-pass wide path, the
+ * counting-only pass and the pass with penalties cut there); a quarter to two fifths of the reference's
  * scratch.  It does not grow with T.  (A call is also accepted with a
  * workspace that lacks the room for those slices of 8192 tokens -- the size
  * versions before 414 asked for -- and then works on the long slices.)
@@ -240,9 +240,10 @@ int rs_philox_init(void *state_device, uint64_t seed, int32_t B, void *stream);
  *
  * Calls that share a workspace must be ordered on one stream.
  *
- * The call is one kernel launch (the general kernel: rows of fewer than 8192
- * tokens in calls of fewer than 2^17, and whatever the other paths do not
- * take; with penalties and top_k <= 1024 the one-launch streaming kernel while
+ * The call is one kernel launch (the short-row kernel, one workgroup per row:
+ * rows of fewer than 8192 tokens, with penalties of up to 16384, and most
+ * calls of up to 512 rows of that length without; the general kernel:
+ * whatever the other paths do not take; with penalties and top_k <= 1024 the one-launch streaming kernel while
  * the call fits the GPU at once), two for calls without penalties whose kept
  * set is expected to be small (a wait-free pass over the logits and a per-row
  * finish; see rs_policy; plain temperature sampling -- top_k = V, top_p = 1,
@@ -262,8 +263,8 @@ int rs_philox_init(void *state_device, uint64_t seed, int32_t B, void *stream);
  * 8192 to 65536 tokens when the call has 64 rows (128 from 32768 tokens on)
  * or more (the row kernel: one workgroup of 512 or 1024 threads per row, the
  * row in its registers; not calls of 257 to 319 rows of up to 32768 tokens, nor
- * of 257 to 511 rows of 32769 to 39999 tokens), or three for calls of at least
- * 2^23 tokens with penalties and top_k <= 1024 (a pass over logits and
+ * of 257 to 511 rows of 32769 to 39999 tokens), or three for larger calls, of at
+ * least 2^22 tokens, with penalties and top_k <= 1024 (a pass over logits and
  * penalties that also writes the decayed penalties, the finish, which patches
  * the sampled tokens' penalties, and a fix-up kernel for slices the pass left
  * alone); results are identical either way.  No environment variable is read.
