@@ -97,17 +97,30 @@ __global__ void __launch_bounds__(kW1SampleT) wide_sample_kernel(const Params p,
     for (int i = tid; i < kNB * 8; i += kThreads) s.hm[i] = 0;
     for (int i = tid; i < 128 * 4; i += kThreads) s.sub[i] = 0;
 
+    // A chunk is one wave's groups of one j: chunk j * (waves) + wave, so what lies beyond the sample is left out a wave at a time
+    // (a sample of 16640 tokens fills 4 of the 8 groups a thread has room for; with the rest worked out and masked the kernel took
+    // 12.9 us on 128 rows of 100256).
+    const uint32_t wave_g = uniform((uint32_t)wave) * (uint32_t)kWave;
+    auto sampled = [&](int j) { return wave_g + (uint32_t)j * kThreads < ng; };      // wave-uniform: ng is a whole number of chunks
     uint32_t eb[kW1SampleR * 4];
     float lmax = -3.402823466e+38f;
+    float4 l[kW1SampleR];
 #pragma unroll
     for (int j = 0; j < kW1SampleR; ++j) {
         const uint32_t g = (uint32_t)tid + (uint32_t)j * kThreads;
         const uint32_t src = ((g >> 6) * S + (S >> 1)) * 64u + (g & 63u);
-        const float4 l = load_logits4(lrow, g < ng ? src : 0u, p.dtype);
-        const float x0 = sf(l.x * p.c), x1 = sf(l.y * p.c), x2 = sf(l.z * p.c), x3 = sf(l.w * p.c);
-        if (g < ng) lmax = fmaxf(lmax, fmaxf(fmaxf(x0, x1), fmaxf(x2, x3)));
-        eb[j * 4 + 0] = __float_as_uint(x0); eb[j * 4 + 1] = __float_as_uint(x1);
-        eb[j * 4 + 2] = __float_as_uint(x2); eb[j * 4 + 3] = __float_as_uint(x3);
+        l[j] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+        if (sampled(j)) l[j] = load_logits4(lrow, src, p.dtype);
+    }
+#pragma unroll
+    for (int j = 0; j < kW1SampleR; ++j) {
+        eb[j * 4] = 0; eb[j * 4 + 1] = 0; eb[j * 4 + 2] = 0; eb[j * 4 + 3] = 0;
+        if (sampled(j)) {
+            const float x0 = sf(l[j].x * p.c), x1 = sf(l[j].y * p.c), x2 = sf(l[j].z * p.c), x3 = sf(l[j].w * p.c);
+            lmax = fmaxf(lmax, fmaxf(fmaxf(x0, x1), fmaxf(x2, x3)));
+            eb[j * 4 + 0] = __float_as_uint(x0); eb[j * 4 + 1] = __float_as_uint(x1);
+            eb[j * 4 + 2] = __float_as_uint(x2); eb[j * 4 + 3] = __float_as_uint(x3);
+        }
     }
     uint32_t kmax = wave_max_u32(fkey(lmax));
     if (lane == 0) s.u32[wave] = kmax;
@@ -120,10 +133,13 @@ __global__ void __launch_bounds__(kW1SampleT) wide_sample_kernel(const Params p,
     const Frame frm = frame_of(M, eb);
 #pragma unroll
     for (int j = 0; j < kW1SampleR; ++j) {
-        const bool in = (uint32_t)tid + (uint32_t)j * kThreads < ng;
+        if (!sampled(j)) {
+            eb[j * 4] = 0; eb[j * 4 + 1] = 0; eb[j * 4 + 2] = 0; eb[j * 4 + 3] = 0;
+            continue;
+        }
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const uint32_t b = in ? frm.raw(__uint_as_float(eb[j * 4 + q])) : 0u;
+            const uint32_t b = frm.raw(__uint_as_float(eb[j * 4 + q]));
             eb[j * 4 + q] = b;
             if (b >= kEMinBits)
                 atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * 8u + (uint32_t)(lane & 7)]),
@@ -198,7 +214,7 @@ __global__ void __launch_bounds__(kW1SampleT) wide_sample_kernel(const Params p,
 #pragma unroll
     for (int j = 0; j < kW1SampleR; ++j)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
+        for (int q = 0; q < 4 && sampled(j); ++q) {
             const uint32_t b = eb[j * 4 + q];
             if (b - lo_live < width) atomicAdd(&s.sub[((b - lo_bits) >> sh) * 4u + (uint32_t)(lane & 3)], 1u);
         }
@@ -411,7 +427,7 @@ __global__ void __launch_bounds__(kThreads, (R <= 8 ? 5 : RS_STREAM_WAVES)) wide
         const uint32_t c0 = pack_count(w0), c1 = pack_count(w1);
         const u128 m0 = w0 ? pack_mass(w0, 127u + ex0 - exb_top) : (u128)0, m1 = w1 ? pack_mass(w1, 127u + ex1 - exb_top) : (u128)0;
         const uint32_t ci = wave_inclusive_scan(c0 + c1);
-        const u128 mi = wave_inclusive_scan(m0 + m1);
+        const u128 mi = wide(m96(wave_inclusive_scan(limbs(m96(m0 + m1)))));
         const uint32_t cc_hi = ci - c1, cc_lo = ci;
         const u128 mm_hi = mi - m1, mm_lo = mi;
         uint32_t *cum = v.cum + ((size_t)row * G + part) * kSB;
@@ -482,6 +498,24 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
     const uint64_t h0 = rc->rowhist[tid], h1 = rc->rowhist[tid + kThreads];
     rc->rowhist[tid] = 0; rc->rowhist[tid + kThreads] = 0;          // left clean for the next call
     const WideGuess gs = *reinterpret_cast<const WideGuess *>(rc->A);
+    // What the slices say about the range's sub-bin edges: every thread takes one edge and half of the slices, sixteen slices'
+    // loads in flight at a time.  Where they lie is known from the start, so the first sixteen (all, up to 32 slices) are asked
+    // for here and arrive while level 1 is worked out; which of them count is decided below.  (With the sample's short cut and one
+    // exchange for the three sums around the range: 128 rows of 100256 54.9 -> 51.4 us a call.)
+    const uint32_t edge = (uint32_t)tid & 127u, upper = (uint32_t)tid >> 7;
+    const uint32_t g_mid = (G + 1u) >> 1, g_lo = upper ? g_mid : 0u, g_hi = upper ? G : g_mid;
+    const uint32_t *cp0 = v.cum + (size_t)row * G * kSB + edge;
+    const uint64_t *mp0 = v.stash + (size_t)row * G * kStashCap + 2 + 2 * edge;
+    uint32_t ec[16];
+    ulonglong2 em[16];
+    auto ask = [&](uint32_t g0) {
+#pragma unroll
+        for (int u = 0; u < 16; ++u) {
+            const size_t g = min(g0 + (uint32_t)u, G - 1u);
+            ec[u] = cp0[g * kSB]; em[u] = *reinterpret_cast<const ulonglong2 *>(mp0 + g * kStashCap);
+        }
+    };
+    ask(g_lo);
     const bool drawer = tid == kWave && !p.inj_u;
     if (drawer) {
         uint32_t *rng_st = p.rng + (size_t)row * 16;
@@ -574,32 +608,27 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
         if (bin > bt) { c_ab = pack_count(w); if (w) m_ab = pack_mass(w, (uint32_t)bin >> 2); }
         else if (bin >= lo_bin) c_in = pack_count(w);
     }
-    const uint32_t cnt_ar = block_sum_u32(s, c_ab, lane, wave);
-    const uint32_t cnt_in = block_sum_u32(s, c_in, lane, wave);
-    const u128 mass_ar = block_sum_u128(s, m_ab, lane, wave);
-    // The row's running sums at the sub-bin edges: the slices' added up (edge 128 is zero by definition).
-    // Every thread takes one edge and half of the slices, sixteen slices' loads in flight at a time; what a
-    // slice that said nothing left behind is not added.
+    uint32_t cnt_ar = 0, cnt_in = 0;
+    u128 mass_ar = 0;
     if ((uint32_t)tid < G) t.take[tid] = ph.window & kWideValid;
-    __syncthreads();
+    {
+        c_ab = wave_sum(c_ab); c_in = wave_sum(c_in); m_ab = wave_sum(m_ab);
+        __syncthreads();
+        if (lane == 0) { s.u32[wave] = c_ab; s.u32[kWaves + wave] = c_in; s.q128[wave] = m_ab; }
+        __syncthreads();
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) { cnt_ar += s.u32[w]; cnt_in += s.u32[kWaves + w]; mass_ar += s.q128[w]; }
+    }
+    // The row's running sums at the sub-bin edges: the slices' added up (edge 128 is zero by definition); what a
+    // slice that said nothing left behind is not added.
     uint32_t Rc = 0;
     u128 Rm = 0;
     {
-        const uint32_t edge = (uint32_t)tid & 127u, upper = (uint32_t)tid >> 7;
-        const uint32_t g_mid = (G + 1u) >> 1, g_lo = upper ? g_mid : 0u, g_hi = upper ? G : g_mid;
-        const uint32_t *cp0 = v.cum + (size_t)row * G * kSB + edge;
-        const uint64_t *mp0 = v.stash + (size_t)row * G * kStashCap + 2 + 2 * edge;
         for (uint32_t g0 = g_lo; g0 < g_hi; g0 += 16u) {
-            uint32_t c[16];
-            uint64_t m0[16], m1[16];
-#pragma unroll
-            for (int u = 0; u < 16; ++u) {
-                const size_t g = min(g0 + (uint32_t)u, G - 1u);
-                c[u] = cp0[g * kSB]; m0[u] = mp0[g * kStashCap]; m1[u] = mp0[g * kStashCap + 1];
-            }
+            if (g0 != g_lo) ask(g0);
 #pragma unroll
             for (int u = 0; u < 16; ++u)
-                if (g0 + (uint32_t)u < g_hi && t.take[g0 + (uint32_t)u]) { Rc += c[u]; Rm += (u128)m0[u] | ((u128)m1[u] << 64); }
+                if (g0 + (uint32_t)u < g_hi && t.take[g0 + (uint32_t)u]) { Rc += ec[u]; Rm += (u128)em[u].x | ((u128)em[u].y << 64); }
         }
         if (upper) { t.blo[edge] = (uint64_t)Rm; t.bhi[edge] = (uint64_t)(Rm >> 64); t.m4[edge] = Rc; }
     }
@@ -731,7 +760,7 @@ __device__ __forceinline__ void wide1_finish_row(const Params &p, const StreamVi
         const uint32_t a = tid ? t.take[tid - 1] : 0u, e = t.take[tid];
         for (uint32_t i = a; i < e; ++i) kept_g += weight((uint32_t)(t.list[i] >> 32));
     }
-    u128 inc = wave_inclusive_scan(kept_g);
+    u128 inc = wide(m96(wave_inclusive_scan(limbs(m96(kept_g)))));
     __syncthreads();
     if (lane == kWave - 1) s.q128[wave] = inc;
     __syncthreads();

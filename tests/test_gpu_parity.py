@@ -2062,3 +2062,27 @@ def test_penalties_on_the_streaming_path_in_slices_of_8192_tokens(torch_cuda, or
                 assert res["diag"]["rounds"][1] == 8 and res["diag"]["rounds"][0] == 0, res["diag"]["rounds"]
             assert smp.status() == 0
         smp.close()
+
+
+@pytest.mark.parametrize("V", [260, 4100, 16384, 16640, 50304, 262148, 524292])
+def test_one_pass_wide_path_with_samples_that_end_within_a_round_of_waves(torch_cuda, oracle, V):
+    """The one-pass wide path where the sample fills one wave, whole rounds of sixteen waves, and one wave more (1, 16, 64 and 65
+    chunks), and where a finishing thread adds up more than sixteen slices: every row against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    B = 3
+    rng = np.random.default_rng(V)
+    lg_np = (rng.random((B, V)) * 4.0).astype(np.float32)
+    lg_np[1] = (rng.standard_normal(V) * 1.5 - 200.0).astype(np.float32)     # a frame beyond 2^100
+    lg_np[2, : V // 2] = -np.inf
+    u_np = H.uniforms(B, 77)
+    lg, u = torch.from_numpy(lg_np).cuda(), torch.from_numpy(u_np).cuda()
+    smp = capi.Sampler(B, V)
+    for top_k, top_p in ((V // 8, 0.9), (-1, 0.5)):
+        rc, c, k, p = capi.normalize(1.0, top_k, top_p, V, B, 1)
+        ref_out, ref_diag = oracle.sample_batch(lg_np, c, k, p, injected_u=u_np)
+        print("one-pass wide path:", V, top_k, top_p, flush=True)
+        res = smp.sample(lg, c, k, p, uniforms=u, path="wide1")
+        _check(res, ref_out, ref_diag, "one-pass wide path, %d tokens, top_k %d" % (V, top_k))
+        assert smp.status() == 0
+    smp.close()
