@@ -95,10 +95,15 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     for (int w = 0; w < (NT / kWave); ++w) k = max(k, s.u32[w]);
     const float M = __builtin_floorf(fkey_inv(k));
 
-    // e in the slice's frame, not yet clamped at 2^-40, and its histogram.  Slots past the end of the row (the row's last slice
-    // only, so that the others are spared the test: 256 x 151936 bfloat16 32.6 -> 31.2 us a call) become dead tokens, spread over the bins of 32 octaves.
+    // e in the slice's frame, not yet clamped at 2^-40, and its histogram.  Slots past the end of the row are in its last slice
+    // only.  In slices of 4096 and 16384 tokens the others are spared the test per group (256 x 151936 bfloat16 32.6 -> 31.2 us a call)
+    // and those slots become dead tokens, spread over the bins of 32 octaves.  Slices of 8192 tokens, which wait for memory rather
+    // than for instructions, keep the test and leave such slots out: 512 x 50304 with every token kept, a seventh of whose last slices
+    // is filled, 29.6 against 30.1 us a call, 64 x 152064 18.0 against 18.5.  (Both forms behind one branch: the pass over slices of 16384
+    // tokens was 7 % slower.)
     const Frame fr = frame_of(M, eb);
-    if ((part + 1u) * (uint32_t)(NT * R) > (uint32_t)p.V >> 2) {
+    constexpr bool kTest = R == 8;
+    if (!kTest && (part + 1u) * (uint32_t)(NT * R) > (uint32_t)p.V >> 2) {
         const float dead = (__builtin_fabsf(M) <= 100.0f ? M : 0.0f) - 48.0f - (float)(lane & 31);
 #pragma unroll
         for (int j = 0; j < R; ++j)
@@ -108,11 +113,18 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
             }
     }
 #pragma unroll
-    for (int i = 0; i < R * 4; ++i) {
-        const uint32_t b = fr.raw(__uint_as_float(eb[i]));
-        eb[i] = b;
-        atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * kRep + (lane & (kRep - 1))]),
-                  (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
+    for (int j = 0; j < R; ++j) {
+        if (!kTest || j < nv) {
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const uint32_t b = fr.raw(__uint_as_float(eb[j * 4 + q]));
+                eb[j * 4 + q] = b;
+                atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * kRep + (lane & (kRep - 1))]),
+                          (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
+            }
+        } else {
+            eb[j * 4] = 0; eb[j * 4 + 1] = 0; eb[j * 4 + 2] = 0; eb[j * 4 + 3] = 0;
+        }
     }
     if (p.e_bits) {
         // diagnostics: e of every token, still in the slice's frame; the finishing workgroup re-bases it
