@@ -108,6 +108,11 @@ int rs_workspace_bytes(int32_t B, int32_t V, size_t *bytes);
  * fill kernel on `stream`.  Call once after allocation, and again after a call
  * reported RS_ERR_DEVICE; rs_sample leaves the workspace ready for the next
  * call on the same stream.  Allocates nothing.
+ * After RS_ERR_DEVICE the tokens, generator states and penalties of that call
+ * are those of a call that stopped somewhere: a slice whose workgroup gave up
+ * keeps its penalties as they were, one that had learnt its row's token has
+ * rewritten them.  A caller that wants to repeat the call restores penalties
+ * and states from copies of its own.
  */
 int rs_workspace_init(void *workspace_device, size_t bytes, void *stream);
 

@@ -69,6 +69,7 @@ struct alignas(256) RowCtl {
     uint64_t h[kLevels + 1][kNB];   // cluster histograms, packed (see kPackOne); one spare for the re-framed level 1
     uint64_t rowhist[kNB];          // streaming path: the row's bins by absolute octave (mod 128), summed over its slices
 };
+static_assert(sizeof(RowCtl) == 38144 && offsetof(RowCtl, arrived) == 12, "a test that spoils a row's count: tests/capi.py ROW_RECORD_BYTES");
 
 struct Params {
     const void  *logits;       // fp32, or bf16 / fp16 (dtype): converted exactly on load

@@ -1862,18 +1862,20 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
     // Every penalty but the sampled token's becomes fma(pen, decay, 0) whatever is sampled: the workgroups that wait write theirs
     // while they do, the last one behind its verdict.  Groups of four that are all +0.0 stay that under a finite decay.  (Written
     // behind the verdict, all of them: 32 rows of 131072 20.8 us a call, 19.4 this way.)  A row that falls back writes them once more.
-    auto decayed = [&]() {
+    // A workgroup whose wait gives up puts its penalties back: no token was sampled for it.
+    auto rewrite = [&](auto fn) {
         if constexpr (PEN) {
             const bool finite = p.decay - p.decay == 0.0f;
 #pragma unroll
             for (int j = 0; j < R; ++j) {
                 const float4 q = sl.pen[j];
                 if (j < sl.nv && (!finite || (__float_as_uint(q.x) | __float_as_uint(q.y) | __float_as_uint(q.z) | __float_as_uint(q.w)) != 0u))
-                    sl.pn4[sl.base4 + (uint32_t)j * kThreads] = make_float4(__builtin_fmaf(q.x, p.decay, 0.0f), __builtin_fmaf(q.y, p.decay, 0.0f),
-                                                                            __builtin_fmaf(q.z, p.decay, 0.0f), __builtin_fmaf(q.w, p.decay, 0.0f));
+                    sl.pn4[sl.base4 + (uint32_t)j * kThreads] = make_float4(fn(q.x), fn(q.y), fn(q.z), fn(q.w));
             }
         }
     };
+    auto decayed = [&]() { rewrite([&](float q) { return __builtin_fmaf(q, p.decay, 0.0f); }); };
+    auto put_back = [&]() { rewrite([](float q) { return q; }); };
     uint32_t verdict = 0;
     if (last) {
         // the token list: the cluster rounds' histogram copies, which are not in use while a row is
@@ -1901,11 +1903,12 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
             s.bc32[7] = w;
         }
         __syncthreads();
-        if (s.abort) return;
+        if (s.abort) { put_back(); return; }
         verdict = s.bc32[7];
     }
     if (verdict == kVerdictFallback) {
-        fused_fallback<R, PEN>(p, v, s, sl, key);       // ends with the cluster path's own leaving protocol
+        // (ends with the cluster path's own leaving protocol; a wait that gives up there comes before its write of the penalties)
+        if (!fused_fallback<R, PEN>(p, v, s, sl, key)) put_back();
         return;
     }
     const uint32_t idx = verdict - 1u;

@@ -92,6 +92,7 @@ def normalize(temperature, top_k, top_p, V, B=1, T=1):
 
 
 HEADER_BYTES = 2304          # the workspace's launch header (sizeof(rs::WsHeader)); tests that spoil a workspace leave it alone
+ROW_RECORD_BYTES = 38144     # a row's record, counted from the workspace's end (sizeof(rs::RowCtl))
 
 
 def workspace_bytes(B, V):

@@ -1561,6 +1561,44 @@ def test_bounded_wait_reports_error_and_recovers(torch_cuda, oracle):
     smp.close()
 
 
+def test_one_launch_path_that_gives_up_leaves_the_penalties_as_they_were(torch_cuda, oracle):
+    """The workgroups of the one-launch path write the decayed penalties while they wait for the sampled token.  When
+    that wait gives up (here: every row's count of arrived workgroups begins at 1000, so that none is ever the last one and
+    no token is posted) no token was sampled, and the penalties must be what they were, bit for bit; after
+    rs_workspace_init the call does what it should from them."""
+    torch = torch_cuda
+    from tests import capi
+    B, V = 3, 65536
+    lg_np = H.logits_normal(B, V, 1.5, seed=84)
+    pen0 = H.penalties_sparse(B, V, seed=85)
+    pen0[1] = np.random.default_rng(86).exponential(0.1, V).astype(np.float32)
+    pen0[2, ::7] = -0.0
+    rc, c, k, p = capi.normalize(0.8, 50, 0.9, V, B, 1)
+    u_np = H.uniforms(B, 87)
+    lg, u = torch.from_numpy(lg_np).cuda(), torch.from_numpy(u_np).cuda()
+    for decay in (0.95, float("inf")):
+        pen_ref = pen0.copy()
+        ref_out, ref_diag = oracle.sample_batch(lg_np, c, k, p, injected_u=u_np, penalties=pen_ref, presence=0.1, repetition=0.2, decay=decay)
+        smp = capi.Sampler(B, V, init=True)
+        smp.set_wait_limit(20)
+        words = smp.ws[: smp.ws.numel() & ~255].view(torch.int32)
+        for row in range(B):
+            words[words.numel() - (row + 1) * (capi.ROW_RECORD_BYTES // 4) + 3] = 1000          # RowCtl::arrived
+        pen = torch.from_numpy(pen0.copy()).cuda()
+        torch.cuda.synchronize()
+        print("no workgroup arrives last, expecting the wait for the sampled token to give up: decay", decay, flush=True)
+        res = smp.sample(lg, c, k, p, uniforms=u, penalties=pen, presence=0.1, repetition=0.2, decay=decay, want_diag=False, path="fused")
+        assert res["rc"] == 0 and smp.status() == -9 and smp.where()[0] == 6, smp.where()
+        assert np.array_equal(pen.cpu().numpy().view(np.uint32), pen0.view(np.uint32)), decay
+        smp.reinit()
+        res = smp.sample(lg, c, k, p, uniforms=u, penalties=pen, presence=0.1, repetition=0.2, decay=decay, path="fused")
+        _check(res, ref_out, ref_diag, "after re-initialisation")
+        got = pen.cpu().numpy()
+        same = (got.view(np.uint32) == pen_ref.view(np.uint32)) | (np.isnan(got) & np.isnan(pen_ref))
+        assert same.all() and smp.status() == 0
+        smp.close()
+
+
 def test_python_module_raises_after_a_failed_call_and_recovers(torch_cuda, oracle):
     """The same failure through the drop-in module, whose workspace is private: the call whose kernel gave
     up returns (its result is garbage), the next call on that stream raises RuntimeError and sets the
