@@ -403,6 +403,19 @@ struct LdsB {
     uint32_t result;             // sampled token + 1 once the row is finished
 };
 
+// The call's parameters, read from the kernel's arguments once more (they are the first of them in every kernel): for the
+// ways that almost no row takes.  Otherwise what only those need is loaded at the kernel's start and kept, in scalar
+// registers that the usual chain is short of: the finishing kernel of eight slices a wave spilled 36 of them, 7 this way, and
+// over 192 shapes of 1 to 256 rows its calls take 0.991 of their time (64 rows of 152064 19.66 -> 19.26 us a call, of 65540 15.65 -> 15.31).
+__device__ __forceinline__ Params params_again()
+{
+    auto *args = __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(args));
+    Params p;
+    __builtin_memcpy(&p, (const void *)args, sizeof(Params));
+    return p;
+}
+
 // A row the stashes cannot finish (a nucleus or a tie of thousands of tokens, more kept tokens than
 // the list holds): the finishing workgroup does it alone, from the logits, in a few passes over the
 // row -- the level-1 histogram in the row's frame (M = floor of the row's maximum is known), the
@@ -926,7 +939,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
     // What the stashes cannot finish, this workgroup does alone from the logits.  Such rows are
     // counted, and the first of a call tells the caller's policy at once (that a call went well is
     // reported by the call after it, see report_begin).
-    auto tell_policy = [&]() {
+    auto tell_policy = [&](const Params &p) {
         if (tid == 0) {
             const uint32_t c = __hip_atomic_fetch_add(&p.hdr->n_need, 1u, __ATOMIC_RELAXED, RS_AGENT);
             if (c == 0u && p.host_words)                 // the call's first such row tells the caller's policy at once
@@ -1179,7 +1192,7 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
                 // 44 against 38 us; 128 rows of 262144, 68 against 116): such a call says so to the caller's
                 // policy, as it did when these rows still went the slow way.
                 // (p.tell_lists: calls of fewer than 2^24 tokens, and calls whose rows the row kernel would take)
-                if (p.tell_lists) tell_policy();
+                if (p.tell_lists) tell_policy(params_again());
             }
         } else {                                         // plan B, the stashes whole
             slow = all > v.list_cap || all == 0u;
@@ -1205,15 +1218,16 @@ __device__ __forceinline__ bool finish_row(const Params &p, const StreamView &v,
             if (FUSED) return false;
             __syncthreads();                             // the random number is there
             if (NT > kThreads && tid >= kThreads) return true;
-            if (p.penalties && p.defer_pen == 2) pen_restore(p, v, row);
-            finish_row_slow(p, s, t, row, xmax, p.inj_u ? 0ull : t.rand64);
-            tell_policy();
+            const Params q = params_again();
+            if (q.penalties && q.defer_pen == 2) pen_restore(q, v, row);
+            finish_row_slow(q, s, t, row, xmax, q.inj_u ? 0ull : t.rand64);
+            tell_policy(q);
             return true;
         }
     }
 
     // a list so long that another kernel is faster (the host's rule): said to the caller's policy
-    if (!FUSED && n > p.long_list) tell_policy();
+    if (!FUSED && n > p.long_list) tell_policy(params_again());
 
     if (n <= (uint32_t)kWave) {
         // ---- a short list: every pair of its tokens ----
