@@ -74,7 +74,9 @@ template <bool FUSED, typename T> __device__ __forceinline__ T get(const T *p)
 // in eb), the packed histogram added to the row's and kept under the slice's own name, cumulative
 // counts, and the stash of its largest tokens with the value down to which it is complete.
 // Returns the key of the slice's maximum.
-template <int R, int NT, int kRep, bool FUSED, bool KEEP = false, int kCap = kStashCap>     // KEEP: a call that keeps every live token (top_k = V, top_p = 1); kCap: room of the stash
+// KEEP: a call that keeps every live token (top_k = V, top_p = 1); kCap: room of the stash; PAD: much of the last slices lies past the
+// end of their rows.
+template <int R, int NT, int kRep, bool FUSED, bool KEEP = false, int kCap = kStashCap, bool PAD = false>
 __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const StreamView &v, LdsA<kRep> &s, uint32_t (&eb)[R * 4],
                                                           const float lmax, const uint32_t row, const uint32_t part,
                                                           const uint32_t base4, const int nv)
@@ -96,34 +98,38 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     const float M = __builtin_floorf(fkey_inv(k));
 
     // e in the slice's frame, not yet clamped at 2^-40, and its histogram.  Slots past the end of the row are in its last slice
-    // only.  In slices of 4096 and 16384 tokens the others are spared the test per group (256 x 151936 bfloat16 32.6 -> 31.2 us a call)
-    // and those slots become dead tokens, spread over the bins of 32 octaves.  Slices of 8192 tokens, which wait for memory rather
-    // than for instructions, keep the test and leave such slots out: 512 x 50304 with every token kept, a seventh of whose last slices
-    // is filled, 29.6 against 30.1 us a call, 64 x 152064 18.0 against 18.5.  (Both forms behind one branch: the pass over slices of 16384
-    // tokens was 7 % slower.)
+    // only.  A wave is spared them kChunk groups at a time, by a scalar test, where there is nothing of the row in any; those beside
+    // live tokens become dead ones, spread over the bins of 32 octaves.  (A test per group and lane, slots left out one by one,
+    // keeps the groups' instructions apart: 256 x 151936 bfloat16 32.6 us a call against 31.2, 64 x 152064 bfloat16, in slices of 8192
+    // tokens, 18.9 against 18.3.)  Slices of 16384 tokens are not tested at all unless a quarter of the call's slots lie past the end of
+    // their rows (PAD, the host's rule, rs_stream.hip): the tests cost such a call 1 % (512 x 50304, 23 % of the slots, 34.9 us a call without,
+    // 35.2 with), the slots 2 to 8 % (1024 x 8196 25.1 and 23.2, 512 x 32772 with top_k 1000 51.7 and 50.5).
     const Frame fr = frame_of(M, eb);
-    constexpr bool kTest = R == 8;
-    if (!kTest && (part + 1u) * (uint32_t)(NT * R) > (uint32_t)p.V >> 2) {
-        const float dead = (__builtin_fabsf(M) <= 100.0f ? M : 0.0f) - 48.0f - (float)(lane & 31);
+    constexpr int kChunk = PAD || (R == 4 && !FUSED) ? 2 : R;
+    constexpr bool kSkip = PAD || (R <= 8 && !FUSED);    // (the one-launch kernel: 0.6 % slower with them over 92 shapes)
+    const uint32_t first = uniform(base4), left = ((uint32_t)p.V >> 2) - min(first, (uint32_t)p.V >> 2);      // groups of the row from the wave's first one on
+    const float dead = (__builtin_fabsf(M) <= 100.0f ? M : 0.0f) - 48.0f - (float)(lane & 31);
 #pragma unroll
-        for (int j = 0; j < R; ++j)
-            if (j >= nv) {
+    for (int jc = 0; jc < R; jc += kChunk) {
+        if (kSkip && (uint32_t)(jc * NT) >= left) {
 #pragma unroll
-                for (int q = 0; q < 4; ++q) eb[j * 4 + q] = __float_as_uint(dead);
-            }
-    }
+            for (int i = jc * 4; i < (jc + kChunk) * 4; ++i) eb[i] = 0;
+            continue;
+        }
+        if ((uint32_t)((jc + kChunk - 1) * NT + kWave) > left) {
 #pragma unroll
-    for (int j = 0; j < R; ++j) {
-        if (!kTest || j < nv) {
+            for (int j = jc; j < jc + kChunk; ++j)
+                if (j >= nv) {
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const uint32_t b = fr.raw(__uint_as_float(eb[j * 4 + q]));
-                eb[j * 4 + q] = b;
-                atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * kRep + (lane & (kRep - 1))]),
-                          (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
-            }
-        } else {
-            eb[j * 4] = 0; eb[j * 4 + 1] = 0; eb[j * 4 + 2] = 0; eb[j * 4 + 3] = 0;
+                    for (int q = 0; q < 4; ++q) eb[j * 4 + q] = __float_as_uint(dead);
+                }
+        }
+#pragma unroll
+        for (int i = jc * 4; i < (jc + kChunk) * 4; ++i) {
+            const uint32_t b = fr.raw(__uint_as_float(eb[i]));
+            eb[i] = b;
+            atomicAdd(reinterpret_cast<unsigned long long *>(&s.hm[(b >> 21) * kRep + (lane & (kRep - 1))]),
+                      (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
         }
     }
     if (p.e_bits) {
@@ -323,7 +329,7 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     return k;
 }
 
-template <int R, int NT, int DT, bool KEEP = false>     // NT threads, each with R groups of four tokens of the slice; DT the logits' type
+template <int R, int NT, int DT, bool KEEP = false, bool PAD = false>     // NT threads, each with R groups of four tokens of the slice; DT the logits' type
 __global__ void __launch_bounds__(NT, (R <= 8 ? 5 : RS_STREAM_WAVES)) stream_kernel(const Params p, const StreamView v)
 {
     constexpr int kRep = stream_copies<R>();
@@ -387,7 +393,7 @@ __global__ void __launch_bounds__(NT, (R <= 8 ? 5 : RS_STREAM_WAVES)) stream_ker
     }
     // a call that keeps everything has no rows to report on; the counting-only pass of the wide path does
     if (reporter) report_end(p, prev, !KEEP || p.report != 0u);
-    slice_count_and_stash<R, NT, kRep, false, KEEP>(p, v, s, eb, lmax, row, part, base4, nv);
+    slice_count_and_stash<R, NT, kRep, false, KEEP, kStashCap, PAD>(p, v, s, eb, lmax, row, part, base4, nv);
 }
 
 struct LdsB {

@@ -30,15 +30,21 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
 #ifndef RS_LONG_NT
 #define RS_LONG_NT 256
 #endif
-#define RS_STREAM(Rv, NTv, Lv, KEEPv) do {                                                                                         \
-        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F32, KEEPv>), sgrid, dim3(NTv), 0, st, p, v);       \
-        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_BF16, KEEPv>), sgrid, dim3(NTv), 0, st, p, v); \
-        else hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F16, KEEPv>), sgrid, dim3(NTv), 0, st, p, v);                             \
+#define RS_STREAM(Rv, NTv, Lv, KEEPv, PADv) do {                                                                                         \
+        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F32, KEEPv, PADv>), sgrid, dim3(NTv), 0, st, p, v);       \
+        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_BF16, KEEPv, PADv>), sgrid, dim3(NTv), 0, st, p, v); \
+        else hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F16, KEEPv, PADv>), sgrid, dim3(NTv), 0, st, p, v);                             \
         if (KEEPv) hipLaunchKernelGGL((keep_finish_kernel<Lv>), dim3(B), dim3(kKeepT + kWave), 0, st, p, v);                              \
         else launch_finish(B, finish_lds_bytes, st, p, v); } while (0)
-    if (slice_r == 4) { if (keep) RS_STREAM(4, 256, 12, true); else RS_STREAM(4, 256, 12, false); }
-    else if (slice_r == 8) { if (keep) RS_STREAM(8, 256, 13, true); else RS_STREAM(8, 256, 13, false); }
-    else { if (keep) RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, true); else RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, false); }
+    if (slice_r == 4) { if (keep) RS_STREAM(4, 256, 12, true, false); else RS_STREAM(4, 256, 12, false, false); }
+    else if (slice_r == 8) { if (keep) RS_STREAM(8, 256, 13, true, false); else RS_STREAM(8, 256, 13, false, false); }
+    else if (keep) RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, true, false);
+    else {
+        // (a quarter of the slots past the ends of their rows: see slice_count_and_stash)
+        const uint32_t slots = v.G << kStreamLongLog2;
+        if (slots - (uint32_t)p.V >= slots >> 2) RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, false, true);
+        else RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, false, false);
+    }
 #undef RS_STREAM
     return hipGetLastError();
 }

@@ -2124,3 +2124,39 @@ def test_one_pass_wide_path_with_samples_that_end_within_a_round_of_waves(torch_
         _check(res, ref_out, ref_diag, "one-pass wide path, %d tokens, top_k %d" % (V, top_k))
         assert smp.status() == 0
     smp.close()
+
+
+@pytest.mark.parametrize("fmt", ["float32", "bfloat16"])
+@pytest.mark.parametrize("B,V", [(9, 4), (9, 2052), (9, 4100), (9, 6140), (520, 8196), (392, 12292), (776, 8196), (776, 10236), (776, 12288), (776, 12292),
+                                 (776, 16380), (520, 16388), (520, 18436)])
+def test_streaming_pass_rows_that_end_within_a_slice(torch_cuda, oracle, B, V, fmt):
+    """Last slices that end inside a wave's group of tokens, a wave's two groups, or a few tokens in, in slices of 4096, 8192 and 16384
+    tokens, these on both sides of a quarter of slots past the end of the row (8196, 12288 | 12292 tokens): eight kinds of rows --
+    far from zero, masked but for the last token, one tie, all of them in the last slots -- over and over, e of every token and
+    every field against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    rng = np.random.default_rng(V + B)
+    lg = (rng.standard_normal((8, V)) * 2.0).astype(np.float32)
+    lg[1] -= 300.0
+    lg[2, :-1] = -np.inf
+    lg[3] = 0.5
+    lg[4] = rng.random(V, dtype=np.float32)
+    lg[5, -3:] += 40.0
+    lg[6] = np.sort(lg[6]) + 1000.0
+    lg[7, : V // 2] = -1e30
+    dt = getattr(torch, fmt)
+    lg = torch.from_numpy(lg).to(dt).float().numpy()
+    u8 = H.uniforms(8, 31)
+    reps = (B + 7) // 8
+    x = torch.from_numpy(lg).cuda().to(dt).repeat(reps, 1)[:B].contiguous()
+    u = torch.from_numpy(np.tile(u8, reps)[:B]).cuda()
+    smp = capi.Sampler(B, V)
+    for top_k, top_p in ((50, 0.9), (1000, 0.95)):
+        rc, c, k, p = capi.normalize(0.8, min(top_k, V), top_p, V, B, 1)
+        ref_out, ref_diag, ref_e = oracle.sample_batch(lg, c, k, p, injected_u=u8, want_e=True)
+        print("streaming pass:", B, V, fmt, top_k, flush=True)
+        res = smp.sample(x, c, k, p, uniforms=u, path="stream", want_e=True)
+        _check(res, np.tile(ref_out, reps)[:B], np.tile(ref_diag, reps)[:B], "rows of %d tokens, top_k %d" % (V, top_k), np.tile(ref_e, (reps, 1))[:B])
+        assert smp.status() == 0
+    smp.close()
