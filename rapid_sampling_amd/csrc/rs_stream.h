@@ -101,22 +101,28 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     // only.  A wave is spared them kChunk groups at a time, by a scalar test, where there is nothing of the row in any; those beside
     // live tokens become dead ones, spread over the bins of 32 octaves.  (A test per group and lane, slots left out one by one,
     // keeps the groups' instructions apart: 256 x 151936 bfloat16 32.6 us a call against 31.2, 64 x 152064 bfloat16, in slices of 8192
-    // tokens, 18.9 against 18.3.)  Slices of 16384 tokens are not tested at all unless a quarter of the call's slots lie past the end of
+    // tokens, 18.9 against 18.3.)  In slices of 8192 tokens four groups at a time: all eight at once take 82 registers instead of 74, with
+    // which five workgroups share a compute unit and not six, and calls of 1281 to 1536 of them need another round (512 x 20480 with
+    // top_k 1000 43.1 us a call against 39.9).  Slices of 16384 tokens are not tested at all unless a quarter of the call's slots lie past the end of
     // their rows (PAD, the host's rule, rs_stream.hip): the tests cost such a call 1 % (512 x 50304, 23 % of the slots, 34.9 us a call without,
     // 35.2 with), the slots 2 to 8 % (1024 x 8196 25.1 and 23.2, 512 x 32772 with top_k 1000 51.7 and 50.5).
+    // Calls that keep every token, which have no stash to select, hide the test per lane behind their loads and lose more by the registers
+    // of groups that are worked out together: 512 x 50304 bfloat16, in slices of 8192, 27.2 us a call against 28.6 with one test of all eight,
+    // in shorter slices nothing tested 10.4 against 10.5 (32 x 65536 bfloat16).
     const Frame fr = frame_of(M, eb);
-    constexpr int kChunk = PAD || (R == 4 && !FUSED) ? 2 : R;
-    constexpr bool kSkip = PAD || (R <= 8 && !FUSED);    // (the one-launch kernel: 0.6 % slower with them over 92 shapes)
+    constexpr bool kLane = KEEP && R == 8;
+    constexpr int kChunk = kLane ? 1 : PAD || (R == 4 && !FUSED && !KEEP) ? 2 : R == 8 && !FUSED ? 4 : R;
+    constexpr bool kSkip = PAD || (R <= 8 && !FUSED && !KEEP);   // (the one-launch kernel: 0.6 % slower with them over 92 shapes)
     const uint32_t first = uniform(base4), left = ((uint32_t)p.V >> 2) - min(first, (uint32_t)p.V >> 2);      // groups of the row from the wave's first one on
     const float dead = (__builtin_fabsf(M) <= 100.0f ? M : 0.0f) - 48.0f - (float)(lane & 31);
 #pragma unroll
     for (int jc = 0; jc < R; jc += kChunk) {
-        if (kSkip && (uint32_t)(jc * NT) >= left) {
+        if (kLane ? jc >= nv : kSkip && (uint32_t)(jc * NT) >= left) {
 #pragma unroll
             for (int i = jc * 4; i < (jc + kChunk) * 4; ++i) eb[i] = 0;
             continue;
         }
-        if ((uint32_t)((jc + kChunk - 1) * NT + kWave) > left) {
+        if (!kLane && (uint32_t)((jc + kChunk - 1) * NT + kWave) > left) {
 #pragma unroll
             for (int j = jc; j < jc + kChunk; ++j)
                 if (j >= nv) {
