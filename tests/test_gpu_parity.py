@@ -462,6 +462,27 @@ def test_row_kernel_unusual_rows(torch_cuda, oracle):
         _run_case(torch, oracle, capi, lg, 1.0, -1, 0.9, u_np=H.uniforms(6, 63), dtype=fmt, what="row kernel %s" % fmt)
 
 
+@pytest.mark.parametrize("B,V,k,one", [
+    (256, 8196, 1024, True), (257, 8192, 1024, True), (513, 8192, 300, True), (600, 8188, 1000, True), (257, 8196, 50, True),
+    (257, 8196, 51, False), (257, 16384, 300, False), (512, 12288, 50, True), (512, 16384, 65, False), (513, 12288, 50, False),
+    (64, 16384, 1000, True), (64, 16388, 1000, False)])
+def test_rows_of_up_to_16384_tokens_with_a_bounding_top_k_take_the_kernel_that_suits_them(torch_cuda, B, V, k, one):
+    """Which calls with a bounding top_k one workgroup per row does by itself (diag.rounds == 10) and which the streaming
+    path (0): rows of up to 8192 tokens all of them, longer ones up to 256 rows, or 512 with a top_k of up to 50.  Calls of 257 to
+    512 rows of 8196 to 16384 tokens with more were 5 to 40 % slower in one workgroup per row."""
+    from tests import capi
+    lg = torch_cuda.from_numpy(H.logits_normal(B, V, 1.5, seed=B)).cuda()
+    rc, c, kk, pp = capi.normalize(1.0, k, 0.95, V, B, 1)
+    smp = capi.Sampler(B, V, with_policy=True, init=True)
+    u = torch_cuda.from_numpy(H.uniforms(B, 64)).cuda()
+    res = smp.sample(lg, c, kk, pp, uniforms=u)
+    assert rc == 0 and res["rc"] == 0 and smp.status() == 0
+    assert (res["diag"]["rounds"] == (10 if one else 0)).all(), np.unique(res["diag"]["rounds"], return_counts=True)
+    ref = smp.sample(lg, c, kk, pp, uniforms=u, path="cluster")
+    for f in FIELDS:
+        assert np.array_equal(res["diag"][f], ref["diag"][f]), f
+
+
 def test_row_kernel_takes_the_wide_kept_sets_of_calls_of_many_short_rows(torch_cuda, oracle):
     """Calls of 128 rows and more (64 in rows of fewer than 32768 tokens) of 8192 to 65536 tokens whose kept
     sets the stashes cannot hold go to the row kernel by themselves (diag.rounds == 10): a top_k of
