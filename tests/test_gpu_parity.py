@@ -1863,23 +1863,38 @@ def test_row_kernel_512_threads_in_every_format_at_the_bounds_of_the_lists(torch
         assert np.array_equal(res["e_bits"][:12], ref_e)
 
 
-def _us_per_call(torch, sample, fn):
-    """Microseconds per call of fn, back to back on the current stream, routed as a program's calls are: the best of
-    seven batches of 30, after twelve calls that settle the route."""
+def _us_per_call(torch, sample, fn, path="auto"):
+    """Microseconds per call of fn, back to back on the current stream, routed as a program's calls are or by the path
+    named: the best of seven batches of 30, after twelve calls that settle the route."""
     sample.reset_routing()
-    for _ in range(12):
-        fn()
-        torch.cuda.synchronize()
-    best = float("inf")
-    for _ in range(7):
-        e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-        e0.record()
-        for _ in range(30):
+    sample._sample.force_path(path)
+    try:
+        for _ in range(12):
             fn()
-        e1.record()
-        e1.synchronize()
-        best = min(best, e0.elapsed_time(e1) * 1000.0 / 30)
+            torch.cuda.synchronize()
+        best = float("inf")
+        for _ in range(7):
+            e0, e1 = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+            e0.record()
+            for _ in range(30):
+                fn()
+            e1.record()
+            e1.synchronize()
+            best = min(best, e0.elapsed_time(e1) * 1000.0 / 30)
+    finally:
+        sample._sample.force_path("auto")
     return best
+
+
+def _rounds_by(sample, path, logits, states, k, p, penalties=None):
+    """diag.rounds of every row of a call at temperature 1 on the path named: which kernel finished it."""
+    from tests import capi
+    sample._sample.force_path(path)
+    try:
+        _, diag, _ = sample._sample.batch_sampling_debug(logits, penalties, states, 0.1, 0.1, 0.95, 1.0, k, p)
+    finally:
+        sample._sample.force_path("auto")
+    return diag.cpu().numpy().view(capi.DIAG_DTYPE)["rounds"].ravel()
 
 
 def _top_tokens_per_slice(rng, B, V, slice_tokens, counts):
@@ -1964,22 +1979,25 @@ def test_streaming_finish_short_lists_of_whole_stashes(torch_cuda, oracle, V, fi
 
 def test_streaming_finish_of_flat_rows_in_calls_of_many(torch_cuda):
     """Flat rows of 4096 tokens with a small top_k, whose lists come out of whole stashes, against rows of the same call
-    that leave short lists at once: short lists are finished the same way wherever they come from.  Time ratio,
-    measured 1.40; 1.83 when lists out of whole stashes took the digits of longer ones."""
+    that leave short lists at once, on the streaming path (by themselves such calls take the short-row kernel): short lists are
+    finished the same way wherever they come from.  Time ratio, measured 1.34; 1.83 when lists out of whole stashes took the digits of longer ones."""
     torch = torch_cuda
     import rapid_sampling_amd as sample
     gen = torch.Generator(device="cuda").manual_seed(4)
     flat = torch.rand((1024, 4096), generator=gen, device="cuda")
     peaked = torch.randn((1024, 4096), generator=gen, device="cuda").mul_(3.0)
     st = sample.setup_rand(1, 1024)
-    a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_temperature_topk_topp(x, st, 1.0, 1, 1.0)) for x in (flat, peaked))
+    for x in (flat, peaked):
+        assert (_rounds_by(sample, "stream", x, st, 1, 1.0) == 0).all()
+    a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_temperature_topk_topp(x, st, 1.0, 1, 1.0), "stream")
+            for x in (flat, peaked))
     print("flat %.1f us, peaked %.1f us: %.2f" % (a, b, a / b), flush=True)
     assert a < 1.6 * b, (a, b)
 
 
 def test_one_launch_path_of_rows_of_few_slices(torch_cuda):
     """320 flat rows of two slices each with penalties and a small top_k, on the one-launch path, against the same rows with
-    a nucleus alone, on the general kernel.  Time ratio, measured 0.85; 0.94 when every finish asked ahead for 64 slices
+    a nucleus alone, on the general kernel (by themselves both take the short-row kernel).  Time ratio, measured 0.84; 0.94 when every finish asked ahead for 64 slices
     whatever the row, drew its random number before its slice and went back to memory for tokens it had been sent."""
     torch = torch_cuda
     import rapid_sampling_amd as sample
@@ -1988,8 +2006,12 @@ def test_one_launch_path_of_rows_of_few_slices(torch_cuda):
     pen = torch.rand((320, 8192), generator=gen, device="cuda")
     pen = torch.where(pen < 0.02, 50.0 * pen, torch.zeros_like(pen))
     st = sample.setup_rand(1, 320)
+    calls = (("fused", 50, 0.95), ("cluster", -1, 0.9))
+    for (path, k, p) in calls:
+        rounds = _rounds_by(sample, path, lg, st, k, p, penalties=pen.clone())
+        assert ((rounds == 0) if path == "fused" else (rounds >= 1) & (rounds < 7)).all(), (path, np.unique(rounds))
     a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_repetition_temperature_topk_topp(
-        lg, pen, st, 0.1, 0.1, 0.95, 1.0, k, p)) for k, p in ((50, 0.95), (-1, 0.9)))
+        lg, pen, st, 0.1, 0.1, 0.95, 1.0, k, p), path) for path, k, p in calls)
     print("one launch %.1f us, general kernel %.1f us: %.2f" % (a, b, a / b), flush=True)
     assert a < 0.93 * b, (a, b)
 
