@@ -231,14 +231,11 @@ __device__ __forceinline__ uint32_t dpp0_u32(uint32_t v)
 template <int CTRL, int ROW_MASK, typename T>
 __device__ __forceinline__ T dpp0(T v)
 {
-    static_assert(sizeof(T) == 4 || sizeof(T) == 8 || sizeof(T) == 16, "32-, 64- or 128-bit integers");
+    static_assert(sizeof(T) == 4 || sizeof(T) == 8, "32- or 64-bit integers (128-bit sums have scans of their own below)");
     if constexpr (sizeof(T) == 4) return (T)dpp0_u32<CTRL, ROW_MASK>((uint32_t)v);
-    else if constexpr (sizeof(T) == 8) {
+    else {
         const uint32_t lo = dpp0_u32<CTRL, ROW_MASK>((uint32_t)v), hi = dpp0_u32<CTRL, ROW_MASK>((uint32_t)((uint64_t)v >> 32));
         return (T)(((uint64_t)hi << 32) | lo);
-    } else {
-        const uint64_t lo = dpp0<CTRL, ROW_MASK>((uint64_t)v), hi = dpp0<CTRL, ROW_MASK>((uint64_t)((u128)v >> 64));
-        return (T)(((u128)hi << 64) | lo);
     }
 }
 

@@ -5,13 +5,14 @@
 
 namespace rs {
 
-// Mass of a packed bin whose tokens share the exponent ex (87 <= ex <= 127): 44 bits shifted by up to 40.
-__device__ __forceinline__ M96 pack_m96(uint64_t w, uint32_t ex)
+// The mass of a sum of weights in units of the exponent ex (87 <= ex <= 127): 44 bits shifted by up to 40.
+__device__ __forceinline__ M96 mass_of(uint64_t sum, uint32_t ex)
 {
-    const uint64_t sum = (w & kPackMask) + ((w >> 43) << 23);
     const uint32_t sh = ex - 87u;
     return M96{sum << sh, (uint32_t)((sum >> 24) >> (40u - sh))};
 }
+// The same of a packed bin whose tokens share the exponent ex.
+__device__ __forceinline__ M96 pack_m96(uint64_t w, uint32_t ex) { return mass_of((w & kPackMask) + ((w >> 43) << 23), ex); }
 
 // ceil(f * s) for a uniform s < 2^96 and a float 0 < f <= 1 (see ceil_mul), the usual 2^-7 <= f < 1 by one 32-bit multiplication
 // per word.
@@ -94,12 +95,6 @@ __device__ __forceinline__ uint64_t need_of(M96 P, M96 above, uint32_t ex)
     const uint32_t sh = ex - 87u;
     const M96 left = (P - above) + M96{(1ull << sh) - 1ull, 0u};
     return (uint64_t)left.hi >> sh ? ~0ull : (left.lo >> sh) | (((uint64_t)left.hi << 1) << (63u - sh));
-}
-// A sum in those units as a mass.
-__device__ __forceinline__ M96 mass_of(uint64_t sum, uint32_t ex)
-{
-    const uint32_t sh = ex - 87u;
-    return M96{sum << sh, (uint32_t)((sum >> 24) >> (40u - sh))};
 }
 // Where a scan in order of falling e stopped: the first place at which there are top_k tokens or the mass P, what lies before
 // it and what is there (wave-uniform).
@@ -186,9 +181,8 @@ __device__ __forceinline__ bool fine_search(const int lane, F word, const Edge &
 // Scan the level-1 histogram s.g (the first wave; the others wait) for the first bin, largest e first, at which
 // (count so far >= top_k) or (mass so far >= P).  The total mass of the histogram is the row total D, and P = ceil(top_p * D)
 // is derived from it here.  With LOCAL this workgroup's own histogram s.hm is scanned along and its mass above the
-// boundary bin returned in local_above.  With GIVEN_P the histogram is that of a subset of the row which is complete above some
-// value: P stands as it is, D is left alone, and the scan may end without the set becoming sufficient (bin 0 then).
-template <bool LOCAL, bool GIVEN_P = false, typename L = Lds>
+// boundary bin returned in local_above.
+template <bool LOCAL, typename L = Lds>
 __device__ __forceinline__ Found hist_find_level1(L &s, uint64_t top_k, float top_p, int lane, int wave)
 {
     if (wave == 0) {
@@ -201,13 +195,8 @@ __device__ __forceinline__ Found hist_find_level1(L &s, uint64_t top_k, float to
         OctScan sc, own;
         sc.load(lane, bins(s.g));
         if constexpr (LOCAL) own.load(lane, bins(s.hm));
-        M96 P;
-        if constexpr (GIVEN_P) P = m96((u128)s.P);
-        else {
-            const M96 D = sc.total();
-            P = ceil_mul(top_p, D);
-            if (lane == 0) { s.D = wide(D); s.P = wide(P); }
-        }
+        const M96 D = sc.total(), P = ceil_mul(top_p, D);
+        if (lane == 0) { s.D = wide(D); s.P = wide(P); }
         Edge e{0u, 0u, 0u, 0ull, M96{0ull, 0u}, 0ull};
         const bool found = sc.search((uint32_t)min(top_k, (uint64_t)0xFFFFFFFFull), P, e);
         M96 mine{0ull, 0u};

@@ -200,7 +200,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     }
     __syncthreads();
     const uint64_t top_k = (uint64_t)p.top_k;
-    Found f = hist_find_level1<false, false, LdsRowS>(s, top_k, p.top_p, lane, wave);
+    Found f = hist_find_level1<false, LdsRowS>(s, top_k, p.top_p, lane, wave);
     // (what is the same for all threads stays in scalar registers, or in LDS until it is used)
     f.bin = uniform(f.bin); f.cnt_above = uniform(f.cnt_above); f.cnt_bin = uniform(f.cnt_bin);
     auto target = [&](uint32_t thr, uint32_t n_gt, uint32_t n_eq, u128 above, uint32_t rounds) {

@@ -138,7 +138,7 @@ __global__ void __launch_bounds__(kThreads) wide_plan_kernel(const Params p, con
     }
     __syncthreads();
     level1_to_row_frame(s, v, row, M, mixed, h0, h1, s.delta, s.m4);
-    const Found f = hist_find_level1<false, false, LdsP>(s, (uint64_t)p.top_k, p.top_p, lane, wave);
+    const Found f = hist_find_level1<false, LdsP>(s, (uint64_t)p.top_k, p.top_p, lane, wave);
     if (tid == 0) {
         WidePlan *pl = reinterpret_cast<WidePlan *>(rc->A);
         pl->kmax = kmax; pl->b1 = f.bin; pl->cnt_above = f.cnt_above; pl->cnt_bin = f.cnt_bin;

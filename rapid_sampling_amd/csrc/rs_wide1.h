@@ -153,7 +153,7 @@ __global__ void __launch_bounds__(kW1SampleT) wide_sample_kernel(const Params p,
     __syncthreads();
     // the sample's share of top_k
     const uint64_t k_s = p.top_k >= p.V ? (uint64_t)n_s : ((uint64_t)p.top_k * n_s + (uint64_t)p.V - 1u) / (uint64_t)p.V;
-    const Found f = hist_find_level1<false, false, LdsS>(s, max(k_s, (uint64_t)1), p.top_p, lane, wave);
+    const Found f = hist_find_level1<false, LdsS>(s, max(k_s, (uint64_t)1), p.top_p, lane, wave);
     // A sample that is one tie (rows of equal logits) says nothing about a threshold, and a range around it
     // would queue every token of the row up at one sub-bin: no guess.  (A row that is one tie of all its
     // tokens is recognised by the finishing workgroup from the row's bins alone.)
