@@ -27,8 +27,13 @@
 //     add up, words that are non-zero once written), every wait is bounded.
 //     Any top_k / top_p, penalties, any batch.
 //
+//   short-row kernel (short_kernel, one launch, no workspace, no waits): one workgroup
+//     per row of up to 16384 tokens, the row in its registers; any kept set, with or
+//     without penalties.  All rows of fewer than 8192 tokens, all calls with penalties in
+//     longer ones, and without them the calls that short_suits says.
+//
 //   streaming path (stream_kernel + finish_kernel, two launches, no waits): for
-//     calls of 2^17 tokens and more without penalties whose kept set is small
+//     calls without penalties that the short-row kernel leaves and whose kept set is small
 //     next to the row (top_k <= 1024, or a small nucleus), and, as a counting-only
 //     variant, for calls that keep every token.  One pass over the logits leaves
 //     per-row histograms and per-slice stashes of the largest tokens; one
@@ -551,10 +556,7 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
     if (force == RS_PATH_WIDE) return keep_all ? kPathKeep : kPathWide;
     if (force == RS_PATH_WIDE1) return keep_all ? kPathKeep : kPathWide1;
     if (force == RS_PATH_ROW) return V <= kRowMaxV ? kPathRow : kPathCluster;
-    // Small calls: rows of fewer than 8192 tokens are one or two workgroups of the general kernel each, with
-    // few or no exchanges (8.5 us for a row of 256 tokens); from 8192 tokens per row on the streaming
-    // path's two launches are faster whatever the batch (one row of 8192 to 100256 tokens: 13.6-14.7
-    // against 16.1-17.9 us, 16 rows: 14.5-15.8 against 16.8-21.3; measured per call between events).
+    // (small calls with a forced slice length: the short-row kernel has taken all the others)
     if ((uint64_t)B * (uint64_t)V < (1ull << 17) && V < 8192) return kPathCluster;
     if (keep_all && V >= 32768) return kPathKeep;              // shorter rows: one workgroup of the general kernel does a row in one go
     // kept sets the stashes cannot hold: the wide path from kWideMin tokens on, unless its rows have been
@@ -605,7 +607,7 @@ using namespace rs;
 
 extern "C" {
 
-int rs_version(void) { return 417; }
+int rs_version(void) { return 418; }
 
 const char *rs_error_string(int code)
 {

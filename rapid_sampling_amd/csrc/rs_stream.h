@@ -1732,8 +1732,7 @@ __global__ void __launch_bounds__(kThreads) penalty_fix_kernel(const Params p, c
 // ------------------------------------------------------------ one-launch path --
 // The streaming pass and the finish in ONE launch, for calls small enough that a second and a third
 // launch (and the cold start of the finishing workgroup) cost as much as the work itself, and for
-// calls with penalties, whose every workgroup needs the sampled token to rewrite its penalties from
-// the registers.  A row is worked by G workgroups (logical ids follow the order in which workgroups
+// calls with penalties, whose every workgroup holds its penalties in registers and rewrites them from there.  A row is worked by G workgroups (logical ids follow the order in which workgroups
 // start once the launch is larger than the GPU holds at once).  Each reads its slice once, publishes
 // the slice's record exactly as the streaming pass does -- with device-scope atomic stores -- and
 // counts itself in (release).  The workgroup that arrives last finishes the row from the records
@@ -1741,8 +1740,9 @@ __global__ void __launch_bounds__(kThreads) penalty_fix_kernel(const Params p, c
 // the verdict -- that is the only wait, and it is for a workgroup that is already running.  On "fall
 // back" (a nucleus or a tie too large for the stashes) all G workgroups go on with the cluster path's
 // rounds from the tokens they still hold in registers: the row's level-1 histogram is already
-// complete in memory, so they start at the boundary search.  With penalties every workgroup then
-// rewrites its slice of them.  The last workgroup to leave cleans the row's record.
+// complete in memory, so they start at the boundary search.  With penalties the workgroups that wait write
+// theirs, decayed, while they do, the last one once it has posted the verdict; the sampled token's is written again when
+// it is known.  The last workgroup to leave cleans the row's record.
 template <int R, bool PEN>
 struct FusedLds {
     union {
