@@ -74,8 +74,8 @@ template <bool FUSED, typename T> __device__ __forceinline__ T get(const T *p)
 // in eb), the packed histogram added to the row's and kept under the slice's own name, cumulative
 // counts, and the stash of its largest tokens with the value down to which it is complete.
 // Returns the key of the slice's maximum.
-// KEEP: a call that keeps every live token (top_k = V, top_p = 1); kCap: room of the stash; PAD: much of the last slices lies past the
-// end of their rows.
+// KEEP: a call that keeps every live token (top_k = V, top_p = 1); kCap: room of the stash; PAD: slots past the end of the row
+// are looked for (the host's rule, rs_stream.hip).
 template <int R, int NT, int kRep, bool FUSED, bool KEEP = false, int kCap = kStashCap, bool PAD = false>
 __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const StreamView &v, LdsA<kRep> &s, uint32_t (&eb)[R * 4],
                                                           const float lmax, const uint32_t row, const uint32_t part,
@@ -103,16 +103,18 @@ __device__ __forceinline__ uint32_t slice_count_and_stash(const Params &p, const
     // keeps the groups' instructions apart: 256 x 151936 bfloat16 32.6 us a call against 31.2, 64 x 152064 bfloat16, in slices of 8192
     // tokens, 18.9 against 18.3.)  In slices of 8192 tokens four groups at a time: all eight at once take 82 registers instead of 74, with
     // which five workgroups share a compute unit and not six, and calls of 1281 to 1536 of them need another round (512 x 20480 with
-    // top_k 1000 43.1 us a call against 39.9).  Slices of 16384 tokens are not tested at all unless a quarter of the call's slots lie past the end of
-    // their rows (PAD, the host's rule, rs_stream.hip): the tests cost such a call 1 % (512 x 50304, 23 % of the slots, 34.9 us a call without,
+    // top_k 1000 43.1 us a call against 39.9).  Slices of 4096 tokens are tested, two groups at a time, in calls of more workgroups than compute
+    // units (PAD): 300 x 16388 15.1 us a call against 16.1, 100 x 50304 14.4 against 14.9; a call whose workgroups have a compute unit each waits for
+    // one chain, which the tests make longer (1 x 262144 10.43 with none, 10.51).  Slices of 16384 tokens are not tested at all unless a
+    // quarter of the call's slots lie past the end of their rows (PAD, too): the tests cost such a call 1 % (512 x 50304, 23 % of the slots, 34.9 us a call without,
     // 35.2 with), the slots 2 to 8 % (1024 x 8196 25.1 and 23.2, 512 x 32772 with top_k 1000 51.7 and 50.5).
     // Calls that keep every token, which have no stash to select, hide the test per lane behind their loads and lose more by the registers
     // of groups that are worked out together: 512 x 50304 bfloat16, in slices of 8192, 27.2 us a call against 28.6 with one test of all eight,
     // in shorter slices nothing tested 10.4 against 10.5 (32 x 65536 bfloat16).
     const Frame fr = frame_of(M, eb);
     constexpr bool kLane = KEEP && R == 8;
-    constexpr int kChunk = kLane ? 1 : PAD || (R == 4 && !FUSED && !KEEP) ? 2 : R == 8 && !FUSED ? 4 : R;
-    constexpr bool kSkip = PAD || (R <= 8 && !FUSED && !KEEP);   // (the one-launch kernel: 0.6 % slower with them over 92 shapes)
+    constexpr int kChunk = kLane ? 1 : PAD ? 2 : R == 8 && !FUSED ? 4 : R;
+    constexpr bool kSkip = PAD || (R == 8 && !FUSED && !KEEP);   // (the one-launch kernel: 0.6 % slower with them over 92 shapes)
     const uint32_t first = uniform(base4), left = ((uint32_t)p.V >> 2) - min(first, (uint32_t)p.V >> 2);      // groups of the row from the wave's first one on
     const float dead = (__builtin_fabsf(M) <= 100.0f ? M : 0.0f) - 48.0f - (float)(lane & 31);
 #pragma unroll

@@ -36,7 +36,11 @@ hipError_t launch_stream(int slice_r, int32_t dtype, bool keep, uint32_t B, size
         else hipLaunchKernelGGL((stream_kernel<Rv, NTv, RS_DTYPE_F16, KEEPv, PADv>), sgrid, dim3(NTv), 0, st, p, v);                             \
         if (KEEPv) hipLaunchKernelGGL((keep_finish_kernel<Lv>), dim3(B), dim3(kKeepT + kWave), 0, st, p, v);                              \
         else launch_finish(B, finish_lds_bytes, st, p, v); } while (0)
-    if (slice_r == 4) { if (keep) RS_STREAM(4, 256, 12, true, false); else RS_STREAM(4, 256, 12, false, false); }
+    if (slice_r == 4) {
+        if (keep) RS_STREAM(4, 256, 12, true, false);
+        else if (B * v.G > 256u) RS_STREAM(4, 256, 12, false, true);     // (more workgroups than compute units: see slice_count_and_stash)
+        else RS_STREAM(4, 256, 12, false, false);
+    }
     else if (slice_r == 8) { if (keep) RS_STREAM(8, 256, 13, true, false); else RS_STREAM(8, 256, 13, false, false); }
     else if (keep) RS_STREAM((kStreamLongR * 256 / RS_LONG_NT), RS_LONG_NT, kStreamLongLog2, true, false);
     else {

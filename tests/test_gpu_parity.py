@@ -2170,11 +2170,12 @@ def test_one_pass_wide_path_with_samples_that_end_within_a_round_of_waves(torch_
 
 
 @pytest.mark.parametrize("fmt", ["float32", "bfloat16"])
-@pytest.mark.parametrize("B,V", [(9, 4), (9, 2052), (9, 4100), (9, 6140), (520, 8196), (392, 12292), (776, 8196), (776, 10236), (776, 12288), (776, 12292),
+@pytest.mark.parametrize("B,V", [(9, 4), (9, 2052), (9, 4100), (9, 6140), (128, 6140), (129, 6140), (300, 4100), (300, 8188),
+                                 (520, 8196), (520, 10236), (520, 12288), (392, 12292), (392, 16380), (776, 8196), (776, 10236), (776, 12288), (776, 12292),
                                  (776, 16380), (520, 16388), (520, 18436)])
 def test_streaming_pass_rows_that_end_within_a_slice(torch_cuda, oracle, B, V, fmt):
-    """Last slices that end inside a wave's group of tokens, a wave's two groups, or a few tokens in, in slices of 4096, 8192 and 16384
-    tokens, these on both sides of a quarter of slots past the end of the row (8196, 12288 | 12292 tokens): eight kinds of rows --
+    """Last slices that end inside a wave's group of tokens, a wave's two or four groups, or a few tokens in, in slices of 4096 (256
+    and 258 workgroups, not tested for the end of the row and tested), 8192 and 16384 tokens, these on both sides of a quarter of slots past the end of the row (8196, 12288 | 12292 tokens): eight kinds of rows --
     far from zero, masked but for the last token, one tie, all of them in the last slots -- over and over, e of every token and
     every field against the oracle."""
     torch = torch_cuda
