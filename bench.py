@@ -44,7 +44,7 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E, vendor figure
 # HBM bytes per call of the bandwidth configuration from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs
 # summarised in the file named here, valid for the library version they were taken with: a library
 # that has moved on reports traffic as null rather than a stale figure.
-TRAFFIC_PROFILE = {"file": "profiles/bench_kernels_hbm_traffic_pmc.md", "rs_version": 416, "bytes": 576170803}
+TRAFFIC_PROFILE = {"file": "profiles/bench_kernels_hbm_traffic_pmc.md", "rs_version": 418, "bytes": 575099802}
 
 
 def event_times_us(torch, fn, steps, warmup):
@@ -152,7 +152,7 @@ def main():
                          "kernel that rocprofv3 FETCH_SIZE / WRITE_SIZE readings are scaled by")
     args = ap.parse_args()
     if args.gpus != 1:
-        print("bench.py: this build runs on one GPU only (rows shard over GPUs without communication; "
+        print("bench.py: this library runs on one GPU only (rows shard over GPUs without communication; "
               "no multi-GPU path is part of it). Run with --gpus 1.", file=sys.stderr)
         sys.exit(2)
 

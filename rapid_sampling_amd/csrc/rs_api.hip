@@ -314,7 +314,8 @@ static int wide_r(int32_t B, int32_t V, size_t workspace_bytes)
 // 262144 when the workspace has room for them (a workspace of rs_workspace_bytes has) and each stash leaves room for the slice's
 // notes behind it, else 16384, whose notes have room of their own.  A thread holds its
 // tokens and their penalties, so slices half as long let twice the workgroups share a compute unit and load in each other's scans:
-// 128 x 262144 73.0 -> 63.9 us a call, 256 x 131072 73.1 -> 64.0, 128 x 100256 42.2 -> 35.0, 512 x 32768 48.0 -> 41.1.  Rows of a million tokens would be cut into more slices than
+// us a call, the same inputs again and again / new ones from HBM each time: 128 x 262144 71.6 -> 64.1 / 86.2 -> 84.6, 256 x 131072
+// 72.5 -> 63.8 / 86.7 -> 84.2, 128 x 100256 41.2 -> 35.1 / 48.5 -> 42.7, 512 x 32768 47.9 -> 40.9 / 54.6 -> 50.3.  Rows of a million tokens would be cut into more slices than
 // their finish handles quickly (16 x 1048576: 55 us a call with slices of 16384, 67 with 8192).
 static uint32_t stash_aim(uint32_t top_k, uint32_t G) { return min(top_k, max(32u, 8u * top_k / G)); }    // eight times a slice's share of the row's top_k
 static int pen_r(int32_t B, int32_t V, int32_t top_k, size_t workspace_bytes)

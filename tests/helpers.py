@@ -1,6 +1,6 @@
 """Shared input builders for the tests: the five BASELINE configurations at
 reduced or full size, always from fixed numpy seeds (no torch RNG, so CPU and
-GPU boxes build identical tensors)."""
+GPU machines build identical tensors)."""
 import numpy as np
 
 

@@ -42,7 +42,7 @@ def test_no_kernel_keeps_registers_in_memory():
 def test_the_streaming_finish_keeps_its_scalars(kernel, most):
     """The way almost no row takes (finish_row_slow) shares the finishing kernels with the usual one, a chain of
     dependent steps.  With 36 spilled scalars in the place of 22, brought about by a change to the slow way alone, calls of
-    64 rows of 152064 were 1 to 2 % slower.  Bounds: the counts of this build (0, 5, 7 and 33) with some room."""
+    64 rows of 152064 were 1 to 2 % slower.  Bounds: the counts when this was written (0, 5, 7 and 33) with some room."""
     k = _kernels()["rs::" + kernel]
     assert k[".sgpr_spill_count"] <= most, k[".sgpr_spill_count"]
 
