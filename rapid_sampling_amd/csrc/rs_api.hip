@@ -454,27 +454,24 @@ static bool row_suits(int32_t B, int32_t V)
 //   1024 x 16384     28.5 / 31.5 / 64.3 / 68.9    29.2 / 46.7 / 47.0 / 62.6
 // So it takes every call with penalties and every call in rows below 8192 tokens; in longer ones, the kept sets of thousands
 // stay with the row kernel where that takes them, and calls of more than 512 rows where they were.  A bounding top_k does not
-// bound the list to the 64 tokens that are resolved by pairs: with more, a call that has more rows than there are compute units
-// is faster on the streaming path (streaming / here, N(0,1.5), us a call):
-//   rows x tokens     top_k 10       40 (0)        64      64 (1)       100       300
-//    257 x  8196   11.9 / 11.4   13.0 / 12.3   14.0 / 14.7   15.8 / 18.3   15.8 / 18.3   17.3 / 18.2
-//    512 x  8196   14.1 / 13.7   15.4 / 15.5   16.8 / 19.9   18.4 / 25.0   19.0 / 23.4   20.7 / 23.5
-//    512 x 12288   16.1 / 14.5   17.2 / 15.7   18.8 / 20.3   19.1 / 26.1   20.0 / 24.2   23.1 / 24.5
-//    257 x 16384   13.7 / 13.9   14.8 / 15.3   15.8 / 17.7   17.1 / 19.1   16.8 / 22.0   19.4 / 21.7
-//    512 x 16384   16.0 / 16.4   17.2 / 17.5   18.9 / 21.9   19.9 / 27.3   21.0 / 25.9   23.5 / 26.4
-// ((0): peaked rows the same or better, 512 x 12288 16.8 / 15.1, flat ones 23.9 / 19.4; (1): bfloat16, whose ties go past 64), so
-// such calls come here with a top_k of up to kShortListK only, which leaves ties some room (over 20 such shapes at 48 and 50: float32 0.86 to
-// 1.05 of the streaming path's time, peaked float16 0.82 to 0.96; flat rows of bfloat16, with ties of hundreds, 0.91 to 1.19).  With up to 256 rows the host cannot
-// tell: peaked rows are a quarter faster here whatever top_k is (128 x 16384, top_k 40 11.4 / 9.0), rows whose list is long are faster from a
-// top_k of some 200 on (128 x 16384, top_k 300 16.4 / 13.6) and up to a tenth slower between 64 and there (64 x 16384, top_k 100 12.3 / 13.1, 64
-// in bfloat16 13.3 / 14.8): they come here.  The same with penalties and more than 1280 rows of 8196 to 10240 tokens, where the long lists of
-// float32 logits are 2 to 8 % slower than on the general kernel and peaked rows 20 to 30 % faster (2048 x 8196: 96 / 102, 90 / 70).
+// bound the list to the 64 tokens that are resolved by pairs.  Calls of 257 to 512 rows, streaming path / here, N(0,1.5), us a call:
+//   rows x tokens     top_k 48 (0)      65         100         300        1000       300 (0)   peaked 40  flat 50 (0)
+//    257 x  8196   14.5 / 11.0  14.5 / 14.1  15.8 / 13.6  17.3 / 13.8  29.7 / 15.2  18.7 / 16.8  12.4 /  9.3  19.0 / 16.1
+//    512 x  8196   17.0 / 11.9  17.4 / 16.1  18.9 / 16.0  20.8 / 16.4  35.1 / 16.8  21.4 / 17.5  14.8 / 10.0  22.2 / 17.5
+//    257 x 12288   14.7 / 10.6  14.9 / 14.9  15.4 / 15.7  17.9 / 15.2  30.3 / 16.1  19.2 / 17.5  13.0 / 10.1  19.8 / 16.6
+//    512 x 12288   18.1 / 12.5  19.3 / 17.4  20.0 / 17.8  23.2 / 17.9  37.8 / 18.1  22.8 / 18.7  16.9 / 11.3  23.8 / 18.8
+//    257 x 16384   15.7 / 12.1  16.2 / 18.3  16.7 / 19.4  19.4 / 18.6  32.7 / 19.9  20.3 / 20.1  14.1 / 11.7  21.5 / 20.2
+//    512 x 16384   18.7 / 14.2  19.4 / 20.8  21.1 / 21.3  23.5 / 21.4  37.7 / 21.9  23.9 / 21.7  17.1 / 13.5  24.7 / 21.9
+// ((0): bfloat16.)  Rows of more than 12288 tokens come here with a top_k of up to kShortListK only, which leaves ties some room.  With
+// up to 256 rows the host cannot tell long lists from short ones: peaked rows are a quarter faster here whatever top_k is (64 x 16384, top_k 40 10.0 /
+// 7.8), rows whose list is long are faster from a top_k of some 200 on (300: 15.3 / 13.3) and 5 to 8 % slower between 64 and there in up to 128
+// rows of more than 12288 tokens (64 x 16384, top_k 65 12.0 / 13.0; 256 x 16384 15.7 / 14.6): they come here.
 constexpr int32_t kShortListK = 50;
 static bool short_suits(int32_t B, int32_t V, int32_t top_k, bool pen)
 {
     if (V > kShortMaxV) return false;
     if (pen || V < 8192) return true;
-    if (top_k <= kStreamK) return B <= 256 || V == 8192 || (B <= 512 && top_k <= kShortListK);
+    if (top_k <= kStreamK) return B <= 256 || V == 8192 || (B <= 512 && (V <= 12288 || top_k <= kShortListK));
     return B <= 256 && (V == 8192 || !row_suits(B, V));
 }
 // Plain temperature sampling (top_k = V, top_p = 1: every live token is kept) has no kept set to

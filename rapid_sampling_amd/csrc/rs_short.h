@@ -38,8 +38,12 @@ struct LdsShort {
 // (j < R): index order is wave, then j, then lane, then token.  Up to two waves per SIMD work the one-wave steps out each
 // for itself and leave the random number to a wave of its own; of sixteen the first does them for all and the last draws.
 template <int W> constexpr int short_threads() { return (W <= 8 ? W + 1 : W) * kWave; }
+// Waves a SIMD must hold: two workgroups of sixteen waves share a compute unit in 64 registers.  The four groups of a thread took 66
+// when left alone, one workgroup a compute unit: 512 rows of 16384, top_k 40 16.9 us a call, in 64 13.5; 384 with a top_k of 300 25.2
+// and 20.6 (with penalties 88 are needed, which no bound brings down to 64).
+template <bool PEN, int W, int R> constexpr int short_waves() { return W == 16 && !PEN ? 8 : 1; }
 template <int DT, bool PEN, int W, int R>
-__global__ void __launch_bounds__(short_threads<W>()) short_kernel(const Params p)
+__global__ void __launch_bounds__(short_threads<W>(), (short_waves<PEN, W, R>())) short_kernel(const Params p)
 {
     constexpr bool kEach = W <= 8;
     constexpr uint32_t kCopies = LdsShort<W, R>::kCopies, kPlane = LdsShort<W, R>::kPlane;

@@ -463,13 +463,14 @@ def test_row_kernel_unusual_rows(torch_cuda, oracle):
 
 
 @pytest.mark.parametrize("B,V,k,one", [
-    (256, 8196, 1024, True), (257, 8192, 1024, True), (513, 8192, 300, True), (600, 8188, 1000, True), (257, 8196, 50, True),
-    (257, 8196, 51, False), (257, 16384, 300, False), (512, 12288, 50, True), (512, 16384, 65, False), (513, 12288, 50, False),
-    (64, 16384, 1000, True), (64, 16388, 1000, False)])
+    (256, 8196, 1024, True), (257, 8192, 1024, True), (513, 8192, 300, True), (600, 8188, 1000, True), (257, 8196, 51, True),
+    (512, 12288, 1024, True), (513, 12288, 50, False), (257, 12292, 50, True), (257, 12292, 51, False), (512, 16384, 50, True),
+    (512, 16384, 65, False), (256, 16384, 300, True), (64, 16388, 1000, False)])
 def test_rows_of_up_to_16384_tokens_with_a_bounding_top_k_take_the_kernel_that_suits_them(torch_cuda, B, V, k, one):
     """Which calls with a bounding top_k one workgroup per row does by itself (diag.rounds == 10) and which the streaming
-    path (0): rows of up to 8192 tokens all of them, longer ones up to 256 rows, or 512 with a top_k of up to 50.  Calls of 257 to
-    512 rows of 8196 to 16384 tokens with more were 5 to 40 % slower in one workgroup per row."""
+    path (0): rows of up to 8192 tokens all of them, longer ones up to 256 rows, or 512 of up to 12288 tokens, or of more with a top_k of up
+    to 50.  Calls of 257 to 512 rows with longer lists were 5 to 40 % slower in one workgroup per row while two workgroups did
+    not share a compute unit, and are up to 16 % slower in rows of more than 12288 tokens."""
     from tests import capi
     lg = torch_cuda.from_numpy(H.logits_normal(B, V, 1.5, seed=B)).cuda()
     rc, c, kk, pp = capi.normalize(1.0, k, 0.95, V, B, 1)
@@ -2017,9 +2018,9 @@ def test_one_launch_path_of_rows_of_few_slices(torch_cuda):
 
 
 @pytest.mark.parametrize("pen_on", [False, True])
-@pytest.mark.parametrize("V", [4, 12, 252, 256, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8188, 8192, 8196, 16384])
+@pytest.mark.parametrize("V", [4, 12, 252, 256, 1020, 1024, 1028, 2048, 2052, 4096, 4100, 8188, 8192, 8196, 12284, 12288, 12292, 16384])
 def test_short_row_kernel(torch_cuda, oracle, V, pen_on):
-    """Rows of up to 16384 tokens, at the edges of the kernel's variants (4, 8 and 16 waves with 1, 2 and 4 groups of four per
+    """Rows of up to 16384 tokens, at the edges of the kernel's variants (4, 8 and 16 waves with 1 to 4 groups of four per
     thread; waves without a token in the shortest rows): lists of 1, 16, 17, 64 and 65 tokens, kept sets of thousands, ties (of all tokens,
     of the largest, of a few values), masked and sorted rows, frames far from zero, NaNs; penalties that are -0.0, infinite,
     dense, and a decay that is not finite.  Every field against the oracle, and with the generator's own draws against
