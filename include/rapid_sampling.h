@@ -248,7 +248,8 @@ int rs_philox_init(void *state_device, uint64_t seed, int32_t B, void *stream);
  * The call is one kernel launch (the short-row kernel, one workgroup per row:
  * rows of fewer than 8192 tokens, with penalties of up to 16384, and most
  * calls of up to 256 rows of that length without, of up to 512 of up to 12288
- * tokens with top_k <= 1024, of the longer ones with top_k <= 50; the general kernel:
+ * tokens with top_k <= 1024, of the longer ones with top_k <= 50 or from 200
+ * to 1024; the general kernel:
  * whatever the other paths do not take; with penalties and top_k <= 1024 the one-launch streaming kernel while
  * the call fits the GPU at once), two for calls without penalties whose kept
  * set is expected to be small (a wait-free pass over the logits and a per-row

@@ -462,16 +462,19 @@ static bool row_suits(int32_t B, int32_t V)
 //    512 x 12288   18.1 / 12.5  19.3 / 17.4  20.0 / 17.8  23.2 / 17.9  37.8 / 18.1  22.8 / 18.7  16.9 / 11.3  23.8 / 18.8
 //    257 x 16384   15.7 / 12.1  16.2 / 18.3  16.7 / 19.4  19.4 / 18.6  32.7 / 19.9  20.3 / 20.1  14.1 / 11.7  21.5 / 20.2
 //    512 x 16384   18.7 / 14.2  19.4 / 20.8  21.1 / 21.3  23.5 / 21.4  37.7 / 21.9  23.9 / 21.7  17.1 / 13.5  24.7 / 21.9
-// ((0): bfloat16.)  Rows of more than 12288 tokens come here with a top_k of up to kShortListK only, which leaves ties some room.  With
+// ((0): bfloat16.)  Rows of more than 12288 tokens come here with a top_k of up to kShortListK, which leaves ties some room, and from
+// kShortLongK on: in 36 sets of such calls (257 to 512 rows of 12292, 14336 and 16384 tokens, three kinds of rows) the kernel takes 0.78 to 1.16 of the
+// streaming path's time with a top_k of 64, 0.88 to 1.16 with 100, 0.79 to 1.13 with 160, 0.76 to 1.01 with 200, 0.75 to 0.99 with 300, 0.55 to 0.71
+// with 1024.  With
 // up to 256 rows the host cannot tell long lists from short ones: peaked rows are a quarter faster here whatever top_k is (64 x 16384, top_k 40 10.0 /
 // 7.8), rows whose list is long are faster from a top_k of some 200 on (300: 15.3 / 13.3) and 5 to 8 % slower between 64 and there in up to 128
 // rows of more than 12288 tokens (64 x 16384, top_k 65 12.0 / 13.0; 256 x 16384 15.7 / 14.6): they come here.
-constexpr int32_t kShortListK = 50;
+constexpr int32_t kShortListK = 50, kShortLongK = 200;
 static bool short_suits(int32_t B, int32_t V, int32_t top_k, bool pen)
 {
     if (V > kShortMaxV) return false;
     if (pen || V < 8192) return true;
-    if (top_k <= kStreamK) return B <= 256 || V == 8192 || (B <= 512 && (V <= 12288 || top_k <= kShortListK));
+    if (top_k <= kStreamK) return B <= 256 || V == 8192 || (B <= 512 && (V <= 12288 || top_k <= kShortListK || top_k >= kShortLongK));
     return B <= 256 && (V == 8192 || !row_suits(B, V));
 }
 // Plain temperature sampling (top_k = V, top_p = 1: every live token is kept) has no kept set to

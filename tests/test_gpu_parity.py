@@ -465,11 +465,11 @@ def test_row_kernel_unusual_rows(torch_cuda, oracle):
 @pytest.mark.parametrize("B,V,k,one", [
     (256, 8196, 1024, True), (257, 8192, 1024, True), (513, 8192, 300, True), (600, 8188, 1000, True), (257, 8196, 51, True),
     (512, 12288, 1024, True), (513, 12288, 50, False), (257, 12292, 50, True), (257, 12292, 51, False), (512, 16384, 50, True),
-    (512, 16384, 65, False), (256, 16384, 300, True), (64, 16388, 1000, False)])
+    (512, 16384, 199, False), (512, 16384, 200, True), (257, 16384, 1024, True), (256, 16384, 100, True), (64, 16388, 1000, False)])
 def test_rows_of_up_to_16384_tokens_with_a_bounding_top_k_take_the_kernel_that_suits_them(torch_cuda, B, V, k, one):
     """Which calls with a bounding top_k one workgroup per row does by itself (diag.rounds == 10) and which the streaming
     path (0): rows of up to 8192 tokens all of them, longer ones up to 256 rows, or 512 of up to 12288 tokens, or of more with a top_k of up
-    to 50.  Calls of 257 to 512 rows with longer lists were 5 to 40 % slower in one workgroup per row while two workgroups did
+    to 50 or from 200 on.  Calls of 257 to 512 rows with longer lists were 5 to 40 % slower in one workgroup per row while two workgroups did
     not share a compute unit, and are up to 16 % slower in rows of more than 12288 tokens."""
     from tests import capi
     lg = torch_cuda.from_numpy(H.logits_normal(B, V, 1.5, seed=B)).cuda()
