@@ -1905,6 +1905,7 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
     auto decayed = [&]() { rewrite([&](float q) { return __builtin_fmaf(q, p.decay, 0.0f); }); };
     auto put_back = [&]() { rewrite([](float q) { return q; }); };
     uint32_t verdict = 0;
+    bool gave_up = false;
     if (last) {
         // the token list: the cluster rounds' histogram copies, which are not in use while a row is
         // finished from the stashes (no dynamic LDS in this kernel: see rs_sample_ex)
@@ -1931,12 +1932,12 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
             s.bc32[7] = w;
         }
         __syncthreads();
-        if (s.abort) { put_back(); return; }
-        verdict = s.bc32[7];
+        gave_up = s.abort != 0u;
+        verdict = gave_up ? kVerdictFallback : s.bc32[7];
     }
     if (verdict == kVerdictFallback) {
         // (ends with the cluster path's own leaving protocol; a wait that gives up there comes before its write of the penalties)
-        if (!fused_fallback<R, PEN>(p, v, s, sl, key)) put_back();
+        if (gave_up || !fused_fallback<R, PEN>(p, v, s, sl, key)) put_back();
         return;
     }
     const uint32_t idx = verdict - 1u;
