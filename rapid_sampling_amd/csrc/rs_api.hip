@@ -437,6 +437,33 @@ static bool row_suits(int32_t B, int32_t V)
     if (V <= 32768) return B >= 320;
     return B >= 512 || V >= 40000;                            // 257 to 511 rows: two rounds pay off in long rows only
 }
+// The row kernel with a bounding top_k of hundreds, whose lists the streaming path's finish goes through in one workgroup per row as well:
+// streaming path / row kernel, us a call, N(0,1.5), top_p 0.95:
+//   rows x tokens   top_k 65       128         200         300        1000       200 (0)    flat 200
+//    64 x 20000   12.6 / 13.6  12.8 / 13.7  14.2 / 13.7  15.7 / 13.8  19.4 / 14.4  14.9 / 15.0  16.9 / 14.1
+//   128 x 20000   13.5 / 13.7  13.7 / 13.9  16.0 / 13.7  16.9 / 13.9  20.7 / 14.5  17.1 / 15.0  18.2 / 14.1
+//   256 x 20000   15.8 / 14.1  15.9 / 14.1  18.4 / 14.1  19.0 / 14.1  24.1 / 14.8  19.1 / 15.2  21.1 / 14.8
+//    64 x 32768   12.8 / 14.6  12.9 / 14.4  13.8 / 14.5  14.4 / 14.5  19.2 / 14.9  15.4 / 15.8  19.2 / 15.6
+//   128 x 32768   14.7 / 15.1  14.7 / 14.9  15.7 / 15.0  17.1 / 15.2  22.1 / 15.4  17.2 / 15.8  20.5 / 15.8
+//   256 x 32768   17.4 / 15.5  17.4 / 15.2  20.9 / 15.4  21.4 / 15.8  25.3 / 16.1  21.7 / 16.3  25.2 / 16.3
+//   300 x 32768   19.1 / 21.7  20.2 / 21.5  23.5 / 21.8  23.2 / 21.6  36.6 / 23.2
+//   512 x 32768   24.2 / 23.6  25.1 / 23.5  28.8 / 23.5  30.1 / 23.8  43.6 / 24.9  28.3 / 22.9  33.0 / 24.9
+//  1024 x 16388   44.7 / 33.1  47.1 / 33.6  49.3 / 33.5  54.9 / 33.7  80.8 / 36.5
+//   128 x 50304   17.1 / 20.1  17.4 / 20.2  19.3 / 19.9  20.5 / 20.0  25.0 / 20.7  20.1 / 19.8  27.0 / 21.2
+//   256 x 50304   22.1 / 21.8  25.1 / 21.8  26.4 / 21.6  27.6 / 21.8  32.1 / 22.4  26.9 / 20.2  30.9 / 22.9
+//   512 x 50304   29.4 / 43.6  32.5 / 44.0  40.2 / 43.4  42.5 / 43.9  57.8 / 45.2  39.2 / 40.3  46.6 / 46.0
+//   128 x 65536   17.7 / 21.6  17.6 / 21.5  19.8 / 21.4  21.0 / 21.7  25.3 / 22.0
+//   256 x 65536   21.4 / 25.4  22.5 / 25.5  27.5 / 25.3  29.2 / 25.8  32.8 / 25.8
+//   300 x 65536   24.2 / 45.6  25.3 / 45.9  31.2 / 45.5  33.8 / 45.8  47.4 / 47.1
+// ((0): bfloat16.)  One round of 256 workgroups costs the same whatever top_k is, the streaming path's finish grows with both: the line for up
+// to 256 rows is their product.  Below 128 rows the gain is small and ends early in longer rows.  (Calls of more than 256 rows of more than 32768
+// tokens with a top_k near 1024 stay where they were, though they would gain up to a quarter: their finish tells the policy of flat rows.)
+static bool row_suits_list(int32_t B, int32_t V, int32_t top_k)
+{
+    if (V > kRowMaxV || V < 8192 || B < 128) return false;
+    if (B <= 256) return (uint32_t)B * (uint32_t)top_k >= (V <= 32768 ? 25600u : 51200u);
+    return V <= 32768 && top_k >= 200;
+}
 // The short-row kernel (one workgroup per row, one launch, any kept set) against what such calls took before it -- the general
 // kernel, the streaming path, the row kernel -- us a call, top_k 40 of peaked rows / top_p 0.9 of N(0,3) / the same two with
 // penalties:
@@ -572,6 +599,7 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
         return (int)kPathCluster;
     };
     if (!bounded && !(top_p < 1.0f)) return wide_or_general(); // a top_k of thousands and no nucleus: more than the stashes hold
+    if (bounded && !(opt && opt->slice_r) && row_suits_list(B, V, top_k)) return kPathRow;
     if (!pol) return bounded ? kPathStream : wide_or_general();
     if (!routed_away(bounded ? 0 : 1)) {
         if (bounded) return kPathStream;

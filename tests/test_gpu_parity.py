@@ -484,6 +484,37 @@ def test_rows_of_up_to_16384_tokens_with_a_bounding_top_k_take_the_kernel_that_s
         assert np.array_equal(res["diag"][f], ref["diag"][f]), f
 
 
+@pytest.mark.parametrize("B,V,k,dtype,one", [
+    (127, 32768, 1024, "float32", False), (128, 16388, 199, "float32", False), (128, 16388, 200, "float32", True), (128, 32768, 1024, "bfloat16", True),
+    (256, 32768, 99, "float32", False), (256, 32764, 100, "float16", True), (128, 32772, 399, "float32", False), (128, 32772, 400, "float32", True),
+    (255, 65536, 202, "float32", True), (256, 65540, 1024, "float32", False), (257, 32768, 199, "float32", False), (257, 32768, 200, "float32", True),
+    (257, 32772, 1024, "float32", False), (513, 12288, 200, "float32", True), (700, 8196, 1024, "float32", True)])
+def test_rows_with_a_bounding_top_k_of_hundreds_take_the_row_kernel(torch_cuda, B, V, k, dtype, one):
+    """Which calls of 128 rows and more with a bounding top_k one workgroup per row does by itself (diag.rounds == 10): the edges of
+    rows, tokens and top_k, rows of ties and masked stretches among them, against the general kernel in every field."""
+    from tests import capi
+    torch = torch_cuda
+    lg_np = H.logits_normal(B, V, 1.5, seed=B)
+    lg_np[1] = 0.25
+    lg_np[2] = np.round(lg_np[2] * 8) / 8
+    lg_np[3, V // 4:] = -np.inf
+    lg_np[4, 100:400] = 9.0
+    lg = torch.from_numpy(lg_np).cuda().to(getattr(torch, dtype))
+    rc, c, kk, pp = capi.normalize(1.0, k, 0.95, V, B, 1)
+    smp = capi.Sampler(B, V, with_policy=True, init=True)
+    u = torch.from_numpy(H.uniforms(B, 66)).cuda()
+    res = smp.sample(lg, c, kk, pp, uniforms=u)
+    assert rc == 0 and res["rc"] == 0 and smp.status() == 0
+    rounds = res["diag"]["rounds"]
+    rounds = np.delete(rounds, 1)                        # (a row of one tie says 0 everywhere)
+    assert ((rounds == 10).all() if one else (rounds != 10).all()), np.unique(rounds, return_counts=True)
+    ref = smp.sample(lg, c, kk, pp, uniforms=u, path="cluster")
+    for f in FIELDS:
+        assert np.array_equal(res["diag"][f], ref["diag"][f]), f
+    assert np.array_equal(res["out"], ref["out"])
+    smp.close()
+
+
 def test_row_kernel_takes_the_wide_kept_sets_of_calls_of_many_short_rows(torch_cuda, oracle):
     """Calls of 128 rows and more (64 in rows of fewer than 32768 tokens) of 8192 to 65536 tokens whose kept
     sets the stashes cannot hold go to the row kernel by themselves (diag.rounds == 10): a top_k of
