@@ -36,7 +36,7 @@ def _run(cmd, verbose):
     subprocess.check_call(cmd)
 
 
-KERNEL_SOURCES = ["rs_api.hip", "rs_cluster.hip", "rs_stream.hip", "rs_wide.hip", "rs_row.hip", "rs_short.hip"]
+KERNEL_SOURCES = ["rs_api.hip", "rs_cluster.hip", "rs_stream.hip", "rs_wide.hip", "rs_row.hip", "rs_short.hip", "rs_sieve.hip"]
 
 
 def build_kernels(verbose=False):

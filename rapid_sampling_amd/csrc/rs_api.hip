@@ -41,6 +41,11 @@
 //     way it does alone, from the logits (finish_row_slow), and says so to the
 //     caller's rs_policy, which routes the next calls of that kind.
 //
+//   sieve path (sieve_kernel + sieve_finish_kernel, two launches, no waits): the streaming
+//     path's calls with a top_k of up to 64, and larger calls with more.  The pass sums the
+//     row approximately and sets its largest tokens aside; the finish makes sure that nothing
+//     it decides depends on what the sum is off by.
+//
 //   wide path (stream_kernel counting only + wide_kernel + wide_finish_kernel,
 //     three launches, no waits): kept sets of thousands of tokens (top_k > 1024,
 //     flat distributions under top_p).  The second pass reads the rows again with
@@ -57,12 +62,14 @@
 //   penalties at scale (stream_pen_kernel + finish_kernel + penalty_fix_kernel).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <math.h>
 #include <stdlib.h>
 
 #include <atomic>
 #include <new>
 
 #include "rs_common.h"
+#include "rs_sieve_view.h"
 
 // Workspace of rs_sample_static: one array per GPU inside the library's code object.  In host code
 // this name is only a handle for hipGetSymbolAddress, never an address.
@@ -438,7 +445,7 @@ static bool row_suits(int32_t B, int32_t V)
     return B >= 512 || V >= 40000;                            // 257 to 511 rows: two rounds pay off in long rows only
 }
 // The row kernel with a bounding top_k of hundreds, whose lists the streaming path's finish goes through in one workgroup per row as well:
-// streaming path / row kernel, us a call, N(0,1.5), top_p 0.95:
+// streaming (or sieve) path / row kernel, us a call, N(0,1.5), top_p 0.95:
 //   rows x tokens   top_k 65       128         200         300        1000       200 (0)    flat 200
 //    64 x 20000   12.6 / 13.6  12.8 / 13.7  14.2 / 13.7  15.7 / 13.8  19.4 / 14.4  14.9 / 15.0  16.9 / 14.1
 //   128 x 20000   13.5 / 13.7  13.7 / 13.9  16.0 / 13.7  16.9 / 13.9  20.7 / 14.5  17.1 / 15.0  18.2 / 14.1
@@ -532,6 +539,44 @@ static int fused_r(int32_t B, int32_t V, bool pen, bool any_size)
     }
     if (any_size && small_call && stream_parts(V, 4) >= 2u) return 4;
     return 0;
+}
+
+// The sieve path (rs_sieve.h) in the place of the streaming path: calls with a bounding top_k, without penalties.  Slice length of its pass (float4
+// groups per thread), 0 when the call stays on the streaming path.  There / here, us a call (N(0,1.5), top_p 1 and, from a top_k of 100 on,
+// 0.95; float32, (0): bfloat16):
+//   rows x tokens     top_k 50      1 (0)       100          300         1000      16 spikes, top_k 40, top_p 0.95
+//      1 x  50304    9.9 / 9.1   8.8 / 8.3  10.9 / 12.6                             9.2 / 9.0
+//     16 x 131072   12.9 / 10.9 10.6 / 9.6  13.3 / 13.9  15.6 / 19.0               11.4 / 10.2
+//     64 x  50304   13.8 / 11.1 11.9 / 9.9  14.9 / 15.4                            12.3 / 10.9
+//     64 x 131072   17.3 / 13.4 13.7 / 11.0 17.8 / 17.9  19.7 / 23.1               15.7 / 13.5
+//     64 x 262144   23.8 / 18.8 19.2 / 14.3 24.4 / 22.4  25.7 / 27.2  32.1 / 31.0  22.1 / 18.8
+//    256 x 131072   35.6 / 28.2 28.5 / 18.6 37.9 / 33.0  43.7 / 40.6
+//    512 x  50304   33.2 / 24.9 27.1 / 18.1 36.8 / 32.3
+//    512 x 131072   58.9 / 49.9 45.2 / 28.5 61.4 / 55.4  75.7 / 63.5               57.0 / 50.0
+//    128 x 1048576   103 / 92    78 / 50     104 / 96     105 / 100    112 / 105    104 / 94
+//   1024 x  20000   39.3 / 28.1 31.0 / 21.8                                        35.2 / 28.2
+// (1 x 32768: 8.9 there and 9.7 here with 16 spikes.)  Its finish compares up to 64 tokens with each other, for which it is as short as the streaming
+// path's; longer lists are faster there until the pass outweighs them.  Slices of 4096 tokens while 32 of them make a row, else of
+// 8192, and of 16384 in a few rows of a million (1 x 1048576 12.0 us against 14.1); shorter when one would hold more than 8 of the row's top_k on
+// average, since a slice sets aside 64 tokens: at least four times its share.  (Up to 16 in slices of 4096, which then set aside 128.)
+// Without a bounding top_k the kept set may be of hundreds of tokens, the longer list's time, and each is one more place where D is too close to
+// call: 16 x 131072 with 455 kept 15.0 there, 46.7 here.
+static uint32_t sieve_share(int32_t top_k, int32_t V, int R) { return (uint32_t)(((uint64_t)(uint32_t)top_k * 1024u * (uint32_t)R + (uint32_t)V - 1u) / (uint32_t)V); }
+static int sieve_r(int32_t B, int32_t V, int32_t top_k)
+{
+    const uint64_t tokens = (uint64_t)B * (uint64_t)V;
+    if (tokens < (top_k <= 64 ? 49152u : top_k <= 128 ? 1u << 24 : V <= kMidMaxV ? 1u << 25 : 1u << 26)) return 0;
+    const uint32_t g4 = stream_parts(V, 4), g8 = stream_parts(V, 8);
+    int R = g4 <= 32u && (uint64_t)B * g4 <= kStreamSmallParts ? 4 : g8 <= 64u || (uint64_t)B * g8 > 8192u ? 8 : 16;
+    while (R > 4 && sieve_share(top_k, V, R) > 8u && stream_parts(V, R / 2) <= 128u) R /= 2;
+    return sieve_share(top_k, V, R) <= 16u ? R : 0;
+}
+// Of a slice's 128 pairs of threads, how many reach the bound of what is set aside: as many as hold one of eight times the slice's share of the
+// top_k tokens (of all of them, if they are fewer), each in a pair by chance, and some more; as far as there is room.
+static uint32_t sieve_reach(int32_t V, int32_t top_k, int R, uint32_t units)
+{
+    const double all = (double)top_k, m = min(8.0 * all * 1024.0 * R / V, all);
+    return min((uint32_t)(128.0 * (1.0 - exp(-m / 128.0)) + 2.0 * sqrt(m) + 4.0), units == 1u ? 48u : 78u);
 }
 
 static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pen, const rs_options *opt)
@@ -636,7 +681,7 @@ using namespace rs;
 
 extern "C" {
 
-int rs_version(void) { return 418; }
+int rs_version(void) { return 419; }
 
 const char *rs_error_string(int code)
 {
@@ -872,6 +917,20 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
     const int path = choose_path(B, V, top_k, top_p, pen, opt);
     if (path == kPathShort) return launch_short(pen, logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     if (path == kPathRow) return launch_row(logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
+    if (const int R = !pen && path == kPathStream ? sieve_r(B, V, top_k) : 0) {
+        SieveView v;
+        v.G = stream_parts(V, R);
+        v.units = sieve_share(top_k, V, R) <= 8u ? 1u : 2u;
+        v.reach = sieve_reach(V, top_k, R, v.units);
+        const size_t slices = (size_t)B * v.G, hdr = align256(sizeof(WsHeader)), stash = align256(hdr + slices * sizeof(SieveHdr));
+        const size_t end = align256(stash + slices * v.units * kWave * sizeof(uint64_t));
+        // (a workspace of rs_workspace_bytes has room, 0.25 bytes a token at most; one without takes the streaming path)
+        if (end + (size_t)B * sizeof(RowCtl) <= (workspace_bytes & ~(size_t)255)) {
+            v.hdr = (SieveHdr *)((char *)workspace + hdr); v.stash = (uint64_t *)((char *)workspace + stash);
+            p.report = (uint32_t)policy_word(0, size_class(B, V));
+            return launch_sieve(R, logits_dtype, (uint32_t)B, (hipStream_t)stream, p, v) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
+        }
+    }
     if (path != kPathCluster) {
         const int sr = path == kPathFused ? fused_r(B, V, pen, opt && opt->path == RS_PATH_FUSED)
                      : (path == kPathWide1 || path == kPathKeep) ? wide_r(B, V, workspace_bytes)

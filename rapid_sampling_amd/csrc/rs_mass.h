@@ -258,9 +258,17 @@ struct LdsFew {
 // of the workgroup together (more may call; all meet at its barrier); one wave does it alone when there are few tokens.  Each token is
 // compared with every other: its place by falling e, where one scan finds the threshold, and its place by index, where
 // another finds the sampled token.  Returns that token + 1 in one lane of wave 0, 0 elsewhere.
+// D and P are those of `totals(mass of the whole list)`; `look` is told by wave 0, in every lane, what was decided: the call's D and P, whether the list
+// is enough, tokens above the threshold and at it, the threshold, the mass above it, tie weight and target, the running sum before the lane's
+// token and with it, and whether that is the sampled one.
+struct Totals { M96 D, P; };
+struct LooksAtNothing {
+    template <typename... A> __device__ __forceinline__ void operator()(const A &...) const {}
+};
+template <typename T, typename F = LooksAtNothing>
 __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const uint32_t row, const int lane, const int wave, const uint64_t *list,
-                                             const uint32_t n, const uint32_t top_k, const M96 D, const M96 P, const float xmax,
-                                             const uint64_t *rand64, const uint32_t rounds)
+                                             const uint32_t n, const uint32_t top_k, T totals, const float xmax,
+                                             const uint64_t *rand64, const uint32_t rounds, F look = F())
 {
     const uint64_t e = list[min((uint32_t)lane, n - 1u)];
     const bool split = n > 16u, in = (uint32_t)lane < n;
@@ -285,11 +293,14 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const uint32_t b = in ? (uint32_t)(s.sorted[lane] >> 32) : 0u;
     const Limbs own = limbs(M96{in ? w_of_bits(b) : 0ull, 0u}), upto = wave_inclusive_scan(own);
+    const Totals t = totals(upto);
+    const M96 D = t.D, P = t.P;
     const uint64_t enough = __builtin_amdgcn_ballot_w64(in && ((uint32_t)lane + 1u >= top_k || m96(upto) >= P));
     const uint32_t thr = lane_of(b, enough ? (uint32_t)__builtin_ctzll(enough) : n - 1u);
     const uint32_t n_gt = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b > thr));
     const uint32_t n_eq = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b == thr));
-    const Target tg = tie_and_target(p, row, uniform(*rand64), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(m96(lane_of(upto - own, n_gt))), rounds, lane == 0);
+    const M96 above = m96(lane_of(upto - own, n_gt));
+    const Target tg = tie_and_target(p, row, uniform(*rand64), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(above), rounds, lane == 0);
     const M96 r = m96(tg.r);
     if (in) {
         const uint32_t be = (uint32_t)(e >> 32);
@@ -298,7 +309,10 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const Limbs mine = limbs(M96{in ? s.w[lane] : 0ull, 0u}), run = wave_inclusive_scan(mine);
-    return in && m96(run - mine) < r && m96(run) >= r ? s.idx[lane] + 1u : 0u;
+    const M96 bef = m96(run - mine), with = m96(run);
+    const bool is_it = in && bef < r && with >= r;
+    look(t, enough != 0ull, n_gt, n_eq, thr, above, tg, bef, with, is_it);
+    return is_it ? s.idx[lane] + 1u : 0u;
 }
 
 }  // namespace rs

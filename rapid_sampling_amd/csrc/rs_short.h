@@ -287,7 +287,7 @@ __global__ void __launch_bounds__(short_threads<W>(), (short_waves<PEN, W, R>())
                 if (eb[i] >= lo) L.list[at++] = ((uint64_t)eb[i] << 32) | (group(i >> 2) * 4u + (uint32_t)(i & 3));
         }
         __syncthreads();
-        token = few_pick(p, L.few, row, lane, wave, L.list, n, top_k, D, P, xmax, &L.rand64, kShortRounds);
+        token = few_pick(p, L.few, row, lane, wave, L.list, n, top_k, [&](const Limbs &) { return Totals{D, P}; }, xmax, &L.rand64, kShortRounds);
     } else {
         // ---- a longer one: everything from the registers ----
         if (span != 0u) {                                // a single token left in the range: the threshold itself

@@ -1,0 +1,963 @@
+// The sieve path: one pass over the logits in which every wave works a slice of its own, a finishing workgroup per row.
+#pragma once
+
+#include "rs_common.h"
+#include "rs_mass.h"
+#include "rs_sieve_view.h"
+#include "rs_stream.h"
+
+namespace rs {
+
+// ---------------------------------------------------------------- sieve path --
+// For kept sets that are small next to the row two things are needed of it: its largest tokens, and its total mass D, of
+// which P = ceil(top_p * D) is the mass that is enough.  The tokens must be exact.  D need not be, as long as nothing that is
+// decided by it lies within its error: then the exact D decides the same.  So
+//
+//   sieve_kernel         a workgroup per slice, no histogram, two barriers.  It sums 2^x with the hardware's exponential and sets aside every token at
+//                        or above a value that a given number of its threads, pair by pair, reach with their largest token: between that
+//                        many and some half more, whatever the distribution.
+//   sieve_finish_kernel  a workgroup per row.  It takes D from the slices' sums, works out threshold and token from the tokens set
+//                        aside -- complete above the largest of the slices' bounds -- and then compares the distance of every
+//                        decision on the way from its alternative with the error that D can have.  If one is too close (a row in some
+//                        ten thousands, more when hundreds of tokens are kept) it sums the row again, from the logits, in double
+//                        precision, and decides again.
+//
+// The results are the same integers as on every other path.
+//
+// The error of D, in units of 2^-24 of it: v_exp_f32(x) is larger than e of x by 0 to 3.45 (every float |x| < 127 compared), of which 2 are
+// taken off; 16 tokens are summed in a tree of four roundings, their sums in double precision, the slice's sum is
+// rounded once to a float, and the slices' are added as integers of 2^-40 of the frame: 6.5, for which 7 are allowed.  A wave with a value
+// out of v_exp_f32's range, or with a NaN or an infinity, sums 2^(x - M), M the floor of its maximum, whose x - M is
+// rounded: |v_exp_f32(x - M) / e - 1| is at most 5.4 units for tokens up to 8 octaves below the frame, 8.7 to 16, 14.1 to 32, 25.2 to 40 (every float
+// |x| < 128 compared; larger |x| have less of it), so for 4096 tokens, one of them in the frame's octave, at most 9.1; with 3 roundings 12.1, and 32
+// are allowed.  Tokens more than 40 octaves below the row's frame weigh nothing but are in the sums: 2^-40 each at most.
+//
+// What bounds it: in large calls the pass reads float32 at the rate of a kernel that only reads.  A token costs 4.6 vector instructions (one of
+// them the exponential, 2.7 issue slots), and a wave some 200 for bound and staging, where the pass with exact e and a histogram (stream_kernel)
+// takes 22 and an LDS atomic.  us of a pass, there / here: 128 rows of 1048576 106 / 86, 64 of 152064 12.7 / 10.1, 256 of 151936 bfloat16
+// 28 / 16.8, of which 12 are the read.
+constexpr uint32_t kSieveErrOdd = 19;                    // D is known to 2^-19 of itself when waves were summed in a frame, else to 7 * 2^-24
+
+// Sum over the wave in double precision, in every lane.
+__device__ __forceinline__ double wave_sum_f64(double v)
+{
+    auto step = [&](auto ctrl, auto mask) {
+        v += __builtin_bit_cast(double, dpp0<decltype(ctrl)::value, decltype(mask)::value>(__builtin_bit_cast(uint64_t, v)));
+    };
+    step(std::integral_constant<int, 0x111>{}, std::integral_constant<int, 0xf>{}); step(std::integral_constant<int, 0x112>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x114>{}, std::integral_constant<int, 0xf>{}); step(std::integral_constant<int, 0x118>{}, std::integral_constant<int, 0xf>{});
+    step(std::integral_constant<int, 0x142>{}, std::integral_constant<int, 0xa>{}); step(std::integral_constant<int, 0x143>{}, std::integral_constant<int, 0xc>{});
+    return __builtin_bit_cast(double, lane63(__builtin_bit_cast(uint64_t, v)));
+}
+
+struct LdsSieve {
+    float4   grp[kWaves][kWave];                         // groups of four tokens that hold one to set aside
+    uint32_t gidx[kWaves][kWave];
+    double   mass[kThreads];                             // the threads' sums
+    float    top[kThreads];                              // and largest tokens
+    float    frame[kWaves];                              // the frames of the sums
+    uint32_t wmax[kWaves], odd[kWaves], n[2][kWaves], tie;
+};
+
+// A workgroup's slice to its record.  group(j, x): the scaled logits of the thread's j-th group of four tokens, group j * 256 + tid of the
+// slice, from the registers that the loads fill; those past the end of the row, `left` groups from the slice's first, are copies of its last;
+// g0: the slice's first group.
+// The terms of the sum need no frame: 2^x is a float for every x in question, and so they are worked out in the order in which
+// the loads arrive.  A wave whose largest x is beyond 120 or below -80 (the tokens 40 octaves below it would no longer be floats), or
+// that holds a NaN or an infinity, does it again, cleaned up and in a frame.
+template <int R, typename G>
+__device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G group, const size_t slice, const uint32_t g0, const uint32_t left, const int tid)
+{
+    const float kInf = __builtin_inff();
+    const int lane = tid & (kWave - 1), wave = (int)uniform((uint32_t)tid >> 6);
+    bool odd = false;
+    double mass = 0.0;
+    float x[R * 4], gm[R], lm = -kInf, M = 0.0f;            // gm: the largest of every group, lm: of all; of the wave: the frame, the sum in it
+    auto top = [&](int j) {
+        float m;                                         // (fmaxf quiets its operands first, an instruction each; products are quiet)
+        asm("v_max3_f32 %0, %1, %2, %3" : "=v"(m) : "v"(x[j * 4]), "v"(x[j * 4 + 1]), "v"(x[j * 4 + 2]));
+        asm("v_max_f32 %0, %1, %2" : "=v"(m) : "v"(m), "v"(x[j * 4 + 3]));
+        return m;
+    };
+    if ((uint32_t)(wave * kWave) >= left) {              // nothing of the row
+#pragma unroll
+        for (int j = 0; j < R; ++j) gm[j] = -kInf;
+    } else {
+        const bool ragged = left < (uint32_t)(R * kThreads);             // some of the groups may lie past the end of the row
+        float part[R / 4], q[4];                         // (a tree: log2 of the tokens' number of roundings)
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            group(j, &x[j * 4]);
+            gm[j] = top(j);
+            q[j % 4] = (__builtin_amdgcn_exp2f(x[j * 4]) + __builtin_amdgcn_exp2f(x[j * 4 + 1])) +
+                       (__builtin_amdgcn_exp2f(x[j * 4 + 2]) + __builtin_amdgcn_exp2f(x[j * 4 + 3]));
+            if (j % 2 == 1) {
+                if (ragged) {
+                    const uint32_t at = (uint32_t)((j - 1) * kThreads) + opaque((uint32_t)tid);
+                    if (at >= left) { gm[j - 1] = -kInf; q[j % 4 - 1] = 0.0f; }
+                    if (at + (uint32_t)kThreads >= left) { gm[j] = -kInf; q[j % 4] = 0.0f; }
+                }
+                lm = fmaxf(fmaxf(lm, gm[j - 1]), gm[j]);
+                __builtin_amdgcn_sched_barrier(0);       // (group after group, as they arrive: side by side they would take 30 registers more)
+            }
+            if (j % 4 == 3) part[j / 4] = (q[0] + q[1]) + (q[2] + q[3]);
+        }
+#pragma unroll
+        for (int i = 0; i < R / 4; ++i) mass += (double)part[i];
+        odd = __builtin_amdgcn_ballot_w64(!(mass < (double)kInf) || lm > 120.0f) != 0ull || __builtin_amdgcn_ballot_w64(lm >= -80.0f) == 0ull;
+        if (__builtin_expect(odd, 0)) {
+            // (the clean-up of sampling.cu:553 on the products in the registers)
+            const uint32_t t = opaque((uint32_t)tid);
+            lm = -kInf;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+#pragma unroll
+                for (int q = 0; q < 4; ++q) x[j * 4 + q] = sf(x[j * 4 + q]);
+                gm[j] = (uint32_t)(j * kThreads) + t < left ? top(j) : -kInf;
+                lm = fmaxf(lm, gm[j]);
+            }
+            M = __builtin_floorf(fkey_inv(wave_max_u32(fkey(lm))));
+            mass = 0.0;
+#pragma unroll
+            for (int j = 0; j < R; ++j) {
+                auto e = [&](int q) { return __builtin_amdgcn_exp2f(x[j * 4 + q] - M); };
+                mass += (uint32_t)(j * kThreads) + t < left ? (double)((e(0) + e(1)) + (e(2) + e(3))) : 0.0;
+            }
+        }
+    }
+    s.top[tid] = lm; s.mass[tid] = mass;
+    {
+        const uint32_t k = wave_max_u32(fkey(lm));
+        if (lane == 0) { s.frame[wave] = M; s.wmax[wave] = k; s.odd[wave] = odd ? 1u : 0u; }
+    }
+    if (tid == 0) s.tie = 1u;
+    __syncthreads();
+
+    // The bound: a value that at least `reach` of 128 pairs of threads reach with their largest token, and not many more, by halving
+    // the range of these (of their order-preserving keys: on scalars).  Every wave for itself.  (Tokens 41 octaves below the slice's frame
+    // are dead wherever the row's frame is.)
+    const float4 t4 = reinterpret_cast<const float4 *>(s.top)[lane];
+    const uint4 k4 = *reinterpret_cast<const uint4 *>(s.wmax);
+    const uint32_t one = fkey(fmaxf(t4.x, t4.y)), two = fkey(fmaxf(t4.z, t4.w));
+    const uint32_t key = uniform(max(max(k4.x, k4.y), max(k4.z, k4.w)));
+    const float xmax = fkey_inv(key), Ms = __builtin_floorf(xmax);
+    auto reached = [&](uint32_t t) {
+        return (uint32_t)(__builtin_popcountll(__builtin_amdgcn_ballot_w64(one >= t)) + __builtin_popcountll(__builtin_amdgcn_ballot_w64(two >= t)));
+    };
+    uint32_t want = v.reach, hi = key;
+    const uint32_t dead = uniform(fkey(Ms - 41.0f));
+    // (from the least of a few of them, which is below the bound nearly always; else from the least of all)
+    uint32_t lo = max(min(min(lane_of(one, 0u), lane_of(two, 16u)), min(lane_of(one, 32u), lane_of(two, 48u))), dead), reach = reached(lo);
+    if (reach < want) { lo = max(~wave_max_u32(~min(one, two)), dead); reach = reached(lo); }
+    const uint32_t room = v.units * (uint32_t)kWave;
+    bool full = false;
+    float bound = 0.0f;
+    uint32_t c[kWaves] = {0u, 0u, 0u, 0u};               // of each wave, its groups that reach the bound
+    for (uint32_t turn = 0;; turn ^= 1u) {
+#pragma unroll 1
+        while (reach > want + 3u && hi - lo > 1u) {
+            const uint32_t mid = lo + ((hi - lo) >> 1), r = reached(mid);
+            if (r >= want) { lo = mid; reach = r; } else hi = mid;
+        }
+        bound = fkey_inv(lo);
+        // the wave's groups that reach it, side by side
+        uint32_t fill = 0;
+        const uint32_t first = opaque(g0 + (uint32_t)tid);          // (or sixteen sums of it are kept from the loads on)
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const bool in = gm[j] >= bound;
+            const uint64_t vote = __builtin_amdgcn_ballot_w64(in);
+            if (vote != 0ull) {
+                const uint32_t at = fill + __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0u));
+                if (in && at < (uint32_t)kWave) {
+                    s.grp[wave][at] = make_float4(x[j * 4], x[j * 4 + 1], x[j * 4 + 2], x[j * 4 + 3]);
+                    s.gidx[wave][at] = first + (uint32_t)(j * kThreads);
+                }
+                fill += (uint32_t)__builtin_popcountll(vote);
+            }
+        }
+        if (lane == 0) s.n[turn][wave] = fill;
+        __syncthreads();
+        const uint4 f4 = *reinterpret_cast<const uint4 *>(s.n[turn]);
+        c[0] = uniform(f4.x); c[1] = uniform(f4.y); c[2] = uniform(f4.z); c[3] = uniform(f4.w);
+        const uint32_t most = max(max(c[0], c[1]), max(c[2], c[3]));
+        if (__builtin_expect(most <= (uint32_t)kWave && c[0] + c[1] + c[2] + c[3] <= room, 1)) break;
+        // more groups than there is room for (threads with many of them, ties): fewer threads; in the end none, and no token above the maximum
+        if (want <= 8u || lo == key) { full = true; break; }
+        want -= 8u;
+        hi = key;
+    }
+    if (wave == 1) {
+        // the slice's sum: lane l those of threads 4 l to 4 l + 3, all of one wave
+        const double2 m2 = reinterpret_cast<const double2 *>(s.mass)[lane * 2], m3 = reinterpret_cast<const double2 *>(s.mass)[lane * 2 + 1];
+        const int down = (int)fmaxf(s.frame[lane >> 4] - Ms, -1000.0f);
+        const double all = wave_sum_f64(__builtin_ldexp((m2.x + m2.y) + (m3.x + m3.y), down));
+        if (lane == 0) v.hdr[slice].mass = __float_as_uint((float)all);
+    }
+    uint32_t n = 0, cut = key;
+    if (__builtin_expect(full, 0)) {
+        float least = xmax;
+        const uint32_t t0 = opaque((uint32_t)tid);
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const float m = fminf(fminf(x[j * 4], x[j * 4 + 1]), fminf(x[j * 4 + 2], x[j * 4 + 3]));
+            if ((uint32_t)(j * kThreads) + t0 < left) least = fminf(least, m);
+        }
+        if (least != xmax) s.tie = 0u;
+        __syncthreads();
+        n = s.tie ? kSieveTie : 0u;
+    } else if (wave == 0) {
+        // the tokens of those groups, by the first wave, a group to a lane
+        const uint32_t all = c[0] + c[1] + c[2] + c[3];
+        uint64_t *st = v.stash + slice * room;
+        for (;;) {
+            n = 0;
+            for (uint32_t g = (uint32_t)lane; g < room; g += kWave) {
+                uint32_t w = 0, at = g;
+                if (at >= c[0]) { at -= c[0]; w = 1u; }
+                if (w == 1u && at >= c[1]) { at -= c[1]; w = 2u; }
+                if (w == 2u && at >= c[2]) { at -= c[2]; w = 3u; }
+                const bool have = g < all;
+                const float4 q4 = s.grp[w][at & 63u];
+                const uint32_t i0 = s.gidx[w][at & 63u] * 4u;
+                const float t[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const bool in = have && t[q] >= bound;
+                    const uint64_t vote = __builtin_amdgcn_ballot_w64(in);
+                    const uint32_t o = n + __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0u));
+                    if (in && o < room) st[o] = ((uint64_t)__float_as_uint(t[q]) << 32) | (i0 + (uint32_t)q);
+                    n += (uint32_t)__builtin_popcountll(vote);
+                }
+            }
+            if (__builtin_expect(n <= room, 1)) { cut = lo - 1u; break; }
+            // several tokens of most groups: a bound between this one and the largest token that fewer reach
+            if (lo == key) { n = 0; break; }
+            lo += max((key - lo) >> 2, 1u);
+            bound = fkey_inv(lo);
+        }
+    }
+    if (tid == 0) {
+        const uint4 o4 = *reinterpret_cast<const uint4 *>(s.odd);
+        *reinterpret_cast<uint2 *>(&v.hdr[slice]) = make_uint2(key, n | ((o4.x | o4.y | o4.z | o4.w) != 0u ? kSieveOdd : 0u));
+        v.hdr[slice].cut = cut;
+    }
+}
+
+// A workgroup of 256 threads to a slice of R * 256 groups of four tokens.
+template <int R, int DT>
+__global__ void __launch_bounds__(kThreads, R == 16 ? 4 : 8) sieve_kernel(const Params p, const SieveView v)
+{
+    __shared__ LdsSieve s;
+    const int tid = threadIdx.x;
+    const uint32_t row = blockIdx.x / v.G, part = blockIdx.x - row * v.G;
+    const bool reporter = blockIdx.x == 0 && tid == 0;
+    PrevCall prev;
+    prev.slow_rows = 0; prev.meta = 0;
+    if (reporter) prev = report_begin(p);
+    const uint32_t g0 = part * (uint32_t)(R * kThreads), left = ((uint32_t)p.V >> 2) - g0;
+    // the thread's j-th group is group j * 256 + tid; past the end of the row its last one
+    typedef typename std::conditional<DT == RS_DTYPE_F32, rs_u32x4, rs_u32x2>::type T;
+    typedef const __attribute__((address_space(1))) T GlobalT;
+    GlobalT *from = (GlobalT *)reinterpret_cast<const T *>(logits_row(p, row)) + g0;
+    T l[R];
+    if (left >= (uint32_t)(R * kThreads)) {              // (a scalar address and the thread's offset: none is worked out per thread)
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            GlobalT *q = from + j * kThreads;
+            asm("" : "+s"(q));
+            l[j] = __builtin_nontemporal_load(q + (uint32_t)tid);
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < R; ++j) l[j] = __builtin_nontemporal_load(from + min((uint32_t)(j * kThreads + tid), left - 1u));
+    }
+    if (reporter) report_end(p, prev, true);
+    sieve_slice<R>(v, s, [&](int j, float *x) {
+        uint32_t w[4];
+        if constexpr (DT == RS_DTYPE_F32) { w[0] = l[j].x; w[1] = l[j].y; w[2] = l[j].z; w[3] = l[j].w; }
+        else widen4(make_uint2(l[j].x, l[j].y), DT, w);
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = __uint_as_float(w[q]) * p.c;
+    }, (size_t)row * v.G + part, g0, left, tid);
+}
+
+// ---- the finish ----
+constexpr uint32_t kSieveList = 2048;                    // tokens at or above the boundary bin that are listed at most
+constexpr int      kSieveCopies = 4;                     // of each level-1 bin while it is counted
+constexpr uint32_t kSieveSteps = 256;                    // between the bound and the row's largest token, where the short way counts
+template <int NT>
+struct LdsSieveFin {
+    alignas(16) uint64_t bins[kSieveCopies][kNB + 4];    // (all of e's exponents: the row's exact total is counted here, too)
+    alignas(16) uint64_t lev[3][128];
+    alignas(16) uint32_t step[NT / 128][kSieveSteps];    // copies, for lanes that add to one address
+    LdsFew   few;
+    uint64_t list[kSieveList], small[kWave];             // bits of e << 32 | index
+    uint64_t blo[NT], bhi[NT];                           // kept weights by bucket of the token index, halves summed apart
+    M96      mass[16];
+    struct { M96 D, P, r, err, shift; Edge f; uint64_t w_tie; uint32_t found; } one;  // what one wave worked out for all
+    uint64_t sum[16];
+    uint64_t rand64;
+    uint32_t wmax[16], wcut[16], flag[16];
+    uint32_t n, few_n, thr, bucket, unsure;
+};
+
+// Is a decision that was made with D, and with P = ceil(top_p * D), the one that the exact D makes?  Both may be off by less than
+// `err` (0: they are exact).  What comes out is how far the target r and the running sums may shift against each other for
+// the pick; `unsure` when threshold or tie weight themselves are in doubt.
+struct Doubt { M96 shift; bool unsure; };
+__device__ __forceinline__ Doubt doubt_of(const M96 P, const M96 err, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq, const M96 above,
+                                          const uint32_t thr, const uint64_t w_tie)
+{
+    Doubt d{M96{0ull, 0u}, false};
+    if (!(err.lo | err.hi)) return d;
+    const M96 least = P >= err ? P - err : M96{0ull, 0u}, most = P + err;
+    // the tokens above the threshold are not enough, those down to it are
+    if (n_gt && !(above < least)) d.unsure = true;
+    const M96 down = above + m96((u128)w_of_bits(thr) * n_eq);
+    if (n_gt + n_eq < top_k && !(down >= most)) d.unsure = true;
+    // The tie weight is (P - above) / n_eq unless that is more than it can be.  If it is, S and with it r move by u and the running sum by t times
+    // what P is off by, u and t between 0 and 1 (the random number; the ties before the token): by no more than that against each other, and what
+    // the divisions round.
+    const M96 S = above + m96((u128)w_tie * n_eq), n{(uint64_t)n_eq, 0u};
+    if (!(least >= S + n)) d.shift = err + n + M96{2ull, 0u};
+    return d;
+}
+// ... and the token whose weight lies at (before, upto] in the running sum, for the target r
+__device__ __forceinline__ bool pick_is_sure(const M96 shift, const M96 before, const M96 upto, const M96 r, const bool first, const bool last)
+{
+    if (!(shift.lo | shift.hi)) return true;
+    return (first || before + shift < r) && (last || upto >= r + shift);
+}
+
+// The level-1 bins of one wave's scan, an octave a lane, from their copies.
+template <typename L>
+__device__ __forceinline__ void sieve_octaves(OctScan &sc, L &l, const int lane)
+{
+    sc.load(lane, [&](uint32_t o, uint64_t (&w)[4]) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = 0ull;
+#pragma unroll
+        for (int c = 0; c < kSieveCopies; ++c) {
+            const ulonglong2 *two = reinterpret_cast<const ulonglong2 *>(&l.bins[c][o * 4u]);
+            const ulonglong2 a = two[0], q = two[1];
+            w[0] += a.x; w[1] += a.y; w[2] += q.x; w[3] += q.y;
+        }
+    });
+}
+
+// fn(group of four, bits of their e) over the row, from the logits (x by the definition, sampling.cu:553), eight loads in flight per thread.
+template <int NT, typename F>
+__device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t row, const float M, F fn)
+{
+    const uint32_t V4 = (uint32_t)p.V >> 2;
+    const char *lrow = logits_row(p, row);
+    const bool far = !(__builtin_fabsf(M) <= 100.0f);
+    const Frame fr(far ? 0 : (int)M);
+    auto e = [&](uint32_t l) {
+        const float x = sf(__uint_as_float(l) * p.c);
+        return fr.raw(far ? fmaxf(x - M, -1000.0f) : x);
+    };
+    constexpr int kAhead = 8;
+#pragma unroll 1
+    for (uint32_t base = threadIdx.x; base < V4; base += kAhead * NT) {
+        uint4 l[kAhead];                                 // (the format is asked once a round: a branch about every load waits for it)
+        if (p.dtype == RS_DTYPE_F32) {
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) l[u] = reinterpret_cast<const uint4 *>(lrow)[min(base + (uint32_t)(u * NT), V4 - 1u)];
+        } else {
+            uint2 q[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) q[u] = reinterpret_cast<const uint2 *>(lrow)[min(base + (uint32_t)(u * NT), V4 - 1u)];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                uint32_t w[4];
+                widen4(q[u], p.dtype, w);
+                l[u] = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u)
+            if (base + (uint32_t)(u * NT) < V4) fn(base + (uint32_t)(u * NT), make_uint4(e(l[u].x), e(l[u].y), e(l[u].z), e(l[u].w)));
+    }
+}
+
+// The row's D in double precision: 2^-40 of it off at most (D >= 1; a thread adds fewer than 2^13 terms).
+template <int NT>
+__device__ __forceinline__ M96 sieve_closer(const Params &p, LdsSieveFin<NT> &L, const uint32_t row, const float M)
+{
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    sieve_row_pass<NT>(p, row, M, [&](uint32_t, const uint4 b) {
+        auto e = [](uint32_t w) { return w < kEMinBits ? 0.0 : (double)__uint_as_float(w); };
+        s[0] += e(b.x); s[1] += e(b.y); s[2] += e(b.z); s[3] += e(b.w);
+    });
+    const double mine = wave_sum_f64((s[0] + s[1]) + (s[2] + s[3]));
+    __syncthreads();
+    if (lane == 0) L.sum[wave] = __builtin_bit_cast(uint64_t, mine);
+    __syncthreads();
+    double all = 0.0;
+    for (int w = 0; w < NT / kWave; ++w) all += __builtin_bit_cast(double, L.sum[w]);
+    const uint64_t q = uniform((uint64_t)(all * 0x1p40));
+    return M96{q << 23, (uint32_t)(q >> 41)};
+}
+
+// The row's exact D: all of its tokens counted into L.bins, which is left that way (with e_bits also the e of every token, dead ones as 0).
+template <int NT>
+__device__ __forceinline__ M96 sieve_exact(const Params &p, LdsSieveFin<NT> &L, const uint32_t row, const float M)
+{
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    uint4 *eb4 = p.e_bits ? reinterpret_cast<uint4 *>(p.e_bits + (int64_t)row * p.V) : nullptr;
+    for (int i = tid; i < kSieveCopies * (kNB + 4); i += NT) (&L.bins[0][0])[i] = 0ull;
+    __syncthreads();
+    uint64_t *bins = L.bins[lane & (kSieveCopies - 1)];
+    sieve_row_pass<NT>(p, row, M, [&](uint32_t i4, const uint4 b) {
+        auto add = [&](uint32_t w) { atomicAdd(reinterpret_cast<unsigned long long *>(&bins[w >> 21]), (unsigned long long)(kPackOne | (w & 0x7FFFFFu))); };
+        add(b.x); add(b.y); add(b.z); add(b.w);
+        auto live = [](uint32_t w) { return w < kEMinBits ? 0u : w; };
+        if (eb4) eb4[i4] = make_uint4(live(b.x), live(b.y), live(b.z), live(b.w));
+    });
+    __syncthreads();
+    OctScan sc;
+    sieve_octaves(sc, L, lane);
+    return sc.total();
+}
+
+// NT threads (256 and a wave that draws the random number, or 1024), PRE units to a wave.
+//
+// What bounds it: the length of its chain, as finish_row's.  The tokens set aside, some hundreds or thousands, are counted in 256 steps of e
+// between the bound and the row's largest, and one scan of the counts says down to which step top_k of them lie: these are listed.  A list of
+// at most 64 is finished by comparing them with each other; a longer one by level-1 bins with masses, and further digits, of the listed
+// tokens alone.  Only when what is listed turns out not to hold the kept set (more tokens in one step than the list takes) are all
+// tokens set aside looked at, bins first; and when those do not, the row itself.
+template <int NT, int PRE>
+__global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(const Params p, const SieveView v)
+{
+    constexpr int  W = NT / kWave;
+    constexpr bool kEach = NT == kThreads;               // every wave works the one-wave steps out for itself
+    union LdsAll { LdsSieveFin<NT> f; struct { Lds s; LdsB t; } slow; };
+    __shared__ LdsAll u;
+    LdsSieveFin<NT> &L = u.f;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int wave = (int)uniform((uint32_t)tid >> 6);
+    const uint32_t row = blockIdx.x, G = v.G;
+
+    uint32_t rs[6] = {0u, 0u, 0u, 0u, 0u, 0u};
+    uint32_t *rng_st = p.rng + (size_t)row * 16;
+    const bool draws = wave == (kEach ? W : W - 1);
+    if (draws && !p.inj_u) {
+#pragma unroll
+        for (int i = 0; i < 6; ++i) rs[i] = rng_st[i];
+    }
+    auto draw = [&]() __attribute__((always_inline)) {
+        if (!p.inj_u) {
+            uint32_t o[4];
+            philox4x32_10(rs[2], rs[3], rs[4], rs[5], rs[0], rs[1], o);
+            if (lane == 0) {
+                L.rand64 = ((uint64_t)o[0] << 32) | o[1];
+                rng_st[2] = rs[2] + 1u;
+                if (rs[2] + 1u == 0u) rng_st[3] = rs[3] + 1u;
+            }
+        }
+    };
+    const SieveHdr *hdrs = v.hdr + (size_t)row * G;
+    // a slice's mass in units of 2^-40 of the row's frame
+    auto mass_in = [&](const uint4 &h, const float M) __attribute__((always_inline)) {
+        const float d = M - __builtin_floorf(fkey_inv(h.x));
+        const int down = d >= 64.0f ? 64 : (int)d;
+        const int sh = (int)(h.w >> 23) - 110 - down;    // 2^(ex - 150) in units of 2^-40
+        const uint64_t m = (h.w & 0x7FFFFFu) | 0x800000u;
+        return sh >= 0 ? m << (sh & 63) : sh > -32 ? m >> (-sh & 63) : 0ull;
+    };
+    M96 D{0ull, 0u}, P{0ull, 0u}, err{0ull, 0u};
+    auto estimate = [&](const uint64_t all, const bool odd) __attribute__((always_inline)) {             // D from the slices' sums, and what it may be off by
+        auto part = [&](uint32_t sh) { return M96{(D.lo >> sh) | ((uint64_t)D.hi << (64u - sh)), D.hi >> sh}; };
+        D = M96{all << 23, (uint32_t)(all >> 41)};
+        if (odd) err = part(kSieveErrOdd);
+        else { D = D - part(23u); err = part(22u) + part(23u) + part(24u); }
+        err = err + M96{((uint64_t)p.V << 23) + 2ull, 0u};
+        P = ceil_mul(p.top_p, D);
+    };
+    if (kEach && wave == W) {
+        // the wave that draws the random number also adds up the row's mass: neither is wanted before the tokens are listed
+        // (bare barriers: what was asked for need not have arrived)
+        uint4 h[2];
+#pragma unroll
+        for (int k = 0; k < 2; ++k) h[k] = *reinterpret_cast<const uint4 *>(&hdrs[min((uint32_t)(lane + k * kWave), G - 1u)]);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();
+        draw();
+        const float M = __builtin_floorf(fkey_inv(wave_max_u32(max(h[0].x, h[1].x))));
+        uint64_t q = 0;
+        bool odd = false;
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+            if ((uint32_t)(lane + k * kWave) < G) { q += mass_in(h[k], M); odd = odd || (h[k].y & kSieveOdd) != 0u; }
+        estimate(wave_sum(q), __builtin_amdgcn_ballot_w64(odd) != 0ull);
+        if (lane == 0) { L.one.D = D; L.one.P = P; L.one.err = err; }
+        __syncthreads();
+        return;
+    }
+    // lane i looks after the wave's i-th unit of 64 tokens set aside, unit wave + W i of the row
+    const uint32_t sl = (uint32_t)(wave + W * lane) >> (v.units - 1u), half = (uint32_t)(wave + W * lane) & (v.units - 1u), GU = G * v.units;
+    const uint64_t *stash = v.stash + (size_t)row * GU * kWave;
+    const bool mine = lane < PRE && sl < G;
+    uint4 h = *reinterpret_cast<const uint4 *>(&hdrs[min(sl, G - 1u)]);
+    uint64_t pre[PRE];                                   // (units beyond the row's read its last one again)
+    auto ask = [&]() __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < PRE; ++i) pre[i] = stash[(size_t)min((uint32_t)(wave + W * i), GU - 1u) * kWave + lane];
+    };
+    ask();
+    auto clear_bins = [&]() __attribute__((always_inline)) {
+        for (int c = 0; c < kSieveCopies; ++c)
+            for (int i = (int)kBin0 + tid; i < kNB; i += NT) L.bins[c][i] = 0ull;
+        for (int i = tid; i < 3 * 128; i += NT) (&L.lev[0][0])[i] = 0ull;
+        L.blo[tid] = 0ull; L.bhi[tid] = 0ull;
+    };
+    for (int i = tid; i < NT / 128 * (int)kSieveSteps; i += NT) (&L.step[0][0])[i] = 0u;
+    if (tid == 0) { L.n = 0u; L.few_n = 0u; L.unsure = 0u; }
+    if (!mine) h = make_uint4(0u, 0u, 0u, 0u);
+    {
+        const uint32_t a = wave_max_u32(h.x), b = wave_max_u32(h.z);
+        if (lane == 0) { L.wmax[wave] = a; L.wcut[wave] = b; }
+    }
+    __syncthreads();
+    uint32_t kmax = L.wmax[0], kcut = L.wcut[0];
+#pragma unroll
+    for (int w = 1; w < W; ++w) { kmax = max(kmax, L.wmax[w]); kcut = max(kcut, L.wcut[w]); }
+    kmax = uniform(kmax); kcut = uniform(kcut);
+    if (!kEach && draws) draw();
+    const float xmax = fkey_inv(kmax);
+    const float M = __builtin_floorf(xmax);
+    // Complete: every token whose e is larger than that of the largest bound.  (Two values of x may share one e.)
+    const uint32_t e_cut = e_bits_of(fkey_inv(max(kcut, 0x00800000u)), M);
+    const bool whole = e_cut < kEMinBits;                // ... that is, every live token
+    const uint32_t from = max(e_cut + 1u, kEMinBits);
+    if constexpr (!kEach) {
+        const uint64_t coarse = __builtin_amdgcn_ballot_w64(mine && (h.y & kSieveOdd) != 0u);
+        const uint64_t q = wave_sum(mine && half == 0u ? mass_in(h, M) : 0ull);
+        if (lane == 0) L.sum[wave] = q | (coarse != 0ull ? 1ull << 63 : 0ull);
+    }
+    uint32_t b[PRE];                                     // bits of e, 0 for what is not a token of the complete part
+    auto look_at = [&](auto each) __attribute__((always_inline)) {
+        const bool far = !(__builtin_fabsf(M) <= 100.0f);
+        const Frame fr(far ? 0 : (int)M);
+        const uint32_t len = max(mine ? h.y & 255u : 0u, half * (uint32_t)kWave) - half * (uint32_t)kWave;     // (of the unit, more than 64 when there is another)
+#pragma unroll
+        for (int i = 0; i < PRE; ++i) {
+            float x = __uint_as_float((uint32_t)(pre[i] >> 32));
+            if (far) x = fmaxf(x - M, -1000.0f);
+            const uint32_t e = fr.raw(x);
+            const bool in = (uint32_t)lane < lane_of(len, (uint32_t)i) && e >= from;
+            b[i] = in ? e : 0u;
+            if (in) each(e);
+        }
+    };
+    auto to_bins = [&]() __attribute__((always_inline)) {
+        const int copy = lane & (kSieveCopies - 1);
+        look_at([&](uint32_t e) {
+            atomicAdd(reinterpret_cast<unsigned long long *>(&L.bins[copy][e >> 21]), (unsigned long long)(kPackOne | (e & 0x7FFFFFu)));
+        });
+    };
+    const uint32_t top_k = (uint32_t)p.top_k;
+    auto total = [&]() __attribute__((always_inline)) {                                 // by then somebody has added up the slices' sums
+        if constexpr (kEach) { D = uniform(L.one.D); P = uniform(L.one.P); err = uniform(L.one.err); }
+        else {
+            uint64_t all = 0, odd = 0;
+#pragma unroll
+            for (int w = 0; w < W; ++w) { all += L.sum[w] & ~(1ull << 63); odd |= L.sum[w] >> 63; }
+            estimate(uniform(all), uniform((uint32_t)odd) != 0u);
+        }
+    };
+    // a row finished from a list of at most 64 tokens that holds its kept set: the token + 1 in one lane of the first wave; 0 in `doubts` when
+    // nothing is in doubt, 1 when D must be exact, 2 when the list is too short (first wave)
+    uint32_t doubts = 0;
+    auto from_few = [&](const uint64_t *list, const uint32_t n, const bool all_of_it, const uint32_t rounds) __attribute__((always_inline)) -> uint32_t {
+        M96 e = err;
+        return few_pick(p, L.few, row, lane, wave, list, n, top_k,
+                        [&](const Limbs &upto) {
+                            if (!all_of_it) return Totals{D, P};
+                            e = M96{0ull, 0u};           // every live token of the row is there
+                            const M96 d = m96(lane_of(upto, 63u));
+                            return Totals{d, ceil_mul(p.top_p, d)};
+                        }, xmax, &L.rand64, rounds,
+                        [&](const Totals &t, bool enough, uint32_t n_gt, uint32_t n_eq, uint32_t thr, const M96 &above, const Target &tg, const M96 &before,
+                            const M96 &upto, bool is_it) {
+                            const Doubt d = doubt_of(t.P, e, top_k, n_gt, n_eq, above, thr, tg.w_tie);
+                            const M96 S = above + m96((u128)tg.w_tie * n_eq);
+                            const bool sure = !d.unsure && (!is_it || pick_is_sure(d.shift, before, upto, m96(tg.r), !(before.lo | before.hi), upto >= S));
+                            doubts = !enough ? 2u : sure ? 0u : 1u;
+                        });
+    };
+    auto put = [&](uint32_t token) __attribute__((always_inline)) {
+        if (wave == 0 && doubts) L.unsure = doubts;
+        if (token) {
+            p.out[row] = (int32_t)(token - 1u);
+            if (p.diag) p.diag[row].index = (int32_t)(token - 1u);
+        }
+        __syncthreads();
+        return uniform(L.unsure);
+    };
+    // the tokens for which in(i) says so, side by side
+    auto list_them = [&](auto in) __attribute__((always_inline)) {
+        uint32_t own = 0;
+#pragma unroll
+        for (int i = 0; i < PRE; ++i) own += in(i) ? 1u : 0u;
+        const uint32_t upto = wave_inclusive_scan(own), of_wave = lane63(upto);
+        if (of_wave) {
+            uint32_t at = 0;
+            if (lane == 0) at = atomicAdd(&L.n, of_wave);
+            at = uniform(at) + upto - own;
+#pragma unroll
+            for (int i = 0; i < PRE; ++i)
+                if (in(i)) L.list[at++] = ((uint64_t)b[i] << 32) | (uint32_t)pre[i];
+        }
+    };
+    auto tell_policy = [&](const Params &q) {
+        if (tid == 0) {
+            const uint32_t c = __hip_atomic_fetch_add(&q.hdr->n_need, 1u, __ATOMIC_RELAXED, RS_AGENT);
+            if (c == 0u && q.host_words)                 // the call's first such row tells the caller's policy at once
+                __hip_atomic_store(q.host_words + q.report, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+        }
+    };
+    // ---- the boundary bin, among the tokens set aside ----
+    Edge f{0u, 0u, 0u, 0ull, M96{0ull, 0u}, 0ull};
+    M96 goal{0ull, 0u};
+    bool found = false;
+    auto edge_for_all = [&]() __attribute__((always_inline)) {
+        if constexpr (!kEach) {
+            if (tid == 0) { L.one.f = f; L.one.D = D; L.one.P = P; L.one.err = err; L.one.found = found ? 1u : 0u; }
+            __syncthreads();
+            f.at = uniform(L.one.f.at); f.cnt_above = uniform(L.one.f.cnt_above); f.cnt_bin = uniform(L.one.f.cnt_bin);
+            f.sum = uniform(L.one.f.sum); f.above = uniform(L.one.f.above); f.bin_sum = uniform(L.one.f.bin_sum);
+            D = uniform(L.one.D); P = uniform(L.one.P); err = uniform(L.one.err); found = uniform(L.one.found) != 0u;
+        }
+    };
+    auto level1 = [&](bool known, bool complete) __attribute__((always_inline)) {       // known: D and err are; complete: every live token of the row has been counted
+        if (kEach || wave == 0) {
+            OctScan sc;
+            sieve_octaves(sc, L, lane);
+            if (known) P = ceil_mul(p.top_p, D);
+            else if (complete) { err = M96{0ull, 0u}; D = sc.total(); P = ceil_mul(p.top_p, D); }
+            else total();
+            // (the largest that P may be: what is listed then holds the kept set whatever the exact D is, and whether another
+            // threshold than this one comes of that is asked behind it)
+            goal = P + err;
+            found = sc.search(top_k, goal, f);
+        }
+        edge_for_all();
+    };
+    // the next digits of the boundary, while more than `most` tokens lie at or above it; tokens(fn): fn(bits of e) for this thread's
+    uint32_t lo = 0, span = 0, lv = 2;
+    auto digits = [&](uint32_t most, auto tokens) __attribute__((always_inline)) {
+#pragma unroll 1
+        for (; found && lv <= (uint32_t)kLevels && f.cnt_bin > 1u && f.cnt_above + f.cnt_bin > most; ++lv) {
+            const uint32_t dsh = level_shift(lv), exb = lo >> 23;
+            uint64_t *hist = L.lev[lv - 2u];
+            tokens([&](uint32_t e) {
+                if (e - lo <= span) atomicAdd(reinterpret_cast<unsigned long long *>(&hist[(e >> dsh) & 127u]), (unsigned long long)(kPackOne | (e & 0x7FFFFFu)));
+            });
+            __syncthreads();
+            if (kEach || wave == 0) {
+                const Edge at = f;
+                found = fine_search(lane, [&](int i) { return hist[i]; }, at, top_k, need_of(goal, f.above, exb), f);
+            }
+            edge_for_all();
+            lo |= f.at << dsh;
+            span = (1u << dsh) - 1u;
+        }
+    };
+    auto begin = [&]() __attribute__((always_inline)) { lo = f.at << 21; span = (1u << 21) - 1u; lv = 2u; };
+    // ---- the steps, and the list ----
+    bool again = p.diag != nullptr || p.e_bits != nullptr;               // with the exact D
+    bool listed = false;
+    uint32_t n_list = 0;
+    {
+        const uint32_t e_max = e_bits_of(xmax, M);
+        const float scale = 255.9f * __builtin_amdgcn_rcpf((float)max(e_max - min(e_max, from), 1u));
+        auto step_of = [&](uint32_t e) { return min((uint32_t)((float)(e - from) * scale), kSieveSteps - 1u); };
+        look_at([&](uint32_t e) { atomicAdd(&L.step[lane & (NT / 128 - 1)][step_of(e)], 1u); });
+        __syncthreads();
+        // four steps a lane, the largest first: at which of them top_k tokens are reached, as far as they fit
+        const uint32_t aim = top_k, most = aim <= (uint32_t)kWave ? (uint32_t)kWave : kSieveList;
+        uint32_t n = 0, step = 0, all = 0;
+        if (kEach || wave == 0) {
+            uint32_t c[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+            for (int k = 0; k < NT / 128; ++k) {
+                const uint4 q = reinterpret_cast<const uint4 *>(L.step[k])[63 - lane];
+                c[0] += q.w; c[1] += q.z; c[2] += q.y; c[3] += q.x;
+            }
+            const uint32_t upto = wave_inclusive_scan(c[0] + c[1] + c[2] + c[3]);
+            all = lane63(upto);
+            n = all;
+            if (all > aim) {
+                const uint32_t l = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= aim));
+                n = lane_of(upto - c[0] - c[1] - c[2] - c[3], l); step = 256u - 4u * l;
+                uint32_t more = n;
+#pragma unroll
+                for (int k = 0; k < 4; ++k) {
+                    more += lane_of(c[k], l);
+                    if (n < aim && more <= most) { n = more; step = 255u - 4u * l - (uint32_t)k; }
+                    else if (n < aim) break;
+                }
+            }
+        }
+        if constexpr (!kEach) {
+            if (tid == 0) { L.one.f.at = n; L.one.f.cnt_above = step; L.one.f.cnt_bin = all; }
+            __syncthreads();
+            n = uniform(L.one.f.at); step = uniform(L.one.f.cnt_above); all = uniform(L.one.f.cnt_bin);
+        }
+        // (short of top_k, it may still be P)
+        listed = n != 0u && n <= most && (n >= top_k || n == all || p.top_p < 1.0f);
+        if (listed) {
+            list_them([&](int i) { return b[i] != 0u && step_of(b[i]) >= step; });
+            n_list = n;
+            if (n > (uint32_t)kWave) clear_bins();
+        }
+        __syncthreads();
+        if (listed && n <= (uint32_t)kWave && !again) {
+            total();
+            const uint32_t token = from_few(L.list, n, whole && n == all, 0u), in_doubt = put(token);
+            if (__builtin_expect(in_doubt == 0u, 1)) return;
+            again = in_doubt == 1u;
+            listed = again;
+            __syncthreads();
+            if (tid == 0) L.unsure = 0u;
+            doubts = 0u;
+        }
+        if (listed && n > (uint32_t)kWave) {
+            for (uint32_t i = (uint32_t)tid; i < n; i += NT) {
+                const uint32_t e = (uint32_t)(L.list[i] >> 32);
+                atomicAdd(reinterpret_cast<unsigned long long *>(&L.bins[lane & (kSieveCopies - 1)][e >> 21]), (unsigned long long)(kPackOne | (e & 0x7FFFFFu)));
+            }
+            __syncthreads();
+            level1(false, whole && n == all);
+            listed = found;
+            begin();
+        }
+    }
+    if (__builtin_expect(!listed, 0)) {
+        // all tokens set aside, by their bins
+        __syncthreads();
+        ask();
+        clear_bins();
+        if (tid == 0) L.n = 0u;
+        __syncthreads();
+        to_bins();
+        __syncthreads();
+        level1(false, whole);
+        listed = found;
+        if (found) {
+            begin();
+            // a list so long that another kernel is faster (the host's rule): said to the caller's policy
+            if (f.cnt_above + f.cnt_bin > min(p.long_list, p.tell_lists ? max(2048u, 3u * top_k) : 0xFFFFFFFFu)) tell_policy(params_again());
+            digits(kSieveList, [&](auto fn) {
+#pragma unroll
+                for (int i = 0; i < PRE; ++i) fn(b[i]);
+            });
+            n_list = f.cnt_above + f.cnt_bin;
+            listed = found && n_list <= kSieveList;
+        }
+        if (listed) list_them([&](int i) { return b[i] >= lo; });
+        __syncthreads();
+        if (__builtin_expect(!listed, 0)) {
+            // One tie of all the row's tokens (rows of equal logits): every token weighs the tie weight, and the token at which the running sum
+            // reaches r follows by division.
+            const Params q = params_again();
+            const uint64_t rand64 = q.inj_u ? 0ull : L.rand64;
+            const bool tie = !mine || ((h.y & kSieveTie) && h.x == kmax);
+            const uint64_t not_all = __builtin_amdgcn_ballot_w64(!tie);
+            if (lane == 0) L.flag[wave] = not_all != 0ull ? 1u : 0u;
+            __syncthreads();
+            uint32_t differ = 0;
+            for (int w = 0; w < W; ++w) differ |= L.flag[w];
+            if (uniform(differ) == 0u) {
+                const uint32_t emax = e_bits_of(xmax, M);
+                if (q.e_bits)
+                    for (uint32_t i = (uint32_t)tid; i < (uint32_t)q.V >> 2; i += NT)
+                        reinterpret_cast<uint4 *>(q.e_bits + (int64_t)row * q.V)[i] = make_uint4(emax, emax, emax, emax);
+                if (tid == 0) {
+                    const u128 all = (u128)w_of_bits(emax) * (uint32_t)q.V;
+                    const Target tg = tie_and_target(q, row, rand64, xmax, all, ceil_mul(q.top_p, all), emax, 0u, (uint32_t)q.V, (u128)0, 0u, true);
+                    uint32_t lo_i = 0, hi_i = (uint32_t)q.V - 1u;                  // smallest i with (i + 1) * w_tie >= r; r <= V * w_tie
+                    while (lo_i < hi_i) {
+                        const uint32_t mid = (lo_i + hi_i) >> 1;
+                        if ((u128)(mid + 1u) * tg.w_tie >= tg.r) hi_i = mid; else lo_i = mid + 1u;
+                    }
+                    q.out[row] = (int32_t)lo_i;
+                    if (q.diag) q.diag[row].index = (int32_t)lo_i;
+                }
+                return;
+            }
+        }
+    }
+    // ---- threshold and token from the list; a decision too close to call is made again with the row's exact total ----
+    bool tell = false;
+    for (;; again = true) {
+        auto from_list = [&](auto fn) {
+            for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) fn((uint32_t)(L.list[i] >> 32));
+        };
+        if (__builtin_expect(again || !listed, 0)) {
+            const bool close = listed && !p.diag && !p.e_bits;
+            D = close ? sieve_closer<NT>(params_again(), L, row, M) : sieve_exact<NT>(params_again(), L, row, M);
+            err = close ? M96{(D.lo >> 38) | ((uint64_t)D.hi << 26), 0u} + M96{1ull << 24, 0u} : M96{0ull, 0u};
+            if (!listed) {
+                // the tokens set aside were not enough, or more than the list holds: the row's own bins, and its tokens at or above the boundary bin
+                tell = true;
+                __syncthreads();
+                level1(true, false);
+                n_list = f.cnt_above + f.cnt_bin;
+                if (!found || n_list > kSieveList) break;
+                const uint32_t edge = f.at << 21;
+                if (tid == 0) L.n = 0u;
+                __syncthreads();
+                sieve_row_pass<NT>(params_again(), row, M, [&](uint32_t i4, const uint4 e) {
+                    auto take = [&](uint32_t w, uint32_t q) {
+                        if (w < edge) return;
+                        const uint32_t o = atomicAdd(&L.n, 1u);
+                        if (o < kSieveList) L.list[o] = ((uint64_t)w << 32) | (i4 * 4u + q);
+                    };
+                    take(e.x, 0u); take(e.y, 1u); take(e.z, 2u); take(e.w, 3u);
+                });
+                listed = true;
+            }
+            __syncthreads();                             // (the bins have been looked at)
+            clear_bins();
+            if (tid == 0) { L.few_n = 0u; L.unsure = 0u; }
+            doubts = 0u;
+            __syncthreads();
+            from_list([&](uint32_t e) {
+                atomicAdd(reinterpret_cast<unsigned long long *>(&L.bins[lane & (kSieveCopies - 1)][e >> 21]), (unsigned long long)(kPackOne | (e & 0x7FFFFFu)));
+            });
+            __syncthreads();
+            level1(true, false);
+            begin();
+            again = true;
+        }
+        if (__builtin_expect(!found, 0)) break;
+        digits((uint32_t)kWave, from_list);
+        if (__builtin_expect(!found, 0)) break;
+        const uint32_t n = f.cnt_above + f.cnt_bin;
+        uint32_t token = 0;                              // of the wave that finds it, in one lane: the sampled token + 1
+        if (n <= (uint32_t)kWave) {
+            // ---- a short list ----
+            const uint64_t *list = L.list;
+            if (n_list > (uint32_t)kWave) {
+                for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) {
+                    const uint64_t e = L.list[i];
+                    if ((uint32_t)(e >> 32) >= lo) {
+                        const uint32_t o = atomicAdd(&L.few_n, 1u);
+                        if (o < (uint32_t)kWave) L.small[o] = e;
+                    }
+                }
+                __syncthreads();
+                list = L.small;
+            }
+            token = from_few(list, n_list > (uint32_t)kWave ? n : n_list, false, 0u);
+        } else {
+            // ---- a longer one ----
+            if (span != 0u) {                            // a single token left in the range: the threshold itself
+                from_list([&](uint32_t e) { if (e - lo <= span) L.thr = e; });
+                __syncthreads();
+                lo = uniform(L.thr);
+            }
+            const uint32_t thr = lo;
+            uint64_t w_tie = 0;
+            M96 r{0ull, 0u}, shift{0ull, 0u};
+            if (kEach || wave == 0) {
+                const M96 above = f.above + mass_of(f.sum, thr >> 23);
+                const Target tg = tie_and_target(p, row, uniform(L.rand64), xmax, wide(D), wide(P), thr, f.cnt_above, f.cnt_bin, wide(above), 0u, tid == 0);
+                w_tie = uniform(tg.w_tie); r = uniform(m96(tg.r));
+                const Doubt d = doubt_of(P, err, top_k, f.cnt_above, f.cnt_bin, above, thr, w_tie);
+                shift = d.shift;
+                doubts = d.unsure ? 1u : 0u;
+            }
+            if constexpr (!kEach) {
+                if (tid == 0) { L.one.w_tie = w_tie; L.one.r = r; L.one.shift = shift; }
+                __syncthreads();
+                w_tie = uniform(L.one.w_tie); r = uniform(L.one.r); shift = uniform(L.one.shift);
+            }
+            // the pick: kept weights by bucket of the token index, NT buckets a step, then the bucket's tokens
+            auto weight = [=](uint32_t e) -> uint64_t { return e > thr ? w_of_bits(e) : e == thr ? w_tie : 0ull; };
+            constexpr uint32_t kLogNT = NT == 256 ? 8u : 10u;
+            uint32_t sh = 32u - (uint32_t)__builtin_clz((uint32_t)p.V - 1u | 1u);
+            sh = sh > kLogNT ? sh - kLogNT : 0u;
+            uint32_t lo_idx = 0, len = (uint32_t)p.V;
+            for (;;) {
+                for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) {
+                    const uint64_t e = L.list[i];
+                    const uint32_t off = (uint32_t)e - lo_idx;
+                    if ((uint32_t)(e >> 32) >= thr && off < len) {
+                        const uint64_t w = weight((uint32_t)(e >> 32));
+                        atomicAdd(reinterpret_cast<unsigned long long *>(&L.blo[off >> sh]), (unsigned long long)(w & 0xFFFFFFFFull));
+                        atomicAdd(reinterpret_cast<unsigned long long *>(&L.bhi[off >> sh]), (unsigned long long)(w >> 32));
+                    }
+                }
+                __syncthreads();
+                const M96 own = m96((u128)L.blo[tid] + ((u128)L.bhi[tid] << 32));
+                L.blo[tid] = 0ull; L.bhi[tid] = 0ull;
+                if (tid == 0) L.few_n = 0u;
+                M96 inc = m96(wave_inclusive_scan(limbs(own)));
+                if (lane == kWave - 1) L.mass[wave] = inc;
+                __syncthreads();
+                {
+                    const Limbs tot = wave_inclusive_scan(limbs(lane < W ? L.mass[lane] : M96{0ull, 0u}));
+                    if (wave) inc = inc + m96(lane_of(tot, (uint32_t)wave - 1u));
+                }
+                const M96 exc = inc - own;
+                if (exc < r && inc >= r) { L.bucket = (uint32_t)tid; L.one.r = r - exc; }
+                __syncthreads();
+                lo_idx += uniform(L.bucket) << sh; len = 1u << sh;
+                r = uniform(L.one.r);
+                for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) {
+                    const uint64_t e = L.list[i];
+                    if ((uint32_t)(e >> 32) >= thr && (uint32_t)e - lo_idx < len) {
+                        const uint32_t o = atomicAdd(&L.few_n, 1u);
+                        if (o < (uint32_t)kWave) L.small[o] = e;
+                    }
+                }
+                __syncthreads();
+                const uint32_t ns = uniform(L.few_n);
+                if (ns <= (uint32_t)kWave) {
+                    if (wave == 0) {
+                        const uint64_t e = L.small[min((uint32_t)lane, ns - 1u)];
+                        uint32_t rank = 0;
+#pragma unroll 4
+                        for (uint32_t j = 0; j < ns; ++j) rank += (uint32_t)L.small[j] < (uint32_t)e ? 1u : 0u;
+                        if ((uint32_t)lane < ns) { L.few.w[rank] = weight((uint32_t)(e >> 32)); L.few.idx[rank] = (uint32_t)e; }
+                        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                        const Limbs one = limbs(M96{(uint32_t)lane < ns ? L.few.w[lane] : 0ull, 0u}), run = wave_inclusive_scan(one);
+                        const M96 up = m96(run), bef = m96(run - one);
+                        if ((uint32_t)lane < ns && bef < r && up >= r) {
+                            token = L.few.idx[lane] + 1u;
+                            if (!pick_is_sure(shift, bef, up, r, false, false)) doubts = 1u;
+                        }
+                    }
+                    break;
+                }
+                sh = sh > kLogNT ? sh - kLogNT : 0u;
+                __syncthreads();
+            }
+        }
+        const uint32_t in_doubt = put(token);
+        if (__builtin_expect(in_doubt == 0u, 1)) {
+            if (tell) tell_policy(params_again());
+            return;
+        }
+        if (in_doubt != 1u || again) break;              // (a list that is too short after all)
+    }
+    // Thousands of tokens in the boundary bin: the slow way.
+    {
+        const Params q = params_again();
+        const uint64_t rand64 = q.inj_u ? 0ull : L.rand64;
+        __syncthreads();
+        if (NT > kThreads && tid >= kThreads) return;
+        __syncthreads();                                 // the LDS is given over
+        finish_row_slow(q, u.slow.s, u.slow.t, row, xmax, rand64);
+        tell_policy(q);
+    }
+}
+
+}  // namespace rs

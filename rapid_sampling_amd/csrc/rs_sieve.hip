@@ -1,0 +1,36 @@
+// Instantiations and launchers of the sieve path.
+#include "rs_sieve.h"
+
+namespace rs {
+
+// The finishing workgroup's size: as launch_finish, by the units of 64 tokens that the row's slices may set aside.
+static void launch_sieve_finish(uint32_t B, hipStream_t st, const Params &p, const SieveView &v)
+{
+    const uint32_t n = v.G * v.units;
+#define RS_FIN(NTv, PREv) hipLaunchKernelGGL((sieve_finish_kernel<NTv, PREv>), dim3(B), dim3(finish_threads<NTv>()), 0, st, p, v)
+    if (n > 128u) RS_FIN(1024, 16);
+    else if (p.top_k > 256 && B <= 256u && n >= 32u) RS_FIN(1024, 8);
+    else if (n <= 16u) RS_FIN(256, 4);
+    else if (n <= 32u) RS_FIN(256, 8);
+    else if (n <= 64u) RS_FIN(256, 16);
+    else RS_FIN(256, 32);
+#undef RS_FIN
+}
+
+hipError_t launch_sieve(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v)
+{
+    const dim3 grid(B * v.G);
+    if (v.G * v.units > 256u) return hipErrorInvalidValue;               // what the finishing workgroup asks for
+#define RS_SIEVE(Rv) do {                                                                                                                \
+        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_F32>), grid, dim3(kThreads), 0, st, p, v);                 \
+        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_BF16>), grid, dim3(kThreads), 0, st, p, v);          \
+        else hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_F16>), grid, dim3(kThreads), 0, st, p, v); } while (0)
+    if (R == 16) RS_SIEVE(16);
+    else if (R == 8) RS_SIEVE(8);
+    else RS_SIEVE(4);
+#undef RS_SIEVE
+    launch_sieve_finish(B, st, p, v);
+    return hipGetLastError();
+}
+
+}  // namespace rs

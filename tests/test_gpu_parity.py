@@ -2236,3 +2236,132 @@ def test_streaming_pass_rows_that_end_within_a_slice(torch_cuda, oracle, B, V, f
         _check(res, np.tile(ref_out, reps)[:B], np.tile(ref_diag, reps)[:B], "rows of %d tokens, top_k %d" % (V, top_k), np.tile(ref_e, (reps, 1))[:B])
         assert smp.status() == 0
     smp.close()
+
+
+def _sieve_rows(V, n_kinds=12):
+    """One row of each kind that the sieve path (rs_sieve.h) may meet, its slices being up to 16384 tokens."""
+    rng = np.random.default_rng(V)
+    lg = (rng.standard_normal((n_kinds, V)) * 2.0).astype(np.float32)
+    lg[1, rng.choice(V, 16, replace=False)] += 10.0                     # a few candidates over a broad floor
+    lg[2] = rng.random(V, dtype=np.float32) * 4                         # flat
+    lg[3] = np.sort(lg[3])                                              # the largest all in the last slots
+    lg[4] = np.sin(np.arange(V, dtype=np.float32) / 300.0) * 5          # neighbours alike: groups of four all set aside
+    lg[5] = -np.inf
+    lg[5, [7, V // 2, V - 1]] = [1.0, 2.0, 1.5]                         # three live tokens
+    lg[6, rng.random(V) < 0.97] = -np.inf
+    lg[7, V // 3] = np.nan
+    lg[7, V // 5] = np.inf                                              # a NaN, an infinity
+    lg[8] = lg[8] * 15 - 300.0                                          # cold, below what needs no frame
+    lg[9] = 0.25                                                        # one tie
+    lg[10] = np.round(lg[10])                                           # ties of thousands below some of tens
+    lg[11, : V // 16] += 5.0                                            # the largest in a sixteenth of the row
+    return lg
+
+
+@pytest.mark.parametrize("V,fmt,k", [(16388, "float32", 40), (49152, "float32", 1), (50260, "bfloat16", 50), (65536, "float16", 64), (131072, "float32", 64), (131076, "bfloat16", 20),
+                                     (262148, "float32", 50), (528384, "float32", 40), (1048576, "bfloat16", 40), (65540, "float32", 100), (131072, "float32", 128),
+                                     (131072, "bfloat16", 300), (262144, "float32", 1000), (1048576, "float32", 1024)])
+def test_sieve_path(torch_cuda, oracle, V, fmt, k):
+    """The sieve path in slices of 4096, 8192 and 16384 tokens that set 64 or 128 of them aside, its short lists (top_k up to 64) and its long
+    ones: every kind of row over and over, as many as the path is taken for, tokens against the oracle without the diagnostics record -- which
+    has the finish sum every row exactly -- and with it every field, the largest and the smallest random number among them."""
+    torch = torch_cuda
+    from tests import capi
+    dt = getattr(torch, fmt)
+    lg = torch.from_numpy(_sieve_rows(V)).to(dt).float().numpy()
+    n = lg.shape[0]
+    least = 49152 if k <= 64 else 1 << 24 if k <= 128 else 1 << 25 if V <= 262144 else 1 << 26
+    B = max(n, (least + V - 1) // V)
+    reps = (B + n - 1) // n
+    B = reps * n
+    x = torch.from_numpy(lg).to(dt).cuda().repeat(reps, 1).contiguous()
+    smp = capi.Sampler(B, V)
+    for temperature, top_p in ((1.0, 0.9), (0.6, 1.0), (0.02, 0.5), (1.3, 0.3)):
+        u_np = H.uniforms(n, k + int(top_p * 100))
+        u_np[: n // 3] = [1.0, 1e-30, 0.5, 1e-7][: n // 3]
+        rc, c, kk, p = capi.normalize(temperature, k, top_p, V, B, 1)
+        ref_out, ref_diag, ref_e = oracle.sample_batch(lg, c, kk, p, injected_u=u_np, want_e=True)
+        u = torch.from_numpy(np.tile(u_np, reps)).cuda()
+        print("sieve path:", B, V, fmt, k, temperature, top_p, flush=True)
+        res = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, path="stream")
+        assert res["rc"] == 0
+        bad = np.nonzero(res["out"] != np.tile(ref_out, reps))[0]
+        assert bad.size == 0, "rows %s: %s, not %s" % (bad[:8] % n, res["out"][bad[:8]], ref_out[bad[:8] % n])
+    few = x[:n] if n * V >= least else x
+    m = few.shape[0] // n
+    res = smp.sample(few, c, kk, p, uniforms=u[: few.shape[0]], want_e=m == 1, path="stream")
+    _check(res, np.tile(ref_out, m), np.tile(ref_diag, m), "sieve path", np.tile(ref_e, (m, 1)) if m == 1 else None)
+    assert smp.status() == 0
+    smp.close()
+
+
+@pytest.mark.parametrize("V,k", [(65536, 64), (262144, 50), (1048576, 40)])
+def test_sieve_path_decisions_too_close_to_call(torch_cuda, oracle, V, k):
+    """Rows in which a decision hangs on the last bits of the row's total, which the pass knows to some 2^-21 only: one token whose weight
+    is exactly top_p of the row, or a last bit more or less, then the threshold is it or the next one; and a target at the very end of a
+    token's share.  c is 1: x is the logit, weights are powers of two."""
+    torch = torch_cuda
+    from tests import capi
+    half, n_low = 0.5, V // 2
+    octaves = int(np.log2(n_low))
+    rows = []
+    for delta in (0.0, 1e-7, -1e-7, 3e-6, -3e-6, 1e-3, -1e-3):
+        for second in (False, True):
+            r = np.full(V, -np.inf, dtype=np.float32)
+            r[V // 4: V // 4 + n_low] = 0.0                              # as heavy together as the one token
+            r[5] = octaves + delta
+            if second:
+                r[V - 3] = octaves - 20.0
+            rows.append(r)
+    lg = np.stack(rows)
+    B = lg.shape[0]
+    temperature = 1.4426950408889634
+    rc, c, kk, p = capi.normalize(temperature, k, half, V, B, 1)
+    assert c == 1.0
+    smp = capi.Sampler(B, V)
+    x = torch.from_numpy(lg).cuda()
+    for seed in range(3):
+        u_np = H.uniforms(B, seed)
+        if seed == 0:
+            u_np[:] = 1.0
+        ref_out, ref_diag = oracle.sample_batch(lg, c, kk, p, injected_u=u_np)
+        res = smp.sample(x, c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_diag=False, path="stream")
+        assert np.array_equal(res["out"], ref_out), (seed, np.nonzero(res["out"] != ref_out)[0])
+    # a kept set of equal tokens, the target within a few parts in 2^24 of every token's end
+    r = np.full((1, V), -30.0, dtype=np.float32)
+    r[0, ::V // 16] = 3.0
+    rc, c, kk, p = capi.normalize(temperature, k, 0.999, V, 64, 1)
+    ends = (np.arange(64) // 4 + 1) / 16.0 + np.array([-2.0 ** -24, 0.0, 2.0 ** -24, -2.0 ** -21])[np.arange(64) % 4]
+    u_np = np.clip(ends, 1e-9, 1.0).astype(np.float32)
+    lg = np.repeat(r, 64, axis=0)
+    ref_out, ref_diag = oracle.sample_batch(lg, c, kk, p, injected_u=u_np)
+    smp64 = capi.Sampler(64, V)
+    res = smp64.sample(torch.from_numpy(lg).cuda(), c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_diag=False, path="stream")
+    assert np.array_equal(res["out"], ref_out), np.nonzero(res["out"] != ref_out)[0]
+    assert smp.status() == 0 and smp64.status() == 0
+    smp.close()
+    smp64.close()
+
+
+def test_hardware_exponential_against_the_tokens_own(torch_cuda, oracle):
+    """What the sieve path's sums are off by rests on the hardware's 2^x being larger than e of x by 0 to 3.45 parts in 2^24.  The path is
+    asked with rows that would show twice that: one token against V - 1 equal ones at a temperature that puts them anywhere, a nucleus whose
+    bound lies within 2^-17 of the one token's share, on both sides."""
+    torch = torch_cuda
+    from tests import capi
+    V, B = 65536, 64
+    rng = np.random.default_rng(7)
+    low = (rng.random(B) * 30 - 15).astype(np.float32)
+    lg = np.repeat(low[:, None], V, axis=1).astype(np.float32)
+    lg[:, 9] = low + np.float32(16.0 * np.log(2.0)) + (rng.standard_normal(B) * 0.01).astype(np.float32)
+    smp = capi.Sampler(B, V)
+    x = torch.from_numpy(lg).cuda()
+    share = np.exp(lg[:, 9].astype(np.float64) - low) / (np.exp(lg[:, 9].astype(np.float64) - low) + V - 1)
+    for b in range(0, B, 4):
+        for off in (-2.0 ** -17, -2.0 ** -22, 0.0, 2.0 ** -22, 2.0 ** -17):
+            u_np = H.uniforms(B, b)
+            rc, c, kk, p = capi.normalize(1.0, 50, float(share[b] * (1 + off)), V, B, 1)
+            ref_out, _ = oracle.sample_batch(lg, c, kk, p, injected_u=u_np)
+            res = smp.sample(x, c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_diag=False, path="stream")
+            assert np.array_equal(res["out"], ref_out), (b, off)
+    smp.close()
