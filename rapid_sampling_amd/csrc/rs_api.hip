@@ -579,6 +579,22 @@ static uint32_t sieve_reach(int32_t V, int32_t top_k, int R, uint32_t units)
     return min((uint32_t)(128.0 * (1.0 - exp(-m / 128.0)) + 2.0 * sqrt(m) + 4.0), units == 1u ? 48u : 78u);
 }
 
+// With penalties, the histogram's pass / here (N(0,1.5), top_p 0.9, one token in a hundred penalised):
+//   rows x tokens     top_k 50        100          300         1000
+//    128 x  50304   25.3 / 19.8
+//     64 x 131072   27.5 / 22.8
+//    128 x 262144   60.2 / 56.5  61.2 / 59.3   63.7 / 67.9  68.2 / 70.4
+//    256 x 131072   54.1 / 48.1  60.9 / 59.7                               (top_k 50: bfloat16)
+//    512 x  32768   40.8 / 38.5
+//    256 x 262144                             149.1 / 111.8
+//     16 x 1048576  45.0 / 37.5
+//     64 x 1048576                            151.2 / 108.3 152.3 / 109.2
+// (1024 x 20000 55.9 / 48.1; flat rows 256 x 50304 42.4 / 29.6.)  Slices of 8192 tokens at most: a thread holds tokens and penalties.
+static int sieve_pen_r(int32_t B, int32_t V, int32_t top_k)
+{
+    return top_k > 128 && (uint64_t)B * (uint64_t)V < (1u << 26) ? 0 : min(sieve_r(B, V, top_k), 8);
+}
+
 static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pen, const rs_options *opt)
 {
     const bool bounded = top_k <= kStreamK;
@@ -586,11 +602,6 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
     if (force == RS_PATH_SHORT) return V <= kShortMaxV ? kPathShort : kPathCluster;
     if (force == RS_PATH_AUTO && !(opt && opt->slice_r) && short_suits(B, V, top_k, pen)) return kPathShort;
     if (force == RS_PATH_FUSED) return fused_r(B, V, pen, true) ? kPathFused : kPathCluster;
-    // The one-launch path by default: calls with penalties whose kept set is bounded by top_k (the
-    // general kernel, the only other way with penalties, spends most of its time in exchanges).
-    if (force == RS_PATH_AUTO && pen && bounded && fused_r(B, V, pen, false)) return kPathFused;
-    // Larger calls with penalties: the streaming pass that also writes the decayed penalties, its finish and a fix-up, three
-    // launches, from kPenStreamMin tokens on.
     rs_policy *pol = opt ? opt->policy : nullptr;
     const int cls = size_class(B, V);
     // after a call of this kind with a slow row: the general kernel for a while, then another try
@@ -616,6 +627,17 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
         retry = true;
         return false;
     };
+    // The one-launch path by default: calls with penalties whose kept set is bounded by top_k (the
+    // general kernel, the only other way with penalties, spends most of its time in exchanges).  Where the sieve path suits the call its three
+    // launches, most of it at the memory's rate, are shorter from a million tokens on, one launch / three, us a call (top_k 50):
+    //     8 x  50304 12.1 / 12.7     8 x 131072 13.3 / 12.8     1 x 1048576 16.4 / 16.7    16 x 131072 14.8 / 13.6    64 x 32768 14.3 / 14.1
+    //    64 x  50304 16.4 / 15.4    32 x 131072 17.1 / 16.1     4 x 1048576 22.0 / 19.3   128 x  50304 25.6 / 20.1    48 x 131072 24.4 / 19.0
+    const bool one_launch = force == RS_PATH_AUTO && pen && bounded && fused_r(B, V, pen, false) != 0;
+    if (one_launch && sieve_pen_r(B, V, top_k) && (uint64_t)B * (uint64_t)V >= (V <= kMidMaxV ? 1u << 20 : 1u << 21) && !(opt && opt->slice_r) &&
+        !routed_away(0)) return kPathStream;
+    if (one_launch) return kPathFused;
+    // Larger calls with penalties: the streaming pass that also writes the decayed penalties, its finish and a fix-up, three
+    // launches, from kPenStreamMin tokens on.
     if (pen && bounded && stream_parts(V, kStreamLongR) >= 2u) {
         if (force == RS_PATH_STREAM || force == RS_PATH_ATTEMPT) return kPathStream;
         if (force == RS_PATH_AUTO && (uint64_t)B * (uint64_t)V >= kPenStreamMin && !routed_away(0)) return kPathStream;
@@ -917,17 +939,27 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
     const int path = choose_path(B, V, top_k, top_p, pen, opt);
     if (path == kPathShort) return launch_short(pen, logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     if (path == kPathRow) return launch_row(logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
-    if (const int R = !pen && path == kPathStream ? sieve_r(B, V, top_k) : 0) {
+    // (with penalties: a decay that leaves +0.0 as it is)
+    if (const int R = path != kPathStream || (pen && decay - decay != 0.0f) ? 0 : pen ? sieve_pen_r(B, V, top_k) : sieve_r(B, V, top_k)) {
         SieveView v;
         v.G = stream_parts(V, R);
         v.units = sieve_share(top_k, V, R) <= 8u ? 1u : 2u;
         v.reach = sieve_reach(V, top_k, R, v.units);
         const size_t slices = (size_t)B * v.G, hdr = align256(sizeof(WsHeader)), stash = align256(hdr + slices * sizeof(SieveHdr));
-        const size_t end = align256(stash + slices * v.units * kWave * sizeof(uint64_t));
-        // (a workspace of rs_workspace_bytes has room, 0.25 bytes a token at most; one without takes the streaming path)
+        v.note_cap = sieve_pen_cap(R);
+        const size_t noted = align256(stash + slices * v.units * kWave * sizeof(uint64_t)), waves = slices * kWaves;
+        const size_t note_at = align256(noted + waves * sizeof(uint32_t)), note_old = align256(note_at + waves * v.note_cap * sizeof(uint32_t));
+        const size_t end = pen ? align256(note_old + waves * v.note_cap * sizeof(float4)) : noted;
+        // (a workspace of rs_workspace_bytes has room, 0.25 bytes a token at most, 1.1 with penalties; one without takes the streaming path)
         if (end + (size_t)B * sizeof(RowCtl) <= (workspace_bytes & ~(size_t)255)) {
-            v.hdr = (SieveHdr *)((char *)workspace + hdr); v.stash = (uint64_t *)((char *)workspace + stash);
+            char *w = (char *)workspace;
+            v.hdr = (SieveHdr *)(w + hdr); v.stash = (uint64_t *)(w + stash);
+            v.noted = (uint32_t *)(w + noted); v.note_at = (uint32_t *)(w + note_at); v.note_old = (float4 *)(w + note_old);
             p.report = (uint32_t)policy_word(0, size_class(B, V));
+            if (pen) {
+                p.defer_pen = 2;
+                return launch_sieve_pen(R, logits_dtype, (uint32_t)B, (hipStream_t)stream, p, v) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
+            }
             return launch_sieve(R, logits_dtype, (uint32_t)B, (hipStream_t)stream, p, v) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
         }
     }

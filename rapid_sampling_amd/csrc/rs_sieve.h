@@ -61,12 +61,13 @@ struct LdsSieve {
 
 // A workgroup's slice to its record.  group(j, x): the scaled logits of the thread's j-th group of four tokens, group j * 256 + tid of the
 // slice, from the registers that the loads fill; those past the end of the row, `left` groups from the slice's first, are copies of its last;
+// strange(): the thread has seen input that must be cleaned up; redo(j, x): the group again, cleaned up; then(): behind the last of these;
 // g0: the slice's first group.
 // The terms of the sum need no frame: 2^x is a float for every x in question, and so they are worked out in the order in which
 // the loads arrive.  A wave whose largest x is beyond 120 or below -80 (the tokens 40 octaves below it would no longer be floats), or
 // that holds a NaN or an infinity, does it again, cleaned up and in a frame.
-template <int R, typename G>
-__device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G group, const size_t slice, const uint32_t g0, const uint32_t left, const int tid)
+template <int R, typename G, typename Z, typename A, typename E>
+__device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G group, Z strange, A redo, E then, const size_t slice, const uint32_t g0, const uint32_t left, const int tid)
 {
     const float kInf = __builtin_inff();
     const int lane = tid & (kWave - 1), wave = (int)uniform((uint32_t)tid >> 6);
@@ -104,15 +105,13 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         }
 #pragma unroll
         for (int i = 0; i < R / 4; ++i) mass += (double)part[i];
-        odd = __builtin_amdgcn_ballot_w64(!(mass < (double)kInf) || lm > 120.0f) != 0ull || __builtin_amdgcn_ballot_w64(lm >= -80.0f) == 0ull;
+        odd = __builtin_amdgcn_ballot_w64(!(mass < (double)kInf) || lm > 120.0f || strange()) != 0ull || __builtin_amdgcn_ballot_w64(lm >= -80.0f) == 0ull;
         if (__builtin_expect(odd, 0)) {
-            // (the clean-up of sampling.cu:553 on the products in the registers)
             const uint32_t t = opaque((uint32_t)tid);
             lm = -kInf;
 #pragma unroll
             for (int j = 0; j < R; ++j) {
-#pragma unroll
-                for (int q = 0; q < 4; ++q) x[j * 4 + q] = sf(x[j * 4 + q]);
+                redo(j, &x[j * 4]);
                 gm[j] = (uint32_t)(j * kThreads) + t < left ? top(j) : -kInf;
                 lm = fmaxf(lm, gm[j]);
             }
@@ -125,6 +124,7 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
             }
         }
     }
+    then();
     s.top[tid] = lm; s.mass[tid] = mass;
     {
         const uint32_t k = wave_max_u32(fkey(lm));
@@ -279,7 +279,170 @@ __global__ void __launch_bounds__(kThreads, R == 16 ? 4 : 8) sieve_kernel(const 
         else widen4(make_uint2(l[j].x, l[j].y), DT, w);
 #pragma unroll
         for (int q = 0; q < 4; ++q) x[q] = __uint_as_float(w[q]) * p.c;
-    }, (size_t)row * v.G + part, g0, left, tid);
+    }, [] { return false; }, [](int, float *x) {
+        // (the clean-up of sampling.cu:553 on the products in the registers)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = sf(x[q]);
+    }, [] {}, (size_t)row * v.G + part, g0, left, tid);
+}
+
+// The same with penalties: x = sf((sf(l) - pen) * c) (sampling.cu:220).  The pass also writes what every penalty will be unless its token is
+// sampled, fma(pen, decay, 0), and sieve_pen_fix_kernel patches the sampled token's once it is known.  Penalties are non-zero only
+// where tokens have been generated, and a finite decay leaves +0.0 as it is: so a wave lists its groups with a bit set in one of their penalties, in
+// LDS, and writes from the list: the new values where they belong, the old ones into its notes, from which the sampled token's is looked up and a
+// row that must be read again gets its old values back.  A wave with more such groups than the list takes leaves its penalties to the fix-up kernel
+// and says so.
+//
+// What bounds it: the memory.  128 x 262144 tokens, two in a hundred penalised, inputs from HBM: 65.5 us, of which 50 are the read (the writes left out
+// of a copy of it) and 15 the lines of the penalties that change, half of all lines; written in whole groups of 64 or 128 bytes 65.0 and 68.5, with
+// non-temporal stores 67.0, with slices of 4096 tokens 66.0.  The pass with a histogram and a vote about every single penalty (stream_pen_kernel), 35
+// vector instructions a token, takes 74.
+template <int R, int DT>
+__global__ void __launch_bounds__(kThreads, R == 8 ? 4 : 6) sieve_pen_kernel(const Params p, const SieveView v)
+{
+    constexpr uint32_t kCap = sieve_pen_cap(R);
+    __shared__ LdsSieve s;
+    __shared__ float4 old[kWaves][kCap];
+    __shared__ uint32_t at[kWaves][kCap];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = (int)uniform((uint32_t)tid >> 6);
+    const uint32_t row = blockIdx.x / v.G, part = blockIdx.x - row * v.G;
+    const bool reporter = blockIdx.x == 0 && tid == 0;
+    PrevCall prev;
+    prev.slow_rows = 0; prev.meta = 0;
+    if (reporter) prev = report_begin(p);
+    const uint32_t g0 = part * (uint32_t)(R * kThreads), left = ((uint32_t)p.V >> 2) - g0;
+    typedef typename std::conditional<DT == RS_DTYPE_F32, rs_u32x4, rs_u32x2>::type T;
+    typedef const __attribute__((address_space(1))) T GlobalT;
+    typedef const __attribute__((address_space(1))) rs_u32x4 GlobalP;
+    GlobalT *from = (GlobalT *)reinterpret_cast<const T *>(logits_row(p, row)) + g0;
+    rs_u32x4 *pens = reinterpret_cast<rs_u32x4 *>(p.penalties + (int64_t)row * p.V) + g0;
+    GlobalP *pfrom = (GlobalP *)pens;
+    const bool ragged = left < (uint32_t)(R * kThreads);
+    T l[R];
+    rs_u32x4 pn[R];
+    if (!ragged) {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            GlobalT *q = from + j * kThreads;
+            GlobalP *b = pfrom + j * kThreads;
+            asm("" : "+s"(q), "+s"(b));
+            l[j] = __builtin_nontemporal_load(q + (uint32_t)tid);
+            pn[j] = b[(uint32_t)tid];
+        }
+    } else {
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            const uint32_t i = min((uint32_t)(j * kThreads + tid), left - 1u);
+            l[j] = __builtin_nontemporal_load(from + i);
+            pn[j] = pfrom[i];
+        }
+    }
+    if (reporter) report_end(p, prev, true);
+    const size_t slice = (size_t)row * v.G + part;
+    auto widen = [&](const T &t, uint32_t (&w)[4]) __attribute__((always_inline)) {
+        if constexpr (DT == RS_DTYPE_F32) { w[0] = t.x; w[1] = t.y; w[2] = t.z; w[3] = t.w; }
+        else widen4(make_uint2(t.x, t.y), DT, w);
+    };
+    uint32_t fill = 0;
+    uint32_t low = 0u;                                   // bit pattern of the most negative penalty
+    sieve_slice<R>(v, s, [&](int j, float *x) __attribute__((always_inline)) {
+        uint32_t w[4];
+        widen(l[j], w);
+        const uint32_t b[4] = {pn[j].x, pn[j].y, pn[j].z, pn[j].w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = (__uint_as_float(w[q]) - __uint_as_float(b[q])) * p.c;
+        bool any = ((b[0] | b[1] | b[2]) | b[3]) != 0u;
+        if (ragged) any = any && (uint32_t)(j * kThreads) + opaque((uint32_t)tid) < left;
+        const uint64_t vote = __builtin_amdgcn_ballot_w64(any);
+        if (vote != 0ull) {
+            const uint32_t o = fill + __builtin_amdgcn_mbcnt_hi((uint32_t)(vote >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)vote, 0u));
+            if (any && o < kCap) {
+                old[wave][o] = make_float4(__uint_as_float(b[0]), __uint_as_float(b[1]), __uint_as_float(b[2]), __uint_as_float(b[3]));
+                at[wave][o] = (uint32_t)(j * kThreads + tid);
+            }
+            fill += (uint32_t)__builtin_popcountll(vote);
+            // (a logit of -inf is the lowest float before the penalty is taken off: only with a penalty of its size, here -1e30, does it matter)
+            low = max(low, max(max(b[0], b[1]), max(b[2], b[3])));
+        }
+    }, [&] { return low > 0xF149F2CAu; }, [&](int j, float *x) __attribute__((always_inline)) {
+        const uint32_t i = min((uint32_t)(j * kThreads) + opaque((uint32_t)tid), left - 1u);
+        uint32_t w[4];
+        const T t = from[i];
+        widen(t, w);
+        const rs_u32x4 q4 = pfrom[i];
+        const uint32_t b[4] = {q4.x, q4.y, q4.z, q4.w};
+#pragma unroll
+        for (int q = 0; q < 4; ++q) x[q] = sf((sf(__uint_as_float(w[q])) - __uint_as_float(b[q])) * p.c);
+    }, [&]() __attribute__((always_inline)) {
+        const size_t mine = slice * kWaves + (size_t)wave;
+        const bool fits = fill <= kCap;
+        if (lane == 0) v.noted[mine] = fits ? fill : kSievePenLeft;
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        if (fits)
+            for (uint32_t i = (uint32_t)lane; i < fill; i += kWave) {
+                const float4 q = old[wave][i];
+                const uint32_t g = at[wave][i];
+                v.note_at[mine * kCap + i] = g0 + g;
+                v.note_old[mine * kCap + i] = q;
+                reinterpret_cast<float4 *>(pens)[g] = make_float4(__builtin_fmaf(q.x, p.decay, 0.0f), __builtin_fmaf(q.y, p.decay, 0.0f),
+                                                                  __builtin_fmaf(q.z, p.decay, 0.0f), __builtin_fmaf(q.w, p.decay, 0.0f));
+            }
+    }, slice, g0, left, tid);
+}
+
+// The sampled token's penalty, pen <- fma(pen, decay, pen == 0 ? presence : repetition) (sampling.cu:427-437), the old value from the notes
+// (+0.0 when its group is not among them), and all penalties of the waves that left theirs.  kSieveFixers workgroups to a row, each for every
+// kSieveFixers-th slice, wave w for wave w's part of them: mostly it is one look at some words and a chain of two loads for the one token (4.7 us
+// behind 128 x 262144 tokens, with 2, 8 or a workgroup per slice alike).
+template <int R>
+__global__ void __launch_bounds__(kThreads) sieve_pen_fix_kernel(const Params p, const SieveView v)
+{
+    constexpr uint32_t kCap = sieve_pen_cap(R);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = (int)uniform((uint32_t)tid >> 6);
+    const uint32_t row = blockIdx.x / kSieveFixers, first = blockIdx.x - row * kSieveFixers, G = v.G;
+    const uint32_t part = first + (uint32_t)lane * kSieveFixers;         // the lane's slice (at most 64 of them: G <= 256)
+    const uint32_t *noted = v.noted + (size_t)row * G * kWaves;
+    const uint32_t n = noted[min(part, G - 1u) * (uint32_t)kWaves + (uint32_t)wave], token = uniform((uint32_t)p.out[row]);
+    const uint32_t V4 = (uint32_t)p.V >> 2, group = token >> 2;
+    float *pens = p.penalties + (int64_t)row * p.V;
+    uint64_t to_do = __builtin_amdgcn_ballot_w64(part < G && n == kSievePenLeft);
+    // the sampled token's slice, if it is one of this workgroup's and its group this wave's, and the penalties have been written
+    const uint32_t its = group / (uint32_t)(R * kThreads), l = its / kSieveFixers;
+    if (token < (uint32_t)p.V && its - l * kSieveFixers == first && ((group >> 6) & (uint32_t)(kWaves - 1)) == (uint32_t)wave && !(to_do >> l & 1ull)) {
+        const size_t rec = (((size_t)row * G + its) * kWaves + (size_t)wave) * kCap;
+        const uint32_t have = min(lane_of(n, l), kCap);
+        constexpr uint32_t kLooks = (kCap + kWave - 1u) / kWave;
+        uint32_t is[kLooks];
+        float old[kLooks], o = 0.0f;                     // (asked for before it is known which: a chain of two loads, not of three)
+        bool mine = false;
+#pragma unroll
+        for (uint32_t u = 0; u < kLooks; ++u) {
+            const size_t i = rec + min(u * kWave + (uint32_t)lane, kCap - 1u);
+            is[u] = v.note_at[i]; old[u] = reinterpret_cast<const float *>(&v.note_old[i])[token & 3u];
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < kLooks; ++u)
+            if (u * kWave + (uint32_t)lane < have && is[u] == group) { o = old[u]; mine = true; }
+        const uint64_t found = __builtin_amdgcn_ballot_w64(mine);
+        if (found ? mine : lane == 0) pens[token] = __builtin_fmaf(o, p.decay, o == 0.0f ? p.presence : p.repetition);
+    }
+    while (to_do) {
+        const uint32_t at = first + (uint32_t)__builtin_ctzll(to_do) * kSieveFixers;
+        to_do &= to_do - 1ull;
+        float4 w[R];
+        uint32_t g[R];
+#pragma unroll
+        for (int j = 0; j < R; ++j) {
+            g[j] = at * (uint32_t)(R * kThreads) + (uint32_t)(j * kThreads + tid);
+            w[j] = reinterpret_cast<const float4 *>(pens)[min(g[j], V4 - 1u)];
+        }
+#pragma unroll
+        for (int j = 0; j < R; ++j)
+            if (g[j] < V4) {
+                auto next = [&](float o, uint32_t i) { return __builtin_fmaf(o, p.decay, g[j] * 4u + i != token ? 0.0f : o == 0.0f ? p.presence : p.repetition); };
+                reinterpret_cast<float4 *>(pens)[g[j]] = make_float4(next(w[j].x, 0u), next(w[j].y, 1u), next(w[j].z, 2u), next(w[j].w, 3u));
+            }
+    }
 }
 
 // ---- the finish ----
@@ -354,10 +517,8 @@ __device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t r
     const char *lrow = logits_row(p, row);
     const bool far = !(__builtin_fabsf(M) <= 100.0f);
     const Frame fr(far ? 0 : (int)M);
-    auto e = [&](uint32_t l) {
-        const float x = sf(__uint_as_float(l) * p.c);
-        return fr.raw(far ? fmaxf(x - M, -1000.0f) : x);
-    };
+    auto e = [&](float x) { return fr.raw(far ? fmaxf(x - M, -1000.0f) : x); };
+    const uint4 *pens = p.penalties ? reinterpret_cast<const uint4 *>(p.penalties + (int64_t)row * p.V) : nullptr;
     constexpr int kAhead = 8;
 #pragma unroll 1
     for (uint32_t base = threadIdx.x; base < V4; base += kAhead * NT) {
@@ -376,9 +537,18 @@ __device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t r
                 l[u] = make_uint4(w[0], w[1], w[2], w[3]);
             }
         }
+        if (pens) {
+            uint4 q[kAhead];
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) q[u] = pens[min(base + (uint32_t)(u * NT), V4 - 1u)];
+            auto less = [&](uint32_t &w, uint32_t pen) { w = __float_as_uint(sf(__uint_as_float(w)) - __uint_as_float(pen)); };
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) { less(l[u].x, q[u].x); less(l[u].y, q[u].y); less(l[u].z, q[u].z); less(l[u].w, q[u].w); }
+        }
+        auto x = [&](uint32_t w) { return sf(__uint_as_float(w) * p.c); };
 #pragma unroll
         for (int u = 0; u < kAhead; ++u)
-            if (base + (uint32_t)(u * NT) < V4) fn(base + (uint32_t)(u * NT), make_uint4(e(l[u].x), e(l[u].y), e(l[u].z), e(l[u].w)));
+            if (base + (uint32_t)(u * NT) < V4) fn(base + (uint32_t)(u * NT), make_uint4(e(x(l[u].x)), e(x(l[u].y)), e(x(l[u].z)), e(x(l[u].w))));
     }
 }
 
@@ -421,6 +591,25 @@ __device__ __forceinline__ M96 sieve_exact(const Params &p, LdsSieveFin<NT> &L, 
     OctScan sc;
     sieve_octaves(sc, L, lane);
     return sc.total();
+}
+
+// The old penalties of a row that is read again, from the notes; its waves then all count as having left theirs to the fix-up kernel.
+template <int NT>
+__device__ __forceinline__ void sieve_pens_back(const Params &p, const SieveView &v, const uint32_t row)
+{
+    if (!p.penalties) return;
+    const int tid = threadIdx.x;
+    float4 *pens = reinterpret_cast<float4 *>(p.penalties + (int64_t)row * p.V);
+    const size_t first = (size_t)row * v.G * kWaves;
+    for (uint32_t w = 0; w < v.G * (uint32_t)kWaves; ++w) {
+        const uint32_t n = v.noted[first + w];
+        if (n != kSievePenLeft)
+            for (uint32_t i = (uint32_t)tid; i < min(n, v.note_cap); i += NT) pens[v.note_at[(first + w) * v.note_cap + i]] = v.note_old[(first + w) * v.note_cap + i];
+    }
+    __syncthreads();
+    for (uint32_t w = (uint32_t)tid; w < v.G * (uint32_t)kWaves; w += NT) v.noted[first + w] = kSievePenLeft;
+    wait_vmem();
+    __syncthreads();
 }
 
 // NT threads (256 and a wave that draws the random number, or 1024), PRE units to a wave.
@@ -800,6 +989,7 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
             for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) fn((uint32_t)(L.list[i] >> 32));
         };
         if (__builtin_expect(again || !listed, 0)) {
+            sieve_pens_back<NT>(params_again(), v, row);
             const bool close = listed && !p.diag && !p.e_bits;
             D = close ? sieve_closer<NT>(params_again(), L, row, M) : sieve_exact<NT>(params_again(), L, row, M);
             err = close ? M96{(D.lo >> 38) | ((uint64_t)D.hi << 26), 0u} + M96{1ull << 24, 0u} : M96{0ull, 0u};
@@ -952,6 +1142,7 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
     {
         const Params q = params_again();
         const uint64_t rand64 = q.inj_u ? 0ull : L.rand64;
+        sieve_pens_back<NT>(q, v, row);
         __syncthreads();
         if (NT > kThreads && tid >= kThreads) return;
         __syncthreads();                                 // the LDS is given over

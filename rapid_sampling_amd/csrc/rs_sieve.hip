@@ -33,4 +33,21 @@ hipError_t launch_sieve(int R, int32_t dtype, uint32_t B, hipStream_t st, const 
     return hipGetLastError();
 }
 
+hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v)
+{
+    const dim3 grid(B * v.G);
+    if (v.G * v.units > 256u || (R != 4 && R != 8) || v.note_cap != sieve_pen_cap(R)) return hipErrorInvalidValue;
+#define RS_SIEVE(Rv) do {                                                                                                                     \
+        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F32>), grid, dim3(kThreads), 0, st, p, v);                  \
+        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_BF16>), grid, dim3(kThreads), 0, st, p, v);           \
+        else hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F16>), grid, dim3(kThreads), 0, st, p, v); } while (0)
+    if (R == 8) RS_SIEVE(8);
+    else RS_SIEVE(4);
+#undef RS_SIEVE
+    launch_sieve_finish(B, st, p, v);
+    if (R == 8) hipLaunchKernelGGL((sieve_pen_fix_kernel<8>), dim3(B * kSieveFixers), dim3(kThreads), 0, st, p, v);
+    else hipLaunchKernelGGL((sieve_pen_fix_kernel<4>), dim3(B * kSieveFixers), dim3(kThreads), 0, st, p, v);
+    return hipGetLastError();
+}
+
 }  // namespace rs

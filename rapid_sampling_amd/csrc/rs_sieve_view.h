@@ -19,9 +19,19 @@ struct SieveView {
     uint32_t  G;             // slices per row
     uint32_t  units;         // a slice sets aside at most 64 tokens (1) or 128 (2)
     uint32_t  reach;         // pairs of threads, of a slice's 128, whose largest token is set aside
+    // calls with penalties: the groups of four of which one penalty's bit pattern is not +0.0, as they were
+    uint32_t *noted;         // [B][G][4]            how many a wave has noted, or kSievePenLeft
+    uint32_t *note_at;       // [B][G][4][note_cap]  which groups of the row
+    float4   *note_old;      // [B][G][4][note_cap]  their penalties
+    uint32_t  note_cap;      // sieve_pen_cap of the slices' length
 };
+constexpr uint32_t kSievePenLeft = 0xFFFFFFFFu;          // the wave's penalties are still the old ones: to be rewritten by the fix-up kernel
+constexpr uint32_t kSieveFixers = 8;                      // workgroups of the fix-up kernel to a row
+// Of a wave's 64 R groups, 3 in 16: 4 to 5 % of the tokens by chance, or 19 % side by side.
+__host__ __device__ constexpr uint32_t sieve_pen_cap(int R) { return 12u * (uint32_t)R; }
 
-// R: groups of four tokens of a lane, 4, 8 or 16: slices of 256 R tokens
+// R: groups of four tokens of a thread, 4, 8 or 16: slices of 1024 R tokens; with penalties 4 or 8
+hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v);
 hipError_t launch_sieve(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v);
 
 }  // namespace rs

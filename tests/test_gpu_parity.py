@@ -2365,3 +2365,47 @@ def test_hardware_exponential_against_the_tokens_own(torch_cuda, oracle):
             res = smp.sample(x, c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_diag=False, path="stream")
             assert np.array_equal(res["out"], ref_out), (b, off)
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,fmt,k", [(24, 16388, "float32", 40), (12, 50260, "bfloat16", 64), (36, 131072, "float32", 1), (12, 262148, "float16", 50),
+                                       (12, 1048576, "float32", 50), (132, 131076, "float32", 100), (72, 1048572, "float32", 300)])
+def test_sieve_path_with_penalties(torch_cuda, oracle, B, V, fmt, k):
+    """The sieve path with penalties, slices of 4096 and 8192 tokens: rows of every kind with none, few, scattered, many and only non-zero
+    penalties, a stretch of them, and infinities, NaN, -0.0 and the lowest floats among them; tokens and penalties against the oracle, without the
+    diagnostics record -- the pass writes the penalties, the fix-up kernel the sampled token's and the waves' with too many of them -- and with
+    it, for which the finish plays the old penalties back.  Then by itself, where the one-launch path gives way to it."""
+    torch = torch_cuda
+    from tests import capi
+    dt = getattr(torch, fmt)
+    lg = torch.from_numpy(_sieve_rows(V)).to(dt).float().numpy()
+    n = lg.shape[0]
+    rng = np.random.default_rng(V + k)
+    pen = rng.exponential(1.0, (n, V)).astype(np.float32)
+    share = np.array([0.0, 0.001, 0.02, 0.05, 0.3, 1.0, 0.01, 0.02, 0.02, 0.02, 0.02, 0.01])
+    pen *= rng.random((n, V)) < share[:, None]
+    pen[2, : V // 16] = 0.5                                             # a stretch
+    pen[1, 77] = -0.0
+    pen[7, [3, 5000, V - 2]] = [np.inf, -np.inf, np.nan]
+    pen[6, 100:4000:50] = -3.4e38                                       # some of their logits are -inf
+    pen[11, 9] = 3.4e38
+    reps = B // n
+    x = torch.from_numpy(lg).to(dt).cuda().repeat(reps, 1).contiguous()
+    u_np = H.uniforms(n, k)
+    u_np[:3] = [1.0, 1e-30, 0.5]
+    u = torch.from_numpy(np.tile(u_np, reps)).cuda()
+    smp = capi.Sampler(B, V)
+    for temperature, top_p in ((1.0, 0.9), (0.6, 1.0), (1.3, 0.3)):
+        rc, c, kk, p = capi.normalize(temperature, k, top_p, V, B, 1)
+        want = pen.copy()
+        ref_out, ref_diag = oracle.sample_batch(lg, c, kk, p, injected_u=u_np, penalties=want, presence=0.1, repetition=0.2, decay=0.95)[:2]
+        for path, diag in (("stream", False), ("stream", True), ("auto", False)):
+            print("sieve path with penalties:", B, V, fmt, k, temperature, top_p, path, diag, flush=True)
+            have = torch.from_numpy(np.tile(pen, (reps, 1))).cuda()
+            res = smp.sample(x, c, kk, p, uniforms=u, penalties=have, presence=0.1, repetition=0.2, decay=0.95, want_diag=diag, path=path)
+            assert res["rc"] == 0 and smp.status() == 0
+            if diag:
+                _check(res, np.tile(ref_out, reps), np.tile(ref_diag, reps), "sieve path with penalties")
+            assert np.array_equal(res["out"], np.tile(ref_out, reps)), np.nonzero(res["out"] != np.tile(ref_out, reps))
+            bad = np.argwhere(have.cpu().numpy().view(np.uint32) != np.tile(want, (reps, 1)).view(np.uint32))
+            assert bad.size == 0, bad[:8]
+    smp.close()
