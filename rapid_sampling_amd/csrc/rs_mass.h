@@ -258,25 +258,25 @@ struct LdsFew {
 // of the workgroup together (more may call; all meet at its barrier); one wave does it alone when there are few tokens.  Each token is
 // compared with every other: its place by falling e, where one scan finds the threshold, and its place by index, where
 // another finds the sampled token.  Returns that token + 1 in one lane of wave 0, 0 elsewhere.
-// D and P are those of `totals(mass of the whole list)`; `look` is told by wave 0, in every lane, what was decided: the call's D and P, whether the list
-// is enough, tokens above the threshold and at it, the threshold, the mass above it, tie weight and target, the running sum before the lane's
-// token and with it, and whether that is the sampled one.
+// D and P are those of `totals(mass of the whole list)`.  Unless they are LooksAtNothing, `decided` and `picked` are told the outcome: decided() by the second wave,
+// which works it out for itself while the first goes on to the token -- the call's P, whether the list is enough, tokens above the threshold and at
+// it, the threshold, the mass above it, the tie weight -- and picked() in the sampled token's lane, by how much the target may move either way
+// against the running sum.
 struct Totals { M96 D, P; };
-struct LooksAtNothing {
-    template <typename... A> __device__ __forceinline__ void operator()(const A &...) const {}
-};
-template <typename T, typename F = LooksAtNothing>
+struct LooksAtNothing {};
+template <typename T, typename F = LooksAtNothing, typename K = LooksAtNothing>
 __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const uint32_t row, const int lane, const int wave, const uint64_t *list,
                                              const uint32_t n, const uint32_t top_k, T totals, const float xmax,
-                                             const uint64_t *rand64, const uint32_t rounds, F look = F())
+                                             const uint64_t *rand64, const uint32_t rounds, F decided = F(), K picked = K())
 {
+    constexpr bool kLook = !std::is_same<F, LooksAtNothing>::value;
     const uint64_t e = list[min((uint32_t)lane, n - 1u)];
     const bool split = n > 16u, in = (uint32_t)lane < n;
     uint32_t larger = 0, before = 0;
-    if (wave < (split ? 4 : 1)) {
-        const uint32_t each = split ? (n + 3u) >> 2 : n, j1 = min(n, ((uint32_t)wave + 1u) * each);
+    if (wave < (split ? 4 : kLook ? 2 : 1)) {
+        const uint32_t each = split ? (n + 3u) >> 2 : n, j0 = split ? (uint32_t)wave * each : 0u, j1 = min(n, j0 + each);
 #pragma unroll 4
-        for (uint32_t j = (uint32_t)wave * each; j < j1; ++j) {
+        for (uint32_t j = j0; j < j1; ++j) {
             const uint64_t o = list[j];
             larger += o > e ? 1u : 0u;                   // (equal e: the larger index first)
             before += (uint32_t)o < (uint32_t)e ? 1u : 0u;
@@ -284,12 +284,12 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
         if (split) s.part[wave][lane] = larger | before << 16;
     }
     if (split) __syncthreads();
-    if (wave != 0) return 0u;
+    if (wave > (kLook ? 1 : 0)) return 0u;
     if (split) {
         const uint32_t c = s.part[0][lane] + s.part[1][lane] + s.part[2][lane] + s.part[3][lane];
         larger = c & 0xFFFFu; before = c >> 16;
     }
-    if (in) s.sorted[larger] = e;
+    if (in) s.sorted[larger] = e;                        // (two waves: the same words)
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const uint32_t b = in ? (uint32_t)(s.sorted[lane] >> 32) : 0u;
     const Limbs own = limbs(M96{in ? w_of_bits(b) : 0ull, 0u}), upto = wave_inclusive_scan(own);
@@ -300,7 +300,10 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     const uint32_t n_gt = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b > thr));
     const uint32_t n_eq = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b == thr));
     const M96 above = m96(lane_of(upto - own, n_gt));
-    const Target tg = tie_and_target(p, row, uniform(*rand64), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(above), rounds, lane == 0);
+    const Target tg = tie_and_target(p, row, uniform(*rand64), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(above), rounds, lane == 0 && wave == 0);
+    if constexpr (kLook) {
+        if (wave != 0) { decided(P, enough != 0ull, n_gt, n_eq, thr, above, tg.w_tie); return 0u; }
+    }
     const M96 r = m96(tg.r);
     if (in) {
         const uint32_t be = (uint32_t)(e >> 32);
@@ -311,7 +314,15 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     const Limbs mine = limbs(M96{in ? s.w[lane] : 0ull, 0u}), run = wave_inclusive_scan(mine);
     const M96 bef = m96(run - mine), with = m96(run);
     const bool is_it = in && bef < r && with >= r;
-    look(t, enough != 0ull, n_gt, n_eq, thr, above, tg, bef, with, is_it);
+    if constexpr (kLook) {
+        if (is_it) {
+            M96 less = r - bef - M96{1ull, 0u}, more = with - r;
+            if (!(bef.lo | bef.hi)) { less.lo = ~0ull; less.hi = ~0u; }                      // (the first kept token)
+            if (with >= m96(lane_of(run, 63u))) { more.lo = ~0ull; more.hi = ~0u; }          // (the last)
+            const bool m = more >= less;
+            picked(M96{m ? less.lo : more.lo, m ? less.hi : more.hi});
+        }
+    }
     return is_it ? s.idx[lane] + 1u : 0u;
 }
 

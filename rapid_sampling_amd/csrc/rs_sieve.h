@@ -458,10 +458,10 @@ struct LdsSieveFin {
     uint64_t list[kSieveList], small[kWave];             // bits of e << 32 | index
     uint64_t blo[NT], bhi[NT];                           // kept weights by bucket of the token index, halves summed apart
     M96      mass[16];
-    struct { M96 D, P, r, err, shift; Edge f; uint64_t w_tie; uint32_t found; } one;  // what one wave worked out for all
+    struct { M96 D, P, r, err, shift, slack; Edge f; uint64_t w_tie; uint32_t found; } one;  // what one wave worked out for all
     uint64_t sum[16];
     uint64_t rand64;
-    uint32_t wmax[16], wcut[16], flag[16];
+    uint32_t flag[16];
     uint32_t n, few_n, thr, bucket, unsure;
 };
 
@@ -509,7 +509,7 @@ __device__ __forceinline__ void sieve_octaves(OctScan &sc, L &l, const int lane)
     });
 }
 
-// fn(group of four, bits of their e) over the row, from the logits (x by the definition, sampling.cu:553), eight loads in flight per thread.
+// fn(group of four, bits of their e) over the row, from the logits (x by the definition, sampling.cu:553), eight loads in flight per thread, or four of 1024 threads.
 template <int NT, typename F>
 __device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t row, const float M, F fn)
 {
@@ -519,7 +519,7 @@ __device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t r
     const Frame fr(far ? 0 : (int)M);
     auto e = [&](float x) { return fr.raw(far ? fmaxf(x - M, -1000.0f) : x); };
     const uint4 *pens = p.penalties ? reinterpret_cast<const uint4 *>(p.penalties + (int64_t)row * p.V) : nullptr;
-    constexpr int kAhead = 8;
+    constexpr int kAhead = NT == kThreads ? 8 : 4;
 #pragma unroll 1
     for (uint32_t base = threadIdx.x; base < V4; base += kAhead * NT) {
         uint4 l[kAhead];                                 // (the format is asked once a round: a branch about every load waits for it)
@@ -691,6 +691,10 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
     const uint32_t sl = (uint32_t)(wave + W * lane) >> (v.units - 1u), half = (uint32_t)(wave + W * lane) & (v.units - 1u), GU = G * v.units;
     const uint64_t *stash = v.stash + (size_t)row * GU * kWave;
     const bool mine = lane < PRE && sl < G;
+    constexpr int kHdrs = PRE * W > kWave ? 2 : 1;       // (128 slices at most)
+    uint4 keys[kHdrs];
+#pragma unroll
+    for (int k = 0; k < kHdrs; ++k) keys[k] = *reinterpret_cast<const uint4 *>(&hdrs[min((uint32_t)(lane + k * kWave), G - 1u)]);
     uint4 h = *reinterpret_cast<const uint4 *>(&hdrs[min(sl, G - 1u)]);
     uint64_t pre[PRE];                                   // (units beyond the row's read its last one again)
     auto ask = [&]() __attribute__((always_inline)) {
@@ -706,16 +710,13 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
     };
     for (int i = tid; i < NT / 128 * (int)kSieveSteps; i += NT) (&L.step[0][0])[i] = 0u;
     if (tid == 0) { L.n = 0u; L.few_n = 0u; L.unsure = 0u; }
+    // the row's largest token and largest bound, every wave from all headers, behind a bare barrier: what has been asked for need not have arrived
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     if (!mine) h = make_uint4(0u, 0u, 0u, 0u);
-    {
-        const uint32_t a = wave_max_u32(h.x), b = wave_max_u32(h.z);
-        if (lane == 0) { L.wmax[wave] = a; L.wcut[wave] = b; }
-    }
-    __syncthreads();
-    uint32_t kmax = L.wmax[0], kcut = L.wcut[0];
+    uint32_t kmax = keys[0].x, kcut = keys[0].z;
 #pragma unroll
-    for (int w = 1; w < W; ++w) { kmax = max(kmax, L.wmax[w]); kcut = max(kcut, L.wcut[w]); }
-    kmax = uniform(kmax); kcut = uniform(kcut);
+    for (int k = 1; k < kHdrs; ++k) { kmax = max(kmax, keys[k].x); kcut = max(kcut, keys[k].z); }
+    kmax = wave_max_u32(kmax); kcut = wave_max_u32(kcut);
     if (!kEach && draws) draw();
     const float xmax = fkey_inv(kmax);
     const float M = __builtin_floorf(xmax);
@@ -760,33 +761,32 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
         }
     };
     // a row finished from a list of at most 64 tokens that holds its kept set: the token + 1 in one lane of the first wave; 0 in `doubts` when
-    // nothing is in doubt, 1 when D must be exact, 2 when the list is too short (first wave)
+    // nothing is in doubt, 1 when D must be exact, 2 when the list is too short (second wave)
     uint32_t doubts = 0;
     auto from_few = [&](const uint64_t *list, const uint32_t n, const bool all_of_it, const uint32_t rounds) __attribute__((always_inline)) -> uint32_t {
         M96 e = err;
         return few_pick(p, L.few, row, lane, wave, list, n, top_k,
-                        [&](const Limbs &upto) {
+                        [&](const Limbs &upto) __attribute__((always_inline)) {
                             if (!all_of_it) return Totals{D, P};
                             e = M96{0ull, 0u};           // every live token of the row is there
                             const M96 d = m96(lane_of(upto, 63u));
                             return Totals{d, ceil_mul(p.top_p, d)};
                         }, xmax, &L.rand64, rounds,
-                        [&](const Totals &t, bool enough, uint32_t n_gt, uint32_t n_eq, uint32_t thr, const M96 &above, const Target &tg, const M96 &before,
-                            const M96 &upto, bool is_it) {
-                            const Doubt d = doubt_of(t.P, e, top_k, n_gt, n_eq, above, thr, tg.w_tie);
-                            const M96 S = above + m96((u128)tg.w_tie * n_eq);
-                            const bool sure = !d.unsure && (!is_it || pick_is_sure(d.shift, before, upto, m96(tg.r), !(before.lo | before.hi), upto >= S));
-                            doubts = !enough ? 2u : sure ? 0u : 1u;
-                        });
+                        [&](const M96 &P, bool enough, uint32_t n_gt, uint32_t n_eq, uint32_t thr, const M96 &above, uint64_t w_tie) __attribute__((always_inline)) {
+                            const Doubt d = doubt_of(P, e, top_k, n_gt, n_eq, above, thr, w_tie);
+                            doubts = !enough ? 2u : d.unsure ? 1u : 0u;
+                            if (lane == 0) L.one.shift = d.shift;
+                        }, [&](const M96 &slack) __attribute__((always_inline)) { L.one.slack = slack; });
     };
-    auto put = [&](uint32_t token) __attribute__((always_inline)) {
-        if (wave == 0 && doubts) L.unsure = doubts;
+    auto put = [&](uint32_t token, bool few) __attribute__((always_inline)) {
+        if (wave <= 1 && doubts) L.unsure = doubts;
         if (token) {
             p.out[row] = (int32_t)(token - 1u);
             if (p.diag) p.diag[row].index = (int32_t)(token - 1u);
         }
         __syncthreads();
-        return uniform(L.unsure);
+        const uint32_t u = uniform(L.unsure);
+        return few && u == 0u && !(L.one.slack >= L.one.shift) ? 1u : u;
     };
     // the tokens for which in(i) says so, side by side
     auto list_them = [&](auto in) __attribute__((always_inline)) {
@@ -908,7 +908,7 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
         __syncthreads();
         if (listed && n <= (uint32_t)kWave && !again) {
             total();
-            const uint32_t token = from_few(L.list, n, whole && n == all, 0u), in_doubt = put(token);
+            const uint32_t token = from_few(L.list, n, whole && n == all, 0u), in_doubt = put(token, true);
             if (__builtin_expect(in_doubt == 0u, 1)) return;
             again = in_doubt == 1u;
             listed = again;
@@ -1131,7 +1131,7 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
                 __syncthreads();
             }
         }
-        const uint32_t in_doubt = put(token);
+        const uint32_t in_doubt = put(token, n <= (uint32_t)kWave);
         if (__builtin_expect(in_doubt == 0u, 1)) {
             if (tell) tell_policy(params_again());
             return;
