@@ -31,6 +31,7 @@ constexpr uint32_t kRowListW  = 768u;                    // tokens of the bounda
 constexpr uint32_t kRowList   = kRowListW * 12u;         // the row's boundary bin is listed when it holds no more than this (16 waves: room to spare for uneven shares)
 constexpr uint32_t kRowKeptW  = kRowListW / 2u;          // the same lists with 64-bit entries: tokens at or above the boundary bin, with their places
 constexpr uint32_t kRowKept   = kRowKeptW * 12u;         // listed when there are no more than this in the row
+constexpr uint32_t kRowFew    = 16u;                     // tokens of a boundary that are compared with each other
 constexpr uint32_t kRowRounds = 10u;                     // DiagRow::rounds of a row finished here
 
 struct LdsRowS {                      // what the shared helpers work on
@@ -51,16 +52,22 @@ struct LdsRow {
     u128     wq[kRowW];               // per wave: kept weight of its stretch of the row
     u128     wq4[kRowW][4];           // the same, a quarter of the wave's groups at a time
     uint32_t nolist;                  // a wave's share of the boundary bin did not fit its list
+    uint32_t nsmall, small[kRowFew];  // the last few tokens among which the threshold is
     uint32_t nokept;                  // the same for the list of all tokens at or above the boundary bin
     uint32_t wu[kRowW];
     uint64_t rand64;
+};
+
+constexpr uint32_t kRowStage = 128u;                     // groups on their way to a wave's list
+template <int W> struct LdsRowStage {
+    alignas(16) uint4 grp[W][kRowStage];
+    uint32_t at[W][kRowStage];
 };
 
 template <int W>
 __device__ __forceinline__ uint32_t row_max_u32(LdsRow &L, uint32_t v, int lane, int wave)
 {
     v = wave_max_u32(v);
-    __syncthreads();
     if (lane == 0) L.wu[wave] = v;
     __syncthreads();
     uint32_t r = L.wu[0];
@@ -78,6 +85,7 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     constexpr int kRowT = NT, kRowW = NT / kWave, kRowR = R;
     constexpr uint32_t kRowListW = rs::kRowListW * (uint32_t)(rs::kRowW / kRowW), kRowKeptW = rs::kRowKeptW * (uint32_t)(rs::kRowW / kRowW);
     __shared__ LdsRow L;
+    __shared__ LdsRowStage<NT / kWave> stage;
     LdsRowS &s = L.s;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     const uint32_t row = blockIdx.x;
@@ -92,7 +100,8 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     prev.slow_rows = 0; prev.meta = 0;
     if (reporter) prev = report_begin(p);
     for (int i = (int)kBin0 * 4 + tid; i < kNB * 4; i += kRowT) reinterpret_cast<uint4 *>(L.hr8)[i] = make_uint4(0u, 0u, 0u, 0u);       // (the bins of live tokens)
-    if (tid == 0) { L.nolist = 0u; L.nokept = 0u; }
+    if (tid < 128 * 4) L.lev[tid] = 0ull;
+    if (tid == 0) { L.nolist = 0u; L.nokept = 0u; L.nsmall = 0u; }
 
     // token (g0 + j * 64) * 4 + q sits in register j * 4 + q; slots past the end of the stretch read the
     // row's last group again (harmless for the maximum and the probe) and are set aside before anything is counted
@@ -236,32 +245,51 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
     }
     // A moderate number of tokens at or above the boundary bin: every wave lists its own, bits of e and place in its
     // stretch, and everything behind -- the levels, the sums of the pick -- reads a few list entries per thread instead
-    // of the registers (the first pass of the pick alone takes 15 instructions per token, listing 8).  Up to a sixth of
+    // of the registers (the first pass of the pick alone takes 15 instructions per token, listing some 4).  Up to a sixth of
     // the row, that is: where more is kept the lists themselves cost as much as the registers (1024 rows of 8192, more
     // than half of each kept: 28 us from the registers, 38 from lists).  512 x 32768 float16, 4 % kept: 31.3 -> 26.8
     // us a call; 512 x 50304: 55.5 -> 46.3; 200 x 50304: 27.6 -> 22.9; flat rows with top_k 1000, 512 x 32768: 38.3 -> 30.4.
     // (The bits are copied out of the compiler's sight: it kept what it had worked out from them in 200 registers.)
-    uint64_t *kept = L.hr8 + (uint32_t)wave * kRowKeptW;             // group by group, then token of the group, then lane
-    uint32_t nkept = 0u, kept_from = 0u;                             // kept_from: lane j, where those of the wave's group j begin
+    uint64_t *kept = L.hr8 + (uint32_t)wave * kRowKeptW;             // (in no order)
+    uint32_t nkept = 0u;
     const uint32_t bin_lo = f.bin << 21;
     const uint32_t at_or_above = f.cnt_above + f.cnt_bin;
     bool have_kept = at_or_above <= kRowKept && at_or_above * 6u <= (uint32_t)p.V;
     if (have_kept) {
+        // (The groups of four that hold such a token first, side by side, and of 64 of these at a time their tokens: with votes about every token
+        // 512 x 32768 float16, 4 % kept, took 26.8 us, like this 25.9.)
+        uint32_t staged = 0u, done = 0u;                             // groups of the wave
+        uint4 *ring = stage.grp[wave];
+        uint32_t *where = stage.at[wave];
+        auto take = [&](const uint32_t n) __attribute__((always_inline)) {           // the tokens of the next n <= 64 groups
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            const uint32_t i = (done + (uint32_t)lane) & (kRowStage - 1u);
+            const uint4 g = ring[i];
+            const uint32_t at4 = where[i], b4[4] = {g.x, g.y, g.z, g.w};
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const bool in = (uint32_t)lane < n && b4[q] >= bin_lo;
+                const uint64_t cand = __builtin_amdgcn_ballot_w64(in);
+                const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(cand >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cand, nkept));
+                if (in && at < kRowKeptW) kept[at] = ((uint64_t)b4[q] << 32) | (at4 + (uint32_t)q);
+                nkept += (uint32_t)__builtin_popcountll(cand);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            done += n;
+        };
         uint32_t lane4 = (uint32_t)lane * 4u;
 #pragma unroll
         for (int j = 0; j < kRowR; ++j) {
-            asm volatile("" : "+s"(nkept), "+v"(lane4));
-            kept_from = lane == j ? nkept : kept_from;
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                uint32_t b = eb[j * 4 + q];
-                asm volatile("" : "+v"(b));
-                const uint64_t cand = __builtin_amdgcn_ballot_w64(b >= bin_lo);
-                const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(cand >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cand, nkept));
-                if (b >= bin_lo && at < kRowKeptW) kept[at] = ((uint64_t)b << 32) | (lane4 + (uint32_t)(j * 256 + q));
-                nkept += (uint32_t)__builtin_popcountll(cand);
-            }
+            uint32_t b0 = eb[j * 4], b1 = eb[j * 4 + 1], b2 = eb[j * 4 + 2], b3 = eb[j * 4 + 3];
+            asm volatile("" : "+s"(staged), "+v"(lane4), "+v"(b0), "+v"(b1), "+v"(b2), "+v"(b3));
+            const bool in = max(max(b0, b1), max(b2, b3)) >= bin_lo;
+            const uint64_t cand = __builtin_amdgcn_ballot_w64(in);
+            const uint32_t at = __builtin_amdgcn_mbcnt_hi((uint32_t)(cand >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)cand, staged)) & (kRowStage - 1u);
+            if (in) { ring[at] = make_uint4(b0, b1, b2, b3); where[at] = lane4 + (uint32_t)(j * 256); }
+            staged += (uint32_t)__builtin_popcountll(cand);
+            if (staged - done >= (uint32_t)kWave) take((uint32_t)kWave);
         }
+        if (staged != done) take(staged - done);
         if (nkept > kRowKeptW && lane == 0) L.nokept = 1u;
         __syncthreads();
         have_kept = L.nokept == 0u;
@@ -274,33 +302,51 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
                 fn((uint32_t)(e >> 32), (uint32_t)e);
             }
         };
-        for (uint32_t lv = 2; lv <= (uint32_t)kLevels && !one_tie && f.cnt_bin > 1u; ++lv) {
+        // Levels while there are more than a few tokens in the boundary bin, each in words of its own (cleared at the start) and looked at where they were
+        // counted; of the few the first wave ranks every one against every other.  (Down to a single token, a level taking four barriers instead of two
+        // and its single token a fifth: 512 x 32768 float16 25.9 us, like this 24.3.)
+        for (uint32_t lv = 2; lv <= (uint32_t)kLevels && !one_tie && f.cnt_bin > kRowFew; ++lv) {
             const uint32_t dsh = level_shift(lv);
-            if (tid < 128 * 4) L.lev[tid] = 0;
-            __syncthreads();
+            uint64_t *hist = L.lev + (lv - 2u) * 128u;
             listed([&](uint32_t b, uint32_t) {
-                if (b - lo <= span)
-                    atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[((b >> dsh) & 127u) * 4u + (uint32_t)(lane & 3)]),
-                              (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
+                if (b - lo <= span) atomicAdd(reinterpret_cast<unsigned long long *>(&hist[(b >> dsh) & 127u]), (unsigned long long)(kPackOne | (b & 0x7FFFFFu)));
             });
             __syncthreads();
-            if (tid < 128) s.hm[tid] = L.lev[tid * 4] + L.lev[tid * 4 + 1] + L.lev[tid * 4 + 2] + L.lev[tid * 4 + 3];
-            __syncthreads();
-            f = hist_find128(s, s.hm, f.cnt_above, f.mass_above, top_k, exb, lane, wave);
+            f = hist_find128(s, hist, f.cnt_above, f.mass_above, top_k, exb, lane, wave);
             lo |= f.bin << dsh;
             span = (1u << dsh) - 1u;
         }
         if (span != 0u) {
-            listed([&](uint32_t b, uint32_t) { if (b - lo <= span) s.bc32[6] = b; });
+            listed([&](uint32_t b, uint32_t) {
+                if (b - lo <= span) L.small[atomicAdd(&L.nsmall, 1u) & (kRowFew - 1u)] = b;
+            });
             __syncthreads();
-            lo = s.bc32[6];
         }
-        const uint32_t thr = lo;
         if (wave == 0) {
-            const Target tg = target(thr, f.cnt_above, f.cnt_bin, f.mass_above, kRowRounds);
-            s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r;
+            uint32_t t = lo, n_gt = f.cnt_above, n_eq = f.cnt_bin;
+            M96 above = uniform(m96(f.mass_above));
+            if (span != 0u) {
+                // (the largest is always kept: what is above the bin is not enough)
+                const uint32_t n = min(uniform(f.cnt_bin), kRowFew), b = (uint32_t)lane < n ? L.small[lane] : 0u;
+                uint32_t larger = 0, sum = 0;
+                for (uint32_t k = 0; k < n; ++k) {
+                    const uint32_t o = lane_of(b, k);
+                    larger += o > b ? 1u : 0u;
+                    sum += o > b ? (o & 0x7FFFFFu) | 0x800000u : 0u;
+                }
+                const uint64_t need = need_of(uniform(m96(s.P)), above, exb);
+                const bool in = (uint32_t)lane < n && n_gt + larger < (uint32_t)min(top_k, (uint64_t)0xFFFFFFFFull) && sum < need;
+                t = ~wave_max_u32(in ? ~b : 0u);
+                const uint64_t at = __builtin_amdgcn_ballot_w64(in && b == t);
+                const uint32_t l = (uint32_t)__builtin_ctzll(at);
+                n_eq = (uint32_t)__builtin_popcountll(at); n_gt += lane_of(larger, l);
+                above = above + mass_of((uint64_t)lane_of(sum, l), exb);
+            }
+            const Target tg = target(t, n_gt, n_eq, wide(above), kRowRounds);
+            s.bc64[1] = tg.w_tie; s.bc128[0] = tg.r; s.bc32[6] = t;
         }
         __syncthreads();
+        const uint32_t thr = uniform(s.bc32[6]);
         const uint64_t w_tie = s.bc64[1];
         const u128 r = s.bc128[0];
         auto weight = [=](uint32_t b) -> uint64_t { return (b > thr) ? w_of_bits(b) : (b == thr ? w_tie : 0ull); };
@@ -314,34 +360,27 @@ __global__ void __launch_bounds__(NT, 4) row_kernel(const Params p)
         const uint32_t wstar = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(winc >= r));
         if ((uint32_t)wave != wstar) return;
         u128 rl = r - wide(lane_of(m96(winc - wt), wstar));
-        // the wave's groups one per lane, then the tokens of one group, four per lane
+        // the wave's stretch in 64 pieces of 64 tokens, one per lane, then the tokens of one piece  (16 groups of 256, four to a lane: 0.25 us more)
         auto in_order = []() { __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront"); };
-        if (lane < 32) L.lev[lane] = 0ull;
+        L.lev[lane] = 0ull; L.lev[kWave + lane] = 0ull;
         in_order();
-        for (uint32_t i = (uint32_t)lane; i < nkept; i += (uint32_t)kWave) {
-            const uint64_t e = kept[i], w = weight((uint32_t)(e >> 32));
-            const uint32_t g = (uint32_t)e >> 8;         // < 16
-            atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[g]), (unsigned long long)(w & 0xFFFFFFFFull));
-            atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[16 + g]), (unsigned long long)(w >> 32));
-        }
+        listed([&](uint32_t b, uint32_t place) {
+            const uint64_t w = weight(b);
+            atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[place >> 6]), (unsigned long long)(w & 0xFFFFFFFFull));
+            atomicAdd(reinterpret_cast<unsigned long long *>(&L.lev[(uint32_t)kWave + (place >> 6)]), (unsigned long long)(w >> 32));
+        });
         in_order();
-        const u128 gm = lane < 16 ? (u128)L.lev[lane] + ((u128)L.lev[16 + lane] << 32) : (u128)0;
-        const u128 ginc = wave_inclusive_scan(gm);
-        const uint32_t j = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(ginc >= rl));       // there is one
-        rl -= wide(lane_of(m96(ginc - gm), j));
-        const uint32_t from = lane_of(kept_from, j), to = j + 1u < (uint32_t)kRowR ? lane_of(kept_from, j + 1u) : nkept;
+        const u128 gm = (u128)L.lev[lane] + ((u128)L.lev[kWave + lane] << 32), ginc = wave_inclusive_scan(gm);
+        const uint32_t piece = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(ginc >= rl));       // there is one
+        rl -= wide(lane_of(m96(ginc - gm), piece));
         in_order();
-#pragma unroll
-        for (int k = 0; k < 4; ++k) L.lev[k * kWave + lane] = 0ull;
+        L.lev[lane] = 0ull;
         in_order();
-        for (uint32_t i = from + (uint32_t)lane; i < to; i += (uint32_t)kWave) L.lev[(uint32_t)kept[i] & 255u] = weight((uint32_t)(kept[i] >> 32));
+        listed([&](uint32_t b, uint32_t place) { if (place >> 6 == piece) L.lev[place & 63u] = weight(b); });
         in_order();
-        const uint64_t w0 = L.lev[lane * 4], w1 = L.lev[lane * 4 + 1], w2 = L.lev[lane * 4 + 2], w3 = L.lev[lane * 4 + 3];
-        const u128 m4 = (u128)w0 + w1 + w2 + w3, inc = wave_inclusive_scan(m4), exc = inc - m4;
-        if (exc < rl && rl <= inc) {                     // exactly one lane
-            const u128 rr = rl - exc;
-            const uint32_t kk = (rr <= w0) ? 0u : (rr <= (u128)w0 + w1) ? 1u : (rr <= (u128)w0 + w1 + w2) ? 2u : 3u;
-            const int32_t idx = (int32_t)(((uint32_t)wave * G + j * (uint32_t)kWave + (uint32_t)lane) * 4u + kk);
+        const u128 own = (u128)L.lev[lane], inc = wave_inclusive_scan(own);
+        if (inc - own < rl && rl <= inc) {               // exactly one lane
+            const int32_t idx = (int32_t)((uint32_t)wave * G * 4u + piece * (uint32_t)kWave + (uint32_t)lane);
             p.out[row] = idx;
             if (p.diag) p.diag[row].index = idx;
         }

@@ -2409,3 +2409,42 @@ def test_sieve_path_with_penalties(torch_cuda, oracle, B, V, fmt, k):
             bad = np.argwhere(have.cpu().numpy().view(np.uint32) != np.tile(want, (reps, 1)).view(np.uint32))
             assert bad.size == 0, bad[:8]
     smp.close()
+
+
+@pytest.mark.parametrize("B,V", [(1, 32768), (260, 32768), (2, 50304), (260, 8192)])
+def test_row_kernel_boundaries_of_a_few_tokens(torch_cuda, oracle, B, V):
+    """The row kernel's threshold among 1 to 40 tokens of one level-1 bin, where it is ranked directly up to 16 of them and found by digits beyond:
+    distinct values and ties, a top_k at either end of them and inside, a top_p inside; workgroups of 1024 and of 512 threads, every field and
+    token against the oracle (integers: equal)."""
+    torch = torch_cuda
+    from tests import capi
+    rng = np.random.default_rng(V + B)
+    n_top = 30
+    rows, ks = [], []
+    for n in (1, 2, 3, 15, 16, 17, 40):
+        for tied in (0, 2, n):                               # of the n, so many alike in the middle
+            r = (rng.standard_normal(V) * 0.5 - 12.0).astype(np.float32)
+            at = rng.choice(V, n_top + n, replace=False)
+            r[at[:n_top]] = 4.0 + rng.random(n_top, dtype=np.float32) * 3
+            b = (1.0 + rng.permutation(n) * np.float32(2.0 ** -12)).astype(np.float32)       # one quarter of an octave
+            m = min(tied, n)
+            if m:
+                b[n // 2 - m // 2: n // 2 - m // 2 + m] = b[n // 2]
+            r[at[n_top:]] = b
+            rows.append(r)
+            ks.append(n)
+    base = np.stack(rows)
+    reps = -(-B // base.shape[0])
+    lg = np.tile(base, (reps, 1))
+    x = torch.from_numpy(lg).cuda()
+    smp = capi.Sampler(lg.shape[0], V)
+    c = 1.0
+    u_np = H.uniforms(base.shape[0], V)
+    u = torch.from_numpy(np.tile(u_np, reps)).cuda()
+    for k, top_p in [(n_top + 1, 1.0), (n_top + 2, 1.0), (n_top + 9, 1.0), (n_top + 16, 1.0), (n_top + 17, 1.0), (n_top + 39, 1.0), (2000, 0.9999), (2000, 0.9)]:
+        ref_out, ref_diag = oracle.sample_batch(base, c, k, top_p, injected_u=u_np)[:2]
+        print("row kernel, few at the boundary:", B, V, k, top_p, flush=True)
+        res = smp.sample(x, c, k, top_p, uniforms=u, path="row")
+        _check(res, np.tile(ref_out, reps), np.tile(ref_diag, reps), "row kernel, few at the boundary")
+        assert smp.status() == 0
+    smp.close()
