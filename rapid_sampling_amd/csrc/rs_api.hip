@@ -555,6 +555,8 @@ static int fused_r(int32_t B, int32_t V, bool pen, bool any_size)
 //    512 x 131072   58.9 / 49.9 45.2 / 28.5 61.4 / 55.4  75.7 / 63.5               57.0 / 50.0
 //    128 x 1048576   103 / 92    78 / 50     104 / 96     105 / 100    112 / 105    104 / 94
 //   1024 x  20000   39.3 / 28.1 31.0 / 21.8                                        35.2 / 28.2
+// and, at the line for longer lists, which used to be finished by 1024 threads: 64 x 262144 top_k 300 25.6 / 25.5, 128 x 131072 29.2 / 26.7, bfloat16
+// 16 x 1048576 24.6 / 23.6, 32 x 1048576 top_k 1000 40.0 / 39.4; below it 64 x 131072 top_k 100 17.7 / 17.8 and, N(0,3) with top_p 0.3, 17.1 / 17.9.
 // (1 x 32768: 8.9 there and 9.7 here with 16 spikes.)  Its finish compares up to 64 tokens with each other, for which it is as short as the streaming
 // path's; longer lists are faster there until the pass outweighs them.  Slices of 4096 tokens while 32 of them make a row, else of
 // 8192, and of 16384 in a few rows of a million (1 x 1048576 12.0 us against 14.1); shorter when one would hold more than 8 of the row's top_k on
@@ -562,10 +564,24 @@ static int fused_r(int32_t B, int32_t V, bool pen, bool any_size)
 // Without a bounding top_k the kept set may be of hundreds of tokens, the longer list's time, and each is one more place where D is too close to
 // call: 16 x 131072 with 455 kept 15.0 there, 46.7 here.
 static uint32_t sieve_share(int32_t top_k, int32_t V, int R) { return (uint32_t)(((uint64_t)(uint32_t)top_k * 1024u * (uint32_t)R + (uint32_t)V - 1u) / (uint32_t)V); }
-static int sieve_r(int32_t B, int32_t V, int32_t top_k)
+constexpr int32_t kSieveK = 320;
+// Whether the pass sums the tokens' own e in double precision.  How often a decision is too close to call goes with the error of D over the weight of
+// the threshold's token: a row in 4000 with 100 kept, in 1000 with 400, and such a row is summed again by one workgroup, 10 us in rows of 131072 tokens
+// and 75 in rows of a million, for which the call waits (128 x 1048576 N(0,3), top_k 1000, top_p 0.3: 255 us a call, 100 with these sums).  With
+// them it is a row in millions, for 10 more issue slots a token: nothing where the pass waits for the memory, us a call, v_exp_f32 / double:
+// 128 x 1048576 top_k 1024 102.4 / 100.7, top_k 50 91.0 / 86.7, with penalties 128 x 262144 58.4 / 58.2; a tenth and more elsewhere (256 x 131072
+// 26.9 / 30.6, 4 x 1048576 12.8 / 14.6, bfloat16 128 x 1048576 50.7 / 76.4), where short lists are rarely in doubt and, in rows of up to 262144
+// tokens, those of more than kSieveK are left to the streaming path.
+static bool sieve_fine(int32_t B, int32_t V, int32_t top_k, int32_t dtype, bool pen)
 {
     const uint64_t tokens = (uint64_t)B * (uint64_t)V;
-    if (tokens < (top_k <= 64 ? 49152u : top_k <= 128 ? 1u << 24 : V <= kMidMaxV ? 1u << 25 : 1u << 26)) return 0;
+    if (pen) return tokens >= 1u << 24;
+    return V > kMidMaxV && (top_k > kSieveK || (dtype == RS_DTYPE_F32 && tokens >= 1u << 26));
+}
+static int sieve_r(int32_t B, int32_t V, int32_t top_k, bool pen)
+{
+    const uint64_t tokens = (uint64_t)B * (uint64_t)V;
+    if (tokens < (top_k <= 64 ? 49152u : 1u << 24) || (!pen && V <= kMidMaxV && top_k > kSieveK)) return 0;
     const uint32_t g4 = stream_parts(V, 4), g8 = stream_parts(V, 8);
     int R = g4 <= 32u && (uint64_t)B * g4 <= kStreamSmallParts ? 4 : g8 <= 64u || (uint64_t)B * g8 > 8192u ? 8 : 16;
     while (R > 4 && sieve_share(top_k, V, R) > 8u && stream_parts(V, R / 2) <= 128u) R /= 2;
@@ -592,7 +608,8 @@ static uint32_t sieve_reach(int32_t V, int32_t top_k, int R, uint32_t units)
 // (1024 x 20000 55.9 / 48.1; flat rows 256 x 50304 42.4 / 29.6.)  Slices of 8192 tokens at most: a thread holds tokens and penalties.
 static int sieve_pen_r(int32_t B, int32_t V, int32_t top_k)
 {
-    return top_k > 128 && (uint64_t)B * (uint64_t)V < (1u << 26) ? 0 : min(sieve_r(B, V, top_k), 8);
+    if (top_k > 128 && (uint64_t)B * (uint64_t)V < (1u << 26)) return 0;
+    return min(sieve_r(B, V, top_k, true), 8);
 }
 
 static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pen, const rs_options *opt)
@@ -940,7 +957,7 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
     if (path == kPathShort) return launch_short(pen, logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     if (path == kPathRow) return launch_row(logits_dtype, (uint32_t)B, (hipStream_t)stream, p) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
     // (with penalties: a decay that leaves +0.0 as it is)
-    if (const int R = path != kPathStream || (pen && decay - decay != 0.0f) ? 0 : pen ? sieve_pen_r(B, V, top_k) : sieve_r(B, V, top_k)) {
+    if (const int R = path != kPathStream || (pen && decay - decay != 0.0f) ? 0 : pen ? sieve_pen_r(B, V, top_k) : sieve_r(B, V, top_k, false)) {
         SieveView v;
         v.G = stream_parts(V, R);
         v.units = sieve_share(top_k, V, R) <= 8u ? 1u : 2u;
@@ -949,11 +966,14 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
         v.note_cap = sieve_pen_cap(R);
         const size_t noted = align256(stash + slices * v.units * kWave * sizeof(uint64_t)), waves = slices * kWaves;
         const size_t note_at = align256(noted + waves * sizeof(uint32_t)), note_old = align256(note_at + waves * v.note_cap * sizeof(uint32_t));
-        const size_t end = pen ? align256(note_old + waves * v.note_cap * sizeof(float4)) : noted;
-        // (a workspace of rs_workspace_bytes has room, 0.25 bytes a token at most, 1.1 with penalties; one without takes the streaming path)
+        const size_t fine = pen ? align256(note_old + waves * v.note_cap * sizeof(float4)) : noted;
+        const bool want_fine = sieve_fine(B, V, top_k, logits_dtype, pen);
+        const size_t end = want_fine ? align256(fine + slices * sizeof(SieveFine)) : fine;
+        // (a workspace of rs_workspace_bytes has room, 0.26 bytes a token at most, 1.1 with penalties; one without takes the streaming path)
         if (end + (size_t)B * sizeof(RowCtl) <= (workspace_bytes & ~(size_t)255)) {
             char *w = (char *)workspace;
             v.hdr = (SieveHdr *)(w + hdr); v.stash = (uint64_t *)(w + stash);
+            v.fine = want_fine ? (SieveFine *)(w + fine) : nullptr;
             v.noted = (uint32_t *)(w + noted); v.note_at = (uint32_t *)(w + note_at); v.note_old = (float4 *)(w + note_old);
             p.report = (uint32_t)policy_word(0, size_class(B, V));
             if (pen) {

@@ -32,6 +32,9 @@ namespace rs {
 // |x| < 128 compared; larger |x| have less of it), so for 4096 tokens, one of them in the frame's octave, at most 9.1; with 3 roundings 12.1, and 32
 // are allowed.  Tokens more than 40 octaves below the row's frame weigh nothing but are in the sums: 2^-40 each at most.
 //
+// Where the pass waits for the memory (the host's rule) it sums the tokens' own e in double precision instead (FINE): 2^-40 of D and of the slices' number
+// is allowed for, and the tokens of no weight only if the least token of a slice is that far down.  Then hardly a row is summed again.
+//
 // What bounds it: in large calls the pass reads float32 at the rate of a kernel that only reads.  A token costs 4.6 vector instructions (one of
 // them the exponential, 2.7 issue slots), and a wave some 200 for bound and staging, where the pass with exact e and a histogram (stream_kernel)
 // takes 22 and an LDS atomic.  us of a pass, there / here: 128 rows of 1048576 106 / 86, 64 of 152064 12.7 / 10.1, 256 of 151936 bfloat16
@@ -56,7 +59,7 @@ struct LdsSieve {
     double   mass[kThreads];                             // the threads' sums
     float    top[kThreads];                              // and largest tokens
     float    frame[kWaves];                              // the frames of the sums
-    uint32_t wmax[kWaves], odd[kWaves], n[2][kWaves], tie;
+    uint32_t wmax[kWaves], odd[kWaves], n[2][kWaves], low[kWaves], tie;
 };
 
 // A workgroup's slice to its record.  group(j, x): the scaled logits of the thread's j-th group of four tokens, group j * 256 + tid of the
@@ -66,13 +69,15 @@ struct LdsSieve {
 // The terms of the sum need no frame: 2^x is a float for every x in question, and so they are worked out in the order in which
 // the loads arrive.  A wave whose largest x is beyond 120 or below -80 (the tokens 40 octaves below it would no longer be floats), or
 // that holds a NaN or an infinity, does it again, cleaned up and in a frame.
-template <int R, typename G, typename Z, typename A, typename E>
+template <int R, bool FINE, typename G, typename Z, typename A, typename E>
 __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G group, Z strange, A redo, E then, const size_t slice, const uint32_t g0, const uint32_t left, const int tid)
 {
     const float kInf = __builtin_inff();
     const int lane = tid & (kWave - 1), wave = (int)uniform((uint32_t)tid >> 6);
     bool odd = false;
     double mass = 0.0;
+    const Frame fr(0);
+    float low = kInf;                                    // FINE: the smallest
     float x[R * 4], gm[R], lm = -kInf, M = 0.0f;            // gm: the largest of every group, lm: of all; of the wave: the frame, the sum in it
     auto top = [&](int j) {
         float m;                                         // (fmaxf quiets its operands first, an instruction each; products are quiet)
@@ -90,8 +95,17 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         for (int j = 0; j < R; ++j) {
             group(j, &x[j * 4]);
             gm[j] = top(j);
-            q[j % 4] = (__builtin_amdgcn_exp2f(x[j * 4]) + __builtin_amdgcn_exp2f(x[j * 4 + 1])) +
-                       (__builtin_amdgcn_exp2f(x[j * 4 + 2]) + __builtin_amdgcn_exp2f(x[j * 4 + 3]));
+            if constexpr (FINE) {
+                float least;                             // (see top)
+                asm("v_min3_f32 %0, %1, %2, %3" : "=v"(least) : "v"(x[j * 4]), "v"(x[j * 4 + 1]), "v"(x[j * 4 + 2]));
+                asm("v_min3_f32 %0, %1, %2, %3" : "=v"(low) : "v"(least), "v"(x[j * 4 + 3]), "v"(low));
+                const bool in = !ragged || (uint32_t)(j * kThreads) + opaque((uint32_t)tid) < left;
+                double d0 = (double)fr.scaled(x[j * 4]) + (double)fr.scaled(x[j * 4 + 1]), d1 = (double)fr.scaled(x[j * 4 + 2]) + (double)fr.scaled(x[j * 4 + 3]);
+                mass += in ? d0 + d1 : 0.0;
+                q[j % 4] = 0.0f;
+            } else
+                q[j % 4] = (__builtin_amdgcn_exp2f(x[j * 4]) + __builtin_amdgcn_exp2f(x[j * 4 + 1])) +
+                           (__builtin_amdgcn_exp2f(x[j * 4 + 2]) + __builtin_amdgcn_exp2f(x[j * 4 + 3]));
             if (j % 2 == 1) {
                 if (ragged) {
                     const uint32_t at = (uint32_t)((j - 1) * kThreads) + opaque((uint32_t)tid);
@@ -103,8 +117,10 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
             }
             if (j % 4 == 3) part[j / 4] = (q[0] + q[1]) + (q[2] + q[3]);
         }
+        if constexpr (!FINE) {
 #pragma unroll
-        for (int i = 0; i < R / 4; ++i) mass += (double)part[i];
+            for (int i = 0; i < R / 4; ++i) mass += (double)part[i];
+        }
         odd = __builtin_amdgcn_ballot_w64(!(mass < (double)kInf) || lm > 120.0f || strange()) != 0ull || __builtin_amdgcn_ballot_w64(lm >= -80.0f) == 0ull;
         if (__builtin_expect(odd, 0)) {
             const uint32_t t = opaque((uint32_t)tid);
@@ -129,6 +145,10 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
     {
         const uint32_t k = wave_max_u32(fkey(lm));
         if (lane == 0) { s.frame[wave] = M; s.wmax[wave] = k; s.odd[wave] = odd ? 1u : 0u; }
+        if constexpr (FINE) {
+            const uint32_t l = wave_max_u32(~fkey(low));
+            if (lane == 0) s.low[wave] = l;
+        }
     }
     if (tid == 0) s.tie = 1u;
     __syncthreads();
@@ -192,7 +212,10 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         const double2 m2 = reinterpret_cast<const double2 *>(s.mass)[lane * 2], m3 = reinterpret_cast<const double2 *>(s.mass)[lane * 2 + 1];
         const int down = (int)fmaxf(s.frame[lane >> 4] - Ms, -1000.0f);
         const double all = wave_sum_f64(__builtin_ldexp((m2.x + m2.y) + (m3.x + m3.y), down));
-        if (lane == 0) v.hdr[slice].mass = __float_as_uint((float)all);
+        if (lane == 0) {
+            v.hdr[slice].mass = __float_as_uint((float)all);
+            if constexpr (FINE) v.fine[slice] = SieveFine{all, ~max(max(s.low[0], s.low[1]), max(s.low[2], s.low[3])), 0u};
+        }
     }
     uint32_t n = 0, cut = key;
     if (__builtin_expect(full, 0)) {
@@ -245,8 +268,8 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
 }
 
 // A workgroup of 256 threads to a slice of R * 256 groups of four tokens.
-template <int R, int DT>
-__global__ void __launch_bounds__(kThreads, R == 16 ? 4 : 8) sieve_kernel(const Params p, const SieveView v)
+template <int R, int DT, bool FINE>
+__global__ void __launch_bounds__(kThreads, R == 16 ? (FINE ? 3 : 4) : !FINE ? 8 : R == 8 ? 5 : 8) sieve_kernel(const Params p, const SieveView v)
 {
     __shared__ LdsSieve s;
     const int tid = threadIdx.x;
@@ -273,7 +296,7 @@ __global__ void __launch_bounds__(kThreads, R == 16 ? 4 : 8) sieve_kernel(const 
         for (int j = 0; j < R; ++j) l[j] = __builtin_nontemporal_load(from + min((uint32_t)(j * kThreads + tid), left - 1u));
     }
     if (reporter) report_end(p, prev, true);
-    sieve_slice<R>(v, s, [&](int j, float *x) {
+    sieve_slice<R, FINE>(v, s, [&](int j, float *x) {
         uint32_t w[4];
         if constexpr (DT == RS_DTYPE_F32) { w[0] = l[j].x; w[1] = l[j].y; w[2] = l[j].z; w[3] = l[j].w; }
         else widen4(make_uint2(l[j].x, l[j].y), DT, w);
@@ -297,7 +320,7 @@ __global__ void __launch_bounds__(kThreads, R == 16 ? 4 : 8) sieve_kernel(const 
 // of a copy of it) and 15 the lines of the penalties that change, half of all lines; written in whole groups of 64 or 128 bytes 65.0 and 68.5, with
 // non-temporal stores 67.0, with slices of 4096 tokens 66.0.  The pass with a histogram and a vote about every single penalty (stream_pen_kernel), 35
 // vector instructions a token, takes 74.
-template <int R, int DT>
+template <int R, int DT, bool FINE>
 __global__ void __launch_bounds__(kThreads, R == 8 ? 4 : 6) sieve_pen_kernel(const Params p, const SieveView v)
 {
     constexpr uint32_t kCap = sieve_pen_cap(R);
@@ -345,7 +368,7 @@ __global__ void __launch_bounds__(kThreads, R == 8 ? 4 : 6) sieve_pen_kernel(con
     };
     uint32_t fill = 0;
     uint32_t low = 0u;                                   // bit pattern of the most negative penalty
-    sieve_slice<R>(v, s, [&](int j, float *x) __attribute__((always_inline)) {
+    sieve_slice<R, FINE>(v, s, [&](int j, float *x) __attribute__((always_inline)) {
         uint32_t w[4];
         widen(l[j], w);
         const uint32_t b[4] = {pn[j].x, pn[j].y, pn[j].z, pn[j].w};
@@ -552,41 +575,37 @@ __device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t r
     }
 }
 
-// The row's D in double precision: 2^-40 of it off at most (D >= 1; a thread adds fewer than 2^13 terms).
+// The row's D from its logits.  `close`: in double precision, 2^-40 of it off at most (D >= 1; a thread adds fewer than 2^13 terms).  Else exactly: all of
+// its tokens are counted into L.bins, which is left that way (with e_bits also the e of every token, dead ones as 0).
 template <int NT>
-__device__ __forceinline__ M96 sieve_closer(const Params &p, LdsSieveFin<NT> &L, const uint32_t row, const float M)
+__device__ __forceinline__ M96 sieve_again(const Params &p, LdsSieveFin<NT> &L, const uint32_t row, const float M, const bool close)
 {
-    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x >> 6;
-    double s[4] = {0.0, 0.0, 0.0, 0.0};
-    sieve_row_pass<NT>(p, row, M, [&](uint32_t, const uint4 b) {
-        auto e = [](uint32_t w) { return w < kEMinBits ? 0.0 : (double)__uint_as_float(w); };
-        s[0] += e(b.x); s[1] += e(b.y); s[2] += e(b.z); s[3] += e(b.w);
-    });
-    const double mine = wave_sum_f64((s[0] + s[1]) + (s[2] + s[3]));
-    __syncthreads();
-    if (lane == 0) L.sum[wave] = __builtin_bit_cast(uint64_t, mine);
-    __syncthreads();
-    double all = 0.0;
-    for (int w = 0; w < NT / kWave; ++w) all += __builtin_bit_cast(double, L.sum[w]);
-    const uint64_t q = uniform((uint64_t)(all * 0x1p40));
-    return M96{q << 23, (uint32_t)(q >> 41)};
-}
-
-// The row's exact D: all of its tokens counted into L.bins, which is left that way (with e_bits also the e of every token, dead ones as 0).
-template <int NT>
-__device__ __forceinline__ M96 sieve_exact(const Params &p, LdsSieveFin<NT> &L, const uint32_t row, const float M)
-{
-    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     uint4 *eb4 = p.e_bits ? reinterpret_cast<uint4 *>(p.e_bits + (int64_t)row * p.V) : nullptr;
     for (int i = tid; i < kSieveCopies * (kNB + 4); i += NT) (&L.bins[0][0])[i] = 0ull;
     __syncthreads();
     uint64_t *bins = L.bins[lane & (kSieveCopies - 1)];
-    sieve_row_pass<NT>(p, row, M, [&](uint32_t i4, const uint4 b) {
-        auto add = [&](uint32_t w) { atomicAdd(reinterpret_cast<unsigned long long *>(&bins[w >> 21]), (unsigned long long)(kPackOne | (w & 0x7FFFFFu))); };
-        add(b.x); add(b.y); add(b.z); add(b.w);
-        auto live = [](uint32_t w) { return w < kEMinBits ? 0u : w; };
-        if (eb4) eb4[i4] = make_uint4(live(b.x), live(b.y), live(b.z), live(b.w));
+    double s[2] = {0.0, 0.0};
+    sieve_row_pass<NT>(p, row, M, [&](uint32_t i4, const uint4 b) __attribute__((always_inline)) {
+        if (close) {
+            auto e = [](uint32_t w) { return w < kEMinBits ? 0.0 : (double)__uint_as_float(w); };
+            s[0] += e(b.x) + e(b.y); s[1] += e(b.z) + e(b.w);
+        } else {
+            auto add = [&](uint32_t w) { atomicAdd(reinterpret_cast<unsigned long long *>(&bins[w >> 21]), (unsigned long long)(kPackOne | (w & 0x7FFFFFu))); };
+            add(b.x); add(b.y); add(b.z); add(b.w);
+            auto live = [](uint32_t w) { return w < kEMinBits ? 0u : w; };
+            if (eb4) eb4[i4] = make_uint4(live(b.x), live(b.y), live(b.z), live(b.w));
+        }
     });
+    if (close) {
+        const double mine = wave_sum_f64(s[0] + s[1]);
+        if (lane == 0) L.sum[wave] = __builtin_bit_cast(uint64_t, mine);
+        __syncthreads();
+        double all = 0.0;
+        for (int w = 0; w < NT / kWave; ++w) all += __builtin_bit_cast(double, L.sum[w]);
+        const uint64_t q = uniform((uint64_t)(all * 0x1p40));
+        return M96{q << 23, (uint32_t)(q >> 41)};
+    }
     __syncthreads();
     OctScan sc;
     sieve_octaves(sc, L, lane);
@@ -612,7 +631,8 @@ __device__ __forceinline__ void sieve_pens_back(const Params &p, const SieveView
     __syncthreads();
 }
 
-// NT threads (256 and a wave that draws the random number, or 1024), PRE units to a wave.
+// NT threads (256 or 512 and a wave that draws the random number, or 1024), PRE units to a wave.
+template <int NT> constexpr int sieve_finish_threads() { return NT == 1024 ? NT : NT + kWave; }
 //
 // What bounds it: the length of its chain, as finish_row's.  The tokens set aside, some hundreds or thousands, are counted in 256 steps of e
 // between the bound and the row's largest, and one scan of the counts says down to which step top_k of them lie: these are listed.  A list of
@@ -620,10 +640,10 @@ __device__ __forceinline__ void sieve_pens_back(const Params &p, const SieveView
 // tokens alone.  Only when what is listed turns out not to hold the kept set (more tokens in one step than the list takes) are all
 // tokens set aside looked at, bins first; and when those do not, the row itself.
 template <int NT, int PRE>
-__global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(const Params p, const SieveView v)
+__global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kernel(const Params p, const SieveView v)
 {
     constexpr int  W = NT / kWave;
-    constexpr bool kEach = NT == kThreads;               // every wave works the one-wave steps out for itself
+    constexpr bool kEach = NT <= 512;                  // every wave works the one-wave steps out for itself
     union LdsAll { LdsSieveFin<NT> f; struct { Lds s; LdsB t; } slow; };
     __shared__ LdsAll u;
     LdsSieveFin<NT> &L = u.f;
@@ -659,13 +679,23 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
         return sh >= 0 ? m << (sh & 63) : sh > -32 ? m >> (-sh & 63) : 0ull;
     };
     M96 D{0ull, 0u}, P{0ull, 0u}, err{0ull, 0u};
-    auto estimate = [&](const uint64_t all, const bool odd) __attribute__((always_inline)) {             // D from the slices' sums, and what it may be off by
+    // D from the slices' sums, and what it may be off by; `dead`: from sums in double precision (bit 1), with tokens that weigh nothing in them (bit 0)
+    auto estimate = [&](const uint64_t all, const bool odd, const uint32_t dead) __attribute__((always_inline)) {
         auto part = [&](uint32_t sh) { return M96{(D.lo >> sh) | ((uint64_t)D.hi << (64u - sh)), D.hi >> sh}; };
         D = M96{all << 23, (uint32_t)(all >> 41)};
         if (odd) err = part(kSieveErrOdd);
+        else if (dead & 2u) err = part(40u) + M96{1ull << 31, 0u};            // (and 128 slices, cut off at 2^-40)
         else { D = D - part(23u); err = part(22u) + part(23u) + part(24u); }
-        err = err + M96{((uint64_t)p.V << 23) + 2ull, 0u};
+        if (odd || dead != 2u) err = err + M96{((uint64_t)p.V << 23) + 2ull, 0u};
         P = ceil_mul(p.top_p, D);
+    };
+    // ... from its sum in double precision, if there are such; `dead`: with tokens that weigh nothing
+    const bool fine = v.fine != nullptr;
+    const uint4 *fines = fine ? reinterpret_cast<const uint4 *>(v.fine + (size_t)row * G) : reinterpret_cast<const uint4 *>(hdrs);
+    auto fine_in = [&](const uint4 &h, const uint4 &f, const float M, bool &dead) __attribute__((always_inline)) {
+        const float d = M - __builtin_floorf(fkey_inv(h.x));
+        dead = dead || fkey_inv(f.z) < M - 39.0f;
+        return (uint64_t)__builtin_ldexp(__builtin_bit_cast(double, ((uint64_t)f.y << 32) | f.x), 40 - (d >= 64.0f ? 64 : (int)d));
     };
     if (kEach && wave == W) {
         // the wave that draws the random number also adds up the row's mass: neither is wanted before the tokens are listed
@@ -673,16 +703,22 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
         uint4 h[2];
 #pragma unroll
         for (int k = 0; k < 2; ++k) h[k] = *reinterpret_cast<const uint4 *>(&hdrs[min((uint32_t)(lane + k * kWave), G - 1u)]);
+        uint4 f[2];                                      // (the headers again where there are no such sums)
+#pragma unroll
+        for (int k = 0; k < 2; ++k) f[k] = fines[min((uint32_t)(lane + k * kWave), G - 1u)];
         __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_s_barrier();
         draw();
         const float M = __builtin_floorf(fkey_inv(wave_max_u32(max(h[0].x, h[1].x))));
         uint64_t q = 0;
-        bool odd = false;
+        bool odd = false, dead = false;
 #pragma unroll
         for (int k = 0; k < 2; ++k)
-            if ((uint32_t)(lane + k * kWave) < G) { q += mass_in(h[k], M); odd = odd || (h[k].y & kSieveOdd) != 0u; }
-        estimate(wave_sum(q), __builtin_amdgcn_ballot_w64(odd) != 0ull);
+            if ((uint32_t)(lane + k * kWave) < G) {
+                q += fine ? fine_in(h[k], f[k], M, dead) : mass_in(h[k], M);
+                odd = odd || (h[k].y & kSieveOdd) != 0u;
+            }
+        estimate(wave_sum(q), __builtin_amdgcn_ballot_w64(odd) != 0ull, (fine ? 2u : 0u) | (__builtin_amdgcn_ballot_w64(dead) != 0ull ? 1u : 0u));
         if (lane == 0) { L.one.D = D; L.one.P = P; L.one.err = err; }
         __syncthreads();
         return;
@@ -695,7 +731,8 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
     uint4 keys[kHdrs];
 #pragma unroll
     for (int k = 0; k < kHdrs; ++k) keys[k] = *reinterpret_cast<const uint4 *>(&hdrs[min((uint32_t)(lane + k * kWave), G - 1u)]);
-    uint4 h = *reinterpret_cast<const uint4 *>(&hdrs[min(sl, G - 1u)]);
+    uint4 h = *reinterpret_cast<const uint4 *>(&hdrs[min(sl, G - 1u)]), fh = make_uint4(0u, 0u, 0u, 0u);
+    if (!kEach) fh = fines[min(sl, G - 1u)];
     uint64_t pre[PRE];                                   // (units beyond the row's read its last one again)
     auto ask = [&]() __attribute__((always_inline)) {
 #pragma unroll
@@ -726,8 +763,10 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
     const uint32_t from = max(e_cut + 1u, kEMinBits);
     if constexpr (!kEach) {
         const uint64_t coarse = __builtin_amdgcn_ballot_w64(mine && (h.y & kSieveOdd) != 0u);
-        const uint64_t q = wave_sum(mine && half == 0u ? mass_in(h, M) : 0ull);
-        if (lane == 0) L.sum[wave] = q | (coarse != 0ull ? 1ull << 63 : 0ull);
+        bool dead = false;
+        const uint64_t q = wave_sum(mine && half == 0u ? fine ? fine_in(h, fh, M, dead) : mass_in(h, M) : 0ull);
+        const uint64_t with_dead = __builtin_amdgcn_ballot_w64(dead);
+        if (lane == 0) L.sum[wave] = q | (coarse != 0ull ? 1ull << 63 : 0ull) | (with_dead != 0ull ? 1ull << 62 : 0ull);
     }
     uint32_t b[PRE];                                     // bits of e, 0 for what is not a token of the complete part
     auto look_at = [&](auto each) __attribute__((always_inline)) {
@@ -754,10 +793,11 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
     auto total = [&]() __attribute__((always_inline)) {                                 // by then somebody has added up the slices' sums
         if constexpr (kEach) { D = uniform(L.one.D); P = uniform(L.one.P); err = uniform(L.one.err); }
         else {
-            uint64_t all = 0, odd = 0;
+            uint64_t all = 0, what = 0;
 #pragma unroll
-            for (int w = 0; w < W; ++w) { all += L.sum[w] & ~(1ull << 63); odd |= L.sum[w] >> 63; }
-            estimate(uniform(all), uniform((uint32_t)odd) != 0u);
+            for (int w = 0; w < W; ++w) { all += L.sum[w] & ~(3ull << 62); what |= L.sum[w] >> 62; }
+            const uint32_t bits = uniform((uint32_t)what);
+            estimate(uniform(all), (bits & 2u) != 0u, (fine ? 2u : 0u) | (bits & 1u));
         }
     };
     // a row finished from a list of at most 64 tokens that holds its kept set: the token + 1 in one lane of the first wave; 0 in `doubts` when
@@ -991,7 +1031,7 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
         if (__builtin_expect(again || !listed, 0)) {
             sieve_pens_back<NT>(params_again(), v, row);
             const bool close = listed && !p.diag && !p.e_bits;
-            D = close ? sieve_closer<NT>(params_again(), L, row, M) : sieve_exact<NT>(params_again(), L, row, M);
+            D = sieve_again<NT>(params_again(), L, row, M, close);
             err = close ? M96{(D.lo >> 38) | ((uint64_t)D.hi << 26), 0u} + M96{1ull << 24, 0u} : M96{0ull, 0u};
             if (!listed) {
                 // the tokens set aside were not enough, or more than the list holds: the row's own bins, and its tokens at or above the boundary bin
@@ -1071,7 +1111,7 @@ __global__ void __launch_bounds__(finish_threads<NT>()) sieve_finish_kernel(cons
             }
             // the pick: kept weights by bucket of the token index, NT buckets a step, then the bucket's tokens
             auto weight = [=](uint32_t e) -> uint64_t { return e > thr ? w_of_bits(e) : e == thr ? w_tie : 0ull; };
-            constexpr uint32_t kLogNT = NT == 256 ? 8u : 10u;
+            constexpr uint32_t kLogNT = NT == 256 ? 8u : NT == 512 ? 9u : 10u;
             uint32_t sh = 32u - (uint32_t)__builtin_clz((uint32_t)p.V - 1u | 1u);
             sh = sh > kLogNT ? sh - kLogNT : 0u;
             uint32_t lo_idx = 0, len = (uint32_t)p.V;

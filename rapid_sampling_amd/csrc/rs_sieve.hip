@@ -3,17 +3,18 @@
 
 namespace rs {
 
-// The finishing workgroup by the units of 64 tokens that the row's slices may set aside.  (1024 threads with top_k beyond 256, as launch_finish has
-// it, were no faster: 128 x 1048576 top_k 1024 104.0 us with them, 103.8 without; 128 x 262144 top_k 300 38.3 / 34.7.)
+// The finishing workgroup by the units of 64 tokens that the row's slices may set aside, 16 to a wave at most.  (1024 threads with top_k beyond 256, as
+// launch_finish has it, were no faster: 128 x 262144 top_k 300 38.3 us a call with them, 34.7 with 256; between 65 and 128 units 128 x 1048576 top_k 1024 takes
+// 102.7 us with 1024 threads, 100.5 with 512, 16 x 1048576 top_k 50 23.0 / 22.8.)
 static void launch_sieve_finish(uint32_t B, hipStream_t st, const Params &p, const SieveView &v)
 {
     const uint32_t n = v.G * v.units;
-#define RS_FIN(NTv, PREv) hipLaunchKernelGGL((sieve_finish_kernel<NTv, PREv>), dim3(B), dim3(finish_threads<NTv>()), 0, st, p, v)
+#define RS_FIN(NTv, PREv) hipLaunchKernelGGL((sieve_finish_kernel<NTv, PREv>), dim3(B), dim3(sieve_finish_threads<NTv>()), 0, st, p, v)
     if (n > 128u) RS_FIN(1024, 16);
+    else if (n > 64u) RS_FIN(512, 16);
     else if (n <= 16u) RS_FIN(256, 4);
     else if (n <= 32u) RS_FIN(256, 8);
-    else if (n <= 64u) RS_FIN(256, 16);
-    else RS_FIN(256, 32);
+    else RS_FIN(256, 16);
 #undef RS_FIN
 }
 
@@ -21,13 +22,12 @@ hipError_t launch_sieve(int R, int32_t dtype, uint32_t B, hipStream_t st, const 
 {
     const dim3 grid(B * v.G);
     if (v.G > 128u || v.G * v.units > 256u) return hipErrorInvalidValue;               // what the finishing workgroup asks for
-#define RS_SIEVE(Rv) do {                                                                                                                \
-        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_F32>), grid, dim3(kThreads), 0, st, p, v);                 \
-        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_BF16>), grid, dim3(kThreads), 0, st, p, v);          \
-        else hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_F16>), grid, dim3(kThreads), 0, st, p, v); } while (0)
-    if (R == 16) RS_SIEVE(16);
-    else if (R == 8) RS_SIEVE(8);
-    else RS_SIEVE(4);
+#define RS_SIEVE(Rv, FINEv) do {                                                                                                                \
+        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_F32, FINEv>), grid, dim3(kThreads), 0, st, p, v);                 \
+        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_BF16, FINEv>), grid, dim3(kThreads), 0, st, p, v);          \
+        else hipLaunchKernelGGL((sieve_kernel<Rv, RS_DTYPE_F16, FINEv>), grid, dim3(kThreads), 0, st, p, v); } while (0)
+    if (v.fine) { if (R == 16) RS_SIEVE(16, true); else if (R == 8) RS_SIEVE(8, true); else RS_SIEVE(4, true); }
+    else { if (R == 16) RS_SIEVE(16, false); else if (R == 8) RS_SIEVE(8, false); else RS_SIEVE(4, false); }
 #undef RS_SIEVE
     launch_sieve_finish(B, st, p, v);
     return hipGetLastError();
@@ -37,12 +37,12 @@ hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, co
 {
     const dim3 grid(B * v.G);
     if (v.G > 128u || v.G * v.units > 256u || (R != 4 && R != 8) || v.note_cap != sieve_pen_cap(R)) return hipErrorInvalidValue;
-#define RS_SIEVE(Rv) do {                                                                                                                     \
-        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F32>), grid, dim3(kThreads), 0, st, p, v);                  \
-        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_BF16>), grid, dim3(kThreads), 0, st, p, v);           \
-        else hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F16>), grid, dim3(kThreads), 0, st, p, v); } while (0)
-    if (R == 8) RS_SIEVE(8);
-    else RS_SIEVE(4);
+#define RS_SIEVE(Rv, FINEv) do {                                                                                                                     \
+        if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F32, FINEv>), grid, dim3(kThreads), 0, st, p, v);                  \
+        else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_BF16, FINEv>), grid, dim3(kThreads), 0, st, p, v);           \
+        else hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F16, FINEv>), grid, dim3(kThreads), 0, st, p, v); } while (0)
+    if (v.fine) { if (R == 8) RS_SIEVE(8, true); else RS_SIEVE(4, true); }
+    else { if (R == 8) RS_SIEVE(8, false); else RS_SIEVE(4, false); }
 #undef RS_SIEVE
     launch_sieve_finish(B, st, p, v);
     if (R == 8) hipLaunchKernelGGL((sieve_pen_fix_kernel<8>), dim3(B * kSieveFixers), dim3(kThreads), 0, st, p, v);

@@ -13,8 +13,15 @@ struct SieveHdr {                                        // 16 bytes
 };
 constexpr uint32_t kSieveTie = 1u << 31, kSieveOdd = 1u << 30;     // kSieveOdd, with any n: a wave's sum was worked out in a frame
 
+struct SieveFine {                                       // 16 bytes
+    double   mass;           // the sum of the slice's e, in its frame
+    uint32_t low;            // fkey(min x of the slice)
+    uint32_t pad;
+};
+
 struct SieveView {
     SieveHdr *hdr;           // [B][G]
+    SieveFine *fine;         // [B][G], or null: the passes' sums are those of the headers
     uint64_t *stash;         // [B][G][64 * units]   bits of x << 32 | index, in no order
     uint32_t  G;             // slices per row
     uint32_t  units;         // a slice sets aside at most 64 tokens (1) or 128 (2)

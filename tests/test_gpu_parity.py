@@ -2260,7 +2260,7 @@ def _sieve_rows(V, n_kinds=12):
 
 @pytest.mark.parametrize("V,fmt,k", [(16388, "float32", 40), (49152, "float32", 1), (50260, "bfloat16", 50), (65536, "float16", 64), (131072, "float32", 64), (131076, "bfloat16", 20),
                                      (262148, "float32", 50), (528384, "float32", 40), (1048576, "bfloat16", 40), (65540, "float32", 100), (131072, "float32", 128),
-                                     (131072, "bfloat16", 300), (262144, "float32", 1000), (1048576, "float32", 1024)])
+                                     (131072, "bfloat16", 300), (262144, "float32", 320), (1048576, "float32", 1024), (1048576, "float32", 50), (300000, "float16", 400)])
 def test_sieve_path(torch_cuda, oracle, V, fmt, k):
     """The sieve path in slices of 4096, 8192 and 16384 tokens that set 64 or 128 of them aside, its short lists (top_k up to 64) and its long
     ones: every kind of row over and over, as many as the path is taken for, tokens against the oracle without the diagnostics record -- which
@@ -2270,7 +2270,9 @@ def test_sieve_path(torch_cuda, oracle, V, fmt, k):
     dt = getattr(torch, fmt)
     lg = torch.from_numpy(_sieve_rows(V)).to(dt).float().numpy()
     n = lg.shape[0]
-    least = 49152 if k <= 64 else 1 << 24 if k <= 128 else 1 << 25 if V <= 262144 else 1 << 26
+    least = 49152 if k <= 64 else 1 << 24
+    if V == 1048576 and fmt == "float32":
+        least = 1 << 26                                                 # the pass that sums in double precision
     B = max(n, (least + V - 1) // V)
     reps = (B + n - 1) // n
     B = reps * n
