@@ -44,7 +44,7 @@ HBM_PEAK_GBS = 8000.0   # MI355X HBM3E, vendor figure
 # HBM bytes per call of the bandwidth configuration from the rocprofv3 FETCH_SIZE / WRITE_SIZE runs
 # summarised in the file named here, valid for the library version they were taken with: a library
 # that has moved on reports traffic as null rather than a stale figure.
-TRAFFIC_PROFILE = {"file": "profiles/bench_kernels_hbm_traffic_pmc.md", "rs_version": 418, "bytes": 575099802}
+TRAFFIC_PROFILE = {"file": "profiles/bench_kernels_hbm_traffic_pmc.md", "rs_version": 419, "bytes": 555307418}
 
 
 def event_times_us(torch, fn, steps, warmup):
@@ -288,8 +288,8 @@ def main():
             "workload": "(B,T,V)=(128,4,1048576) N(0,1.5), top_k 1024, top_p 0.95: 128 sampled rows of 4 MiB, "
                         "stride T*V, algorithmic bytes 4*V per row = 512 MiB per call",
             "us_per_call": round(t_btv, 2), "rows_per_s": round(Bb / (t_btv * 1e-6), 1),
-            "kernels": "streaming path, two launches per call: rs::stream_kernel (reads the logits; dominant) and "
-                       "rs::finish_kernel; achieved = bytes / time of the whole call",
+            "kernels": "sieve path, two launches per call: rs::sieve_kernel (reads the logits; dominant) and "
+                       "rs::sieve_finish_kernel; achieved = bytes / time of the whole call",
             "cluster_path_us_per_call": round(t_cluster, 2),
             "read_peak_GBs": round(bytes_btv / (t_floor * 1e-6) / 1e9, 1),
             "frac_of_read_peak": round(t_floor / t_btv, 4),
@@ -335,8 +335,8 @@ def main():
             "us_per_call": round(t_pen, 2), "achieved": round(Bb * Vb * 12 / (t_pen * 1e-6) / 1e9, 1),
             "frac": round(Bb * Vb * 12 / (t_pen * 1e-6) / 1e9 / HBM_PEAK_GBS, 4),
             "note": "(128,1048576) fp32 rows (stride T*V) with a (128,1048576) penalties tensor, 2 % non-zero: "
-                    "rs::stream_pen_kernel (reads both, writes the decayed penalties), rs::finish_kernel (patches the sampled "
-                    "tokens), rs::penalty_fix_kernel (slices the pass deferred: none here); algorithmic bytes 12*V per row"}
+                    "rs::sieve_pen_kernel (reads both, writes the decayed penalties), rs::sieve_finish_kernel, "
+                    "rs::sieve_pen_fix_kernel (patches the sampled tokens, rewrites what the pass left: nothing here); algorithmic bytes 12*V per row"}
         del pen_b, last
         # kept sets of thousands of tokens (calls of this size take the one-pass wide path: a look at a sample of
         # each row, one pass over the logits, a finish per row): the same rows with top_k 10000, and 512 flat

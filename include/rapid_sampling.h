@@ -53,7 +53,7 @@ typedef struct rs_row_diag {
     uint32_t left_bits;   /* same as thr_bits                                 */
     uint32_t thr_bits;    /* bit pattern of the smallest kept e               */
     uint32_t rounds;      /* histogram levels summed over the cluster; 0 = row
-                             finished by the streaming path, 8 = by its
+                             finished by the streaming or the sieve path, 8 = by its
                              finishing workgroup alone from the logits, 9 = a
                              call that keeps every token (top_k = V, top_p = 1)
                              on the streaming path                            */
@@ -91,7 +91,8 @@ int rs_normalize_args(double temperature, int64_t top_k, double top_p,
  * the non-zero penalties; up to 3.2 bytes per token for the first 6M tokens,
  * where slices are shorter; 1.5 bytes per token in rows of up to 262144
  * tokens, for the slices of 8192 tokens the one-pass wide path, the
- * counting-only pass and the pass with penalties cut there); a quarter to two fifths of the reference's
+ * counting-only pass and the pass with penalties cut there; the sieve path lays
+ * its own records, 1.1 bytes per token at most, over the same space); a quarter to two fifths of the reference's
  * scratch.  It does not grow with T.  (A call is also accepted with a
  * workspace that lacks the room for those slices of 8192 tokens -- the size
  * versions before 414 asked for -- and then works on the long slices.)

@@ -44,7 +44,8 @@
 //   sieve path (sieve_kernel + sieve_finish_kernel, two launches, no waits): the streaming
 //     path's calls with a top_k of up to 64, and larger calls with more.  The pass sums the
 //     row approximately and sets its largest tokens aside; the finish makes sure that nothing
-//     it decides depends on what the sum is off by.
+//     it decides depends on what the sum is off by.  With penalties (sieve_pen_kernel,
+//     the same finish, sieve_pen_fix_kernel): the pass writes the decayed penalties, too.
 //
 //   wide path (stream_kernel counting only + wide_kernel + wide_finish_kernel,
 //     three launches, no waits): kept sets of thousands of tokens (top_k > 1024,
@@ -54,7 +55,8 @@
 //
 //   row kernel (row_kernel, one launch, no workspace, no waits): the same kept sets
 //     in rows of up to 65536 tokens when the call has rows enough to fill the GPU
-//     with one workgroup of 1024 threads per row, the row in its registers.
+//     with one workgroup of 1024 threads per row, the row in its registers; and a
+//     bounding top_k of hundreds in such calls.
 //
 //   one-launch path (fused_kernel): the streaming pass and the finish in one
 //     grid, for calls with penalties that fit the device at once.
