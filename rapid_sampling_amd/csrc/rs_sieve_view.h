@@ -34,8 +34,9 @@ struct SieveView {
 };
 constexpr uint32_t kSievePenLeft = 0xFFFFFFFFu;          // the wave's penalties are still the old ones: to be rewritten by the fix-up kernel
 constexpr uint32_t kSieveFixers = 8;                      // workgroups of the fix-up kernel to a row
-// Of a wave's 64 R groups, 3 in 16: 4 to 5 % of the tokens by chance, or 19 % side by side.
-__host__ __device__ constexpr uint32_t sieve_pen_cap(int R) { return 12u * (uint32_t)R; }
+// Of a wave's 64 R groups, 11 in 64: some 4 % of the tokens by chance, or 17 % side by side; as many as a workspace of rs_workspace_bytes has room
+// for in rows of a million tokens.
+__host__ __device__ constexpr uint32_t sieve_pen_cap(int R) { return 11u * (uint32_t)R; }
 
 // R: groups of four tokens of a thread, 4, 8 or 16: slices of 1024 R tokens; with penalties 4 or 8
 hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v);
