@@ -648,12 +648,12 @@ static int choose_path(int32_t B, int32_t V, int32_t top_k, float top_p, bool pe
     };
     // The one-launch path by default: calls with penalties whose kept set is bounded by top_k (the
     // general kernel, the only other way with penalties, spends most of its time in exchanges).  Where the sieve path suits the call its three
-    // launches, most of it at the memory's rate, are shorter from a million tokens on, one launch / three, us a call (top_k 50):
-    //     8 x  50304 12.1 / 12.7     8 x 131072 13.3 / 12.8     1 x 1048576 16.4 / 16.7    16 x 131072 14.8 / 13.6    64 x 32768 14.3 / 14.1
-    //    64 x  50304 16.4 / 15.4    32 x 131072 17.1 / 16.1     4 x 1048576 22.0 / 19.3   128 x  50304 25.6 / 20.1    48 x 131072 24.4 / 19.0
+    // launches, most of it at the memory's rate, are shorter from some 3 million tokens on; one launch / three, us a call (top_k 50), with 2 % of
+    // the penalties non-zero and, behind it, with all of them, which the fix-up kernel then rewrites:
+    //     8 x 131072 13.3 / 13.6, 13.1 / 15       16 x 131072 14.7 / 14.5, 15.0 / 15.9     64 x  50304 17.3 / 16.3, 18.2 / 18.0
+    //    32 x 131072 18.4 / 17.0, 18.9 / 19.1    100 x  50304 23.6 / 18.2, 24.4 / 20.8    256 x  20000 25.2 / 18.7, 26.4 / 20.7
     const bool one_launch = force == RS_PATH_AUTO && pen && bounded && fused_r(B, V, pen, false) != 0;
-    if (one_launch && sieve_pen_r(B, V, top_k) && (uint64_t)B * (uint64_t)V >= (V <= kMidMaxV ? 1u << 20 : 1u << 21) && !(opt && opt->slice_r) &&
-        !routed_away(0)) return kPathStream;
+    if (one_launch && sieve_pen_r(B, V, top_k) && (uint64_t)B * (uint64_t)V >= 3u << 20 && !(opt && opt->slice_r) && !routed_away(0)) return kPathStream;
     if (one_launch) return kPathFused;
     // Larger calls with penalties: the streaming pass that also writes the decayed penalties, its finish and a fix-up, three
     // launches, from kPenStreamMin tokens on.
@@ -966,6 +966,7 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
         v.reach = sieve_reach(V, top_k, R, v.units);
         const size_t slices = (size_t)B * v.G, hdr = align256(sizeof(WsHeader)), stash = align256(hdr + slices * sizeof(SieveHdr));
         v.note_cap = sieve_pen_cap(R);
+        v.fixers = min(v.G, max(8u, 1536u / (uint32_t)B));           // (a slice each while that is not many workgroups)
         const size_t noted = align256(stash + slices * v.units * kWave * sizeof(uint64_t)), waves = slices * kWaves;
         const size_t note_at = align256(noted + waves * sizeof(uint32_t)), note_old = align256(note_at + waves * v.note_cap * sizeof(uint32_t));
         const size_t fine = pen ? align256(note_old + waves * v.note_cap * sizeof(float4)) : noted;

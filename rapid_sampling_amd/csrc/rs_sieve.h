@@ -414,24 +414,25 @@ __global__ void __launch_bounds__(kThreads, R == 8 ? 4 : 6) sieve_pen_kernel(con
 }
 
 // The sampled token's penalty, pen <- fma(pen, decay, pen == 0 ? presence : repetition) (sampling.cu:427-437), the old value from the notes
-// (+0.0 when its group is not among them), and all penalties of the waves that left theirs.  kSieveFixers workgroups to a row, each for every
-// kSieveFixers-th slice, wave w for wave w's part of them: mostly it is one look at some words and a chain of two loads for the one token (4.7 us
-// behind 128 x 262144 tokens, with 2, 8 or a workgroup per slice alike).
+// (+0.0 when its group is not among them), and all penalties of the waves that left theirs.  v.fixers workgroups to a row, each for every
+// v.fixers-th slice, wave w for wave w's part of them: mostly it is one look at some words and a chain of two loads for the one token (4.7 us
+// behind 128 x 262144 tokens, with 2, 8 or 32 workgroups to a row alike; but rows of nothing but non-zero penalties
+// pay for every slice that a workgroup does after another: 64 x 50304 21.9 us a call with 8, 17.7 with 32).
 template <int R>
 __global__ void __launch_bounds__(kThreads) sieve_pen_fix_kernel(const Params p, const SieveView v)
 {
     constexpr uint32_t kCap = sieve_pen_cap(R);
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = (int)uniform((uint32_t)tid >> 6);
-    const uint32_t row = blockIdx.x / kSieveFixers, first = blockIdx.x - row * kSieveFixers, G = v.G;
-    const uint32_t part = first + (uint32_t)lane * kSieveFixers;         // the lane's slice (at most 64 of them: G <= 256)
+    const uint32_t row = blockIdx.x / v.fixers, first = blockIdx.x - row * v.fixers, G = v.G;
+    const uint32_t part = first + (uint32_t)lane * v.fixers;         // the lane's slice (64 of them at most)
     const uint32_t *noted = v.noted + (size_t)row * G * kWaves;
     const uint32_t n = noted[min(part, G - 1u) * (uint32_t)kWaves + (uint32_t)wave], token = uniform((uint32_t)p.out[row]);
     const uint32_t V4 = (uint32_t)p.V >> 2, group = token >> 2;
     float *pens = p.penalties + (int64_t)row * p.V;
     uint64_t to_do = __builtin_amdgcn_ballot_w64(part < G && n == kSievePenLeft);
     // the sampled token's slice, if it is one of this workgroup's and its group this wave's, and the penalties have been written
-    const uint32_t its = group / (uint32_t)(R * kThreads), l = its / kSieveFixers;
-    if (token < (uint32_t)p.V && its - l * kSieveFixers == first && ((group >> 6) & (uint32_t)(kWaves - 1)) == (uint32_t)wave && !(to_do >> l & 1ull)) {
+    const uint32_t its = group / (uint32_t)(R * kThreads), l = its / v.fixers;
+    if (token < (uint32_t)p.V && its - l * v.fixers == first && ((group >> 6) & (uint32_t)(kWaves - 1)) == (uint32_t)wave && !(to_do >> l & 1ull)) {
         const size_t rec = (((size_t)row * G + its) * kWaves + (size_t)wave) * kCap;
         const uint32_t have = min(lane_of(n, l), kCap);
         constexpr uint32_t kLooks = (kCap + kWave - 1u) / kWave;
@@ -450,7 +451,7 @@ __global__ void __launch_bounds__(kThreads) sieve_pen_fix_kernel(const Params p,
         if (found ? mine : lane == 0) pens[token] = __builtin_fmaf(o, p.decay, o == 0.0f ? p.presence : p.repetition);
     }
     while (to_do) {
-        const uint32_t at = first + (uint32_t)__builtin_ctzll(to_do) * kSieveFixers;
+        const uint32_t at = first + (uint32_t)__builtin_ctzll(to_do) * v.fixers;
         to_do &= to_do - 1ull;
         float4 w[R];
         uint32_t g[R];

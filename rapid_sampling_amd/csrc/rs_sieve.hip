@@ -36,7 +36,7 @@ hipError_t launch_sieve(int R, int32_t dtype, uint32_t B, hipStream_t st, const 
 hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v)
 {
     const dim3 grid(B * v.G);
-    if (v.G > 128u || v.G * v.units > 256u || (R != 4 && R != 8) || v.note_cap != sieve_pen_cap(R)) return hipErrorInvalidValue;
+    if (v.G > 128u || v.G * v.units > 256u || (R != 4 && R != 8) || v.note_cap != sieve_pen_cap(R) || v.fixers == 0u || (v.G + v.fixers - 1u) / v.fixers > 64u) return hipErrorInvalidValue;
 #define RS_SIEVE(Rv, FINEv) do {                                                                                                                     \
         if (dtype == RS_DTYPE_F32) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_F32, FINEv>), grid, dim3(kThreads), 0, st, p, v);                  \
         else if (dtype == RS_DTYPE_BF16) hipLaunchKernelGGL((sieve_pen_kernel<Rv, RS_DTYPE_BF16, FINEv>), grid, dim3(kThreads), 0, st, p, v);           \
@@ -45,8 +45,8 @@ hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, co
     else { if (R == 8) RS_SIEVE(8, false); else RS_SIEVE(4, false); }
 #undef RS_SIEVE
     launch_sieve_finish(B, st, p, v);
-    if (R == 8) hipLaunchKernelGGL((sieve_pen_fix_kernel<8>), dim3(B * kSieveFixers), dim3(kThreads), 0, st, p, v);
-    else hipLaunchKernelGGL((sieve_pen_fix_kernel<4>), dim3(B * kSieveFixers), dim3(kThreads), 0, st, p, v);
+    if (R == 8) hipLaunchKernelGGL((sieve_pen_fix_kernel<8>), dim3(B * v.fixers), dim3(kThreads), 0, st, p, v);
+    else hipLaunchKernelGGL((sieve_pen_fix_kernel<4>), dim3(B * v.fixers), dim3(kThreads), 0, st, p, v);
     return hipGetLastError();
 }
 

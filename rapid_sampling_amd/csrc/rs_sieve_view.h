@@ -31,9 +31,9 @@ struct SieveView {
     uint32_t *note_at;       // [B][G][4][note_cap]  which groups of the row
     float4   *note_old;      // [B][G][4][note_cap]  their penalties
     uint32_t  note_cap;      // sieve_pen_cap of the slices' length
+    uint32_t  fixers;        // workgroups of the fix-up kernel to a row
 };
 constexpr uint32_t kSievePenLeft = 0xFFFFFFFFu;          // the wave's penalties are still the old ones: to be rewritten by the fix-up kernel
-constexpr uint32_t kSieveFixers = 8;                      // workgroups of the fix-up kernel to a row
 // Of a wave's 64 R groups, 11 in 64: some 4 % of the tokens by chance, or 17 % side by side; as many as a workspace of rs_workspace_bytes has room
 // for in rows of a million tokens.
 __host__ __device__ constexpr uint32_t sieve_pen_cap(int R) { return 11u * (uint32_t)R; }
