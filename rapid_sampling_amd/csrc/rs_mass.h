@@ -274,7 +274,7 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     const bool split = n > 16u, in = (uint32_t)lane < n;
     uint32_t larger = 0, before = 0;
     if (wave < (split ? 4 : kLook ? 2 : 1)) {
-        const uint32_t each = split ? (n + 3u) >> 2 : n, j0 = split ? (uint32_t)wave * each : 0u, j1 = min(n, j0 + each);
+        const uint32_t each = split ? (n + 3u) >> 2 : n, j0 = kLook && !split ? 0u : (uint32_t)wave * each, j1 = min(n, j0 + each);
 #pragma unroll 4
         for (uint32_t j = j0; j < j1; ++j) {
             const uint64_t o = list[j];
@@ -293,6 +293,7 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const uint32_t b = in ? (uint32_t)(s.sorted[lane] >> 32) : 0u;
     const Limbs own = limbs(M96{in ? w_of_bits(b) : 0ull, 0u}), upto = wave_inclusive_scan(own);
+    const uint64_t random = *rand64;                     // (asked for here, wanted for the target)
     const Totals t = totals(upto);
     const M96 D = t.D, P = t.P;
     const uint64_t enough = __builtin_amdgcn_ballot_w64(in && ((uint32_t)lane + 1u >= top_k || m96(upto) >= P));
@@ -300,7 +301,7 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     const uint32_t n_gt = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b > thr));
     const uint32_t n_eq = (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(b == thr));
     const M96 above = m96(lane_of(upto - own, n_gt));
-    const Target tg = tie_and_target(p, row, uniform(*rand64), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(above), rounds, lane == 0 && wave == 0);
+    const Target tg = tie_and_target(p, row, uniform(random), xmax, wide(D), wide(P), thr, n_gt, n_eq, wide(above), rounds, lane == 0 && (!kLook || wave == 0));
     if constexpr (kLook) {
         if (wave != 0) { decided(P, enough != 0ull, n_gt, n_eq, thr, above, tg.w_tie); return 0u; }
     }
