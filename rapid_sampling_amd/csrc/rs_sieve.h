@@ -578,11 +578,13 @@ __device__ __forceinline__ void sieve_row_pass(const Params &p, const uint32_t r
 
 // The row's D from its logits.  `close`: in double precision, 2^-40 of it off at most (D >= 1; a thread adds fewer than 2^13 terms).  Else exactly: all of
 // its tokens are counted into L.bins, which is left that way (with e_bits also the e of every token, dead ones as 0).
+// The barrier at its start is between the waves that may still read L.bins (each wave searches them for itself in level1) and those that clear them.
 template <int NT>
 __device__ __forceinline__ M96 sieve_again(const Params &p, LdsSieveFin<NT> &L, const uint32_t row, const float M, const bool close)
 {
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid >> 6;
     uint4 *eb4 = p.e_bits ? reinterpret_cast<uint4 *>(p.e_bits + (int64_t)row * p.V) : nullptr;
+    __syncthreads();
     for (int i = tid; i < kSieveCopies * (kNB + 4); i += NT) (&L.bins[0][0])[i] = 0ull;
     __syncthreads();
     uint64_t *bins = L.bins[lane & (kSieveCopies - 1)];

@@ -2450,3 +2450,26 @@ def test_row_kernel_boundaries_of_a_few_tokens(torch_cuda, oracle, B, V):
         _check(res, np.tile(ref_out, reps), np.tile(ref_diag, reps), "row kernel, few at the boundary")
         assert smp.status() == 0
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,k", [(128, 131072, 65), (128, 131072, 300), (64, 262144, 200), (24, 1048576, 128)])
+def test_sieve_path_diagnostics_of_long_lists(torch_cuda, oracle, B, V, k):
+    """Calls without penalties that ask for diagnostics of lists of more than 64 tokens: every row's total is made again right behind the search of
+    its bins, which all waves must have done before they are cleared.  Rows of many kinds, several times, every field against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    lg = _sieve_rows(V)
+    n = lg.shape[0]
+    reps = -(-B // n)
+    x = torch.from_numpy(lg).cuda().repeat(reps, 1).contiguous()
+    smp = capi.Sampler(reps * n, V)
+    for top_p in (0.9, 0.4):
+        u_np = H.uniforms(n, k)
+        rc, c, kk, p = capi.normalize(1.0, k, top_p, V, reps * n, 1)
+        ref_out, ref_diag = oracle.sample_batch(lg, c, kk, p, injected_u=u_np)
+        u = torch.from_numpy(np.tile(u_np, reps)).cuda()
+        for turn in range(5):
+            print("sieve path, diagnostics:", reps * n, V, k, top_p, turn, flush=True)
+            _check(smp.sample(x, c, kk, p, uniforms=u, path="stream"), np.tile(ref_out, reps), np.tile(ref_diag, reps), "sieve path, diagnostics")
+            assert smp.status() == 0
+    smp.close()
