@@ -156,6 +156,13 @@ class Sampler:
         assert rc == 0
         return st.value
 
+    def rows_again(self):
+        """Rows that the last call, if it took the sieve path, summed again from their logits (WsHeader::n_again): with diagnostics all of
+        them but those of equal tokens.  Sets the word to 0, which other paths leave as it is."""
+        n = int(self.ws[:4].view(self.torch.int32).item())
+        self.ws[:4] = 0
+        return n
+
     def where(self):
         """(wait, row, slice, seen, wanted) of the first wait that gave up; wait 0 = none."""
         w = (C.c_uint32 * 4)()

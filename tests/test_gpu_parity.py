@@ -2473,3 +2473,46 @@ def test_sieve_path_diagnostics_of_long_lists(torch_cuda, oracle, B, V, k):
             _check(smp.sample(x, c, kk, p, uniforms=u, path="stream"), np.tile(ref_out, reps), np.tile(ref_diag, reps), "sieve path, diagnostics")
             assert smp.status() == 0
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,k,dtype,share,path,sieve", [
+    (3, 16380, 40, "float32", 0.0, None, False), (4, 16388, 64, "float32", 0.0, None, True), (2, 16388, 64, "float32", 0.0, None, False),
+    (1, 50304, 50, "bfloat16", 0.0, None, True), (64, 131072, 65, "float32", 0.0, None, False), (128, 131072, 65, "float32", 0.0, None, True),
+    (128, 131072, 320, "float16", 0.0, "stream", True), (128, 131072, 321, "float32", 0.0, "stream", False), (20, 1048576, 1024, "float32", 0.0, None, True),
+    (16, 1048576, 512, "float32", 0.0, None, True), (64, 1048576, 50, "float32", 0.0, None, True), (20, 1048576, 600, "bfloat16", 0.0, None, True),
+    (23, 131072, 50, "float32", 0.02, None, False), (24, 131072, 50, "float32", 0.02, None, True), (24, 131072, 65, "float32", 0.02, None, False),
+    (256, 65536, 128, "float32", 0.02, None, True), (128, 131072, 50, "bfloat16", 0.02, None, True), (128, 131072, 50, "float16", 0.02, None, True),
+    (128, 131072, 129, "float32", 0.02, None, False), (64, 1048576, 1024, "float32", 0.02, None, True)])
+def test_which_calls_take_the_sieve_path(torch_cuda, oracle, B, V, k, dtype, share, path, sieve):
+    """Seen by the rows it sums again for the diagnostics: the edges of its rule, and calls for each of its kernels -- slices of 4096, 8192 and 16384 tokens,
+    the three formats, float and double sums, with penalties and without.  Some kinds of rows over and over, in every field against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    dt = getattr(torch, dtype)
+    n = min(B, 6)
+    lg = torch.from_numpy(_sieve_rows(V)[[0, 1, 11, 6, 7, 5][:n]]).to(dt).float().numpy()
+    reps = -(-B // n)
+    x = torch.from_numpy(lg).to(dt).cuda().repeat(reps, 1)[:B].contiguous()
+    u_np = H.uniforms(n, k)
+    u = torch.from_numpy(np.tile(u_np, reps)[:B]).cuda()
+    rc, c, kk, p = capi.normalize(0.9, k, 0.9, V, B, 1)
+    pen = H.penalties_sparse(n, V, share, seed=V) if share else None
+    want = pen.copy() if share else None
+    more = dict(presence=0.1, repetition=0.2, decay=0.95) if share else {}
+    ref_out, ref_diag = oracle.sample_batch(lg, c, kk, p, injected_u=u_np, **(dict(more, penalties=want) if share else {}))[:2]
+    smp = capi.Sampler(B, V)
+    for diag in (True, False):
+        have = torch.from_numpy(np.tile(pen, (reps, 1))[:B]).cuda() if share else None
+        print("sieve or not:", B, V, k, dtype, share, path, diag, flush=True)
+        smp.rows_again()
+        res = smp.sample(x, c, kk, p, uniforms=u, want_diag=diag, path=path, penalties=have, **more)
+        assert res["rc"] == 0 and np.array_equal(res["out"], np.tile(ref_out, reps)[:B])
+        again = smp.rows_again()
+        if diag:
+            _check(res, np.tile(ref_out, reps)[:B], np.tile(ref_diag, reps)[:B], "sieve or not")
+            assert again == (B if sieve else 0), again
+        if share:
+            bad = np.argwhere(have.cpu().numpy().view(np.uint32) != np.tile(want, (reps, 1))[:B].view(np.uint32))
+            assert bad.size == 0, bad[:8]
+    assert smp.status() == 0
+    smp.close()
