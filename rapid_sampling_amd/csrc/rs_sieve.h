@@ -491,23 +491,30 @@ struct LdsSieveFin {
 
 // Is a decision that was made with D, and with P = ceil(top_p * D), the one that the exact D makes?  Both may be off by less than
 // `err` (0: they are exact).  What comes out is how far the target r and the running sums may shift against each other for
-// the pick; `unsure` when threshold or tie weight themselves are in doubt.
+// the pick; `unsure` when threshold or tie weight themselves are in doubt.  With top_p = 1 P is the row's total, and that is at least the mass of the
+// tokens that have been seen: they are above no such P, however little the rest of the row weighs.
 struct Doubt { M96 shift; bool unsure; };
-__device__ __forceinline__ Doubt doubt_of(const M96 P, const M96 err, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq, const M96 above,
+__device__ __forceinline__ M96 larger_of(const M96 a, const M96 b)
+{
+    const bool m = a >= b;                               // (by its parts: a choice between two objects would be one between addresses)
+    return M96{m ? a.lo : b.lo, m ? a.hi : b.hi};
+}
+__device__ __forceinline__ Doubt doubt_of(const M96 P, const M96 err, const float top_p, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq, const M96 above,
                                           const uint32_t thr, const uint64_t w_tie)
 {
     Doubt d{M96{0ull, 0u}, false};
     if (!(err.lo | err.hi)) return d;
-    const M96 least = P >= err ? P - err : M96{0ull, 0u}, most = P + err;
+    M96 least = P >= err ? P - err : M96{0ull, 0u};
+    const M96 most = P + err, down = above + m96((u128)w_of_bits(thr) * n_eq);
+    if (top_p >= 1.0f) least = larger_of(least, down);
     // the tokens above the threshold are not enough, those down to it are
     if (n_gt && !(above < least)) d.unsure = true;
-    const M96 down = above + m96((u128)w_of_bits(thr) * n_eq);
     if (n_gt + n_eq < top_k && !(down >= most)) d.unsure = true;
-    // The tie weight is (P - above) / n_eq unless that is more than it can be.  If it is, S and with it r move by u and the running sum by t times
-    // what P is off by, u and t between 0 and 1 (the random number; the ties before the token): by no more than that against each other, and what
-    // the divisions round.
-    const M96 S = above + m96((u128)w_tie * n_eq), n{(uint64_t)n_eq, 0u};
-    if (!(least >= S + n)) d.shift = err + n + M96{2ull, 0u};
+    // The tie weight is (P - above) / n_eq unless that is more than it can be (the threshold's own, or the share that top_k leaves of it).  If it is the
+    // former, S and with it r move by u and the running sum by t times what P is off by, u and t between 0 and 1 (the random number; the ties before
+    // the token): by no more than that against each other, and what the divisions round.
+    const M96 n{(uint64_t)n_eq, 0u};
+    if (!(least >= above + m96((u128)w_tie * n_eq) + n) && !(w_tie == w_of_bits(thr) && least >= down)) d.shift = err + n + M96{2ull, 0u};
     return d;
 }
 // ... and the token whose weight lies at (before, upto] in the running sum, for the target r
@@ -810,13 +817,13 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         M96 e = err;
         return few_pick(p, L.few, row, lane, wave, list, n, top_k,
                         [&](const Limbs &upto) __attribute__((always_inline)) {
-                            if (!all_of_it) return Totals{D, P};
+                            if (!all_of_it) return Totals{D, p.top_p >= 1.0f && n >= top_k ? larger_of(m96(lane_of(upto, 63u)), P) : P};     // (see doubt_of)
                             e = M96{0ull, 0u};           // every live token of the row is there
                             const M96 d = m96(lane_of(upto, 63u));
                             return Totals{d, ceil_mul(p.top_p, d)};
                         }, xmax, &L.rand64, rounds,
                         [&](const M96 &P, bool enough, uint32_t n_gt, uint32_t n_eq, uint32_t thr, const M96 &above, uint64_t w_tie) __attribute__((always_inline)) {
-                            const Doubt d = doubt_of(P, e, top_k, n_gt, n_eq, above, thr, w_tie);
+                            const Doubt d = doubt_of(P, e, p.top_p, top_k, n_gt, n_eq, above, thr, w_tie);
                             doubts = !enough ? 2u : d.unsure ? 1u : 0u;
                             if (lane == 0) L.one.shift = d.shift;
                         }, [&](const M96 &slack) __attribute__((always_inline)) { L.one.slack = slack; });
@@ -873,6 +880,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             if (known) P = ceil_mul(p.top_p, D);
             else if (complete) { err = M96{0ull, 0u}; D = sc.total(); P = ceil_mul(p.top_p, D); }
             else total();
+            if (p.top_p >= 1.0f) P = larger_of(sc.total(), P);       // (see doubt_of)
             // (the largest that P may be: what is listed then holds the kept set whatever the exact D is, and whether another
             // threshold than this one comes of that is asked behind it)
             goal = P + err;
@@ -1028,6 +1036,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
     // ---- threshold and token from the list; a decision too close to call is made again with the row's exact total ----
     bool tell = false;
     for (;; again = true) {
+
         auto from_list = [&](auto fn) {
             for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) fn((uint32_t)(L.list[i] >> 32));
         };
@@ -1104,7 +1113,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
                 const M96 above = f.above + mass_of(f.sum, thr >> 23);
                 const Target tg = tie_and_target(p, row, uniform(L.rand64), xmax, wide(D), wide(P), thr, f.cnt_above, f.cnt_bin, wide(above), 0u, tid == 0);
                 w_tie = uniform(tg.w_tie); r = uniform(m96(tg.r));
-                const Doubt d = doubt_of(P, err, top_k, f.cnt_above, f.cnt_bin, above, thr, w_tie);
+                const Doubt d = doubt_of(P, err, p.top_p, top_k, f.cnt_above, f.cnt_bin, above, thr, w_tie);
                 shift = d.shift;
                 doubts = d.unsure ? 1u : 0u;
             }

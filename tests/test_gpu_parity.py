@@ -2516,3 +2516,33 @@ def test_which_calls_take_the_sieve_path(torch_cuda, oracle, B, V, k, dtype, sha
             assert bad.size == 0, bad[:8]
     assert smp.status() == 0
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,k,temperature,share", [(64, 152064, 50, 0.35, 0.0), (64, 152064, 50, 0.25, 0.0), (13, 50260, 40, 0.3, 0.0), (64, 1048576, 40, 0.2, 0.0),
+                                                     (128, 131072, 300, 0.4, 0.0), (32, 131072, 50, 0.3, 0.02), (128, 131072, 50, 0.3, 0.02)])
+def test_sieve_path_with_top_p_of_one_on_peaked_rows(torch_cuda, oracle, B, V, k, temperature, share):
+    """A low temperature leaves less beyond the top_k tokens than the row's total may be off by.  With top_p = 1 nothing hangs on it: the total is at least
+    what the tokens that were seen weigh.  No row is summed again, or done the slow way; tokens and penalties against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    n = 8
+    lg = np.concatenate([H.logits_spiked(n - 2, V, seed=V), H.logits_spiked(2, V, n_spikes=1, boost=20.0, seed=3)])
+    reps = -(-B // n)
+    x = torch.from_numpy(lg).cuda().repeat(reps, 1)[:B].contiguous()
+    u_np = H.uniforms(n, k)
+    u_np[:2] = [1.0, 1e-30]
+    u = torch.from_numpy(np.tile(u_np, reps)[:B]).cuda()
+    rc, c, kk, p = capi.normalize(temperature, k, 1.0, V, B, 1)
+    pen = H.penalties_sparse(n, V, share, seed=V) if share else None
+    want, have = (pen.copy(), torch.from_numpy(np.tile(pen, (reps, 1))[:B]).cuda()) if share else (None, None)
+    more = dict(presence=0.1, repetition=0.2, decay=0.95) if share else {}
+    ref_out = oracle.sample_batch(lg, c, kk, p, injected_u=u_np, **(dict(more, penalties=want) if share else {}))[0]
+    smp = capi.Sampler(B, V, with_policy=True)
+    smp.rows_again()
+    res = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, penalties=have, **more)
+    again = smp.rows_again()
+    assert np.array_equal(res["out"], np.tile(ref_out, reps)[:B])
+    assert again == 0 and smp.policy_state() == 0, again
+    if share:
+        assert np.array_equal(have.cpu().numpy().view(np.uint32), np.tile(want, (reps, 1))[:B].view(np.uint32))
+    smp.close()
