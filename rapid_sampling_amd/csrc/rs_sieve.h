@@ -1034,21 +1034,23 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         }
     }
     // ---- threshold and token from the list; a decision too close to call is made again with the row's exact total ----
-    bool tell = false;
-    for (;; again = true) {
+    bool from_row = false;                               // the list is of the row, not of the tokens set aside
+    for (uint32_t sums = 0;; again = true) {             // sums: of the row made so far
 
         auto from_list = [&](auto fn) {
             for (uint32_t i = (uint32_t)tid; i < n_list; i += NT) fn((uint32_t)(L.list[i] >> 32));
         };
         if (__builtin_expect(again || !listed, 0)) {
-            sieve_pens_back<NT>(params_again(), v, row);
-            if (tid == 0) __hip_atomic_fetch_add(&params_again().hdr->n_again, 1u, __ATOMIC_RELAXED, RS_AGENT);
-            const bool close = listed && !p.diag && !p.e_bits;
+            if (sums == 0u) {
+                sieve_pens_back<NT>(params_again(), v, row);
+                if (tid == 0) __hip_atomic_fetch_add(&params_again().hdr->n_again, 1u, __ATOMIC_RELAXED, RS_AGENT);
+            }
+            const bool close = sums++ == 0u && listed && !p.diag && !p.e_bits;       // (and exactly when that is not close enough)
             D = sieve_again<NT>(params_again(), L, row, M, close);
             err = close ? M96{(D.lo >> 38) | ((uint64_t)D.hi << 26), 0u} + M96{1ull << 24, 0u} : M96{0ull, 0u};
             if (!listed) {
                 // the tokens set aside were not enough, or more than the list holds: the row's own bins, and its tokens at or above the boundary bin
-                tell = true;
+                from_row = true;
                 __syncthreads();
                 level1(true, false);
                 n_list = f.cnt_above + f.cnt_bin;
@@ -1079,9 +1081,12 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             begin();
             again = true;
         }
-        if (__builtin_expect(!found, 0)) break;
-        digits((uint32_t)kWave, from_list);
-        if (__builtin_expect(!found, 0)) break;
+        if (__builtin_expect(found, 1)) digits((uint32_t)kWave, from_list);
+        if (__builtin_expect(!found, 0)) {               // (P may be more than is listed)
+            if (from_row) break;
+            listed = false;
+            continue;
+        }
         const uint32_t n = f.cnt_above + f.cnt_bin;
         uint32_t token = 0;                              // of the wave that finds it, in one lane: the sampled token + 1
         if (n <= (uint32_t)kWave) {
@@ -1186,10 +1191,13 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         }
         const uint32_t in_doubt = put(token, n <= (uint32_t)kWave);
         if (__builtin_expect(in_doubt == 0u, 1)) {
-            if (tell) tell_policy(params_again());
+            if (from_row) tell_policy(params_again());
             return;
         }
-        if (in_doubt != 1u || again) break;              // (a list that is too short after all)
+        if (in_doubt != 1u || !(err.lo | err.hi)) {      // a list that is too short after all
+            if (from_row) break;
+            listed = false;
+        }
     }
     // Thousands of tokens in the boundary bin: the slow way.
     {
