@@ -115,6 +115,18 @@ struct Frame {
         for (int i = 2; i < 6; ++i) p = __builtin_fmaf(p, f, __uint_as_float(c[i]));
         return __builtin_ldexpf(p, n);
     }
+    // The same, and 0 for x = -inf, whose fractional part v_fract_f32 has as a NaN: its clamp to [0, 1], which makes zeros of NaNs, costs nothing.
+    // What x = NaN comes to has no meaning.
+    __device__ __forceinline__ float scaled_or_none(float x) const
+    {
+        int n;
+        asm("v_cvt_flr_i32_f32 %0, %1" : "=v"(n) : "v"(x));
+        const float f = __builtin_amdgcn_fmed3f(__builtin_amdgcn_fractf(x), 0.0f, 1.0f);
+        float p = __builtin_fmaf(__uint_as_float(c[0]), f, __uint_as_float(c[1]));
+#pragma unroll
+        for (int i = 2; i < 6; ++i) p = __builtin_fmaf(p, f, __uint_as_float(c[i]));
+        return __builtin_ldexpf(p, n);
+    }
     __device__ __forceinline__ uint32_t raw(float x) const { return __float_as_uint(scaled(x)); }                    // e_bits_raw
     __device__ __forceinline__ uint32_t bits(float x) const { return __float_as_uint(fmaxf(scaled(x), 0x1p-41f)); }  // e_bits_of
 };

@@ -33,7 +33,10 @@ namespace rs {
 // are allowed.  Tokens more than 40 octaves below the row's frame weigh nothing but are in the sums: 2^-40 each at most.
 //
 // Where the pass waits for the memory (the host's rule) it sums the tokens' own e in double precision instead (FINE): 2^-40 of D and of the slices' number
-// is allowed for, and the tokens of no weight only if the least token of a slice is that far down.  Then hardly a row is summed again.
+// is allowed for, and the tokens of no weight only if the least token of a slice is that far down.  Then hardly a row is summed again.  (Logits of -inf
+// must not make a wave one that is out of range: 128 x 262144 with penalties and one logit in twenty -inf 94.7 us a call, 59.3 as it is; 128 x 1048576
+// N(0,3), top_k 1000, top_p 0.3, some of whose rows were then summed again, 327.)
+// What was summed in a frame counts only where it weighs: not in a wave or a slice all of whose tokens are 41 octaves down, a masked stretch.
 //
 // What bounds it: in large calls the pass reads float32 at the rate of a kernel that only reads.  A token costs 4.6 vector instructions (one of
 // them the exponential, 2.7 issue slots), and a wave some 200 for bound and staging, where the pass with exact e and a histogram (stream_kernel)
@@ -77,7 +80,7 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
     bool odd = false;
     double mass = 0.0;
     const Frame fr(0);
-    float low = kInf;                                    // FINE: the smallest
+    float low = kInf;                                    // FINE: the smallest, or a NaN if there is one
     float x[R * 4], gm[R], lm = -kInf, M = 0.0f;            // gm: the largest of every group, lm: of all; of the wave: the frame, the sum in it
     auto top = [&](int j) {
         float m;                                         // (fmaxf quiets its operands first, an instruction each; products are quiet)
@@ -97,10 +100,11 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
             gm[j] = top(j);
             if constexpr (FINE) {
                 float least;                             // (see top)
-                asm("v_min3_f32 %0, %1, %2, %3" : "=v"(least) : "v"(x[j * 4]), "v"(x[j * 4 + 1]), "v"(x[j * 4 + 2]));
-                asm("v_min3_f32 %0, %1, %2, %3" : "=v"(low) : "v"(least), "v"(x[j * 4 + 3]), "v"(low));
+                asm("v_minimum3_f32 %0, %1, %2, %3" : "=v"(least) : "v"(x[j * 4]), "v"(x[j * 4 + 1]), "v"(x[j * 4 + 2]));
+                asm("v_minimum3_f32 %0, %1, %2, %3" : "=v"(low) : "v"(least), "v"(x[j * 4 + 3]), "v"(low));
                 const bool in = !ragged || (uint32_t)(j * kThreads) + opaque((uint32_t)tid) < left;
-                double d0 = (double)fr.scaled(x[j * 4]) + (double)fr.scaled(x[j * 4 + 1]), d1 = (double)fr.scaled(x[j * 4 + 2]) + (double)fr.scaled(x[j * 4 + 3]);
+                auto e = [&](int q) { return (double)fr.scaled_or_none(x[j * 4 + q]); };
+                const double d0 = e(0) + e(1), d1 = e(2) + e(3);
                 mass += in ? d0 + d1 : 0.0;
                 q[j % 4] = 0.0f;
             } else
@@ -121,7 +125,7 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
 #pragma unroll
             for (int i = 0; i < R / 4; ++i) mass += (double)part[i];
         }
-        odd = __builtin_amdgcn_ballot_w64(!(mass < (double)kInf) || lm > 120.0f || strange()) != 0ull || __builtin_amdgcn_ballot_w64(lm >= -80.0f) == 0ull;
+        odd = __builtin_amdgcn_ballot_w64(!(mass < (double)kInf) || lm > 120.0f || (FINE && low != low) || strange()) != 0ull || __builtin_amdgcn_ballot_w64(lm >= -80.0f) == 0ull;
         if (__builtin_expect(odd, 0)) {
             const uint32_t t = opaque((uint32_t)tid);
             lm = -kInf;
@@ -212,9 +216,16 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         const double2 m2 = reinterpret_cast<const double2 *>(s.mass)[lane * 2], m3 = reinterpret_cast<const double2 *>(s.mass)[lane * 2 + 1];
         const int down = (int)fmaxf(s.frame[lane >> 4] - Ms, -1000.0f);
         const double all = wave_sum_f64(__builtin_ldexp((m2.x + m2.y) + (m3.x + m3.y), down));
+        const uint4 o4 = *reinterpret_cast<const uint4 *>(s.odd);
+        const float4 m4 = *reinterpret_cast<const float4 *>(s.frame);
+        const float from = Ms - 41.0f;
+        const bool any = (o4.x != 0u && m4.x >= from) || (o4.y != 0u && m4.y >= from) || (o4.z != 0u && m4.z >= from) || (o4.w != 0u && m4.w >= from);
         if (lane == 0) {
-            v.hdr[slice].mass = __float_as_uint((float)all);
-            if constexpr (FINE) v.fine[slice] = SieveFine{all, ~max(max(s.low[0], s.low[1]), max(s.low[2], s.low[3])), 0u};
+            v.hdr[slice].mass = __float_as_uint((float)all) | (any ? kSieveOdd : 0u);
+            if constexpr (FINE) {                        // (a wave that was cleaned up may hold anything: -inf)
+                const uint32_t low = (o4.x | o4.y | o4.z | o4.w) != 0u ? 0x007FFFFFu : ~max(max(s.low[0], s.low[1]), max(s.low[2], s.low[3]));
+                v.fine[slice] = SieveFine{all, low, 0u};
+            }
         }
     }
     uint32_t n = 0, cut = key;
@@ -261,8 +272,7 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         }
     }
     if (tid == 0) {
-        const uint4 o4 = *reinterpret_cast<const uint4 *>(s.odd);
-        *reinterpret_cast<uint2 *>(&v.hdr[slice]) = make_uint2(key, n | ((o4.x | o4.y | o4.z | o4.w) != 0u ? kSieveOdd : 0u));
+        *reinterpret_cast<uint2 *>(&v.hdr[slice]) = make_uint2(key, n);
         v.hdr[slice].cut = cut;
     }
 }
@@ -684,10 +694,11 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
     auto mass_in = [&](const uint4 &h, const float M) __attribute__((always_inline)) {
         const float d = M - __builtin_floorf(fkey_inv(h.x));
         const int down = d >= 64.0f ? 64 : (int)d;
-        const int sh = (int)(h.w >> 23) - 110 - down;    // 2^(ex - 150) in units of 2^-40
+        const int sh = (int)(h.w >> 23 & 255u) - 110 - down;    // 2^(ex - 150) in units of 2^-40
         const uint64_t m = (h.w & 0x7FFFFFu) | 0x800000u;
         return sh >= 0 ? m << (sh & 63) : sh > -32 ? m >> (-sh & 63) : 0ull;
     };
+    auto is_odd = [&](const uint4 &h, const float M) __attribute__((always_inline)) { return (h.w & kSieveOdd) != 0u && fkey_inv(h.x) >= M - 41.0f; };
     M96 D{0ull, 0u}, P{0ull, 0u}, err{0ull, 0u};
     // D from the slices' sums, and what it may be off by; `dead`: from sums in double precision (bit 1), with tokens that weigh nothing in them (bit 0)
     auto estimate = [&](const uint64_t all, const bool odd, const uint32_t dead) __attribute__((always_inline)) {
@@ -726,7 +737,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         for (int k = 0; k < 2; ++k)
             if ((uint32_t)(lane + k * kWave) < G) {
                 q += fine ? fine_in(h[k], f[k], M, dead) : mass_in(h[k], M);
-                odd = odd || (h[k].y & kSieveOdd) != 0u;
+                odd = odd || is_odd(h[k], M);
             }
         estimate(wave_sum(q), __builtin_amdgcn_ballot_w64(odd) != 0ull, (fine ? 2u : 0u) | (__builtin_amdgcn_ballot_w64(dead) != 0ull ? 1u : 0u));
         if (lane == 0) { L.one.D = D; L.one.P = P; L.one.err = err; }
@@ -772,7 +783,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
     const bool whole = e_cut < kEMinBits;                // ... that is, every live token
     const uint32_t from = max(e_cut + 1u, kEMinBits);
     if constexpr (!kEach) {
-        const uint64_t coarse = __builtin_amdgcn_ballot_w64(mine && (h.y & kSieveOdd) != 0u);
+        const uint64_t coarse = __builtin_amdgcn_ballot_w64(mine && is_odd(h, M));
         bool dead = false;
         const uint64_t q = wave_sum(mine && half == 0u ? fine ? fine_in(h, fh, M, dead) : mass_in(h, M) : 0ull);
         const uint64_t with_dead = __builtin_amdgcn_ballot_w64(dead);

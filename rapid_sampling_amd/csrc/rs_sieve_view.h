@@ -9,9 +9,9 @@ struct SieveHdr {                                        // 16 bytes
     uint32_t mkey;           // fkey(max x of the slice)
     uint32_t n;              // tokens set aside; kSieveTie: none, and all tokens of the slice equal its maximum
     uint32_t cut;            // every token of the slice with fkey(x) > cut is set aside
-    uint32_t mass;           // float: the sum of 2^(x - floor(max x))
+    uint32_t mass;           // float: the sum of 2^(x - floor(max x)); kSieveOdd in the place of its sign: a wave's was worked out in a frame, one that matters
 };
-constexpr uint32_t kSieveTie = 1u << 31, kSieveOdd = 1u << 30;     // kSieveOdd, with any n: a wave's sum was worked out in a frame
+constexpr uint32_t kSieveTie = 1u << 31, kSieveOdd = 1u << 31;
 
 struct SieveFine {                                       // 16 bytes
     double   mass;           // the sum of the slice's e, in its frame

@@ -2569,3 +2569,35 @@ def test_sieve_path_decisions_within_the_closer_sum(torch_cuda, oracle):
     res = smp.sample(torch.from_numpy(lg).cuda(), c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_diag=False)
     assert np.array_equal(res["out"], ref_out) and smp.rows_again() == 4 and smp.policy_state() == 0
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,k,top_p,share,masked,seed", [(128, 1048576, 1000, 0.3, 0.0, 0.05, 7), (24, 1048576, 1000, 0.3, 0.0, "half", 9), (256, 131072, 320, 0.2, 0.0, "half", 8),
+                                                           (128, 262144, 100, 0.9, 0.02, 0.05, 7)])
+def test_sieve_path_sums_of_masked_rows(torch_cuda, oracle, B, V, k, top_p, share, masked, seed):
+    """Logits of -inf here and there or side by side leave the row's total as well known as it is without them: no more rows are summed again.
+    Tokens against the general kernel's, and some rows against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    gen = torch.Generator(device="cuda").manual_seed(seed)
+    x = torch.randn((B, V), generator=gen, device="cuda") * 3.0
+    if masked == "half":
+        x[:, : V // 2] = -np.inf
+    else:
+        x.masked_fill_(torch.rand((B, V), generator=gen, device="cuda") < masked, -np.inf)
+    u = 1.0 - torch.rand(B, generator=gen, device="cuda")
+    rc, c, kk, p = capi.normalize(1.0, k, top_p, V, B, 1)
+    smp = capi.Sampler(B, V)
+    more = dict(presence=0.1, repetition=0.2, decay=0.95) if share else {}
+    pen = torch.from_numpy(H.penalties_sparse(2, V, share, seed=V)).cuda().repeat(B // 2, 1) if share else None
+    have = pen.clone() if share else None
+    smp.rows_again()
+    res = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, penalties=have, **more)
+    again = smp.rows_again()
+    ref = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, path="cluster", penalties=pen, **more)
+    assert np.array_equal(res["out"], ref["out"]) and smp.status() == 0
+    assert again == 0, again
+    if share:
+        assert torch.equal(have.view(torch.int32), pen.view(torch.int32))
+    else:
+        assert np.array_equal(res["out"][:4], oracle.sample_batch(x[:4].cpu().numpy(), c, kk, p, injected_u=u[:4].cpu().numpy())[0])
+    smp.close()
