@@ -503,20 +503,21 @@ struct LdsSieveFin {
 // `err` (0: they are exact).  What comes out is how far the target r and the running sums may shift against each other for
 // the pick; `unsure` when threshold or tie weight themselves are in doubt.  With top_p = 1 P is the row's total, and that is at least the mass of the
 // tokens that have been seen: they are above no such P, however little the rest of the row weighs.
+__device__ __forceinline__ bool wants_all(const Params &p) { return __float_as_uint(p.top_p) == 0x3F800000u; }        // (of its bits: on scalars)
 struct Doubt { M96 shift; bool unsure; };
 __device__ __forceinline__ M96 larger_of(const M96 a, const M96 b)
 {
     const bool m = a >= b;                               // (by its parts: a choice between two objects would be one between addresses)
     return M96{m ? a.lo : b.lo, m ? a.hi : b.hi};
 }
-__device__ __forceinline__ Doubt doubt_of(const M96 P, const M96 err, const float top_p, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq, const M96 above,
+__device__ __forceinline__ Doubt doubt_of(const M96 P, const M96 err, const bool whole_row, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq, const M96 above,
                                           const uint32_t thr, const uint64_t w_tie)
 {
     Doubt d{M96{0ull, 0u}, false};
     if (!(err.lo | err.hi)) return d;
     M96 least = P >= err ? P - err : M96{0ull, 0u};
     const M96 most = P + err, down = above + m96((u128)w_of_bits(thr) * n_eq);
-    if (top_p >= 1.0f) least = larger_of(least, down);
+    if (whole_row) least = larger_of(least, down);
     // the tokens above the threshold are not enough, those down to it are
     if (n_gt && !(above < least)) d.unsure = true;
     if (n_gt + n_eq < top_k && !(down >= most)) d.unsure = true;
@@ -828,13 +829,14 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         M96 e = err;
         return few_pick(p, L.few, row, lane, wave, list, n, top_k,
                         [&](const Limbs &upto) __attribute__((always_inline)) {
-                            if (!all_of_it) return Totals{D, p.top_p >= 1.0f && n >= top_k ? larger_of(m96(lane_of(upto, 63u)), P) : P};     // (see doubt_of)
+                            // (see doubt_of: more than is listed, whatever that is; without waiting for what it is, which took 0.1 us)
+                            if (!all_of_it) return Totals{D, wants_all(p) && n >= top_k && !p.diag ? M96{~0ull, 0x7FFFFFFFu} : P};
                             e = M96{0ull, 0u};           // every live token of the row is there
                             const M96 d = m96(lane_of(upto, 63u));
                             return Totals{d, ceil_mul(p.top_p, d)};
                         }, xmax, &L.rand64, rounds,
                         [&](const M96 &P, bool enough, uint32_t n_gt, uint32_t n_eq, uint32_t thr, const M96 &above, uint64_t w_tie) __attribute__((always_inline)) {
-                            const Doubt d = doubt_of(P, e, p.top_p, top_k, n_gt, n_eq, above, thr, w_tie);
+                            const Doubt d = doubt_of(P, e, false, top_k, n_gt, n_eq, above, thr, w_tie);
                             doubts = !enough ? 2u : d.unsure ? 1u : 0u;
                             if (lane == 0) L.one.shift = d.shift;
                         }, [&](const M96 &slack) __attribute__((always_inline)) { L.one.slack = slack; });
@@ -891,7 +893,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             if (known) P = ceil_mul(p.top_p, D);
             else if (complete) { err = M96{0ull, 0u}; D = sc.total(); P = ceil_mul(p.top_p, D); }
             else total();
-            if (p.top_p >= 1.0f) P = larger_of(sc.total(), P);       // (see doubt_of)
+            if (wants_all(p)) P = larger_of(sc.total(), P);       // (see doubt_of)
             // (the largest that P may be: what is listed then holds the kept set whatever the exact D is, and whether another
             // threshold than this one comes of that is asked behind it)
             goal = P + err;
@@ -1129,7 +1131,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
                 const M96 above = f.above + mass_of(f.sum, thr >> 23);
                 const Target tg = tie_and_target(p, row, uniform(L.rand64), xmax, wide(D), wide(P), thr, f.cnt_above, f.cnt_bin, wide(above), 0u, tid == 0);
                 w_tie = uniform(tg.w_tie); r = uniform(m96(tg.r));
-                const Doubt d = doubt_of(P, err, p.top_p, top_k, f.cnt_above, f.cnt_bin, above, thr, w_tie);
+                const Doubt d = doubt_of(P, err, wants_all(p), top_k, f.cnt_above, f.cnt_bin, above, thr, w_tie);
                 shift = d.shift;
                 doubts = d.unsure ? 1u : 0u;
             }
