@@ -2601,3 +2601,29 @@ def test_sieve_path_sums_of_masked_rows(torch_cuda, oracle, B, V, k, top_p, shar
     else:
         assert np.array_equal(res["out"][:4], oracle.sample_batch(x[:4].cpu().numpy(), c, kk, p, injected_u=u[:4].cpu().numpy())[0])
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,k", [(64, 1048576, 1024), (64, 1048576, 300), (128, 262144, 320)])
+def test_sieve_path_slices_with_spikes_and_more_tokens_than_they_have_room_for(torch_cuda, oracle, B, V, k):
+    """Rows of 16 spikes over a broad floor with a top_k for which slices set aside nearly all that they have room for, some a token more: the bound
+    that such a slice takes instead does not depend on how far up its spike is, and every row's top_k tokens are found without the row being read
+    again.  With top_p = 1 nothing else is in doubt.  Tokens against the general kernel's, one row against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    smp = capi.Sampler(B, V)
+    rc, c, kk, p = capi.normalize(1.0, k, 1.0, V, B, 1)
+    for seed in (100, 101, 102):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        x = torch.randn((B, V), generator=gen, device="cuda") * 2.0
+        where = torch.randint(0, V, (B, 16), generator=gen, device="cuda")
+        x.scatter_(1, where, x.gather(1, where) + 10.0)
+        u = 1.0 - torch.rand(B, generator=gen, device="cuda")
+        print("sieve path, spikes:", B, V, k, seed, flush=True)
+        smp.rows_again()
+        res = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, path="stream")
+        again = smp.rows_again()
+        ref = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, path="cluster")
+        assert np.array_equal(res["out"], ref["out"]) and smp.status() == 0
+        assert again == 0, again
+    assert res["out"][0] == oracle.sample_batch(x[:1].cpu().numpy(), c, kk, p, injected_u=u[:1].cpu().numpy())[0][0]
+    smp.close()
