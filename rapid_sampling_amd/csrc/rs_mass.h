@@ -314,12 +314,15 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const Limbs mine = limbs(M96{in ? s.w[lane] : 0ull, 0u}), run = wave_inclusive_scan(mine);
     const M96 bef = m96(run - mine), with = m96(run);
+    // (read by all lanes: behind a branch that lane 63 does not take, its sum need not be there)
+    M96 all{0ull, 0u};
+    if constexpr (kLook) all = m96(lane_of(run, 63u));
     const bool is_it = in && bef < r && with >= r;
     if constexpr (kLook) {
         if (is_it) {
             M96 less = r - bef - M96{1ull, 0u}, more = with - r;
             if (!(bef.lo | bef.hi)) { less.lo = ~0ull; less.hi = ~0u; }                      // (the first kept token)
-            if (with >= m96(lane_of(run, 63u))) { more.lo = ~0ull; more.hi = ~0u; }          // (the last)
+            if (with >= all) { more.lo = ~0ull; more.hi = ~0u; }          // (the last)
             const bool m = more >= less;
             picked(M96{m ? less.lo : more.lo, m ? less.hi : more.hi});
         }

@@ -2549,21 +2549,22 @@ def test_sieve_path_with_top_p_of_one_on_peaked_rows(torch_cuda, oracle, B, V, k
 
 
 def test_sieve_path_decisions_within_the_closer_sum(torch_cuda, oracle):
-    """One token whose weight is exactly top_p of the row: the sum in double precision cannot tell either, and the exact one decides, without the
-    slow way -- several passes over the row, which a caller's policy would be told of."""
+    """Two tokens that share the nucleus evenly, and a target right at the end of the first: the sum in double precision cannot tell either, and the
+    exact one decides, without the slow way -- several passes over the row, which a caller's policy would be told of."""
     torch = torch_cuda
     from tests import capi
     V, n_low = 262144, 131072
     lg = np.full((4, V), -np.inf, dtype=np.float32)
     lg[:, V // 4: V // 4 + n_low - 20 * 1024] = 0.0
-    lg[:, 1000: 21000: 1000] = 10.0                      # (20 of them)
-    lg[:, 5] = 17.0                                      # as heavy as the others together (c is 1: x is the logit)
-    lg[1, 5] = np.nextafter(np.float32(17.0), np.float32(0))
+    lg[:, 1000: 21000: 1000] = 10.0                      # (20 of them, c is 1: x is the logit)
+    lg[:, [5, 700]] = 17.0                               # as heavy, each, as the others together
+    lg[1, 9:700] = -3.0
     lg[2, V - 3] = -20.0
-    u_np = np.array([1.0, 0.7, 0.3, 1e-6], dtype=np.float32)
+    u_np = np.array([0.5, 0.5, 0.5, np.nextafter(np.float32(0.5), np.float32(1))], dtype=np.float32)
     rc, c, kk, p = capi.normalize(1.4426950408889634, 50, 0.5, V, 4, 1)
     assert c == 1.0
     ref_out = oracle.sample_batch(lg, c, kk, p, injected_u=u_np)[0]
+    assert ref_out.tolist() == [5, 5, 5, 700]
     smp = capi.Sampler(4, V, with_policy=True)
     smp.rows_again()
     res = smp.sample(torch.from_numpy(lg).cuda(), c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_diag=False)
