@@ -244,12 +244,12 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         // the tokens of those groups, by the first wave, a group to a lane
         const uint32_t all = c[0] + c[1] + c[2] + c[3];
         uint64_t *st = v.stash + slice * room;
-        // Mostly they fit.  If not (several tokens of a group), the bound is raised, by a 64th of itself and twice as much each time, until they do,
+        // Mostly they fit.  If not (several tokens of a group), the bound is raised, by a 64th to a 32nd of itself and twice as much each time, until they do,
         // and lowered again when they fill less than half of the room: `over` is one that too many reach, from `fits` on they fit.  (A fixed part of
         // the way up to the slice's largest token depends on how far up that is: in rows with a few spikes hardly a token was left, and rows whose top_k
         // tokens were then not all there had to be summed again, 64 x 1048576 with a top_k of 1024 457 us a call, 62 like this.)
         const uint32_t first = lo;
-        for (uint32_t over = lo, fits = key + 1u, step = 1u << 17;;) {
+        for (uint32_t over = lo, fits = key + 1u, step = 1u << 18;;) {
             n = 0;
             for (uint32_t g = (uint32_t)lane; g < room; g += kWave) {
                 uint32_t w = 0, at = g;
