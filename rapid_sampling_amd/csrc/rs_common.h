@@ -26,7 +26,7 @@ constexpr uint64_t kValid     = 1ull << 63;   // marks a written exchange word
 constexpr uint32_t kVerdictFallback = 0xFFFFFFFFu;   // the finishing workgroup could not finish the row from the stashes
 
 struct alignas(256) WsHeader {
-    uint32_t n_again;     // rows of the running (or last) call on the sieve path that were summed again from their logits (all of them when it asks for diagnostics)
+    uint32_t n_again;     // rows that calls on the sieve path have summed again from their logits (all of a call that asks for diagnostics); never cleared here
     uint32_t finished;    // workgroups that have left the running launch
     int32_t  error;       // sticky RS_ERR_DEVICE
     uint32_t n_need;      // rows of the running (or last) streaming call that the finishing workgroups did the slow way

@@ -311,7 +311,7 @@ __global__ void __launch_bounds__(kThreads, R == 16 ? (FINE ? 3 : 4) : !FINE ? 8
 #pragma unroll
         for (int j = 0; j < R; ++j) l[j] = __builtin_nontemporal_load(from + min((uint32_t)(j * kThreads + tid), left - 1u));
     }
-    if (reporter) { a_store(&p.hdr->n_again, 0u); report_end(p, prev, true); }
+    if (reporter) report_end(p, prev, true);
     sieve_slice<R, FINE>(v, s, [&](int j, float *x) {
         uint32_t w[4];
         if constexpr (DT == RS_DTYPE_F32) { w[0] = l[j].x; w[1] = l[j].y; w[2] = l[j].z; w[3] = l[j].w; }
@@ -376,7 +376,7 @@ __global__ void __launch_bounds__(kThreads, R == 8 ? 4 : 6) sieve_pen_kernel(con
             pn[j] = pfrom[i];
         }
     }
-    if (reporter) { a_store(&p.hdr->n_again, 0u); report_end(p, prev, true); }
+    if (reporter) report_end(p, prev, true);
     const size_t slice = (size_t)row * v.G + part;
     auto widen = [&](const T &t, uint32_t (&w)[4]) __attribute__((always_inline)) {
         if constexpr (DT == RS_DTYPE_F32) { w[0] = t.x; w[1] = t.y; w[2] = t.z; w[3] = t.w; }

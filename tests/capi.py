@@ -157,8 +157,8 @@ class Sampler:
         return st.value
 
     def rows_again(self):
-        """Rows that the last call, if it took the sieve path, summed again from their logits (WsHeader::n_again): with diagnostics all of
-        them but those of equal tokens.  Sets the word to 0, which other paths leave as it is."""
+        """Rows that calls on the sieve path have summed again from their logits since this was last asked (WsHeader::n_again): of a call with
+        diagnostics all of them but those of equal tokens.  Sets the word to 0, which calls only add to."""
         n = int(self.ws[:4].view(self.torch.int32).item())
         self.ws[:4] = 0
         return n
