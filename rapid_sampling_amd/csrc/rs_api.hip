@@ -567,10 +567,10 @@ static int fused_r(int32_t B, int32_t V, bool pen, bool any_size)
 // call: 16 x 131072 with 455 kept 15.0 there, 46.7 here.
 static uint32_t sieve_share(int32_t top_k, int32_t V, int R) { return (uint32_t)(((uint64_t)(uint32_t)top_k * 1024u * (uint32_t)R + (uint32_t)V - 1u) / (uint32_t)V); }
 constexpr int32_t kSieveK = 320;
-// Whether the pass sums the tokens' own e in double precision.  How often a decision is too close to call goes with the error of D over the weight of
-// the threshold's token: a row in 4000 with 100 kept, in 1000 with 400, and such a row is summed again by one workgroup, 10 us in rows of 131072 tokens
-// and 75 in rows of a million, for which the call waits (128 x 1048576 N(0,3), top_k 1000, top_p 0.3: 255 us a call, 100 with these sums).  With
-// them it is a row in millions, for 10 more issue slots a token: nothing where the pass waits for the memory, us a call, v_exp_f32 / double:
+// Whether the pass sums the tokens' own e in double precision.  How often a target is too close to call goes with the error of D times the tokens kept: a
+// row in 20000 with 50 kept, in 4000 with 300, and more in rows of a million cold tokens; and such a row is summed again by one workgroup, 35 us in rows of
+// 131072 tokens and 275 in rows of a million, for which the call waits.  With these sums it is a row in millions, but for tokens that weigh
+// nothing, for 10 more issue slots a token: nothing where the pass waits for the memory, us a call, v_exp_f32 / double:
 // 128 x 1048576 top_k 1024 102.4 / 100.7, top_k 50 91.0 / 86.7, with penalties 128 x 262144 58.4 / 58.2; a tenth and more elsewhere (256 x 131072
 // 26.9 / 30.6, 4 x 1048576 12.8 / 14.6, bfloat16 128 x 1048576 50.7 / 76.4), where short lists are rarely in doubt and, in rows of up to 262144
 // tokens, those of more than kSieveK are left to the streaming path.

@@ -10,17 +10,17 @@ namespace rs {
 
 // ---------------------------------------------------------------- sieve path --
 // For kept sets that are small next to the row two things are needed of it: its largest tokens, and its total mass D, of
-// which P = ceil(top_p * D) is the mass that is enough.  The tokens must be exact.  D need not be, as long as nothing that is
-// decided by it lies within its error: then the exact D decides the same.  So
+// which P = ceil(top_p * D) is the mass that is enough.  The tokens must be exact.  D need not be, as long as the token that is
+// picked with it is the one that every D within its error picks: then the exact D picks it, too.  So
 //
 //   sieve_kernel         a workgroup per slice, no histogram, two barriers.  It sums 2^x with the hardware's exponential and sets aside every token at
 //                        or above a value that a given number of its threads, pair by pair, reach with their largest token: between that
 //                        many and some half more, whatever the distribution.
 //   sieve_finish_kernel  a workgroup per row.  It takes D from the slices' sums, works out threshold and token from the tokens set
-//                        aside -- complete above the largest of the slices' bounds -- and then compares the distance of every
-//                        decision on the way from its alternative with the error that D can have.  If one is too close (a row in some
-//                        ten thousands, more when hundreds of tokens are kept) it sums the row again, from the logits, in double
-//                        precision, and decides again.
+//                        aside -- complete above the largest of the slices' bounds -- and then compares the target's distance from
+//                        both ends of the token's place with what the error of D can shift them by.  If it is too close (a row in a million for
+//                        each token kept) it sums the row again, from the logits, in double precision, and decides again; exactly, when that
+//                        is too close as well.
 //
 // The results are the same integers as on every other path.
 //
@@ -498,47 +498,51 @@ struct LdsSieveFin {
     uint64_t list[kSieveList], small[kWave];             // bits of e << 32 | index
     uint64_t blo[NT], bhi[NT];                           // kept weights by bucket of the token index, halves summed apart
     M96      mass[16];
-    struct { M96 D, P, r, err, shift, slack; Edge f; uint64_t w_tie; uint32_t found; } one;  // what one wave worked out for all
+    struct { M96 D, P, r, err, shift, slack[2]; Edge f; uint64_t w_tie; uint32_t found, other; } one;  // what one wave worked out for all
     uint64_t sum[16];
     uint64_t rand64;
     uint32_t flag[16];
     uint32_t n, few_n, thr, bucket, unsure;
 };
 
-// Is a decision that was made with D, and with P = ceil(top_p * D), the one that the exact D makes?  Both may be off by less than
-// `err` (0: they are exact).  What comes out is how far the target r and the running sums may shift against each other for
-// the pick; `unsure` when threshold or tie weight themselves are in doubt.  With top_p = 1 P is the row's total, and that is at least the mass of the
-// tokens that have been seen: they are above no such P, however little the rest of the row weighs.
+// Is a token that was picked with D, and with P = ceil(top_p * D), the one that the exact D picks?  Both may be off by less than `err` (0: they are
+// exact).  As P grows, no token's weight falls -- one above the threshold has its own, one at it a share of what is left, one below none -- and the kept
+// mass S grows by what P does, up to what the tie weight's division leaves: so a running sum and the target r, u of S, shift against each other by no
+// more than that, whichever thresholds lie in between, and the token is the same if r is further than that from both ends of its place.
+// With top_p = 1 P is the row's total, and that is at least the mass of the tokens that have been seen: they are above no such P, however little the rest
+// of the row weighs.
 __device__ __forceinline__ bool wants_all(const Params &p) { return __float_as_uint(p.top_p) == 0x3F800000u; }        // (of its bits: on scalars)
-struct Doubt { M96 shift; bool unsure; };
 __device__ __forceinline__ M96 larger_of(const M96 a, const M96 b)
 {
     const bool m = a >= b;                               // (by its parts: a choice between two objects would be one between addresses)
     return M96{m ? a.lo : b.lo, m ? a.hi : b.hi};
 }
-__device__ __forceinline__ Doubt doubt_of(const M96 P, const M96 err, const bool whole_row, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq, const M96 above,
-                                          const uint32_t thr, const uint64_t w_tie)
+__device__ __forceinline__ bool is_zero(const M96 a) { return !(a.lo | a.hi); }
+__device__ __forceinline__ M96 less_by(const M96 a, const M96 b) { return a >= b ? a - b : M96{0ull, 0u}; }
+// Is another threshold possible, P being `least` at least and `most` at most: are the tokens above this one enough, or those down to it not?  Then tokens of
+// no weight may have some.
+__device__ __forceinline__ bool other_threshold(const M96 err, const M96 least, const M96 most, const uint32_t top_k, const uint32_t n_gt, const uint32_t n_eq,
+                                                const M96 above, const M96 down)
 {
-    Doubt d{M96{0ull, 0u}, false};
-    if (!(err.lo | err.hi)) return d;
-    M96 least = P >= err ? P - err : M96{0ull, 0u};
-    const M96 most = P + err, down = above + m96((u128)w_of_bits(thr) * n_eq);
-    if (whole_row) least = larger_of(least, down);
-    // the tokens above the threshold are not enough, those down to it are
-    if (n_gt && !(above < least)) d.unsure = true;
-    if (n_gt + n_eq < top_k && !(down >= most)) d.unsure = true;
-    // The tie weight is (P - above) / n_eq unless that is more than it can be (the threshold's own, or the share that top_k leaves of it).  If it is the
-    // former, S and with it r move by u and the running sum by t times what P is off by, u and t between 0 and 1 (the random number; the ties before
-    // the token): by no more than that against each other, and what the divisions round.
-    const M96 n{(uint64_t)n_eq, 0u};
-    if (!(least >= above + m96((u128)w_tie * n_eq) + n) && !(w_tie == w_of_bits(thr) && least >= down)) d.shift = err + n + M96{2ull, 0u};
-    return d;
+    return !is_zero(err) && ((n_gt && !(above < least)) || (n_gt + n_eq < top_k && !(down >= most)));
 }
-// ... and the token whose weight lies at (before, upto] in the running sum, for the target r
-__device__ __forceinline__ bool pick_is_sure(const M96 shift, const M96 before, const M96 upto, const M96 r, const bool first, const bool last)
+// How far r and the running sums may shift against each other, P being off by less than err.  The tie weight is (P - above) / n_eq unless that is more than
+// it can be, the threshold's own or the share that top_k leaves of it: then S and r do not move.  The divisions leave less than a unit for each of the
+// ties, of one threshold or, if another is possible, of two of up to 2^20 tokens.  (err is 2^25 and more: where no other is possible, above < P - err,
+// no tie weighs nothing, and the first and the last kept token are the first and the last whatever P is.)
+__device__ __forceinline__ M96 shift_of(const M96 err, const bool other, const M96 least, const uint32_t n_eq, const M96 above, const M96 down, const uint32_t thr,
+                                        const uint64_t w_tie)
 {
-    if (!(shift.lo | shift.hi)) return true;
-    return (first || before + shift < r) && (last || upto >= r + shift);
+    if (is_zero(err)) return err;
+    if (other) return err + M96{(1ull << 21) + 2ull, 0u};
+    const M96 n{(uint64_t)n_eq, 0u};
+    if (least >= above + m96((u128)w_tie * n_eq) + n || (w_tie == w_of_bits(thr) && least >= down)) return M96{0ull, 0u};
+    return err + n + M96{2ull, 0u};
+}
+// ... of the token whose weight lies at (before, upto] in the running sum
+__device__ __forceinline__ bool pick_is_sure(const M96 shift, const M96 before, const M96 upto, const M96 r)
+{
+    return is_zero(shift) || (before + shift < r && upto >= r + shift);
 }
 
 // The level-1 bins of one wave's scan, an octave a lane, from their copies.
@@ -835,17 +839,18 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         M96 e = err;
         return few_pick(p, L.few, row, lane, wave, list, n, top_k,
                         [&](const Limbs &upto) __attribute__((always_inline)) {
-                            // (see doubt_of: more than is listed, whatever that is; without waiting for what it is, which took 0.1 us)
+                            // (see above: more than is listed, whatever that is; without waiting for what it is, which took 0.1 us)
                             if (!all_of_it) return Totals{D, wants_all(p) && n >= top_k && !p.diag ? M96{~0ull, 0x7FFFFFFFu} : P};
                             e = M96{0ull, 0u};           // every live token of the row is there
                             const M96 d = m96(lane_of(upto, 63u));
                             return Totals{d, ceil_mul(p.top_p, d)};
                         }, xmax, &L.rand64, rounds,
                         [&](const M96 &P, bool enough, uint32_t n_gt, uint32_t n_eq, uint32_t thr, const M96 &above, uint64_t w_tie) __attribute__((always_inline)) {
-                            const Doubt d = doubt_of(P, e, false, top_k, n_gt, n_eq, above, thr, w_tie);
-                            doubts = !enough ? 2u : d.unsure ? 1u : 0u;
-                            if (lane == 0) L.one.shift = d.shift;
-                        }, [&](const M96 &slack) __attribute__((always_inline)) { L.one.slack = slack; });
+                            const M96 least = less_by(P, e), down = above + m96((u128)w_of_bits(thr) * n_eq);
+                            const bool other = other_threshold(e, least, P + e, top_k, n_gt, n_eq, above, down);
+                            doubts = !enough ? 2u : 0u;
+                            if (lane == 0) { L.one.shift = shift_of(e, other, least, n_eq, above, down, thr, w_tie); L.one.other = other ? 1u : 0u; }
+                        }, [&](const M96 &to_ends, const M96 &to_tokens) __attribute__((always_inline)) { L.one.slack[1] = to_ends; L.one.slack[0] = to_tokens; });
     };
     auto put = [&](uint32_t token, bool few) __attribute__((always_inline)) {
         if (wave <= 1 && doubts) L.unsure = doubts;
@@ -855,7 +860,8 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         }
         __syncthreads();
         const uint32_t u = uniform(L.unsure);
-        return few && u == 0u && !(L.one.slack >= L.one.shift) ? 1u : u;
+        const M96 room = L.one.other ? L.one.slack[1] : L.one.slack[0];
+        return few && u == 0u && !(room >= L.one.shift) ? 1u : u;
     };
     // the tokens for which in(i) says so, side by side
     auto list_them = [&](auto in) __attribute__((always_inline)) {
@@ -899,7 +905,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             if (known) P = ceil_mul(p.top_p, D);
             else if (complete) { err = M96{0ull, 0u}; D = sc.total(); P = ceil_mul(p.top_p, D); }
             else total();
-            if (wants_all(p)) P = larger_of(sc.total(), P);       // (see doubt_of)
+            if (wants_all(p)) P = larger_of(sc.total(), P);       // (see wants_all)
             // (the largest that P may be: what is listed then holds the kept set whatever the exact D is, and whether another
             // threshold than this one comes of that is asked behind it)
             goal = P + err;
@@ -1135,11 +1141,14 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             M96 r{0ull, 0u}, shift{0ull, 0u};
             if (kEach || wave == 0) {
                 const M96 above = f.above + mass_of(f.sum, thr >> 23);
-                const Target tg = tie_and_target(p, row, uniform(L.rand64), xmax, wide(D), wide(P), thr, f.cnt_above, f.cnt_bin, wide(above), 0u, tid == 0);
+                const M96 down = above + m96((u128)w_of_bits(thr) * f.cnt_bin);
+                M96 least = less_by(P, err);
+                if (wants_all(p)) least = larger_of(least, down);
+                // (the threshold is that of the largest P: when it need not be the exact one's, so are tie weight and target)
+                const bool other = other_threshold(err, least, goal, top_k, f.cnt_above, f.cnt_bin, above, down);
+                const Target tg = tie_and_target(p, row, uniform(L.rand64), xmax, wide(D), wide(M96{other ? goal.lo : P.lo, other ? goal.hi : P.hi}), thr, f.cnt_above, f.cnt_bin, wide(above), 0u, tid == 0);
                 w_tie = uniform(tg.w_tie); r = uniform(m96(tg.r));
-                const Doubt d = doubt_of(P, err, wants_all(p), top_k, f.cnt_above, f.cnt_bin, above, thr, w_tie);
-                shift = d.shift;
-                doubts = d.unsure ? 1u : 0u;
+                shift = shift_of(other ? err + err : err, other, least, f.cnt_bin, above, down, thr, w_tie);
             }
             if constexpr (!kEach) {
                 if (tid == 0) { L.one.w_tie = w_tie; L.one.r = r; L.one.shift = shift; }
@@ -1199,7 +1208,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
                         const M96 up = m96(run), bef = m96(run - one);
                         if ((uint32_t)lane < ns && bef < r && up >= r) {
                             token = L.few.idx[lane] + 1u;
-                            if (!pick_is_sure(shift, bef, up, r, false, false)) doubts = 1u;
+                            if (!pick_is_sure(shift, bef, up, r)) doubts = 1u;
                         }
                     }
                     break;

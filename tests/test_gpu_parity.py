@@ -2628,3 +2628,38 @@ def test_sieve_path_slices_with_spikes_and_more_tokens_than_they_have_room_for(t
         assert again == 0, again
     assert res["out"][0] == oracle.sample_batch(x[:1].cpu().numpy(), c, kk, p, injected_u=u[:1].cpu().numpy())[0][0]
     smp.close()
+
+
+@pytest.mark.parametrize("B,V,k,top_p,temperature,share", [(64, 152064, 50, 0.99999, 0.4, 0.0), (13, 50260, 40, 0.99999, 0.4, 0.0), (128, 131072, 300, 0.9999, 0.5, 0.0), (128, 131072, 300, 0.99, 0.7, 0.0),
+                                                           (64, 1048576, 50, 0.99999, 0.3, 0.0), (128, 262144, 50, 0.9999, 0.5, 0.02)])
+def test_sieve_path_nuclei_that_end_among_the_smallest_weights(torch_cuda, oracle, B, V, k, top_p, temperature, share):
+    """A nucleus whose last tokens weigh less than the row's total may be off by: which of them is the last is not known, but as good as no row
+    hangs on it -- the token does only when the target lies within that distance of its place, for some 2 * top_k * 7 / 2^24 of the rows, of which
+    these calls may have ten times as many, and one.  Tokens and penalties against the general kernel's, some rows against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    smp = capi.Sampler(B, V)
+    rc, c, kk, p = capi.normalize(temperature, k, top_p, V, B, 1)
+    more = dict(presence=0.1, repetition=0.2, decay=0.95) if share else {}
+    rows = again = 0
+    for seed in range(100, 104):
+        gen = torch.Generator(device="cuda").manual_seed(seed)
+        x = torch.randn((B, V), generator=gen, device="cuda") * 2.0
+        where = torch.randint(0, V, (B, 16), generator=gen, device="cuda")
+        x.scatter_(1, where, x.gather(1, where) + 10.0)
+        u = 1.0 - torch.rand(B, generator=gen, device="cuda")
+        pen = torch.from_numpy(H.penalties_sparse(2, V, share, seed=V)).cuda().repeat(B // 2, 1) if share else None
+        have = pen.clone() if share else None
+        print("sieve path, end of the nucleus:", B, V, k, top_p, seed, flush=True)
+        smp.rows_again()
+        res = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, penalties=have, path="stream", **more)
+        again += smp.rows_again()
+        rows += B
+        ref = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, penalties=pen, path="cluster", **more)
+        assert np.array_equal(res["out"], ref["out"]) and smp.status() == 0
+        if share:
+            assert torch.equal(have.view(torch.int32), pen.view(torch.int32))
+    if not share:
+        assert np.array_equal(res["out"][:3], oracle.sample_batch(x[:3].cpu().numpy(), c, kk, p, injected_u=u[:3].cpu().numpy())[0])
+    assert again <= 10 * rows * 2 * k * 7 / 2 ** 24 + 1, (again, rows)
+    smp.close()
