@@ -643,21 +643,42 @@ __device__ __forceinline__ M96 sieve_again(const Params &p, LdsSieveFin<NT> &L, 
     return sc.total();
 }
 
-// The old penalties of a row that is read again, from the notes; its waves then all count as having left theirs to the fix-up kernel.
+// The old penalties of a row that is read again, from the notes; its waves then all count as having left theirs to the fix-up kernel.  Every wave plays back
+// lists of its own, four at a time asked for together: one after the other by the whole workgroup each took two trips to memory.
 template <int NT>
 __device__ __forceinline__ void sieve_pens_back(const Params &p, const SieveView &v, const uint32_t row)
 {
     if (!p.penalties) return;
-    const int tid = threadIdx.x;
+    constexpr uint32_t W = NT / kWave, kMost = (sieve_pen_cap(8) + kWave - 1u) / kWave;
+    const uint32_t lane = threadIdx.x & (kWave - 1u), wave = uniform(threadIdx.x >> 6), lists = v.G * (uint32_t)kWaves;
     float4 *pens = reinterpret_cast<float4 *>(p.penalties + (int64_t)row * p.V);
-    const size_t first = (size_t)row * v.G * kWaves;
-    for (uint32_t w = 0; w < v.G * (uint32_t)kWaves; ++w) {
-        const uint32_t n = v.noted[first + w];
-        if (n != kSievePenLeft)
-            for (uint32_t i = (uint32_t)tid; i < min(n, v.note_cap); i += NT) pens[v.note_at[(first + w) * v.note_cap + i]] = v.note_old[(first + w) * v.note_cap + i];
+    const size_t first = (size_t)row * lists;
+    // lane l looks after the wave's l-th list (a finish of W waves has rows of 16 W slices at most)
+    const uint32_t its = wave + W * lane;
+    const bool have = its < lists;
+    uint32_t n = have ? v.noted[first + its] : kSievePenLeft;
+    n = n == kSievePenLeft ? 0u : min(n, v.note_cap);
+    if (have) v.noted[first + its] = kSievePenLeft;
+    for (uint32_t l = 0; l * W < lists; l += 4u) {
+        uint32_t at[4][kMost];
+        float4 old[4][kMost];
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            const size_t rec = (first + min(wave + W * (l + u), lists - 1u)) * v.note_cap;
+#pragma unroll
+            for (uint32_t k = 0; k < kMost; ++k) {
+                const size_t i = rec + min(k * (uint32_t)kWave + lane, v.note_cap - 1u);
+                at[u][k] = v.note_at[i]; old[u][k] = v.note_old[i];
+            }
+        }
+#pragma unroll
+        for (uint32_t u = 0; u < 4u; ++u) {
+            const uint32_t of_list = lane_of(n, min(l + u, (uint32_t)kWave - 1u));
+#pragma unroll
+            for (uint32_t k = 0; k < kMost; ++k)
+                if (wave + W * (l + u) < lists && k * (uint32_t)kWave + lane < of_list) pens[at[u][k]] = old[u][k];
+        }
     }
-    __syncthreads();
-    for (uint32_t w = (uint32_t)tid; w < v.G * (uint32_t)kWaves; w += NT) v.noted[first + w] = kSievePenLeft;
     wait_vmem();
     __syncthreads();
 }
