@@ -1859,7 +1859,13 @@ __global__ void __launch_bounds__(kThreads, 2) fused_kernel(const Params p, cons
 #pragma unroll
         for (int i = 0; i < 6; ++i) rs[i] = st[i];
     }
+    // the call's first thread reports on the streaming call before it, if there was one (report_begin)
+    const bool reporter = blockIdx.x == 0 && tid == 0 && p.host_words != nullptr;
+    PrevCall prev;
+    prev.slow_rows = 0; prev.meta = 0;
+    if (reporter) prev = report_begin(p);
     const float lmax = slice_load(p, sl);
+    if (reporter) report_end(p, prev, false);
     const uint32_t key = slice_count_and_stash<R, kThreads, kRep, true>(p, v, u.a, sl.eb, lmax, row, part, sl.base4, sl.nv);
 
     // Count this slice in.  Everything it published went out as device-scope atomic stores (written

@@ -2712,3 +2712,36 @@ def test_sieve_path_plays_penalties_back_in_little_time(torch_cuda, oracle):
     print("the second sums add %.0f us with penalties to play back, %.0f without" % tuple(added), flush=True)
     assert smp.status() == 0 and added[0] < 1.15 * added[1], added
     smp.close()
+
+
+def test_a_slow_penalty_call_sends_the_next_to_the_one_launch_path_for_one_stay(torch_cuda, oracle):
+    """A call with penalties on the sieve path one of whose rows is done the slow way: the next 64 of its kind take the one-launch path, the first of
+    which reports on it, once; the call after them is a good one, and the path is back with the call behind the one that says so.  (Which path a call
+    took is seen by the rows that the sieve path sums again for the diagnostics.)"""
+    torch = torch_cuda
+    from tests import capi
+    B, V = 32, 131072
+    lg_np = H.logits_normal(B, V, 1.5, seed=60)
+    slow_np = lg_np.copy()
+    slow_np[3, ::2] = 40.0
+    pen_np = H.penalties_sparse(B, V, 0.01, seed=61)
+    pen_np[3] = 0.0
+    u_np = H.uniforms(B, 62)
+    rc, c, k, p = capi.normalize(1.0, 50, 0.9, V, B, 1)
+    more = dict(presence=0.1, repetition=0.2, decay=0.95)
+    smp = capi.Sampler(B, V, with_policy=True, init=True)
+    u, lg, slow, pen0 = (torch.from_numpy(a).cuda() for a in (u_np, lg_np, slow_np, pen_np))
+    refs = {name: oracle.sample_batch(a, c, k, p, injected_u=u_np, penalties=pen_np.copy(), **more) for name, a in (("good", lg_np), ("slow", slow_np))}
+
+    def call(name):
+        smp.rows_again()
+        res = smp.sample(slow if name == "slow" else lg, c, k, p, uniforms=u, penalties=pen0.clone(), **more)
+        _check(res, *refs[name], "penalties after a slow row, " + name)
+        return smp.rows_again()
+
+    assert call("good") == B and smp.policy_state() == 0
+    assert call("slow") == B and smp.policy_state() == 2
+    taken = [call("good") for _ in range(70)]
+    assert taken == [0] * 64 + [B] + [0] + [B] * 4, taken
+    assert smp.policy_state() == 0 and smp.status() == 0
+    smp.close()
