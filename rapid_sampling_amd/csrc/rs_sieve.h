@@ -651,7 +651,7 @@ __device__ __forceinline__ void sieve_pens_back(const Params &p, const SieveView
     if (!p.penalties) return;
     constexpr uint32_t W = NT / kWave, kMost = (sieve_pen_cap(8) + kWave - 1u) / kWave;
     const uint32_t lane = threadIdx.x & (kWave - 1u), wave = uniform(threadIdx.x >> 6), lists = v.G * (uint32_t)kWaves;
-    float4 *pens = reinterpret_cast<float4 *>(p.penalties + (int64_t)row * p.V);
+    rs_u32x4 *pens = reinterpret_cast<rs_u32x4 *>(p.penalties + (int64_t)row * p.V);
     const size_t first = (size_t)row * lists;
     // lane l looks after the wave's l-th list (a finish of W waves has rows of 16 W slices at most)
     const uint32_t its = wave + W * lane;
@@ -661,14 +661,14 @@ __device__ __forceinline__ void sieve_pens_back(const Params &p, const SieveView
     if (have) v.noted[first + its] = kSievePenLeft;
     for (uint32_t l = 0; l * W < lists; l += 4u) {
         uint32_t at[4][kMost];
-        float4 old[4][kMost];
+        rs_u32x4 old[4][kMost];
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
             const size_t rec = (first + min(wave + W * (l + u), lists - 1u)) * v.note_cap;
 #pragma unroll
             for (uint32_t k = 0; k < kMost; ++k) {
                 const size_t i = rec + min(k * (uint32_t)kWave + lane, v.note_cap - 1u);
-                at[u][k] = v.note_at[i]; old[u][k] = v.note_old[i];
+                at[u][k] = v.note_at[i]; old[u][k] = reinterpret_cast<const rs_u32x4 *>(v.note_old)[i];
             }
         }
 #pragma unroll
