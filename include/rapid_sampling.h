@@ -435,6 +435,16 @@ int rs_static_status(int32_t *status, uint32_t where[4], int32_t clear, void *st
 int rs_floor_read(const float *logits_device, int64_t row_stride, int32_t *out_device,
                   int32_t B, int32_t V, int32_t variant, void *stream);
 
+/*
+ * What the error bound of the sieve path's sums rests on, over every float:
+ * by how much the hardware's 2^x is larger than the weight e of x, in units of
+ * 2^-24 of it.  below < 0: of x itself, |x| < 125; 0 to 40: of x - M, rounded,
+ * for the frame M that many octaves above floor(x), |M| <= 100.  The least and the
+ * largest, times 2^20, are min- and max-combined into out_device[0] and [1], which
+ * are not cleared.  For tests; no counterpart in the reference.
+ */
+int rs_exp_error(int32_t below, int64_t *out_device, void *stream);
+
 #ifdef __cplusplus
 }
 #endif

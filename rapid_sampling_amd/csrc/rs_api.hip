@@ -1202,4 +1202,11 @@ int rs_floor_read(const float *logits, int64_t row_stride, int32_t *out, int32_t
     return hipGetLastError() == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
 }
 
+int rs_exp_error(int32_t below, int64_t *out, void *stream)
+{
+    if (!out) return RS_ERR_NULL;
+    if (below > 40) return RS_ERR_ARG;
+    return launch_exp_error(below, (hipStream_t)stream, (long long *)out) == hipSuccess ? RS_OK : RS_ERR_LAUNCH;
+}
+
 }  // extern "C"

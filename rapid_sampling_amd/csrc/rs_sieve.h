@@ -24,12 +24,12 @@ namespace rs {
 //
 // The results are the same integers as on every other path.
 //
-// The error of D, in units of 2^-24 of it: v_exp_f32(x) is larger than e of x by 0 to 3.45 (every float |x| < 127 compared), of which 2 are
-// taken off; 16 tokens are summed in a tree of four roundings, their sums in double precision, the slice's sum is
-// rounded once to a float, and the slices' are added as integers of 2^-40 of the frame: 6.5, for which 7 are allowed.  A wave with a value
-// out of v_exp_f32's range, or with a NaN or an infinity, sums 2^(x - M), M the floor of its maximum, whose x - M is
-// rounded: |v_exp_f32(x - M) / e - 1| is at most 5.4 units for tokens up to 8 octaves below the frame, 8.7 to 16, 14.1 to 32, 25.2 to 40 (every float
-// |x| < 128 compared; larger |x| have less of it), so for 4096 tokens, one of them in the frame's octave, at most 9.1; with 3 roundings 12.1, and 32
+// The error of D, in units of 2^-24 of it: v_exp_f32(x) is larger than e of x by -2.96 to 3.45 (a test compares every float); 16 tokens are
+// summed in a tree of four roundings, of one unit each at most, their sums in double precision, and the slice's sum is rounded once to a float, one more:
+// 8.45, for which 9 are allowed.  The slices' are added as integers of 2^-40 of the frame, cut off, which is less than what is allowed for the tokens of no
+// weight (below).  A wave with a value out of v_exp_f32's range, or with a NaN or an infinity, sums 2^(x - M), M the floor of its maximum, whose x - M is
+// rounded: |v_exp_f32(x - M) / e - 1| is at most 5.9 units for tokens up to 8 octaves below the frame, 8.7 to 16, 14.1 to 32, 25.5 to 40 (the same test; where
+// |x| is 128 and more, x - M is exact), so for 4096 tokens, one of them in the frame's octave, at most 9; with 3 roundings 12, and 32
 // are allowed.  Tokens more than 40 octaves below the row's frame weigh nothing but are in the sums: 2^-40 each at most.
 //
 // Where the pass waits for the memory (the host's rule) it sums the tokens' own e in double precision instead (FINE): 2^-40 of D and of the slices' number
@@ -42,7 +42,7 @@ namespace rs {
 // them the exponential, 2.7 issue slots), and a wave some 200 for bound and staging, where the pass with exact e and a histogram (stream_kernel)
 // takes 22 and an LDS atomic.  us of a pass, there / here: 128 rows of 1048576 106 / 86, 64 of 152064 12.7 / 10.1, 256 of 151936 bfloat16
 // 28 / 16.8, of which 12 are the read.
-constexpr uint32_t kSieveErrOdd = 19;                    // D is known to 2^-19 of itself when waves were summed in a frame, else to 7 * 2^-24
+constexpr uint32_t kSieveErrOdd = 19;                    // D is known to 2^-19 of itself when waves were summed in a frame, else to 9 * 2^-24
 
 // Sum over the wave in double precision, in every lane.
 __device__ __forceinline__ double wave_sum_f64(double v)
@@ -738,7 +738,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         D = M96{all << 23, (uint32_t)(all >> 41)};
         if (odd) err = part(kSieveErrOdd);
         else if (dead & 2u) err = part(40u) + M96{1ull << 31, 0u};            // (and 128 slices, cut off at 2^-40)
-        else { D = D - part(23u); err = part(22u) + part(23u) + part(24u); }
+        else err = part(21u) + part(24u);
         if (odd || dead != 2u) err = err + M96{((uint64_t)p.V << 23) + 2ull, 0u};
         P = ceil_mul(p.top_p, D);
     };

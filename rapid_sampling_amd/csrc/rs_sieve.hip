@@ -50,4 +50,30 @@ hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, co
     return hipGetLastError();
 }
 
+// What the error bounds of the sieve path's sums rest on, for every float: by how much, in units of 2^-24, the hardware's 2^x is larger than
+// e of x, at |x| < 125 (below < 0), or the hardware's 2^(x - M) than e of x for the frame `below` octaves above x, |M| <= 100 (further out x - M is exact,
+// and e of it is asked).  out: the least and the largest, in units of 2^-20 of those (both to be set before).
+__global__ void __launch_bounds__(kThreads) exp_error_kernel(const int below, long long *out)
+{
+    const Frame fr(0);
+    double least = 1e9, most = -1e9;
+    for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < 0x42FA0000u; i += gridDim.x * kThreads)
+#pragma unroll
+        for (uint32_t sign = 0; sign < 2u; ++sign) {
+            const float x = __uint_as_float(i | sign << 31), M = below < 0 ? 0.0f : __builtin_floorf(x) + (float)below;
+            if (__builtin_fabsf(M) > 100.0f) continue;
+            const double e = (double)fr.scaled(x), h = __builtin_ldexp((double)__builtin_amdgcn_exp2f(below < 0 ? x : x - M), (int)M);
+            const double off = (h - e) * 0x1p24 / e;
+            least = fmin(least, off); most = fmax(most, off);
+        }
+    atomicMin(&out[0], (long long)floor(least * 0x1p20));
+    atomicMax(&out[1], (long long)ceil(most * 0x1p20));
+}
+
+hipError_t launch_exp_error(int below, hipStream_t st, long long *out)
+{
+    hipLaunchKernelGGL(exp_error_kernel, dim3(4096), dim3(kThreads), 0, st, below, out);
+    return hipGetLastError();
+}
+
 }  // namespace rs

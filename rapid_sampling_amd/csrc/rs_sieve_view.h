@@ -41,5 +41,6 @@ __host__ __device__ constexpr uint32_t sieve_pen_cap(int R) { return 11u * (uint
 // R: groups of four tokens of a thread, 4, 8 or 16: slices of 1024 R tokens; with penalties 4 or 8
 hipError_t launch_sieve_pen(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v);
 hipError_t launch_sieve(int R, int32_t dtype, uint32_t B, hipStream_t st, const Params &p, const SieveView &v);
+hipError_t launch_exp_error(int below, hipStream_t st, long long *out);
 
 }  // namespace rs

@@ -81,6 +81,8 @@ def lib():
         L.rs_static_status.argtypes = [C.POINTER(i32), C.POINTER(C.c_uint32), i32, vp]
         L.rs_floor_read.restype = C.c_int
         L.rs_floor_read.argtypes = [vp, i64, vp, i32, i32, i32, vp]
+        L.rs_exp_error.restype = C.c_int
+        L.rs_exp_error.argtypes = [i32, vp, vp]
         _lib = L
     return _lib
 
