@@ -1252,8 +1252,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
     {
         const Params q = params_again();
         const uint64_t rand64 = q.inj_u ? 0ull : L.rand64;
-        sieve_pens_back<NT>(q, v, row);
-        __syncthreads();
+        __syncthreads();                                 // (the row has been summed again: its penalties are back)
         if (NT > kThreads && tid >= kThreads) return;
         __syncthreads();                                 // the LDS is given over
         finish_row_slow(q, u.slow.s, u.slow.t, row, xmax, rand64);
