@@ -261,7 +261,7 @@ struct LdsFew {
 // D and P are those of `totals(mass of the whole list)`.  Unless they are LooksAtNothing, `decided` and `picked` are told the outcome: decided() by the second wave,
 // which works it out for itself while the first goes on to the token -- the call's P, whether the list is enough, tokens above the threshold and at
 // it, the threshold, the mass above it, the tie weight -- and picked() in the sampled token's lane, by how much the target may move either way
-// against the running sum: within the token's place, and until it is another kept token's.
+// against the running sum.
 struct Totals { M96 D, P; };
 struct LooksAtNothing {};
 template <typename T, typename F = LooksAtNothing, typename K = LooksAtNothing>
@@ -314,18 +314,12 @@ __device__ __forceinline__ uint32_t few_pick(const Params &p, LdsFew &s, const u
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     const Limbs mine = limbs(M96{in ? s.w[lane] : 0ull, 0u}), run = wave_inclusive_scan(mine);
     const M96 bef = m96(run - mine), with = m96(run);
-    // (read by all lanes: behind a branch that lane 63 does not take its sum need not be there)
-    M96 all{0ull, 0u};
-    if constexpr (kLook) all = m96(lane_of(run, 63u));
     const bool is_it = in && bef < r && with >= r;
     if constexpr (kLook) {
         if (is_it) {
-            M96 less = r - bef - M96{1ull, 0u}, more = with - r;
-            auto smaller = [&]() { const bool m = more >= less; return M96{m ? less.lo : more.lo, m ? less.hi : more.hi}; };
-            const M96 to_ends = smaller();
-            if (!(bef.lo | bef.hi)) { less.lo = ~0ull; less.hi = ~0u; }                      // (the first kept token)
-            if (with >= all) { more.lo = ~0ull; more.hi = ~0u; }          // (the last)
-            picked(to_ends, smaller());
+            const M96 less = r - bef - M96{1ull, 0u}, more = with - r;
+            const bool m = more >= less;
+            picked(M96{m ? less.lo : more.lo, m ? less.hi : more.hi});
         }
     }
     return is_it ? s.idx[lane] + 1u : 0u;

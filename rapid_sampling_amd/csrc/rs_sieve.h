@@ -217,13 +217,17 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         const int down = (int)fmaxf(s.frame[lane >> 4] - Ms, -1000.0f);
         const double all = wave_sum_f64(__builtin_ldexp((m2.x + m2.y) + (m3.x + m3.y), down));
         const uint4 o4 = *reinterpret_cast<const uint4 *>(s.odd);
-        const float4 m4 = *reinterpret_cast<const float4 *>(s.frame);
-        const float from = Ms - 41.0f;
-        const bool any = (o4.x != 0u && m4.x >= from) || (o4.y != 0u && m4.y >= from) || (o4.z != 0u && m4.z >= from) || (o4.w != 0u && m4.w >= from);
+        const uint32_t odds = uniform(o4.x | o4.y | o4.z | o4.w);
+        bool any = false;
+        if (__builtin_expect(odds != 0u, 0)) {
+            const float4 m4 = *reinterpret_cast<const float4 *>(s.frame);
+            const float from = Ms - 41.0f;
+            any = (o4.x != 0u && m4.x >= from) || (o4.y != 0u && m4.y >= from) || (o4.z != 0u && m4.z >= from) || (o4.w != 0u && m4.w >= from);
+        }
         if (lane == 0) {
             v.hdr[slice].mass = __float_as_uint((float)all) | (any ? kSieveOdd : 0u);
             if constexpr (FINE) {                        // (a wave that was cleaned up may hold anything: -inf)
-                const uint32_t low = (o4.x | o4.y | o4.z | o4.w) != 0u ? 0x007FFFFFu : ~max(max(s.low[0], s.low[1]), max(s.low[2], s.low[3]));
+                const uint32_t low = odds != 0u ? 0x007FFFFFu : ~max(max(s.low[0], s.low[1]), max(s.low[2], s.low[3]));
                 v.fine[slice] = SieveFine{all, low, 0u};
             }
         }
@@ -498,7 +502,7 @@ struct LdsSieveFin {
     uint64_t list[kSieveList], small[kWave];             // bits of e << 32 | index
     uint64_t blo[NT], bhi[NT];                           // kept weights by bucket of the token index, halves summed apart
     M96      mass[16];
-    struct { M96 D, P, r, err, shift, slack[2]; Edge f; uint64_t w_tie; uint32_t found, other; } one;  // what one wave worked out for all
+    struct { M96 D, P, r, err, shift, slack; Edge f; uint64_t w_tie; uint32_t found; } one;  // what one wave worked out for all
     uint64_t sum[16];
     uint64_t rand64;
     uint32_t flag[16];
@@ -528,8 +532,7 @@ __device__ __forceinline__ bool other_threshold(const M96 err, const M96 least, 
 }
 // How far r and the running sums may shift against each other, P being off by less than err.  The tie weight is (P - above) / n_eq unless that is more than
 // it can be, the threshold's own or the share that top_k leaves of it: then S and r do not move.  The divisions leave less than a unit for each of the
-// ties, of one threshold or, if another is possible, of two of up to 2^20 tokens.  (err is 2^25 and more: where no other is possible, above < P - err,
-// no tie weighs nothing, and the first and the last kept token are the first and the last whatever P is.)
+// ties, of one threshold or, if another is possible, of two of up to 2^20 tokens.
 __device__ __forceinline__ M96 shift_of(const M96 err, const bool other, const M96 least, const uint32_t n_eq, const M96 above, const M96 down, const uint32_t thr,
                                         const uint64_t w_tie)
 {
@@ -870,8 +873,8 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
                             const M96 least = less_by(P, e), down = above + m96((u128)w_of_bits(thr) * n_eq);
                             const bool other = other_threshold(e, least, P + e, top_k, n_gt, n_eq, above, down);
                             doubts = !enough ? 2u : 0u;
-                            if (lane == 0) { L.one.shift = shift_of(e, other, least, n_eq, above, down, thr, w_tie); L.one.other = other ? 1u : 0u; }
-                        }, [&](const M96 &to_ends, const M96 &to_tokens) __attribute__((always_inline)) { L.one.slack[1] = to_ends; L.one.slack[0] = to_tokens; });
+                            if (lane == 0) L.one.shift = shift_of(e, other, least, n_eq, above, down, thr, w_tie);
+                        }, [&](const M96 &slack) __attribute__((always_inline)) { L.one.slack = slack; });
     };
     auto put = [&](uint32_t token, bool few) __attribute__((always_inline)) {
         if (wave <= 1 && doubts) L.unsure = doubts;
@@ -881,8 +884,7 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         }
         __syncthreads();
         const uint32_t u = uniform(L.unsure);
-        const M96 room = L.one.other ? L.one.slack[1] : L.one.slack[0];
-        return few && u == 0u && !(room >= L.one.shift) ? 1u : u;
+        return few && u == 0u && !(L.one.slack >= L.one.shift) ? 1u : u;
     };
     // the tokens for which in(i) says so, side by side
     auto list_them = [&](auto in) __attribute__((always_inline)) {
