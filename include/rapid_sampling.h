@@ -92,7 +92,8 @@ int rs_normalize_args(double temperature, int64_t top_k, double top_p,
  * where slices are shorter; 1.5 bytes per token in rows of up to 262144
  * tokens, for the slices of 8192 tokens the one-pass wide path, the
  * counting-only pass and the pass with penalties cut there; the sieve path lays
- * its own records, 1.1 bytes per token at most, over the same space); a quarter to two fifths of the reference's
+ * its own records, up to 1.1 bytes per token, over the same space, and calls for
+ * which they do not fit take the streaming path); a quarter to two fifths of the reference's
  * scratch.  It does not grow with T.  (A call is also accepted with a
  * workspace that lacks the room for those slices of 8192 tokens -- the size
  * versions before 414 asked for -- and then works on the long slices.)

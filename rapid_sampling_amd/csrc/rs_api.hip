@@ -974,7 +974,8 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
         const size_t fine = pen ? align256(note_old + waves * v.note_cap * sizeof(float4)) : noted;
         const bool want_fine = sieve_fine(B, V, top_k, logits_dtype, pen);
         const size_t end = want_fine ? align256(fine + slices * sizeof(SieveFine)) : fine;
-        // (a workspace of rs_workspace_bytes has room, 0.26 bytes a token at most, 1.1 with penalties; one without takes the streaming path)
+        // (A workspace of rs_workspace_bytes has room, but for calls with penalties and a top_k of 700 and more in rows of 350000 to 525000 tokens, which set
+        // 128 tokens of a slice of 4096 aside: up to an eighth too little.  They take the streaming path, as calls with a smaller workspace do.)
         if (end + (size_t)B * sizeof(RowCtl) <= (workspace_bytes & ~(size_t)255)) {
             char *w = (char *)workspace;
             v.hdr = (SieveHdr *)(w + hdr); v.stash = (uint64_t *)(w + stash);

@@ -2482,9 +2482,10 @@ def test_sieve_path_diagnostics_of_long_lists(torch_cuda, oracle, B, V, k):
     (16, 1048576, 512, "float32", 0.0, None, True), (64, 1048576, 50, "float32", 0.0, None, True), (20, 1048576, 600, "bfloat16", 0.0, None, True),
     (23, 131072, 50, "float32", 0.02, None, False), (24, 131072, 50, "float32", 0.02, None, True), (24, 131072, 65, "float32", 0.02, None, False),
     (256, 65536, 128, "float32", 0.02, None, True), (128, 131072, 50, "bfloat16", 0.02, None, True), (128, 131072, 50, "float16", 0.02, None, True),
-    (128, 131072, 129, "float32", 0.02, None, False), (64, 1048576, 1024, "float32", 0.02, None, True)])
+    (128, 131072, 129, "float32", 0.02, None, False), (64, 1048576, 1024, "float32", 0.02, None, True),
+    (168, 400000, 640, "float32", 0.02, None, True), (168, 400000, 1024, "float32", 0.02, None, False)])
 def test_which_calls_take_the_sieve_path(torch_cuda, oracle, B, V, k, dtype, share, path, sieve):
-    """Seen by the rows it sums again for the diagnostics: the edges of its rule, and calls for each of its kernels -- slices of 4096, 8192 and 16384 tokens,
+    """Seen by the rows it sums again for the diagnostics: the edges of its rule, of what a workspace has room for, and calls for each of its kernels -- slices of 4096, 8192 and 16384 tokens,
     the three formats, float and double sums, with penalties and without.  Some kinds of rows over and over, in every field against the oracle."""
     torch = torch_cuda
     from tests import capi
@@ -2769,3 +2770,41 @@ def test_hardware_exponential_over_every_float(torch_cuda):
         assert -bound <= least and most <= bound
     out = torch.zeros(2, dtype=torch.int64, device="cuda")
     assert capi.lib().rs_exp_error(41, out.data_ptr(), st) != 0 and capi.lib().rs_exp_error(0, None, st) != 0
+
+
+@pytest.mark.parametrize("V,k,decay", [(16388, 70, 0.95), (40000, 200, 0.95), (131072, 200, float("inf")), (262144, 320, 0.95), (1048576, 200, 0.95), (1048576, 1000, 0.95)])
+def test_streaming_path_where_the_sieve_path_is_not_taken(torch_cuda, oracle, V, k, decay):
+    """Small calls with a top_k of more than 64 keep to the streaming path, its stashes, its notes of penalties and its fix-up: rows of every kind that
+    the sieve path's tests have, without penalties and with none, few, scattered, many and only non-zero ones, a stretch of them, infinities, NaN and
+    -0.0 among them; two chained steps, every field and every penalty against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    lg = _sieve_rows(V)
+    B = lg.shape[0]
+    rng = np.random.default_rng(V + k)
+    pen = rng.exponential(1.0, (B, V)).astype(np.float32)
+    share = np.array([0.0, 0.001, 0.02, 0.05, 0.3, 1.0, 0.01, 0.02, 0.02, 0.02, 0.02, 0.01])
+    pen *= rng.random((B, V)) < share[:, None]
+    pen[2, : V // 16] = 0.5
+    pen[1, 77] = -0.0
+    pen[7, [3, 5000, V - 2]] = [np.inf, -np.inf, np.nan]
+    if decay != 0.95:
+        pen[:] = 0.0                                                    # 0 * inf: every entry becomes NaN, zeros too
+    x = torch.from_numpy(lg).cuda()
+    smp = capi.Sampler(B, V)
+    rc, c, kk, p = capi.normalize(0.8, k, 0.9, V, B, 1)
+    more = dict(presence=0.1, repetition=0.2, decay=decay)
+    for with_pen in (False, True):
+        want = pen.copy()
+        have = torch.from_numpy(pen.copy()).cuda()
+        for step in range(2 if decay == 0.95 else 1):
+            u_np = H.uniforms(B, k + step)
+            u_np[:3] = [1.0, 1e-30, 0.5]
+            ref = oracle.sample_batch(lg, c, kk, p, injected_u=u_np, want_e=True, **(dict(more, penalties=want) if with_pen else {}))
+            print("streaming path:", V, k, decay, with_pen, step, flush=True)
+            smp.rows_again()
+            res = smp.sample(x, c, kk, p, uniforms=torch.from_numpy(u_np).cuda(), want_e=True, path="stream", **(dict(more, penalties=have) if with_pen else {}))
+            _check(res, ref[0], ref[1], "streaming path, top_k %d" % k, ref[2])
+            assert smp.rows_again() == 0 and smp.status() == 0
+            assert not with_pen or np.array_equal(have.cpu().numpy().view(np.uint32), want.view(np.uint32))
+    smp.close()
