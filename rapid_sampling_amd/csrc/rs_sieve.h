@@ -967,8 +967,8 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
         auto step_of = [&](uint32_t e) { return min((uint32_t)((float)(e - from) * scale), kSieveSteps - 1u); };
         look_at([&](uint32_t e) { atomicAdd(&L.step[lane & (NT / 128 - 1)][step_of(e)], 1u); });
         __syncthreads();
-        // four steps a lane, the largest first: at which of them top_k tokens are reached, as far as they fit
-        const uint32_t aim = top_k, most = aim <= (uint32_t)kWave ? (uint32_t)kWave : kSieveList;
+        // four steps a lane, the largest first: at which of them top_k tokens are reached, if they fit then
+        const uint32_t aim = top_k;
         uint32_t n = 0, step = 0, all = 0;
         if (kEach || wave == 0) {
             uint32_t c[4] = {0u, 0u, 0u, 0u};
@@ -983,13 +983,9 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             if (all > aim) {
                 const uint32_t l = (uint32_t)__builtin_ctzll(__builtin_amdgcn_ballot_w64(upto >= aim));
                 n = lane_of(upto - c[0] - c[1] - c[2] - c[3], l); step = 256u - 4u * l;
-                uint32_t more = n;
 #pragma unroll
-                for (int k = 0; k < 4; ++k) {
-                    more += lane_of(c[k], l);
-                    if (n < aim && more <= most) { n = more; step = 255u - 4u * l - (uint32_t)k; }
-                    else if (n < aim) break;
-                }
+                for (int k = 0; k < 4; ++k)
+                    if (n < aim) { n += lane_of(c[k], l); step = 255u - 4u * l - (uint32_t)k; }
             }
         }
         if constexpr (!kEach) {
@@ -997,8 +993,8 @@ __global__ void __launch_bounds__(sieve_finish_threads<NT>()) sieve_finish_kerne
             __syncthreads();
             n = uniform(L.one.f.at); step = uniform(L.one.f.cnt_above); all = uniform(L.one.f.cnt_bin);
         }
-        // (short of top_k, it may still be P)
-        listed = n != 0u && n <= most && (n >= top_k || n == all || p.top_p < 1.0f);
+        // (fewer than top_k, which are all there are, may still be P)
+        listed = n != 0u && n <= kSieveList;
         if (listed) {
             list_them([&](int i) { return b[i] != 0u && step_of(b[i]) >= step; });
             n_list = n;
