@@ -966,6 +966,7 @@ int rs_sample_ex(const void *logits, int32_t logits_dtype, int64_t row_stride, f
         v.G = stream_parts(V, R);
         v.units = sieve_share(top_k, V, R) <= 8u ? 1u : 2u;
         v.reach = sieve_reach(V, top_k, R, v.units);
+        v.keep = (uint32_t)top_k <= v.units * (uint32_t)kWave ? (uint32_t)top_k : v.units * (uint32_t)kWave / 2u;      // (its slice may hold them all)
         const size_t slices = (size_t)B * v.G, hdr = align256(sizeof(WsHeader)), stash = align256(hdr + slices * sizeof(SieveHdr));
         v.note_cap = sieve_pen_cap(R);
         v.fixers = min(v.G, max(8u, 1536u / (uint32_t)B));           // (a slice each while that is not many workgroups)

@@ -206,9 +206,9 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         c[0] = uniform(f4.x); c[1] = uniform(f4.y); c[2] = uniform(f4.z); c[3] = uniform(f4.w);
         const uint32_t most = max(max(c[0], c[1]), max(c[2], c[3]));
         if (__builtin_expect(most <= (uint32_t)kWave && c[0] + c[1] + c[2] + c[3] <= room, 1)) break;
-        // more groups than there is room for (threads with many of them, ties): fewer threads; in the end none, and no token above the maximum
-        if (want <= 8u || lo == key) { full = true; break; }
-        want -= 8u;
+        // more groups than there is room for (threads with many of them, ties): fewer threads, in the end one; if there are too many like it, none
+        if (want == 1u || lo == key) { full = true; break; }
+        want = want > 8u ? want - 8u : 1u;
         hi = key;
     }
     if (wave == 1) {
@@ -248,22 +248,22 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         // the tokens of those groups, by the first wave, a group to a lane
         const uint32_t all = c[0] + c[1] + c[2] + c[3];
         uint64_t *st = v.stash + slice * room;
-        // Mostly they fit.  If not (several tokens of a group), the bound is raised, by a 64th to a 32nd of itself and twice as much each time, until they do,
-        // and lowered again when they fill less than half of the room: `over` is one that too many reach, from `fits` on they fit.  (A fixed part of
-        // the way up to the slice's largest token depends on how far up that is: in rows with a few spikes hardly a token was left, and rows whose top_k
-        // tokens were then not all there had to be summed again, 64 x 1048576 with a top_k of 1024 457 us a call, 62 like this.)
-        const uint32_t first = lo;
-        for (uint32_t over = lo, fits = key + 1u, step = 1u << 18;;) {
+        // the group that is the lane's u-th
+        auto group_of = [&](const uint32_t g, float (&t)[4]) __attribute__((always_inline)) {
+            uint32_t w = 0, at = g;
+            if (at >= c[0]) { at -= c[0]; w = 1u; }
+            if (w == 1u && at >= c[1]) { at -= c[1]; w = 2u; }
+            if (w == 2u && at >= c[2]) { at -= c[2]; w = 3u; }
+            const float4 q4 = s.grp[w][at & 63u];
+            t[0] = q4.x; t[1] = q4.y; t[2] = q4.z; t[3] = q4.w;
+            return s.gidx[w][at & 63u] * 4u;
+        };
+        for (;;) {
             n = 0;
             for (uint32_t g = (uint32_t)lane; g < room; g += kWave) {
-                uint32_t w = 0, at = g;
-                if (at >= c[0]) { at -= c[0]; w = 1u; }
-                if (w == 1u && at >= c[1]) { at -= c[1]; w = 2u; }
-                if (w == 2u && at >= c[2]) { at -= c[2]; w = 3u; }
                 const bool have = g < all;
-                const float4 q4 = s.grp[w][at & 63u];
-                const uint32_t i0 = s.gidx[w][at & 63u] * 4u;
-                const float t[4] = {q4.x, q4.y, q4.z, q4.w};
+                float t[4];
+                const uint32_t i0 = group_of(g, t);
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
                     const bool in = have && t[q] >= bound;
@@ -273,12 +273,32 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
                     n += (uint32_t)__builtin_popcountll(vote);
                 }
             }
-            if (n > room) over = lo; else fits = lo;
-            if (__builtin_expect(n <= room && (lo == first || n * 2u >= room || fits - over <= 1u), 1)) { cut = lo - 1u; break; }
-            if (fits > key && fits - over <= 1u) { n = 0; break; }           // ties of the largest
-            if (fits > key) { lo = key - over > step ? over + step : key; step *= 2u; }
-            else lo = fits - over <= 1u ? fits : over + ((fits - over) >> 1);
-            bound = fkey_inv(lo);
+            if (__builtin_expect(n <= room, 1)) { cut = lo - 1u; break; }
+            // Too many (several tokens of a group): a bound is looked for that no more reach than there is room for, but v.keep all the same, or as many as ties
+            // leave -- upwards in steps of a 64th to a 32nd of it, twice as long each time, until they fit, then by halving.  Too many reach `over`, from
+            // `fits` on they fit.  (A fixed part of the way up to the slice's largest token depends on how far up that is: in rows with a few spikes hardly a
+            // token was left, and rows whose top_k tokens were then not all there had to be summed again, 64 x 1048576 with a top_k of 1024 455 us a call,
+            // 59 like this.  There is always a slice like that in a call of hundreds: what this takes the whole call takes longer.)
+            uint32_t k8[8];
+#pragma unroll
+            for (uint32_t u = 0; u < 2u; ++u) {
+                const uint32_t g = u * kWave + (uint32_t)lane;
+                float t[4];
+                group_of(g, t);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) k8[u * 4u + q] = g < all ? fkey(t[q]) : 0u;
+            }
+            uint32_t over = lo, fits = key + 1u;
+            for (uint32_t step = 1u << 18; fits - over > 1u; step *= 2u) {
+                const uint32_t mid = fits <= key ? over + ((fits - over) >> 1) : key - over > step ? over + step : key;
+                uint32_t r = 0;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) r += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(k8[i] >= mid));
+                if (r > room) over = mid;
+                else { fits = mid; if (r >= v.keep) break; }
+            }
+            if (fits > key) { n = 0; break; }            // ties of the largest
+            lo = fits; bound = fkey_inv(lo);
         }
     }
     if (tid == 0) {

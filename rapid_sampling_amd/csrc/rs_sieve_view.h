@@ -26,6 +26,7 @@ struct SieveView {
     uint32_t  G;             // slices per row
     uint32_t  units;         // a slice sets aside at most 64 tokens (1) or 128 (2)
     uint32_t  reach;         // pairs of threads, of a slice's 128, whose largest token is set aside
+    uint32_t  keep;          // tokens that a slice with more than it has room for sets aside at least
     // calls with penalties: the groups of four of which one penalty's bit pattern is not +0.0, as they were
     uint32_t *noted;         // [B][G][4]            how many a wave has noted, or kSievePenLeft
     uint32_t *note_at;       // [B][G][4][note_cap]  which groups of the row

@@ -2821,3 +2821,44 @@ def test_sieve_path_lists_of_a_few_tokens_more_than_64(torch_cuda):
     a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_temperature_topk_topp(x, st, 0.8, k, 0.95), "stream") for k in (64, 50))
     print("top_k 64 %.1f us, 50 %.1f us: %.2f" % (a, b, a / b), flush=True)
     assert a < 1.32 * b, (a, b)
+
+
+@pytest.mark.parametrize("kind", ["sorted", "block", "ties"])
+@pytest.mark.parametrize("V,k,dtype,share", [(152064, 20, "float32", 0.0), (152064, 50, "float32", 0.0), (50260, 40, "bfloat16", 0.0), (131072, 50, "float32", 0.02), (1048576, 40, "float32", 0.0)])
+def test_sieve_path_rows_whose_largest_tokens_lie_together(torch_cuda, oracle, kind, V, k, dtype, share):
+    """Slices that hold more of a row's largest tokens than they have room for: sorted rows, a block of 100 tokens far above the rest, and a few equal
+    ones, the row's largest, beside hundreds of the next value.  They set aside as many as fit, top_k of them at least, and no row is read again.
+    Tokens against the oracle."""
+    torch = torch_cuda
+    from tests import capi
+    B = 64 if not share else 32
+    rng = np.random.default_rng(V + k)
+    lg = (rng.standard_normal((8, V)) * 2.0).astype(np.float32)
+    if kind == "sorted":
+        lg = np.sort(lg)
+        lg[::2] = lg[::2, ::-1]
+    elif kind == "block":
+        lg[:, V // 3: V // 3 + 100] += 12.0
+    else:
+        lg = np.minimum(np.round(lg), 3.0)
+        lg[:, V // 9] = lg[:, V // 2 + 1] = lg[:, V // 2 + 900] = 9.0
+    lg = torch.from_numpy(lg).to(getattr(torch, dtype)).float().numpy()
+    u_np = H.uniforms(8, k)
+    x = torch.from_numpy(lg).cuda().to(getattr(torch, dtype)).repeat(B // 8, 1).contiguous()
+    u = torch.from_numpy(np.tile(u_np, B // 8)).cuda()
+    pen = H.penalties_sparse(8, V, share, seed=V) if share else None
+    top_k = 2 if kind == "ties" else k
+    rc, c, kk, p = capi.normalize(0.8, top_k, 1.0, V, B, 1)
+    more = dict(presence=0.1, repetition=0.2, decay=0.95) if share else {}
+    have = torch.from_numpy(np.tile(pen, (B // 8, 1))).cuda() if share else None
+    ref = oracle.sample_batch(lg, c, kk, p, injected_u=u_np, **(dict(more, penalties=pen) if share else {}))[0]
+    smp = capi.Sampler(B, V)
+    smp.rows_again()
+    print("largest tokens together:", kind, B, V, k, dtype, share, flush=True)
+    res = smp.sample(x, c, kk, p, uniforms=u, want_diag=False, penalties=have, **more)
+    again = smp.rows_again()
+    assert np.array_equal(res["out"], np.tile(ref, B // 8)) and smp.status() == 0
+    assert again == 0, again
+    if share:
+        assert np.array_equal(have.cpu().numpy().view(np.uint32), np.tile(pen, (B // 8, 1)).view(np.uint32))
+    smp.close()
