@@ -590,13 +590,16 @@ static int sieve_r(int32_t B, int32_t V, int32_t top_k, bool pen)
     return sieve_share(top_k, V, R) <= 16u ? R : 0;
 }
 // Of a slice's 128 pairs of threads, how many reach the bound of what is set aside: as many as hold one of eight times the slice's share of the
-// top_k tokens (of all of them, if they are fewer), each in a pair by chance, and some more; as far as there is room: 44 to 47 pairs hold some 56 of a room of 64,
-// 72 to 75 some 110 of 128.  (48 and 78 filled it to the brim, and half of the slices had a token too many and raised their bound: us a call, with
-// those / now, 128 x 1048576 top_k 1024 109.5 / 103.0, 256 x 131072 top_k 300 40.0 / 38.7.)
+// top_k tokens (of all of them, if they are fewer), each in a pair by chance, and some more; as far as there is room: 40 to 43 pairs hold some 50 of a room of 64,
+// 70 to 73 some 106 of 128.  (48 and 78 filled it to the brim, and half of the slices had a token too many and raised their bound: us a call, with
+// those / now, 128 x 1048576 top_k 1024 109 / 104, 256 x 131072 top_k 300 39.8 / 38.1.)  And with a top_k of up to 42 as many as have all of these tokens
+// among theirs, k pairs and hardly any two in one, so that a row whose largest tokens lie in one slice -- all but a stretch of the vocabulary masked -- need not be
+// read again: 64 x 152064 top_k 20, a sixteenth of each row 5 higher, 100.5 / 16.7, ordinary rows 0 to 0.1 longer.
 static uint32_t sieve_reach(int32_t V, int32_t top_k, int R, uint32_t units)
 {
     const double all = (double)top_k, m = min(8.0 * all * 1024.0 * R / V, all);
-    return min((uint32_t)(128.0 * (1.0 - exp(-m / 128.0)) + 2.0 * sqrt(m) + 4.0), units == 1u ? 44u : 72u);
+    const uint32_t by_share = (uint32_t)(128.0 * (1.0 - exp(-m / 128.0)) + 2.0 * sqrt(m) + 4.0), all_of_them = top_k <= 42 ? (uint32_t)(top_k - top_k * top_k / 640) : 0u;
+    return min(max(by_share, all_of_them), units == 1u ? 40u : 70u);
 }
 
 // With penalties, the histogram's pass / here (N(0,1.5), top_p 0.9, one token in a hundred penalised):

@@ -2823,14 +2823,16 @@ def test_sieve_path_lists_of_a_few_tokens_more_than_64(torch_cuda):
     assert a < 1.32 * b, (a, b)
 
 
-@pytest.mark.parametrize("kind", ["sorted", "block", "ties"])
+@pytest.mark.parametrize("kind", ["sorted", "block", "ties", "masked"])
 @pytest.mark.parametrize("V,k,dtype,share", [(152064, 20, "float32", 0.0), (152064, 50, "float32", 0.0), (50260, 40, "bfloat16", 0.0), (131072, 50, "float32", 0.02), (1048576, 40, "float32", 0.0)])
 def test_sieve_path_rows_whose_largest_tokens_lie_together(torch_cuda, oracle, kind, V, k, dtype, share):
     """Slices that hold more of a row's largest tokens than they have room for: sorted rows, a block of 100 tokens far above the rest, and a few equal
-    ones, the row's largest, beside hundreds of the next value.  They set aside as many as fit, top_k of them at least, and no row is read again.
-    Tokens against the oracle."""
+    ones, the row's largest, beside hundreds of the next value; and rows of which all but the 2000 tokens of one slice is masked (up to a top_k of 42).
+    They set aside as many as fit, top_k of them at least, and no row is read again.  Tokens against the oracle."""
     torch = torch_cuda
     from tests import capi
+    if kind == "masked" and k > 42:
+        k = 30
     B = 64 if not share else 32
     rng = np.random.default_rng(V + k)
     lg = (rng.standard_normal((8, V)) * 2.0).astype(np.float32)
@@ -2839,6 +2841,9 @@ def test_sieve_path_rows_whose_largest_tokens_lie_together(torch_cuda, oracle, k
         lg[::2] = lg[::2, ::-1]
     elif kind == "block":
         lg[:, V // 3: V // 3 + 100] += 12.0
+    elif kind == "masked":
+        lg[:, :16384] = -np.inf
+        lg[:, 16384 + 2000:] = -np.inf
     else:
         lg = np.minimum(np.round(lg), 3.0)
         lg[:, V // 9] = lg[:, V // 2 + 1] = lg[:, V // 2 + 900] = 9.0
