@@ -42,7 +42,7 @@
 //     caller's rs_policy, which routes the next calls of that kind.
 //
 //   sieve path (sieve_kernel + sieve_finish_kernel, two launches, no waits): the streaming
-//     path's calls with a top_k of up to 64, and larger calls with more.  The pass sums the
+//     path's calls with a top_k of up to 58, and larger calls with more.  The pass sums the
 //     row approximately and sets its largest tokens aside; the finish makes sure that nothing
 //     it decides depends on what the sum is off by.  With penalties (sieve_pen_kernel,
 //     the same finish, sieve_pen_fix_kernel): the pass writes the decayed penalties, too.
@@ -560,7 +560,9 @@ static int fused_r(int32_t B, int32_t V, bool pen, bool any_size)
 // and, at the line for longer lists, which used to be finished by 1024 threads: 64 x 262144 top_k 300 25.6 / 25.5, 128 x 131072 29.2 / 26.7, bfloat16
 // 16 x 1048576 24.6 / 23.6, 32 x 1048576 top_k 1000 40.0 / 39.4; below it 64 x 131072 top_k 100 17.7 / 17.8 and, N(0,3) with top_p 0.3, 17.1 / 17.9.
 // (1 x 32768: 8.9 there and 9.7 here with 16 spikes.)  Its finish compares up to 64 tokens with each other, for which it is as short as the streaming
-// path's; longer lists are faster there until the pass outweighs them.  Slices of 4096 tokens while 32 of them make a row, else of
+// path's; longer lists are faster there until the pass outweighs them, and with a top_k of 59 to 64 most are longer by the last step that they are cut at: there /
+// here, top_k 58, 60, 64 of rows with 16 spikes, 1 x 50304 10.4 / 10.3, 10.4 / 12.1, 10.4 / 12.0; 64 x 152064 19.7 / 15.2, 19.6 / 17.8, 19.6 / 18.3; with
+// penalties 32 x 131072 18.5 / 18.1, 18.5 / 19.5, 18.6 / 21.1.  Slices of 4096 tokens while 32 of them make a row, else of
 // 8192, and of 16384 in a few rows of a million (1 x 1048576 12.0 us against 14.1); shorter when one would hold more than 8 of the row's top_k on
 // average, since a slice sets aside 64 tokens: at least four times its share.  (Up to 16 in slices of 4096, which then set aside 128.)
 // Without a bounding top_k the kept set may be of hundreds of tokens, the longer list's time, and each is one more place where D is too close to
@@ -583,7 +585,7 @@ static bool sieve_fine(int32_t B, int32_t V, int32_t top_k, int32_t dtype, bool 
 static int sieve_r(int32_t B, int32_t V, int32_t top_k, bool pen)
 {
     const uint64_t tokens = (uint64_t)B * (uint64_t)V;
-    if (tokens < (top_k <= 64 ? 49152u : 1u << 24) || (!pen && V <= kMidMaxV && top_k > kSieveK)) return 0;
+    if (tokens < (top_k <= 58 ? 49152u : top_k <= 64 ? 1u << 23 : 1u << 24) || (!pen && V <= kMidMaxV && top_k > kSieveK)) return 0;
     const uint32_t g4 = stream_parts(V, 4), g8 = stream_parts(V, 8);
     int R = g4 <= 32u && (uint64_t)B * g4 <= kStreamSmallParts ? 4 : g8 <= 64u || (uint64_t)B * g8 > 8192u ? 8 : 16;
     while (R > 4 && sieve_share(top_k, V, R) > 8u && stream_parts(V, R / 2) <= 128u) R /= 2;

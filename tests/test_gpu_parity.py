@@ -2476,7 +2476,9 @@ def test_sieve_path_diagnostics_of_long_lists(torch_cuda, oracle, B, V, k):
 
 
 @pytest.mark.parametrize("B,V,k,dtype,share,path,sieve", [
-    (3, 16380, 40, "float32", 0.0, None, False), (4, 16388, 64, "float32", 0.0, None, True), (2, 16388, 64, "float32", 0.0, None, False),
+    (3, 16380, 40, "float32", 0.0, None, False), (4, 16388, 58, "float32", 0.0, None, True), (2, 16388, 58, "float32", 0.0, None, False),
+    (4, 16388, 59, "float32", 0.0, None, False), (64, 131072, 64, "float32", 0.0, None, True), (63, 131072, 59, "float32", 0.0, None, False),
+    (63, 131072, 64, "float32", 0.02, None, False),
     (1, 50304, 50, "bfloat16", 0.0, None, True), (64, 131072, 65, "float32", 0.0, None, False), (128, 131072, 65, "float32", 0.0, None, True),
     (128, 131072, 320, "float16", 0.0, "stream", True), (128, 131072, 321, "float32", 0.0, "stream", False), (20, 1048576, 1024, "float32", 0.0, None, True),
     (16, 1048576, 512, "float32", 0.0, None, True), (64, 1048576, 50, "float32", 0.0, None, True), (20, 1048576, 600, "bfloat16", 0.0, None, True),
