@@ -72,7 +72,11 @@ struct LdsSieve {
 // The terms of the sum need no frame: 2^x is a float for every x in question, and so they are worked out in the order in which
 // the loads arrive.  A wave whose largest x is beyond 120 or below -80 (the tokens 40 octaves below it would no longer be floats), or
 // that holds a NaN or an infinity, does it again, cleaned up and in a frame.
-template <int R, bool FINE, typename G, typename Z, typename A, typename E>
+//
+// kGrain: two tokens' keys are equal or further apart than this.  Halving a range ends there: 10 turns less for bfloat16, whose ties hardly ever leave as many
+// threads as are wanted (512 x 32768 with logits near 20, top_k 50: 29.7 us a call with 1, 26.7 like this).
+constexpr uint32_t sieve_grain(int dtype) { return dtype == RS_DTYPE_BF16 ? 1u << 13 : dtype == RS_DTYPE_F16 ? 1u << 10 : 1u; }   // (of products of 8 and 11 bits by one factor)
+template <int R, bool FINE, uint32_t kGrain, typename G, typename Z, typename A, typename E>
 __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G group, Z strange, A redo, E then, const size_t slice, const uint32_t g0, const uint32_t left, const int tid)
 {
     const float kInf = __builtin_inff();
@@ -179,9 +183,18 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
     uint32_t c[kWaves] = {0u, 0u, 0u, 0u};               // of each wave, its groups that reach the bound
     for (uint32_t turn = 0;; turn ^= 1u) {
 #pragma unroll 1
-        while (reach > want + 3u && hi - lo > 1u) {
+        while (reach > want + 3u && hi - lo > kGrain) {
             const uint32_t mid = lo + ((hi - lo) >> 1), r = reached(mid);
             if (r >= want) { lo = mid; reach = r; } else hi = mid;
+        }
+        // (ties at the bound, of more threads than there is room for: none of them)
+        auto leave_ties = [&]() { lo = hi; hi = key; reach = want = reached(lo); };
+        if (__builtin_expect(hi - lo <= kGrain && lo != key && reach * 2u > room, 0)) {
+            const float4 t = reinterpret_cast<const float4 *>(s.top)[opaque((uint32_t)lane)];            // (again: kept, it would cost the usual way registers)
+            uint32_t threads = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) threads += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(fkey(i == 0 ? t.x : i == 1 ? t.y : i == 2 ? t.z : t.w) >= lo));
+            if (threads > room) leave_ties();
         }
         bound = fkey_inv(lo);
         // the wave's groups that reach it, side by side
@@ -208,8 +221,8 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
         if (__builtin_expect(most <= (uint32_t)kWave && c[0] + c[1] + c[2] + c[3] <= room, 1)) break;
         // more groups than there is room for (threads with many of them, ties): fewer threads, in the end one; if there are too many like it, none
         if (want == 1u || lo == key) { full = true; break; }
-        want = want > 8u ? want - 8u : 1u;
-        hi = key;
+        if (hi - lo <= kGrain) leave_ties();
+        else { want = want > 8u ? want - 8u : 1u; hi = key; }
     }
     if (wave == 1) {
         // the slice's sum: lane l those of threads 4 l to 4 l + 3, all of one wave
@@ -289,11 +302,25 @@ __device__ __forceinline__ void sieve_slice(const SieveView &v, LdsSieve &s, G g
                 for (int q = 0; q < 4; ++q) k8[u * 4u + q] = g < all ? fkey(t[q]) : 0u;
             }
             uint32_t over = lo, fits = key + 1u;
-            for (uint32_t step = 1u << 18; fits - over > 1u; step *= 2u) {
-                const uint32_t mid = fits <= key ? over + ((fits - over) >> 1) : key - over > step ? over + step : key;
+            auto next_to = [&](const uint32_t k) __attribute__((always_inline)) {        // the least token's key from k on, all ones if there is none
+                uint32_t least = ~0u;
+#pragma unroll
+                for (int i = 0; i < 8; ++i) least = k8[i] >= k ? min(least, k8[i]) : least;
+                return ~wave_max_u32(~least);
+            };
+            auto reach_it = [&](const uint32_t k) __attribute__((always_inline)) {
                 uint32_t r = 0;
 #pragma unroll
-                for (int i = 0; i < 8; ++i) r += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(k8[i] >= mid));
+                for (int i = 0; i < 8; ++i) r += (uint32_t)__builtin_popcountll(__builtin_amdgcn_ballot_w64(k8[i] >= k));
+                return r;
+            };
+            // (past the least token's value first: there may be many of it)
+            const uint32_t next = next_to(next_to(lo) + 1u);
+            if (next <= key) {
+                if (reach_it(next) <= room) over = (fits = next) - 1u; else over = next;
+            } else over = key;
+            for (uint32_t step = 1u << 18; fits - over > 1u; step *= 2u) {
+                const uint32_t mid = fits <= key ? over + ((fits - over) >> 1) : key - over > step ? over + step : key, r = reach_it(mid);
                 if (r > room) over = mid;
                 else { fits = mid; if (r >= v.keep) break; }
             }
@@ -336,7 +363,7 @@ __global__ void __launch_bounds__(kThreads, R == 16 ? (FINE ? 3 : 4) : !FINE ? 8
         for (int j = 0; j < R; ++j) l[j] = __builtin_nontemporal_load(from + min((uint32_t)(j * kThreads + tid), left - 1u));
     }
     if (reporter) report_end(p, prev, true);
-    sieve_slice<R, FINE>(v, s, [&](int j, float *x) {
+    sieve_slice<R, FINE, sieve_grain(DT)>(v, s, [&](int j, float *x) {
         uint32_t w[4];
         if constexpr (DT == RS_DTYPE_F32) { w[0] = l[j].x; w[1] = l[j].y; w[2] = l[j].z; w[3] = l[j].w; }
         else widen4(make_uint2(l[j].x, l[j].y), DT, w);
@@ -408,7 +435,7 @@ __global__ void __launch_bounds__(kThreads, R == 8 ? 4 : 6) sieve_pen_kernel(con
     };
     uint32_t fill = 0;
     uint32_t low = 0u;                                   // bit pattern of the most negative penalty
-    sieve_slice<R, FINE>(v, s, [&](int j, float *x) __attribute__((always_inline)) {
+    sieve_slice<R, FINE, 1u>(v, s, [&](int j, float *x) __attribute__((always_inline)) {
         uint32_t w[4];
         widen(l[j], w);
         const uint32_t b[4] = {pn[j].x, pn[j].y, pn[j].z, pn[j].w};

@@ -2869,3 +2869,19 @@ def test_sieve_path_rows_whose_largest_tokens_lie_together(torch_cuda, oracle, k
     if share:
         assert np.array_equal(have.cpu().numpy().view(np.uint32), np.tile(pen, (B // 8, 1)).view(np.uint32))
     smp.close()
+
+
+def test_sieve_path_slices_with_ties_at_their_bound(torch_cuda):
+    """Rows of 60 large tokens over whole numbers, whose slices have ties of more threads than there is room for at the bound they look for, against
+    the same over distinct values.  Time ratio, measured 1.21; 1.53 when the bound was tried again and again, for eight threads fewer each time."""
+    torch = torch_cuda
+    import rapid_sampling_amd as sample
+    gen = torch.Generator(device="cuda").manual_seed(7)
+    x = torch.randn((64, 50304), generator=gen, device="cuda").mul_(2.0)
+    y = x.round()
+    for z in (x, y):
+        z[:, torch.arange(60, device="cuda") * 838] = 12.0 + torch.arange(60, device="cuda") * 0.11
+    st = sample.setup_rand(1, 64)
+    a, b = (_us_per_call(torch, sample, lambda: sample.batch_sampling_temperature_topk_topp(z, st, 0.8, 40, 0.95), "stream") for z in (y, x))
+    print("whole numbers %.1f us, distinct %.1f us: %.2f" % (a, b, a / b), flush=True)
+    assert a < 1.35 * b, (a, b)
