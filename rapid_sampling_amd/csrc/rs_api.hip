@@ -729,7 +729,7 @@ using namespace rs;
 
 extern "C" {
 
-int rs_version(void) { return 419; }
+int rs_version(void) { return 420; }
 
 const char *rs_error_string(int code)
 {

@@ -38,10 +38,10 @@ namespace rs {
 // N(0,3), top_k 1000, top_p 0.3, some of whose rows were then summed again, 327.)
 // What was summed in a frame counts only where it weighs: not in a wave or a slice all of whose tokens are 41 octaves down, a masked stretch.
 //
-// What bounds it: in large calls the pass reads float32 at the rate of a kernel that only reads.  A token costs 4.6 vector instructions (one of
-// them the exponential, 2.7 issue slots), and a wave some 200 for bound and staging, where the pass with exact e and a histogram (stream_kernel)
-// takes 22 and an LDS atomic.  us of a pass, there / here: 128 rows of 1048576 106 / 86, 64 of 152064 12.7 / 10.1, 256 of 151936 bfloat16
-// 28 / 16.8, of which 12 are the read.
+// What bounds it: in large calls of float32 the read: 128 rows of 1048576 take 93 to 99 us a pass on average (86 at the fastest), a kernel that only reads them 81
+// to 87; there a token costs some 20 vector instructions (FINE).  Without that it costs 4.6 (one of them the exponential, 2.7 issue slots) and a wave some 200
+// for bound and staging, some 10 a token together, where the pass with exact e and a histogram (stream_kernel) takes 22 and an LDS atomic.  us of a pass,
+// there / here: 128 rows of 1048576 112 / 93 to 99, 64 of 152064 12.7 / 10.4, 256 of 151936 bfloat16 28 / 17, of which 12 are the read.
 constexpr uint32_t kSieveErrOdd = 19;                    // D is known to 2^-19 of itself when waves were summed in a frame, else to 9 * 2^-24
 
 // Sum over the wave in double precision, in every lane.
